@@ -7,6 +7,7 @@
 
 #include "../../include/restir_abi.h"
 #include "rt_traverse.h"
+#include "rt_wide8.h"
 
 namespace rk {
 
@@ -38,6 +39,15 @@ struct SceneView {
     const rt::WNode *wide;  // the 4-entry nodes over `nodes` (same indices), built by the library
     int32_t treeNested;     // 1: every box finite and inside the box stored for its parent
     float maxCoord;         // largest |box coordinate| of the tree
+    // the 8-entry nodes (rt_wide8.h), their triangles (p1.w: the slot that stores the triangle, 2 node
+    // + side; p2.w: its index) and the parent slot of each binary node
+    const rt::W8Node *w8;
+    const float4 *w8Tris;
+    const uint32_t *parent;
+    float invMax;           // clamp of 1 / d in the 8-entry walk
+    int32_t treeTight;      // 1: every leaf box is the bounding box of its triangle
+    int32_t w8Ok;           // 1: the 8-entry nodes cover the tree
+    uint32_t w8Grid;        // workgroups of their tracer
     uint32_t *traceHeads;   // the queue tracer's work counters (the context's): kTraceShards words,
                             // kTraceShardStride apart, cleared by each tracer launch
 };
@@ -83,6 +93,8 @@ int tile_index(uint32_t tx, uint32_t ty);  // -1 if not compiled
 // from one visit; a 4-byte triangle index and an owner byte each) and a tally word per lane.
 constexpr uint32_t kTraceListEntries = 64 + 4 * 64;
 constexpr uint32_t kTraceExtraLds = 4u * kTraceListEntries * 5u + 256u * 4u;
+constexpr uint32_t kTrace8Lds = rt::kW8Stack * 1024u + 4u * 128u * 5u + 2u * 256u * 4u;  // the 8-entry tracer's workgroup
+constexpr uint32_t kTrace8PerCu = 5;  // its 92 VGPRs allow 5 waves per SIMD (its LDS 6 workgroups)
 hipError_t launch_pass_a(int tile, int stack, const restir_uniforms &u, const SceneView &sc,
                          const GView &cur, const GView &prev, const restir_reservoir *prevRes,
                          restir_reservoir *out, const int32_t *candLight, const float *candQ,

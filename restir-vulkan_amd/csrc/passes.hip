@@ -969,6 +969,247 @@ __global__ __launch_bounds__(256) void k_trace_queue(const SceneView sc, const f
     }
 }
 
+// Inclusive sum over the wave's lanes (all active).
+__device__ __forceinline__ uint32_t wave_sum_inclusive(uint32_t x) {
+    const auto add = [&](auto ctrl, auto rows) {
+        x += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), decltype(ctrl)::value,
+                                                               decltype(rows)::value, 0xf, false));
+    };
+    const std::integral_constant<int, 0xf> all;
+    add(std::integral_constant<int, 0x111>{}, all);  // row_shr 1, 2, 4, 8: within rows of 16 lanes
+    add(std::integral_constant<int, 0x112>{}, all);
+    add(std::integral_constant<int, 0x114>{}, all);
+    add(std::integral_constant<int, 0x118>{}, all);
+    add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast 15, 31
+    add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    return x;
+}
+
+// The same tracer over the 8-entry nodes (rt_wide8.h): the tracer of every tree they cover. What
+// differs: a lane's walk state is one word, the first child's index and the mask of the passed
+// entries still to visit (mask 0: nothing to walk), and its stack holds such words. A visit adds one
+// entry to the wave's ring when triangles passed: the first one's index with the owner lane in the
+// upper 6 bits, and their mask relative to it. A round takes the oldest entries, spreads their
+// triangles over the lanes (prefix sum, LDS list) and tests up to 64, one per lane. A triangle that
+// is hit is confirmed against the reference's boxes. The rays the nodes do not cover are walked
+// through the binary tree as they are taken.
+//
+// VALU bound: with the 4-entry nodes a ray took 18 visits and 95 wave instructions at 0.63 lane
+// use; here about 12 and 60. Per launch, 4-entry against 8-entry nodes: a 1080p Pass C (5.5 M rays,
+// 138,000 triangles) 1.16 -> 0.78 ms, a 4K one (2.3 M triangles, whose 300 MB of 4-entry nodes
+// overflow the Infinity Cache) 14.7 -> 9.4 ms, 4 M surface-to-light segments 1.15 -> 0.74 ms, 1,021
+// segments 93 -> 49 us. Measured at the same sizes: one ring entry per triangle instead of per
+// visit 0.90 ms (its appends ran once per triangle of the wave's fullest lane); rounds at 40 and 56
+// entries within 1%; 16 and 24 idle lanes before a refill 1-4% slower; 3 and 4 workgroups per CU
+// 17% and 5% slower; 6 waves per SIMD (80 VGPRs) spills and is 6% slower.
+constexpr uint32_t kTri8Ring = 128, kTri8Round = 48;  // a round starts at kTri8Round entries
+template <int MODE>
+__global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4 *__restrict__ p1,
+                                                const float4 *__restrict__ p2, const uint32_t *__restrict__ count,
+                                                uint32_t nBatch, CQueues q, uint32_t *__restrict__ out) {
+    constexpr bool PER_PIXEL = MODE == kTracePassA, BATCH = MODE == kTraceBatch;
+    __shared__ uint32_t stack[rt::kW8Stack * 256];
+    __shared__ uint32_t ringTri[4 * kTri8Ring];
+    __shared__ uint8_t ringMask[4 * kTri8Ring];
+    __shared__ uint32_t testList[256];
+    __shared__ uint32_t tally[256];  // per lane: 256 x (its tests done in a round) + its hits
+    static_assert(sizeof(stack) + sizeof(ringTri) + sizeof(ringMask) + sizeof(testList) + sizeof(tally) == kTrace8Lds,
+                  "LDS the grid is sized for");
+    static_assert(kTri8Round - 1 + 64 <= kTri8Ring, "a step's entries fit the ring");
+    uint32_t *stk = stack + threadIdx.x;
+    const uint32_t nCentre = MODE == kTracePassC ? count[0] : 0u;
+    const uint32_t n = BATCH ? nBatch : (PER_PIXEL ? count[0] : nCentre + count[1]);
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t *ring = ringTri + (threadIdx.x >> 6) * kTri8Ring;
+    uint8_t *ringM = ringMask + (threadIdx.x >> 6) * kTri8Ring;
+    uint32_t *list = testList + (threadIdx.x & ~63u);
+    uint32_t *tal = tally + (threadIdx.x & ~63u);
+    tally[threadIdx.x] = 0u;  // each wave uses its own 64 words only
+    rt::W8Seg w{};
+    uint32_t grp = 0;    // the entries to visit: first child << 8 | mask; mask 0: nothing to walk
+    int top = 0;         // entries of this lane's stack
+    bool hit = false;
+    int32_t ray = -1;
+    uint32_t tag = 0;
+    uint32_t waiting = 0;            // this lane's tests in the wave's ring
+    uint32_t first = 0, listed = 0;  // wave-uniform: the ring's oldest entry and its length
+    uint32_t next = 0, end = 0;      // wave-uniform: the rays of the wave's chunk not handed out yet
+    const uint32_t nChunks = (n + kTraceChunk - 1) / kTraceChunk;
+    // wave-uniform; no more waves than chunks are needed (each takes at least one)
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+    if (wave >= nChunks) return;
+    uint32_t shard = wave % kTraceShards;
+    bool drained = false;            // wave-uniform: every shard is exhausted
+    for (;;) {
+        const uint64_t idle = __ballot(ray < 0);
+        const uint32_t nIdle = static_cast<uint32_t>(__popcll(idle));
+        if (nIdle >= kTraceRefill) {
+            if (next >= end && !drained) {
+                // every lane is active here: the first active lane is lane 0, and the values stay
+                // in scalar registers, so the loop's tests are seen as wave-uniform
+                for (;;) {
+                    uint32_t v = 0;
+                    if (lane == 0) v = atomicAdd(sc.traceHeads + shard * kTraceShardStride, 1u);
+                    const uint32_t c = __builtin_amdgcn_readfirstlane(v) * kTraceShards + shard;
+                    if (c < nChunks) {
+                        next = c * kTraceChunk;
+                        end = n - next < kTraceChunk ? n : next + kTraceChunk;
+                        break;
+                    }
+                    // exhausted: the next shard in line that is not, all of them looked at together
+                    // (one after another, a launch's last waves would wait for 64 loads in a row)
+                    const uint32_t t = __hip_atomic_load(sc.traceHeads + lane * kTraceShardStride, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT);
+                    const uint64_t left = __ballot(t * kTraceShards + lane < nChunks);
+                    if (left == 0) {
+                        drained = true;
+                        break;
+                    }
+                    // the waves spread over what is left
+                    const uint32_t nth = wave % static_cast<uint32_t>(__popcll(left));
+                    const uint64_t pick = __ballot(((left >> lane) & 1ull) != 0 && lanes_below(left) == nth);
+                    shard = static_cast<uint32_t>(__builtin_ctzll(pick));
+                }
+            }
+            if (next < end) {
+                if (ray < 0) {
+                    const uint32_t i = next + lanes_below(idle);
+                    if (i < end) {
+                        const bool centre = MODE == kTracePassC && i < nCentre;
+                        const float4 a4 = MODE != kTracePassC ? p1[i] : (centre ? q.c1[i] : q.n1[i - nCentre]);
+                        tag = BATCH ? i : __float_as_uint(a4.w);
+                        // a neighbour ray of a pixel whose centre ray was shadowed is not traced
+                        if (MODE != kTracePassC || centre || !(q.bits[tag & 0x07ffffffu] & kBitCentreShadowed)) {
+                            f3 o, d;
+                            const float4 b4 = MODE != kTracePassC
+                                                  ? p2[i]
+                                                  : reinterpret_cast<const float4 *>(q.merged + (tag & 0x07ffffffu))[0];
+                            shadow_segment(xyz(a4), xyz(b4), o, d);
+                            ray = static_cast<int32_t>(i);
+                            hit = false;
+                            top = 0;
+                            grp = 1u;  // node 0
+                            if (!rt::make_w8seg(w, o, d, sc.maxCoord, sc.invMax)) {
+                                hit = rt::occluded_slow(sc.nodes, sc.tris, sc.parent, o, d);
+                                grp = 0u;
+                            }
+                        }
+                    }
+                }
+                next = end - next < nIdle ? end : next + nIdle;
+            }
+        }
+        if (__ballot(ray >= 0) == 0) {
+            if (drained && next >= end) break;
+            continue;
+        }
+        // one visit per walking lane
+        uint32_t pend = 0, triBase = 0;
+        if (grp & 0xffu) {
+            const uint32_t node = (grp >> 8) + static_cast<uint32_t>(__builtin_ctz(grp));
+            grp &= grp - 1u;
+            uint32_t child;
+            pend = rt::w8_visit(w, sc.w8, node, child, triBase);
+            const bool more = (grp & 0xffu) != 0;
+            if (child & 0xffu) {
+                if (more) {
+                    stk[top * 256] = grp;
+                    ++top;
+                }
+                grp = child;
+            } else if (!more && top > 0) {
+                --top;
+                grp = stk[top * 256];
+            }
+        }
+        const uint64_t found = __ballot(pend != 0);
+        if (found) {
+            if (pend) {
+                const uint32_t b = static_cast<uint32_t>(__builtin_ctz(pend));
+                const uint32_t at = (first + listed + lanes_below(found)) & (kTri8Ring - 1u);
+                ring[at] = (triBase + b) | (lane << 26);
+                ringM[at] = static_cast<uint8_t>(pend >> b);
+                waiting += static_cast<uint32_t>(__popc(pend));
+            }
+            listed += static_cast<uint32_t>(__popcll(found));
+        }
+        // rounds of triangle tests: whenever the ring holds enough for one, or what there is once
+        // too few lanes can still walk
+        const uint32_t walkers = static_cast<uint32_t>(__popcll(__ballot((grp & 0xffu) != 0)));
+        while (listed >= kTri8Round || (listed > 0u && walkers < kTriRoundWalkers)) {
+            const uint64_t known = __ballot(hit);
+            const uint32_t at = (first + lane) & (kTri8Ring - 1u);
+            uint32_t e = 0, m = 0;
+            if (lane < listed) {
+                e = ring[at];
+                m = ringM[at];
+            }
+            const uint32_t c = static_cast<uint32_t>(__popc(m));
+            const uint32_t incl = wave_sum_inclusive(c);
+            const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+            const uint32_t take = total < 64u ? total : 64u;
+            uint32_t pos = incl - c;
+            const bool part = m != 0 && pos < 64u && incl > 64u;  // one entry at most is left in part
+            while (__ballot(m != 0 && pos < 64u)) {
+                if (m != 0 && pos < 64u) {
+                    list[pos] = e + static_cast<uint32_t>(__builtin_ctz(m));
+                    m &= m - 1u;
+                    ++pos;
+                }
+            }
+            if (part) ringM[at] = static_cast<uint8_t>(m);
+            const uint32_t done = static_cast<uint32_t>(__popcll(__ballot(lane < listed && m == 0)));
+            first = (first + done) & (kTri8Ring - 1u);
+            listed -= done;
+            const bool mine = lane < take;
+            uint32_t t = 0, o = 0;
+            if (mine) {
+                t = list[lane] & 0x03ffffffu;
+                o = list[lane] >> 26;
+            }
+            const int src = static_cast<int>(o);
+            const f3 ro{__shfl(w.o.x, src), __shfl(w.o.y, src), __shfl(w.o.z, src)};
+            const f3 rd{__shfl(w.d.x, src), __shfl(w.d.y, src), __shfl(w.d.z, src)};
+            bool h = false;
+            if (mine && !((known >> o) & 1ull)) {
+                const float4 *v = sc.w8Tris + 3 * t;
+                const float4 va = v[0], vb = v[1], vc = v[2];
+                h = rt::tri_hit(va, vb, vc, ro, rd);
+                if (h)
+                    h = rt::w8_confirm(sc.nodes, sc.parent, sc.treeNested != 0, sc.treeTight != 0, va, vb, vc, ro, rd);
+            }
+            if (mine) atomicAdd(&tal[o], h ? 257u : 256u);
+            const uint32_t r = atomicExch(&tal[lane], 0u);  // after this wave's adds (LDS keeps a wave's order)
+            waiting -= r >> 8;
+            if (r & 0xffu) {
+                hit = true;
+                grp = 0u;
+            }
+        }
+        if (ray >= 0 && waiting == 0 && (grp & 0xffu) == 0) {
+            if (BATCH) {
+                out[tag] = hit ? 1u : 0u;
+            } else if (hit) {
+                if (PER_PIXEL || (tag & kCentreTag)) q.bits[tag & 0x07ffffffu] |= kBitCentreShadowed;
+                else atomicOr(&q.occ[tag & 0x07ffffffu], 1u << (tag >> 27));
+            }
+            ray = -1;
+        }
+    }
+}
+
+// Launches the queue tracer over the nodes that cover the scene's tree.
+template <int STACK, int MODE>
+static void launch_tracer(const char *name, uint32_t gridCap, const SceneView &sc, const float4 *p1, const float4 *p2,
+                          const uint32_t *count, uint32_t nBatch, const CQueues &q, uint32_t *out, hipStream_t s) {
+    // nBatch rays need no more workgroups than one lane each
+    const uint32_t grid = MODE == kTraceBatch && (nBatch + 255) / 256 < sc.w8Grid ? (nBatch + 255) / 256 : sc.w8Grid;
+    if (sc.w8Ok)
+        RK_LAUNCH(name, k_trace8<MODE>, dim3(grid), dim3(256), 0, s, sc, p1, p2, count, nBatch, q, out);
+    else
+        RK_LAUNCH(name, (k_trace_queue<STACK, MODE>), dim3(gridCap), dim3(256), 0, s, sc, p1, p2, count, nBatch, q, out);
+}
+
 // ---------------------------------------------------------------- Pass A, ray queue ---
 // Pass A with its visibility ray (restirOmni.glsl:148-160) moved out of the per-pixel lanes:
 // (1) RIS per pixel; the reservoir is parked in the output, the random stream's state in
@@ -1393,8 +1634,8 @@ static hipError_t run_a_queued(PassAArgs args, const AQueues &q, uint32_t gridCa
     if (args.u.flags & RESTIR_VISIBILITY_REUSE_FLAG) {
         CQueues cq{};
         cq.bits = q.occ;  // a shadowed ray sets kBitCentreShadowed in occ[pixel]
-        RK_LAUNCH("k_trace_queue(pass_a)", (k_trace_queue<STACK, kTracePassA>), dim3(gridCap), dim3(256), 0, s,
-                  args.sc, q.p1, q.p2, q.counter + 0, 0u, cq, nullptr);
+        launch_tracer<STACK, kTracePassA>("k_trace_queue(pass_a)", gridCap, args.sc, q.p1, q.p2, q.counter + 0, 0u, cq,
+                                          nullptr, s);
     }
     RK_LAUNCH("k_pass_a_finish", (k_pass_a_finish<TX, TY>), tiles, block, 0, s, args, q);
     return hipGetLastError();
@@ -1473,8 +1714,8 @@ static hipError_t run_c_queued(PassCArgs args, const CQueues &q, uint32_t gridCa
         RK_LAUNCH("k_pack_surface", k_pack_surface, dim3((npx + 255) / 256), dim3(256), 0, s, args.g, npx, q.surf);
     RK_LAUNCH("k_pass_c_merge", (k_pass_c_merge<TX, TY>), tiles, block, 0, s, args, q);
     if (args.u.flags & RESTIR_VISIBILITY_REUSE_FLAG) {
-        RK_LAUNCH("k_trace_queue(pass_c)", (k_trace_queue<STACK, kTracePassC>), dim3(gridCap), dim3(256), 0, s,
-                  args.sc, nullptr, nullptr, q.counter + 0, 0u, q, nullptr);
+        launch_tracer<STACK, kTracePassC>("k_trace_queue(pass_c)", gridCap, args.sc, nullptr, nullptr, q.counter + 0, 0u,
+                                          q, nullptr, s);
         RK_LAUNCH("k_pass_c_finish", (k_pass_c_finish<TX, TY>), tiles, block, 0, s, args, q);
     }
     return hipGetLastError();
@@ -1788,8 +2029,8 @@ static void run_trace(bool persistent, uint32_t gridCap, uint32_t *counter, cons
     const uint32_t grid = blocks < gridCap ? blocks : gridCap;
     if (!REF && !args.visits && !args.tests) {
         // no counts asked for: the passes' queue tracer (gathered triangle tests)
-        RK_LAUNCH("k_trace_queue(batch)", (k_trace_queue<STACK, kTraceBatch>), dim3(grid), dim3(256), 0, s, args.sc,
-                  args.p1, args.p2, nullptr, args.n, CQueues{}, args.shadowed);
+        launch_tracer<STACK, kTraceBatch>("k_trace_queue(batch)", grid, args.sc, args.p1, args.p2, nullptr, args.n,
+                                          CQueues{}, args.shadowed, s);
         return;
     }
     RK_LAUNCH("k_trace_pool", (k_trace_pool<STACK, REF>), dim3(grid), dim3(256), 0, s, args, counter);

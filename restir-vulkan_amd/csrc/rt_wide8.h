@@ -1,0 +1,199 @@
+// rt_wide8.h — 8-entry nodes over a bound tree, for the queue tracer and the primary rays.
+//
+// The reference tests a triangle exactly when every box on its path from the root passes, so a
+// segment is occluded exactly when some triangle is hit by the triangle test AND every box of its
+// path passes the box test. The second half has to be known only for triangles that are hit, so
+// the walk may test any boxes in any rounding as long as it never skips such a triangle: a hit is
+// then confirmed against the reference's own boxes (w8_confirm). That frees the layout: a node
+// holds up to 8 entries (internal nodes or triangles) collapsed from the binary tree, with box planes of 11 bits relative to the node, 128 bytes per node against 128 per
+// 4 entries with fp32 planes.
+//
+// Conservative boxes. Every box is grown by s = 192 u C before it is quantised outwards
+// (u = 2^-24, C the largest |box coordinate| of the tree), and the walk forms each slab distance as
+// t(q) = RN(q S + N), S = 2^e inv (exact), N = RN(RN(p - o) inv), inv the hardware's 1/d (within
+// 2u). With |o| <= 16 C the walk's distance differs from the exact one by at most 6u (|q 2^e| +
+// |p - o|) / |d| <= 6u (4.01 C + 17.01 C) / |d|, the reference's RN(RN(b - o)/d) by at most 2.01u
+// (17 C) / |d|: 161 u C / |d| in all, less than the growth s / |d|. So the walk's near distance of a box is at most,
+// and its far distance at least, the reference's for every box inside it, and the walk enters
+// every node on the path of a triangle whose path passes. 1/d is clamped to +-K (SceneView::invMax,
+// s K >= 4): for |d| < 1/K a segment that starts inside the grown slab keeps near < 0 and far > 1,
+// and one that starts outside cannot reach the box itself (its distance exceeds s K), so zero,
+// denormal (the hardware's reciprocal is then infinite) and tiny components are covered too. Segments with a non-finite component or |o| > 16 C walk the
+// binary tree (occluded_slow).
+#pragma once
+
+#include "rt_traverse.h"
+
+namespace rt {
+
+constexpr int kW8Stack = 16;  // entries of a lane's stack: trees of at most 17 levels of 8-entry nodes
+constexpr float kW8Grow = 192.0f * 5.9604645e-8f;  // s / C
+constexpr float kW8Reach = 16.0f;                  // |o| / C at most
+
+struct alignas(128) W8Node {
+    float p[3];         // the node's corner: plane q of axis a lies at p[a] + q 2^e[a]
+    uint32_t child;     // first internal child's index << 8 | mask of the internal entries: they
+                        // take the lowest slots, and the child of slot k is node (child >> 8) + k
+    uint32_t exps;      // signed byte a < 3: e[a]; byte 3: mask of the triangle entries
+    uint32_t triBase;   // the triangle of slot k is triBase + k
+    uint32_t pad[2];
+    uint16_t plane[3][2][8];  // per axis: low and high planes of the 8 slots (halves, 0..2047)
+};
+static_assert(sizeof(W8Node) == 128, "one 128-byte line per node");
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
+// A segment for the 8-entry walk.
+struct W8Seg {
+    f3 o, d, inv;
+    uint32_t ox, oy, oz;  // byte offset of an axis's near planes: 0 for d > 0, else 16
+};
+// False for a segment the walk does not cover.
+__device__ __forceinline__ bool make_w8seg(W8Seg &w, f3 o, f3 d, float maxCoord, float invMax) {
+    constexpr float kInf = __builtin_huge_valf();
+    w.o = o;
+    w.d = d;
+    const f3 inv{__builtin_amdgcn_rcpf(d.x), __builtin_amdgcn_rcpf(d.y), __builtin_amdgcn_rcpf(d.z)};
+    w.inv = f3{fminf(fmaxf(inv.x, -invMax), invMax), fminf(fmaxf(inv.y, -invMax), invMax),
+               fminf(fmaxf(inv.z, -invMax), invMax)};
+    w.ox = w.inv.x > 0.0f ? 0u : 16u;
+    w.oy = w.inv.y > 0.0f ? 0u : 16u;
+    w.oz = w.inv.z > 0.0f ? 0u : 16u;
+    const float reach = kW8Reach * maxCoord;
+    // comparisons are false for NaN
+    return fabsf(d.x) < kInf && fabsf(d.y) < kInf && fabsf(d.z) < kInf && fabsf(o.x) <= reach &&
+           fabsf(o.y) <= reach && fabsf(o.z) <= reach;
+}
+
+// Visits `node`: `child` gets its child word with only the internal entries that the segment passes
+// left in the mask, `triBase` its first triangle; returns the mask of the triangle entries that it
+// passes. 12 VALU per box: 6 FMA with half operands, max3, min3, the clamp to the segment, a
+// subtraction whose sign is shifted into the mask.
+__device__ __forceinline__ uint32_t w8_visit(const W8Seg &w, const W8Node *__restrict__ nodes, uint32_t node,
+                                             uint32_t &child, uint32_t &triBase) {
+    const char *base = reinterpret_cast<const char *>(nodes);
+    const uint32_t row = node << 7;
+    const float4 h0 = *reinterpret_cast<const float4 *>(base + row);
+    const uint2 h1 = *reinterpret_cast<const uint2 *>(base + row + 16);
+    const h8 nx = *reinterpret_cast<const h8 *>(base + (row + w.ox) + 32);
+    const h8 fx = *reinterpret_cast<const h8 *>(base + (row + (w.ox ^ 16u)) + 32);
+    const h8 ny = *reinterpret_cast<const h8 *>(base + (row + w.oy) + 64);
+    const h8 fy = *reinterpret_cast<const h8 *>(base + (row + (w.oy ^ 16u)) + 64);
+    const h8 nz = *reinterpret_cast<const h8 *>(base + (row + w.oz) + 96);
+    const h8 fz = *reinterpret_cast<const h8 *>(base + (row + (w.oz ^ 16u)) + 96);
+    const int32_t e = static_cast<int32_t>(h1.x);
+    const float sx = ldexpf(w.inv.x, (e << 24) >> 24), sy = ldexpf(w.inv.y, (e << 16) >> 24),
+                sz = ldexpf(w.inv.z, (e << 8) >> 24);
+    const float bx = (h0.x - w.o.x) * w.inv.x, by = (h0.y - w.o.y) * w.inv.y, bz = (h0.z - w.o.z) * w.inv.z;
+    uint32_t miss = 0;
+#pragma unroll
+    for (int k = 7; k >= 0; --k) {
+        const float lo = fmaxf(fmaxf(fmaf(static_cast<float>(nx[k]), sx, bx), fmaf(static_cast<float>(ny[k]), sy, by)),
+                               fmaf(static_cast<float>(nz[k]), sz, bz));
+        const float hi = fminf(fminf(fmaf(static_cast<float>(fx[k]), sx, bx), fmaf(static_cast<float>(fy[k]), sy, by)),
+                               fmaf(static_cast<float>(fz[k]), sz, bz));
+        const float gap = fminf(hi, 1.0f) - fmaxf(lo, 0.0f);  // negative: the segment misses the box
+        miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(gap), 31);
+    }
+    child = __float_as_uint(h0.w) & ~miss;
+    triBase = h1.y;
+    return (h1.x >> 24) & ~miss;
+}
+
+// rayTriangleIntersection over given vertices (ray_tri's arithmetic).
+__device__ __forceinline__ bool tri_hit(float4 a, float4 b, float4 c, f3 o, f3 d) {
+    const f3 p1 = xyz(a);
+    const f3 e1 = xyz(b) - p1;
+    const f3 e2 = xyz(c) - p1;
+    const f3 p = cross(d, e2);
+    float f = 1.0f / dot(e1, p);
+    const f3 s = o - p1;
+    const float bx = f * dot(s, p);
+    if (bx < 0.0f || bx > 1.0f) return false;
+    const f3 q = cross(s, e1);
+    const float by = f * dot(d, q);
+    if (by < 0.0f || by + bx > 1.0f) return false;
+    f *= dot(e2, q);
+    return f > 0.0f && f < 1.0f;
+}
+
+__device__ __forceinline__ bool regular_segment(f3 o, f3 d) {
+    constexpr float kInf = __builtin_huge_valf();
+    return fabsf(d.x) > 0.0f && fabsf(d.y) > 0.0f && fabsf(d.z) > 0.0f && fabsf(d.x) < kInf && fabsf(d.y) < kInf &&
+           fabsf(d.z) < kInf && fabsf(o.x) < kInf && fabsf(o.y) < kInf && fabsf(o.z) < kInf;
+}
+
+// Side `side` of node x: its box as stored, and its child.
+__device__ __forceinline__ bool side_passes(const Node *__restrict__ nodes, uint32_t x, uint32_t side, f3 o, f3 d) {
+    const float4 *p = reinterpret_cast<const float4 *>(nodes + x) + 2 * side;
+    return ray_box_div(o, d, p[0], p[1]);
+}
+
+// Whether the reference tests the triangle stored under `slot` (2 node + side) for this segment:
+// every box from that slot up to the root passes. In a nested tree a regular segment that passes a
+// box passes every box around it (the slab distances are monotone in the planes), so the slot's
+// own box decides.
+__device__ __forceinline__ bool path_passes(const Node *__restrict__ nodes, const uint32_t *__restrict__ parent,
+                                            uint32_t slot, f3 o, f3 d, bool leafOnly) {
+    for (;;) {
+        const uint32_t x = slot >> 1;
+        if (!side_passes(nodes, x, slot & 1u, o, d)) return false;
+        if (leafOnly || x == 0) return true;
+        slot = parent[x];
+    }
+}
+
+// Confirms a triangle hit (see the file comment). `tight`: every leaf box of the tree is the
+// bounding box of its triangle, so the box needs no load. Most confirmations are clear from
+// distances formed with the hardware reciprocal (within 4u of the exact quotient of the rounded
+// difference, the reference's within u of it: the slack of 16u covers both).
+__device__ __forceinline__ bool w8_confirm(const Node *__restrict__ nodes, const uint32_t *__restrict__ parent,
+                                           bool treeNested, bool tight, float4 a, float4 b, float4 c, f3 o, f3 d) {
+    const bool leafOnly = treeNested && regular_segment(o, d);
+    if (leafOnly && tight) {
+        const float4 mn = make_float4(fminf(fminf(a.x, b.x), c.x), fminf(fminf(a.y, b.y), c.y),
+                                      fminf(fminf(a.z, b.z), c.z), 0.0f);
+        const float4 mx = make_float4(fmaxf(fmaxf(a.x, b.x), c.x), fmaxf(fmaxf(a.y, b.y), c.y),
+                                      fmaxf(fmaxf(a.z, b.z), c.z), 0.0f);
+        const float ix = __builtin_amdgcn_rcpf(d.x), iy = __builtin_amdgcn_rcpf(d.y), iz = __builtin_amdgcn_rcpf(d.z);
+        const float ax = (mn.x - o.x) * ix, ay = (mn.y - o.y) * iy, az = (mn.z - o.z) * iz;
+        const float bx = (mx.x - o.x) * ix, by = (mx.y - o.y) * iy, bz = (mx.z - o.z) * iz;
+        const float rmin = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz));
+        const float rmax = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
+        constexpr float kRel = 16.0f * 5.9604645e-8f, kAbs = 1e-30f;
+        const float big = fmaxf(fmaxf(fmaxf(fabsf(ax), fabsf(bx)), fmaxf(fabsf(ay), fabsf(by))),
+                                fmaxf(fabsf(az), fabsf(bz)));  // a flushed or infinite reciprocal fails this test
+        const float minHi = rmin + (fabsf(rmin) * kRel + kAbs), maxLo = rmax - (fabsf(rmax) * kRel + kAbs);
+        const float dMax = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
+        if (big < 1e30f && dMax < 1e30f && minHi < 1.0f && maxLo >= minHi && maxLo > 0.0f) return true;
+        return ray_box_div(o, d, mn, mx);
+    }
+    return path_passes(nodes, parent, __float_as_uint(a.w), o, d, leafOnly);
+}
+
+// The reference's answer for any segment, from the binary nodes and their parents, without a stack:
+// for the segments the 8-entry walk does not cover.
+__device__ __forceinline__ bool occluded_slow(const Node *__restrict__ nodes, const float4 *__restrict__ tris,
+                                              const uint32_t *__restrict__ parent, f3 o, f3 d) {
+    uint32_t x = 0, side = 0;
+    for (;;) {
+        if (side_passes(nodes, x, side, o, d)) {
+            const int32_t c = side ? nodes[x].right : nodes[x].left;
+            if (c >= 0) {
+                x = static_cast<uint32_t>(c);
+                side = 0;
+                continue;
+            }
+            if (ray_tri(tris, ~c, o, d)) return true;
+        }
+        while (side == 1u) {  // both sides of x are done: back to the side that led here
+            if (x == 0) return false;
+            const uint32_t up = parent[x];
+            x = up >> 1;
+            side = up & 1u;
+        }
+        side = 1u;
+    }
+}
+
+}  // namespace rt
