@@ -757,6 +757,30 @@ __global__ __launch_bounds__(64) void k_w8_collapse(const rt::Node *__restrict__
         int at = nInt;
         for (int k = 0; k < cnt; ++k)
             if (ref[k][lane] < 0) order[at++] = k;
+        // the internal entries along the axis on which their centres spread most, the largest
+        // centre first: the primary rays take them from the side they come from. The shadow rays
+        // take them in this order (1-11% faster on the terrains than the other way round)
+        uint32_t axis = 0;
+        float spread = -1.0f;
+        for (uint32_t a = 0; a < 3; ++a) {
+            float lo = __builtin_huge_valf(), hi = -__builtin_huge_valf();
+            for (int k = 0; k < nInt; ++k) {
+                const float c = box[a][order[k]][lane] + box[3 + a][order[k]][lane];
+                lo = fminf(lo, c);
+                hi = fmaxf(hi, c);
+            }
+            if (hi - lo > spread) {
+                spread = hi - lo;
+                axis = a;
+            }
+        }
+        for (int k = 1; k < nInt; ++k)
+            for (int j = k; j > 0; --j) {
+                const int u = order[j - 1], v = order[j];
+                if (!(box[axis][u][lane] + box[3 + axis][u][lane] < box[axis][v][lane] + box[3 + axis][v][lane])) break;
+                order[j - 1] = v;
+                order[j] = u;
+            }
         // room in the next level and among the triangles, one atomic pair per wave
         const uint32_t inclInt = rscan::wave_inclusive(static_cast<uint32_t>(nInt));
         const uint32_t inclTri = rscan::wave_inclusive(static_cast<uint32_t>(nTri));
@@ -778,7 +802,8 @@ __global__ __launch_bounds__(64) void k_w8_collapse(const rt::Node *__restrict__
         w.child = (baseInt << 8) | ((1u << nInt) - 1u);
         w.triBase = baseTri - static_cast<uint32_t>(nInt);
         w.exps = (((1u << cnt) - 1u) & ~((1u << nInt) - 1u)) << 24;
-        w.pad[0] = w.pad[1] = 0;
+        w.axis = axis;
+        w.pad = 0;
         for (int k = 0; k < nInt; ++k) work[baseInt + static_cast<uint32_t>(k)] = static_cast<uint32_t>(ref[order[k]][lane]);
         for (int a = 0; a < 3; ++a) {
             double lo = 1e300, hi = -1e300;
@@ -869,8 +894,8 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     RK_LAUNCH("k_w8_clear", k_w8_clear, dim3(1), dim3(64), 0, s, p.flags, p.info);
     RK_LAUNCH("k_wide_build", k_wide_build, dim3(groups(nNodes)), dim3(256), 0, s, bn, nNodes, bt, p.wide, p.parent,
               p.flags);
-    // node indices take 24 bits of a child word, triangles 26 bits of a tracer's list entry
-    const bool w8Fits = maxW8 <= (1u << 24) && nTris <= (1u << 26);
+    // node indices take 23 bits of a child word, triangles 26 bits of a tracer's list entry
+    const bool w8Fits = maxW8 <= (1u << 23) && nTris <= (1u << 26);
     // a level of 8-entry nodes covers at least one level of the tree
     const uint32_t levels = depth < static_cast<uint32_t>(kW8Levels) ? depth : static_cast<uint32_t>(kW8Levels);
     if (w8Fits)

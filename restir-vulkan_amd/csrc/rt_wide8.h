@@ -19,7 +19,8 @@
 // s K >= 4): for |d| < 1/K a segment that starts inside the grown slab keeps near < 0 and far > 1,
 // and one that starts outside cannot reach the box itself (its distance exceeds s K), so zero,
 // denormal (the hardware's reciprocal is then infinite) and tiny components are covered too. Segments with a non-finite component or |o| > 16 C walk the
-// binary tree (occluded_slow).
+// binary tree (occluded_slow). The same holds for unbounded rays (the primary rays) of unit
+// direction, whose boxes all lie within 31 C of the origin: s K >= 31 C.
 #pragma once
 
 #include "rt_traverse.h"
@@ -32,11 +33,12 @@ constexpr float kW8Reach = 16.0f;                  // |o| / C at most
 
 struct alignas(128) W8Node {
     float p[3];         // the node's corner: plane q of axis a lies at p[a] + q 2^e[a]
-    uint32_t child;     // first internal child's index << 8 | mask of the internal entries: they
-                        // take the lowest slots, and the child of slot k is node (child >> 8) + k
+    uint32_t child;     // first internal child's index (23 bits) << 8 | mask of the internal entries:
+                        // they take the lowest slots, and the child of slot k is node (child >> 8) + k
     uint32_t exps;      // signed byte a < 3: e[a]; byte 3: mask of the triangle entries
     uint32_t triBase;   // the triangle of slot k is triBase + k
-    uint32_t pad[2];
+    uint32_t axis;      // the internal entries are in descending order of their centres on this axis
+    uint32_t pad;
     uint16_t plane[3][2][8];  // per axis: low and high planes of the 8 slots (halves, 0..2047)
 };
 static_assert(sizeof(W8Node) == 128, "one 128-byte line per node");
@@ -65,16 +67,28 @@ __device__ __forceinline__ bool make_w8seg(W8Seg &w, f3 o, f3 d, float maxCoord,
            fabsf(o.y) <= reach && fabsf(o.z) <= reach;
 }
 
-// Visits `node`: `child` gets its child word with only the internal entries that the segment passes
-// left in the mask, `triBase` its first triangle; returns the mask of the triangle entries that it
-// passes. 12 VALU per box: 6 FMA with half operands, max3, min3, the clamp to the segment, a
-// subtraction whose sign is shifted into the mask.
-__device__ __forceinline__ uint32_t w8_visit(const W8Seg &w, const W8Node *__restrict__ nodes, uint32_t node,
-                                             uint32_t &child, uint32_t &triBase) {
+// What a visit leaves: the child word with only the internal entries that are passed left in the
+// mask, and the mask of the triangle entries that are passed (slot k: triangle triBase + k). With
+// kOrder also the node's axis, and the slot of the nearest internal entry that is passed.
+struct W8Visit {
+    uint32_t child, tris, triBase, axis, nearest;
+};
+// Visits `node` on [0, tMax]. 12 VALU per box: 6 FMA with half operands, max3, min3, the clamp to
+// the segment, a subtraction whose sign is shifted into the mask.
+template <bool kOrder>
+__device__ __forceinline__ W8Visit w8_visit(const W8Seg &w, const W8Node *__restrict__ nodes, uint32_t node,
+                                            float tMax) {
     const char *base = reinterpret_cast<const char *>(nodes);
     const uint32_t row = node << 7;
     const float4 h0 = *reinterpret_cast<const float4 *>(base + row);
-    const uint2 h1 = *reinterpret_cast<const uint2 *>(base + row + 16);
+    uint3 h1{0u, 0u, 0u};
+    if (kOrder) {
+        h1 = *reinterpret_cast<const uint3 *>(base + row + 16);
+    } else {
+        const uint2 v = *reinterpret_cast<const uint2 *>(base + row + 16);
+        h1.x = v.x;
+        h1.y = v.y;
+    }
     const h8 nx = *reinterpret_cast<const h8 *>(base + (row + w.ox) + 32);
     const h8 fx = *reinterpret_cast<const h8 *>(base + (row + (w.ox ^ 16u)) + 32);
     const h8 ny = *reinterpret_cast<const h8 *>(base + (row + w.oy) + 64);
@@ -85,19 +99,22 @@ __device__ __forceinline__ uint32_t w8_visit(const W8Seg &w, const W8Node *__res
     const float sx = ldexpf(w.inv.x, (e << 24) >> 24), sy = ldexpf(w.inv.y, (e << 16) >> 24),
                 sz = ldexpf(w.inv.z, (e << 8) >> 24);
     const float bx = (h0.x - w.o.x) * w.inv.x, by = (h0.y - w.o.y) * w.inv.y, bz = (h0.z - w.o.z) * w.inv.z;
-    uint32_t miss = 0;
+    const uint32_t inner = __float_as_uint(h0.w);
+    uint32_t miss = 0, near = 0xffffffffu;
 #pragma unroll
     for (int k = 7; k >= 0; --k) {
         const float lo = fmaxf(fmaxf(fmaf(static_cast<float>(nx[k]), sx, bx), fmaf(static_cast<float>(ny[k]), sy, by)),
                                fmaf(static_cast<float>(nz[k]), sz, bz));
         const float hi = fminf(fminf(fmaf(static_cast<float>(fx[k]), sx, bx), fmaf(static_cast<float>(fy[k]), sy, by)),
                                fmaf(static_cast<float>(fz[k]), sz, bz));
-        const float gap = fminf(hi, 1.0f) - fmaxf(lo, 0.0f);  // negative: the segment misses the box
+        const float gap = fminf(hi, tMax) - fmaxf(lo, 0.0f);  // negative: the box is missed
         miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(gap), 31);
+        if (kOrder) {  // entry distances are not negative: they order as their bits
+            const uint32_t key = (__float_as_uint(fmaxf(lo, 0.0f)) & ~7u) | static_cast<uint32_t>(k);
+            near = min(near, gap >= 0.0f && ((inner >> k) & 1u) ? key : 0xffffffffu);
+        }
     }
-    child = __float_as_uint(h0.w) & ~miss;
-    triBase = h1.y;
-    return (h1.x >> 24) & ~miss;
+    return W8Visit{inner & ~miss, (h1.x >> 24) & ~miss, h1.y, h1.z, near & 7u};
 }
 
 // rayTriangleIntersection over given vertices (ray_tri's arithmetic).
@@ -123,21 +140,33 @@ __device__ __forceinline__ bool regular_segment(f3 o, f3 d) {
            fabsf(d.z) < kInf && fabsf(o.x) < kInf && fabsf(o.y) < kInf && fabsf(o.z) < kInf;
 }
 
-// Side `side` of node x: its box as stored, and its child.
+// The box tests of the primary rays (an unbounded ray: no rmin < 1), in the division form.
+__device__ __forceinline__ bool ray_box_div_unbounded(f3 o, f3 d, float4 mn, float4 mx) {
+    const float ax = (mn.x - o.x) / d.x, ay = (mn.y - o.y) / d.y, az = (mn.z - o.z) / d.z;
+    const float bx = (mx.x - o.x) / d.x, by = (mx.y - o.y) / d.y, bz = (mx.z - o.z) / d.z;
+    const float rmin = gmax(gmin(ax, bx), gmax(gmin(ay, by), gmin(az, bz)));
+    const float rmax = gmin(gmax(ax, bx), gmin(gmax(ay, by), gmax(az, bz)));
+    return rmax >= rmin && rmax > 0.0f;
+}
+
+// Side `side` of node x: whether its box, as stored, is passed (kSeg: by the segment, else by the
+// unbounded ray).
+template <bool kSeg>
 __device__ __forceinline__ bool side_passes(const Node *__restrict__ nodes, uint32_t x, uint32_t side, f3 o, f3 d) {
     const float4 *p = reinterpret_cast<const float4 *>(nodes + x) + 2 * side;
-    return ray_box_div(o, d, p[0], p[1]);
+    return kSeg ? ray_box_div(o, d, p[0], p[1]) : ray_box_div_unbounded(o, d, p[0], p[1]);
 }
 
 // Whether the reference tests the triangle stored under `slot` (2 node + side) for this segment:
 // every box from that slot up to the root passes. In a nested tree a regular segment that passes a
 // box passes every box around it (the slab distances are monotone in the planes), so the slot's
 // own box decides.
+template <bool kSeg>
 __device__ __forceinline__ bool path_passes(const Node *__restrict__ nodes, const uint32_t *__restrict__ parent,
                                             uint32_t slot, f3 o, f3 d, bool leafOnly) {
     for (;;) {
         const uint32_t x = slot >> 1;
-        if (!side_passes(nodes, x, slot & 1u, o, d)) return false;
+        if (!side_passes<kSeg>(nodes, x, slot & 1u, o, d)) return false;
         if (leafOnly || x == 0) return true;
         slot = parent[x];
     }
@@ -147,6 +176,7 @@ __device__ __forceinline__ bool path_passes(const Node *__restrict__ nodes, cons
 // bounding box of its triangle, so the box needs no load. Most confirmations are clear from
 // distances formed with the hardware reciprocal (within 4u of the exact quotient of the rounded
 // difference, the reference's within u of it: the slack of 16u covers both).
+template <bool kSeg>
 __device__ __forceinline__ bool w8_confirm(const Node *__restrict__ nodes, const uint32_t *__restrict__ parent,
                                            bool treeNested, bool tight, float4 a, float4 b, float4 c, f3 o, f3 d) {
     const bool leafOnly = treeNested && regular_segment(o, d);
@@ -165,10 +195,10 @@ __device__ __forceinline__ bool w8_confirm(const Node *__restrict__ nodes, const
                                 fmaxf(fabsf(az), fabsf(bz)));  // a flushed or infinite reciprocal fails this test
         const float minHi = rmin + (fabsf(rmin) * kRel + kAbs), maxLo = rmax - (fabsf(rmax) * kRel + kAbs);
         const float dMax = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
-        if (big < 1e30f && dMax < 1e30f && minHi < 1.0f && maxLo >= minHi && maxLo > 0.0f) return true;
-        return ray_box_div(o, d, mn, mx);
+        if (big < 1e30f && dMax < 1e30f && (!kSeg || minHi < 1.0f) && maxLo >= minHi && maxLo > 0.0f) return true;
+        return kSeg ? ray_box_div(o, d, mn, mx) : ray_box_div_unbounded(o, d, mn, mx);
     }
-    return path_passes(nodes, parent, __float_as_uint(a.w), o, d, leafOnly);
+    return path_passes<kSeg>(nodes, parent, __float_as_uint(a.w), o, d, leafOnly);
 }
 
 // The reference's answer for any segment, from the binary nodes and their parents, without a stack:
@@ -177,7 +207,7 @@ __device__ __forceinline__ bool occluded_slow(const Node *__restrict__ nodes, co
                                               const uint32_t *__restrict__ parent, f3 o, f3 d) {
     uint32_t x = 0, side = 0;
     for (;;) {
-        if (side_passes(nodes, x, side, o, d)) {
+        if (side_passes<true>(nodes, x, side, o, d)) {
             const int32_t c = side ? nodes[x].right : nodes[x].left;
             if (c >= 0) {
                 x = static_cast<uint32_t>(c);
