@@ -523,16 +523,20 @@ int restir_gbuffer_from_attachments(restir_ctx *ctx, const restir_gbuffer_attach
  * reference writes it into RestirUniforms::prevFrameProjectionViewMatrix (app.cpp:779). */
 int restir_camera_projection_view(const restir_camera *cam, float aspect, float out_col_major[16]);
 
-/* ---- batched views (no counterpart in the reference, which renders one view): one persistent
- * launch per pass covers the tiles of n views, each with its own uniforms, G-buffers,
- * reservoirs and scene (the lights and BVH set on `scene`, a context on the same device). The
- * pixels are computed by the same code as the single-view entry points, so each view's output is
- * bit-identical to calling restir_initial_temporal / restir_spatial / restir_unbiased (inline
- * schedule) / restir_shade for it alone. Workgroups take tiles from a global counter in view
- * order, so small and large views share the GPU without a tail per view. The per-view records
- * are written to context-owned device memory by kernels on `stream` (no host-memory reads at
- * execution), so a sequence of these calls can be captured in a HIP graph; calls on one context
- * must stay on one stream. Outputs may not overlap each other or any view's inputs. */
+/* ---- batched views (no counterpart in the reference, which renders one view): one call per pass
+ * covers n views, each with its own uniforms, G-buffers, reservoirs and scene (the lights and BVH
+ * set on `scene`, a context on the same device). The pixels are computed by the same code as the
+ * single-view entry points, so each view's output is bit-identical to calling
+ * restir_initial_temporal / restir_spatial / restir_unbiased / restir_shade for it alone
+ * (RESTIR_INPUT_VISIBLE_FLAG is ignored here). restir_spatial_views and restir_shade_views are one
+ * persistent launch over the tiles of all views, so small and large views share the GPU without a
+ * tail per view. The two calls that trace shadow rays run the views one after another on the queued
+ * schedule with ctx's scratch and counters; with launch->schedule = RESTIR_SCHEDULE_INLINE, or where
+ * the scratch cannot grow (under stream capture, or out of memory), they too are one persistent
+ * launch, rays traced per pixel. The per-view records of a persistent launch are written to
+ * context-owned device memory by kernels on `stream` (no host-memory reads at execution), so a
+ * sequence of these calls can be captured in a HIP graph; calls on one context must stay on one
+ * stream. Outputs may not overlap each other or any view's inputs. */
 typedef struct restir_view {
     const restir_ctx *scene;         /* lights + BVH of this view */
     const restir_uniforms *uniforms; /* screenSize, frame, flags, ... of this view */

@@ -126,7 +126,15 @@ uint32_t persistent_blocks(uint32_t cus, int stack) {
 }
 
 int ensure_scratch(restir_ctx *ctx, size_t bytes) {
-    if (bytes > ctx->scratchBytes) ctx->surfValid = false;  // a new allocation holds no records
+    if (bytes > ctx->scratchBytes) {
+        ctx->surfValid = false;  // a new allocation holds no records
+        if (ctx->scratchInGraph) {  // a graph may replay launches over the old one: kept to the end
+            ctx->retired.push_back(ctx->scratch);
+            ctx->scratch = nullptr;
+            ctx->scratchBytes = 0;
+            ctx->scratchInGraph = false;
+        }
+    }
     return ensure(ctx, &ctx->scratch, &ctx->scratchBytes, bytes);
 }
 

@@ -1,7 +1,9 @@
 // abi_views.hip — batched-view entry points (restir_*_views): per-view validation with the same
-// rules as the single-view entry points, then one persistent launch per pass.
+// rules as the single-view entry points, then one persistent launch per pass, or, for the passes that
+// trace shadow rays, the queued schedule view after view.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "ctx.h"
@@ -53,6 +55,37 @@ int prepare(restir_ctx *ctx, uint32_t n) {
 
 uint32_t *view_counter(restir_ctx *ctx) { return ctx->counters + 8; }
 
+// Whether the passes that trace rays run view after view on the queued schedule, with this context's
+// scratch (`bytes`: the largest view's) and work counters: unless the caller asks for the inline
+// schedule, or the scratch is too small and cannot grow (the stream is being captured, or the
+// device is out of memory). Tracing in the pixels' lanes keeps a wave until its longest ray ends
+// and cannot gather triangle tests: 8 views from 640x360 to 1920x1080 over 2 scenes take 21.5 ms of
+// one-launch passes A and C that way, 13.6 ms queued, with a launch sequence per view.
+bool queued_views(restir_ctx *ctx, const restir_launch *launch, size_t bytes, hipStream_t s) {
+    if (launch && launch->schedule == RESTIR_SCHEDULE_INLINE) return false;
+    // what the scratch held of a single-view Pass C will be overwritten
+    ctx->queuedNpx = 0;
+    ctx->surfValid = false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        if (bytes > ctx->scratchBytes) return false;
+        ctx->scratchInGraph = true;
+        return true;
+    }
+    if (ensure_scratch(ctx, bytes) == RESTIR_OK) return true;
+    (void)hipGetLastError();
+    ctx->error.clear();
+    return false;
+}
+
+// The scene of a view as this context's launches see it: a scene may be in use by launches of its
+// own context, so the tracer takes its chunks through this context's counters.
+rk::SceneView own_counters(const restir_ctx *ctx, rk::SceneView sc) {
+    sc.traceHeads = ctx->scene.traceHeads;
+    return sc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -65,6 +98,7 @@ int restir_initial_temporal_views(restir_ctx *ctx, const restir_view *views, uin
     if (int r = pick_tile(ctx, launch, &tile)) return r;
     std::vector<rk::ViewA> rec(n);
     std::vector<Span> outs, ins;
+    size_t queueBytes = 0;
     int stack = 24;  // the smallest compiled stack; raised to the deepest scene's
     for (uint32_t v = 0; v < n; ++v) {
         const restir_view &w = views[v];
@@ -84,12 +118,26 @@ int restir_initial_temporal_views(restir_ctx *ctx, const restir_view *views, uin
         }
         outs.push_back({w.out, bytes});
         if (w.scene->stack > stack) stack = w.scene->stack;
+        queueBytes = std::max(queueBytes, rk::pass_a_queue_bytes(W * H));
         rec[v] = rk::ViewA{*u, w.scene->scene, view_of(w.cur), view_of(temporal ? w.prev : nullptr), w.in, w.out};
     }
     if (int r = check_disjoint(ctx, outs, ins, "initial_temporal_views")) return r;
+    if (int r = use_device(ctx)) return r;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (queued_views(ctx, launch, queueBytes, s)) {
+        for (uint32_t v = 0; v < n; ++v) {
+            const rk::ViewA &w = rec[v];
+            const int st = views[v].scene->stack;
+            const hipError_t e = rk::launch_pass_a(tile, st, w.u, own_counters(ctx, w.sc), w.cur, w.prev, w.prevRes,
+                                                   w.out, nullptr, nullptr, ctx->scratch,
+                                                   persistent_blocks(ctx->cus, st), s);
+            if (e != hipSuccess) return hip_fail(ctx, e, "initial_temporal_views launch");
+        }
+        return RESTIR_OK;
+    }
     if (int r = prepare(ctx, n)) return r;
     const hipError_t e = rk::launch_pass_a_views(tile, stack, rec.data(), n, ctx->viewTable, view_counter(ctx),
-                                                 resident_blocks(ctx->cus, static_cast<uint32_t>(stack) * 1024u), static_cast<hipStream_t>(stream));
+                                                 resident_blocks(ctx->cus, static_cast<uint32_t>(stack) * 1024u), s);
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "initial_temporal_views launch");
 }
 
@@ -129,6 +177,8 @@ int restir_unbiased_views(restir_ctx *ctx, const restir_view *views, uint32_t n,
     if (int r = pick_tile(ctx, launch, &tile)) return r;
     std::vector<rk::ViewC> rec(n);
     std::vector<Span> outs, ins;
+    size_t queueBytes = 0;
+    bool queueable = true;
     int stack = 24;  // the smallest compiled stack; raised to the deepest scene's
     for (uint32_t v = 0; v < n; ++v) {
         const restir_view &w = views[v];
@@ -143,13 +193,29 @@ int restir_unbiased_views(restir_ctx *ctx, const restir_view *views, uint32_t n,
         ins.push_back({w.in, bytes});
         outs.push_back({w.out, bytes});
         if (w.scene->stack > stack) stack = w.scene->stack;
+        queueBytes = std::max(queueBytes, rk::pass_c_queue_bytes(W * H, k));
+        // a queued neighbour ray carries its pixel in 27 bits of its tag
+        queueable = queueable && static_cast<uint64_t>(W) * H < (1ull << 27);
         rec[v] = rk::ViewC{*u, w.scene->scene, view_of(w.cur), w.in, w.out};
     }
     if (int r = check_disjoint(ctx, outs, ins, "unbiased_views")) return r;
+    if (int r = use_device(ctx)) return r;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (queueable && queued_views(ctx, launch, queueBytes, s)) {
+        for (uint32_t v = 0; v < n; ++v) {
+            rk::ViewC &w = rec[v];
+            w.u.flags &= ~RESTIR_INPUT_VISIBLE_FLAG;  // these calls make no use of the promise
+            const int st = views[v].scene->stack;
+            const hipError_t e = rk::launch_pass_c(tile, st, w.u, k, iter, own_counters(ctx, w.sc), w.g, w.in, w.out,
+                                                   ctx->scratch, persistent_blocks(ctx->cus, st), s);
+            if (e != hipSuccess) return hip_fail(ctx, e, "unbiased_views launch");
+        }
+        return RESTIR_OK;
+    }
     if (int r = prepare(ctx, n)) return r;
     const hipError_t e = rk::launch_pass_c_views(tile, stack, rec.data(), n, k, iter, ctx->viewTable,
                                                  view_counter(ctx), resident_blocks(ctx->cus, static_cast<uint32_t>(stack) * 1024u),
-                                                 static_cast<hipStream_t>(stream));
+                                                 s);
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "unbiased_views launch");
 }
 

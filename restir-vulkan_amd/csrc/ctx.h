@@ -37,6 +37,8 @@ struct restir_ctx {
     void *noallocScratch = nullptr;  // this device's copy of abi.hip's static `scratch` array
     void *scratch = nullptr;       // ray queues of the queued Pass C schedule
     size_t scratchBytes = 0;
+    bool scratchInGraph = false;   // a stream capture recorded multi-view launches that use it
+    std::vector<void *> retired;   // earlier scratches that captured graphs still use
     uint32_t queuedNpx = 0;        // shape of the last queued Pass C (its rays stay in scratch)
     const restir_reservoir *queuedOut = nullptr;  // its output (the light end of its neighbour rays)
     int queuedK = 0;
@@ -78,6 +80,7 @@ struct restir_ctx {
     ~restir_ctx() {
         if (counters) (void)hipFree(counters);
         if (scratch) (void)hipFree(scratch);
+        for (void *p : retired) (void)hipFree(p);
         if (mlpScratch) (void)hipFree(mlpScratch);
         if (truthScratch) (void)hipFree(truthScratch);
         if (viewTable) (void)hipFree(viewTable);
@@ -102,6 +105,7 @@ int check_frame(restir_ctx *ctx, const restir_uniforms *u, const char *name);
 int pick_tile(restir_ctx *ctx, const restir_launch *l, int *tile);
 int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, void **queues);
 int ensure(restir_ctx *ctx, void **buf, size_t *have, size_t bytes);
+int ensure_scratch(restir_ctx *ctx, size_t bytes);
 uint32_t resident_blocks(uint32_t cus, uint32_t ldsBytes);
 uint32_t persistent_blocks(uint32_t cus, int stack);
 int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *tris, uint32_t depth, hipStream_t s);

@@ -275,11 +275,12 @@ class BatchRenderer:
     the same Scene object share its device tables (one context per distinct scene). Every view
     has its own G-buffers, reservoirs and image; ``rgb`` holds all images back to back and
     ``images[v]`` is view v's [3 * W * H] slice. Pass B and shading of all views run as one
-    persistent launch each (restir_*_views). The passes that trace shadow rays, A and C, run
-    either the same way (``rays="persistent"``, the default: one launch per pass over all views,
-    rays traced per pixel) or view by view on the queued ray schedule of the view's scene context
-    (``rays="queued"``: each view's rays compacted and traced by the persistent tracer). Both give
-    each view's output bit-identical to a Renderer of that view alone.
+    persistent launch each (restir_*_views). The passes that trace shadow rays, A and C, run either
+    through the multi-view entry points too (``rays="persistent"``, the default: queued view after
+    view with this renderer's own scratch, or, with ``launch.schedule`` = SCHEDULE_INLINE, one
+    persistent launch per pass with the rays traced per pixel) or view by view through each scene's
+    context (``rays="queued"``). All give each view's output bit-identical to a Renderer of that view
+    alone.
 
     On the queued schedule the views of different scenes share nothing (each scene context has its
     own scratch and queues), so with ``concurrent_scenes`` (default) each scene's views run in order
