@@ -529,7 +529,7 @@ int restir_camera_projection_view(const restir_camera *cam, float aspect, float 
  * single-view entry points, so each view's output is bit-identical to calling
  * restir_initial_temporal / restir_spatial / restir_unbiased / restir_shade for it alone
  * (RESTIR_INPUT_VISIBLE_FLAG is ignored here). restir_spatial_views and restir_shade_views are one
- * persistent launch over the tiles of all views, so small and large views share the GPU without a
+ * launch over the tiles of all views, so small and large views share the GPU without a
  * tail per view. The two calls that trace shadow rays run the views one after another on the queued
  * schedule with ctx's scratch and counters; with launch->schedule = RESTIR_SCHEDULE_INLINE, or where
  * the scratch cannot grow (under stream capture, or out of memory), they too are one persistent
