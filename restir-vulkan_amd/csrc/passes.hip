@@ -151,8 +151,8 @@ __device__ __forceinline__ Pcg pass_a_rng(const PassAArgs &a, uint32_t x, uint32
 // depends on the kind; the target function and the reservoir update run once for all lanes of a
 // wave whatever kinds its lanes drew. `valid` false: an empty candidate (p_hat 0, probability 1)
 // that still counts in M and draws its update number.
-__device__ __forceinline__ void add_candidate(Res &res, const Surface &s, f3 pos, const SceneView &sc, bool valid,
-                                              bool tri, int32_t li, float prob, float4 point, float ra, float rb,
+__device__ __forceinline__ void add_candidate(Res &res, RisTaken &taken, const Surface &s, f3 pos,
+                                              const SceneView &sc, bool valid, bool tri, int32_t li, float prob, float4 point, float ra, float rb,
                                               float u, bool areaPdf) {
     f3 L{0.0f, 0.0f, 0.0f}, nl{0.0f, 0.0f, 0.0f};
     float lum = 0.0f;
@@ -178,7 +178,7 @@ __device__ __forceinline__ void add_candidate(Res &res, const Surface &s, f3 pos
     }
     const bool useLN = valid && tri;
     const float ph = valid ? eval_phat(s, L, nl, useLN, lum) : 0.0f;
-    res_add_sample_u(res, L, make_float4(nl.x, nl.y, nl.z, useLN ? 1.0f : 0.0f), lum, index, ph,
+    res_add_sample_u(res, taken, L, make_float4(nl.x, nl.y, nl.z, useLN ? 1.0f : 0.0f), lum, index, ph,
                      valid ? prob : 1.0f, u);
 }
 
@@ -201,6 +201,7 @@ __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurfac
     const f3 pos = ps.pos, n = ps.n;
     const Surface &s = ps.s;
     res = res_zero();
+    RisTaken taken;
     const SceneView &sc = a.sc;
     const bool standard = (a.u.flags & RESTIR_STANDARD_WEIGHTS_FLAG) != 0;
     const uint32_t M = a.u.initialLightSampleCount;
@@ -221,7 +222,7 @@ __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurfac
             }
             const float u = pcg_float(rng);
             const float4 point = valid && !tri ? point_light(sc, li) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            add_candidate(res, s, pos, sc, valid, tri, tri ? li - sc.nPoints : li, q, point, ra, rb, u, standard);
+            add_candidate(res, taken, s, pos, sc, valid, tri, tri ? li - sc.nPoints : li, q, point, ra, rb, u, standard);
         }
     } else if (dot(n, n) != 0.0f && M > 0) {
         // A candidate draws r1, r2 (the alias column and its coin), then a triangle light's two
@@ -287,7 +288,7 @@ __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurfac
             } else {
                 u = pcg_float_at(s2);
             }
-            add_candidate(res, s, pos, sc, true, cur.tri, cur.li, cur.prob, cur.point, ra, rb, u, standard);
+            add_candidate(res, taken, s, pos, sc, true, cur.tri, cur.li, cur.prob, cur.point, ra, rb, u, standard);
             st = stN;
             cur = nxt;
             stN = stNN;
@@ -296,6 +297,7 @@ __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurfac
         }
         rng.state = st;
     }
+    res.w = ris_w(taken, res.pHat);
     // the standard RIS contribution weight instead of the selection-time one
     if (standard && res.w > 0.0f) res.w = res.sumW / (static_cast<float>(res.M) * res.pHat);
 }

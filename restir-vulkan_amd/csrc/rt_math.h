@@ -31,8 +31,96 @@ RT_HD float dot(f3 a, f3 b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
 RT_HD f3 cross(f3 a, f3 b) {
     return f3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
-RT_HD f3 normalize(f3 a) { return a / sqrtf(dot(a, a)); }
 RT_HD f3 xyz(float4 v) { return f3{v.x, v.y, v.z}; }
+
+// ---------------------------------------------------- correctly rounded division and square root
+// The same numbers as `/` and sqrtf, from fewer instructions, for operands away from the ends of
+// the exponent range. The compiler's IEEE division takes 11 instructions whatever its operands; here
+// a divisor's reciprocal is formed once (rcp_near, 3) and each quotient over it takes 3. The square
+// root takes 5 instead of about 15.
+//   rcp_near(b)     = RN(1 / b):   one Newton step on the hardware's reciprocal
+//   div_near(a,b,y) = RN(a / b):   a product and one residual step (Markstein 1990), y = rcp_near(b)
+//   sqrt_near(x)    = RN(sqrt(x)): one residual step on the hardware's reciprocal square root
+//   over_pi(x)      = RN(x / kPi): as div_near, with 1 / kPi rounded at compile time
+// Compared on the MI355X with the IEEE forms for every b in [2^-60, 2^60], every x in [2^-100,
+// 2^100], and every one of the 2^46 pairs of mantissas of a and b: no difference. Scaling by powers of
+// two changes no mantissa while nothing under- or overflows, which the bounds below keep away. With
+// them, and W formed once instead of per candidate, k_pass_a_ris (VALU bound: 0.82 of the issue
+// rate) went from 0.75 to 0.635 ms at 1080p, M = 32.
+#ifdef __HIP_DEVICE_COMPILE__
+#define RT_NEAR_MATH 1
+#endif
+__device__ __forceinline__ float rcp_near(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return fmaf(fmaf(-b, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float div_near(float a, float b, float y) {
+    const float q = a * y;
+    return fmaf(fmaf(-b, q, a), y, q);
+}
+__device__ __forceinline__ float sqrt_near(float x) {
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y;
+    return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+}
+__device__ __forceinline__ float over_pi(float x) {
+    constexpr float c = 1.0f / kPi;
+    const float q = x * c;
+    return fmaf(fmaf(-q, kPi, x), c, q);
+}
+// x in [2^-60, 2^60]; false for negative numbers, NaN and infinity
+__device__ __forceinline__ bool mid_range(float x) {
+    return __float_as_uint(x) - 0x21800000u <= 0x5d800000u - 0x21800000u;
+}
+// Every component of a at least 2^-48 in magnitude and |a|^2 = s2 at most 2^60
+__device__ __forceinline__ bool mid_range3(f3 a, float s2) {
+    return fminf(fminf(fabsf(a.x), fabsf(a.y)), fabsf(a.z)) >= 0x1p-48f && s2 <= 0x1p60f;
+}
+// a / sqrt(s2), s2 = dot(a, a) of a mid_range3 vector
+__device__ __forceinline__ f3 normalize_near(f3 a, float s2) {
+    const float s = sqrt_near(s2), y = rcp_near(s);
+    return f3{div_near(a.x, s, y), div_near(a.y, s, y), div_near(a.z, s, y)};
+}
+RT_HD f3 normalize(f3 a) {
+    const float s2 = dot(a, a);
+#ifdef RT_NEAR_MATH
+    if (mid_range3(a, s2)) return normalize_near(a, s2);
+#endif
+    return a / sqrtf(s2);
+}
+
+// The operations of the BRDF evaluation. Ieee: as written. Near: the forms above; `ok` turns false
+// when an operand lies outside their ranges, and the result is then not used.
+struct Ieee {
+    static constexpr bool ok = true;
+    __device__ __forceinline__ float div(float a, float b) { return a / b; }
+    __device__ __forceinline__ float rcp(float b) { return 1.0f / b; }
+    __device__ __forceinline__ float root(float x) { return sqrtf(x); }
+    __device__ __forceinline__ float div_pi(float x) { return x / kPi; }
+    __device__ __forceinline__ f3 unit(f3 a, float s2) { return a / sqrtf(s2); }
+};
+struct Near {
+    bool ok = true;
+    __device__ __forceinline__ float div(float a, float b) {
+        ok = ok && mid_range(a) && mid_range(b);
+        return div_near(a, b, rcp_near(b));
+    }
+    __device__ __forceinline__ float rcp(float b) {
+        ok = ok && mid_range(b);
+        return rcp_near(b);
+    }
+    __device__ __forceinline__ float root(float x) {
+        ok = ok && mid_range(x);
+        return sqrt_near(x);
+    }
+    __device__ __forceinline__ float div_pi(float x) {  // +0 (a metal) gives +0
+        ok = ok && (mid_range(x) || __float_as_uint(x) == 0u);
+        return over_pi(x);
+    }
+    __device__ __forceinline__ f3 unit(f3 a, float s2) {
+        ok = ok && mid_range3(a, s2);
+        return normalize_near(a, s2);
+    }
+};
 
 RT_HD float gmin(float x, float y) { return (y < x) ? y : x; }
 RT_HD float gmax(float x, float y) { return (x < y) ? y : x; }
@@ -131,15 +219,17 @@ RT_HD float schlick(float c) {  // disneyBRDF.glsl:5-10
     const float sm = m * m;
     return sm * sm * m;
 }
-RT_HD float gtr2(float ndoth, float a) {  // disneyBRDF.glsl:13-18
+template <class A>
+__device__ __forceinline__ float gtr2(A &m, float ndoth, float a) {  // disneyBRDF.glsl:13-18
     const float a2 = a * a;
     const float t = 1.0f + (a2 - 1.0f) * ndoth * ndoth;
-    return a2 / (kPi * t * t);
+    return m.div(a2, kPi * t * t);
 }
-RT_HD float smith_g(float ndotv, float alphaG) {  // disneyBRDF.glsl:20-25
+template <class A>
+__device__ __forceinline__ float smith_g(A &m, float ndotv, float alphaG) {  // disneyBRDF.glsl:20-25
     const float a = alphaG * alphaG;
     const float b = ndotv * ndotv;
-    return 1.0f / (fabsf(ndotv) + gmax(sqrtf(a + b - a * b), 0.0001f));
+    return m.rcp(fabsf(ndotv) + gmax(m.root(a + b - a * b), 0.0001f));
 }
 
 // Per-pixel constants of the BRDF that do not depend on the light: alpha, and the terms of
@@ -152,7 +242,7 @@ struct Surface {
     float gOut;       // smith_g(cosOut, a)
     float oneMinusMetal;
 };
-RT_HD Surface make_surface(f3 pos, f3 n, f3 cam, float albLum, float rough, float metal) {
+__device__ __forceinline__ Surface make_surface(f3 pos, f3 n, f3 cam, float albLum, float rough, float metal) {
     Surface s;
     s.pos = pos;
     s.n = n;
@@ -163,7 +253,12 @@ RT_HD Surface make_surface(f3 pos, f3 n, f3 cam, float albLum, float rough, floa
     s.metal = metal;
     s.a = gmax(0.001f, rough * rough);
     s.fOut = schlick(s.cosOut);
-    s.gOut = smith_g(s.cosOut, s.a);
+    Near near;
+    s.gOut = smith_g(near, s.cosOut, s.a);
+    if (!near.ok) {
+        Ieee ieee;
+        s.gOut = smith_g(ieee, s.cosOut, s.a);
+    }
     s.oneMinusMetal = 1.0f - metal;
     return s;
 }
@@ -173,7 +268,8 @@ struct LightGeom {
     bool below;
 };
 // restirUtils.glsl:7-25 (shared by evaluatePHat and evaluatePHatFull)
-RT_HD LightGeom light_geometry(const Surface &s, f3 L, f3 LN, bool useLN) {
+template <class A>
+__device__ __forceinline__ LightGeom light_geometry(A &m, const Surface &s, f3 L, f3 LN, bool useLN) {
     LightGeom g{};
     f3 wi = L - s.pos;
     if (dot(wi, s.n) < 0.0f) {
@@ -181,53 +277,67 @@ RT_HD LightGeom light_geometry(const Surface &s, f3 L, f3 LN, bool useLN) {
         return g;
     }
     const float sqrDist = dot(wi, wi);
-    wi = wi / sqrtf(sqrDist);
+    wi = m.unit(wi, sqrDist);
     g.cosIn = dot(s.n, wi);
-    const f3 h = normalize(wi + s.wo);
+    const f3 hv = wi + s.wo;
+    const f3 h = m.unit(hv, dot(hv, hv));
     g.cosHalf = dot(s.n, h);
     g.cosInHalf = dot(wi, h);
-    g.geometry = g.cosIn / sqrDist;
+    g.geometry = m.div(g.cosIn, sqrDist);
     if (useLN) g.geometry *= fabsf(dot(wi, LN));
     g.below = false;
     return g;
 }
 // disneyBrdfDiffuseFactor (:27-33) and the specular factor Gs*Ds (:42-55)
-RT_HD float diffuse_factor(const Surface &s, const LightGeom &g) {
+template <class A>
+__device__ __forceinline__ float diffuse_factor(A &m, const Surface &s, const LightGeom &g) {
     const float fin = schlick(g.cosIn);
     const float fd90 = 0.5f + 2.0f * g.cosInHalf * g.cosInHalf * s.rough;
     const float fd = gmix(1.0f, fd90, fin) * gmix(1.0f, fd90, s.fOut);
-    return fd * s.oneMinusMetal / kPi;
+    return m.div_pi(fd * s.oneMinusMetal);
 }
-RT_HD float gs_ds(const Surface &s, const LightGeom &g) {
-    const float ds = gtr2(g.cosHalf, s.a);
-    float gs = smith_g(g.cosIn, s.a);
+template <class A>
+__device__ __forceinline__ float gs_ds(A &m, const Surface &s, const LightGeom &g) {
+    const float ds = gtr2(m, g.cosHalf, s.a);
+    float gs = smith_g(m, g.cosIn, s.a);
     gs *= s.gOut;
     return gs * ds;
 }
 // evaluatePHat, restirUtils.glsl:3-28 with disneyBrdfLuminance (disneyBRDF.glsl:82-90)
-RT_HD float eval_phat(const Surface &s, f3 L, f3 LN, bool useLN, float emLum) {
-    const LightGeom g = light_geometry(s, L, LN, useLN);
+template <class A>
+__device__ __forceinline__ float eval_phat_as(A &m, const Surface &s, f3 L, f3 LN, bool useLN, float emLum) {
+    const LightGeom g = light_geometry(m, s, L, LN, useLN);
     if (g.below) return 0.0f;
     float brdf = 0.0f;
     if (!(g.cosIn < 0.0f)) {
-        const float diffuse = s.albLum * diffuse_factor(s, g);
+        const float diffuse = s.albLum * diffuse_factor(m, s, g);
         const float fih = schlick(g.cosInHalf);
-        const float gsds = gs_ds(s, g);
+        const float gsds = gs_ds(m, s, g);
         const float specLum = gmix(0.04f, s.albLum, s.metal);
         const float fs = gmix(specLum, 1.0f, fih);
         brdf = diffuse + fs * gsds;
     }
     return emLum * brdf * g.geometry;
 }
+__device__ __forceinline__ float eval_phat(const Surface &s, f3 L, f3 LN, bool useLN, float emLum) {
+    Near near;
+    float p = eval_phat_as(near, s, L, LN, useLN, emLum);
+    if (!near.ok) {
+        Ieee ieee;
+        p = eval_phat_as(ieee, s, L, LN, useLN, emLum);
+    }
+    return p;
+}
 // evaluatePHatFull, restirUtils.glsl:30-55 with disneyBrdfColor (disneyBRDF.glsl:73-81)
-RT_HD f3 eval_phat_full(const Surface &s, f3 albedo, f3 L, f3 LN, bool useLN, f3 em) {
-    const LightGeom g = light_geometry(s, L, LN, useLN);
+template <class A>
+__device__ __forceinline__ f3 eval_phat_full_as(A &m, const Surface &s, f3 albedo, f3 L, f3 LN, bool useLN, f3 em) {
+    const LightGeom g = light_geometry(m, s, L, LN, useLN);
     if (g.below) return f3{0.0f, 0.0f, 0.0f};
     f3 brdf{0.0f, 0.0f, 0.0f};
     if (!(g.cosIn < 0.0f)) {
-        const float df = diffuse_factor(s, g);
+        const float df = diffuse_factor(m, s, g);
         const float fih = schlick(g.cosInHalf);
-        const float gsds = gs_ds(s, g);
+        const float gsds = gs_ds(m, s, g);
         const float alb[3] = {albedo.x, albedo.y, albedo.z};
         float out[3];
         for (int c = 0; c < 3; ++c) {
@@ -239,6 +349,15 @@ RT_HD f3 eval_phat_full(const Surface &s, f3 albedo, f3 L, f3 LN, bool useLN, f3
         brdf = f3{out[0], out[1], out[2]};
     }
     return f3{em.x * brdf.x * g.geometry, em.y * brdf.y * g.geometry, em.z * brdf.z * g.geometry};
+}
+__device__ __forceinline__ f3 eval_phat_full(const Surface &s, f3 albedo, f3 L, f3 LN, bool useLN, f3 em) {
+    Near near;
+    f3 p = eval_phat_full_as(near, s, albedo, L, LN, useLN, em);
+    if (!near.ok) {
+        Ieee ieee;
+        p = eval_phat_full_as(ieee, s, albedo, L, LN, useLN, em);
+    }
+    return p;
 }
 
 // ------------------------------------------------------------------------------- reservoirs
@@ -263,10 +382,12 @@ RT_HD Res res_zero() {
 }
 // updateReservoirAt, reservoir.glsl:6-26
 // u: the update's uniform draw; returns true when the sample is taken
-RT_HD bool res_update_u(Res &r, float weight, f3 pos, float4 n, float emLum, int32_t li, float pHat,
-                        float w, float u) {
+__device__ __forceinline__ bool res_update_u(Res &r, float weight, f3 pos, float4 n, float emLum, int32_t li, float pHat,
+                                             float w, float u) {
     r.sumW += weight;
-    const float rp = weight / r.sumW;
+    if (weight == 0.0f) return false;  // u < 0 / sumW never holds
+    const float rp = mid_range(weight) && mid_range(r.sumW) ? div_near(weight, r.sumW, rcp_near(r.sumW))
+                                                            : weight / r.sumW;
     if (u < rp) {
         r.pos = pos;
         r.emLum = emLum;
@@ -278,24 +399,33 @@ RT_HD bool res_update_u(Res &r, float weight, f3 pos, float4 n, float emLum, int
     }
     return false;
 }
-RT_HD void res_update(Res &r, float weight, f3 pos, float4 n, float emLum, int32_t li, float pHat,
-                      float w, Pcg &rng) {
+__device__ __forceinline__ void res_update(Res &r, float weight, f3 pos, float4 n, float emLum, int32_t li, float pHat,
+                                           float w, Pcg &rng) {
     res_update_u(r, weight, pos, n, emLum, li, pHat, w, pcg_float(rng));
 }
-// addSampleToReservoir, reservoir.glsl:28-42 (u: the update's uniform draw)
-RT_HD void res_add_sample_u(Res &r, f3 pos, float4 n, float emLum, int32_t li, float pHat,
-                            float sampleP, float u) {
-    const float weight = pHat / sampleP;
+// addSampleToReservoir, reservoir.glsl:28-42 (u: the update's uniform draw). Its W = sumW / (M
+// pHat), of the moment a sample is taken, is left to ris_w: only the last one taken keeps it.
+struct RisTaken {
+    float sumW = 0.0f;
+    uint32_t M = 0u;  // 0: none was taken
+};
+__device__ __forceinline__ void res_add_sample_u(Res &r, RisTaken &taken, f3 pos, float4 n, float emLum, int32_t li,
+                                                 float pHat, float sampleP, float u) {
+    const float weight = (mid_range(pHat) || __float_as_uint(pHat) == 0u) && mid_range(sampleP)
+                             ? div_near(pHat, sampleP, rcp_near(sampleP))
+                             : pHat / sampleP;
     r.M += 1u;
-    const float w = (r.sumW + weight) / (static_cast<float>(r.M) * pHat);
-    res_update_u(r, weight, pos, n, emLum, li, pHat, w, u);
+    if (res_update_u(r, weight, pos, n, emLum, li, pHat, 0.0f, u)) {
+        taken.sumW = r.sumW;
+        taken.M = r.M;
+    }
 }
-RT_HD void res_add_sample(Res &r, f3 pos, float4 n, float emLum, int32_t li, float pHat,
-                          float sampleP, Pcg &rng) {
-    res_add_sample_u(r, pos, n, emLum, li, pHat, sampleP, pcg_float(rng));
+// W of the sample taken last (0 when none was)
+__device__ __forceinline__ float ris_w(const RisTaken &taken, float pHat) {
+    return taken.M ? taken.sumW / (static_cast<float>(taken.M) * pHat) : 0.0f;
 }
 // combineReservoirs, reservoir.glsl:44-64
-RT_HD void res_combine(Res &self, const Res &o, float pHat, Pcg &rng) {
+__device__ __forceinline__ void res_combine(Res &self, const Res &o, float pHat, Pcg &rng) {
     self.M += o.M;
     const float weight = pHat * o.w * static_cast<float>(o.M);
     if (weight > 0.0f) res_update(self, weight, o.pos, o.normal, o.emLum, o.lightIndex, pHat, o.w, rng);
