@@ -971,6 +971,14 @@ __global__ __launch_bounds__(256) void k_trace_queue(const SceneView sc, const f
     }
 }
 
+// What the wave's lanes stored to LDS before it, its other lanes read after it: a wave's LDS accesses
+// take effect in order, and the barrier (no instruction) keeps the compiler from reordering them.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Inclusive sum over the wave's lanes (all active).
 __device__ __forceinline__ uint32_t wave_sum_inclusive(uint32_t x) {
     const auto add = [&](auto ctrl, auto rows) {
@@ -1135,6 +1143,7 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
                 waiting += static_cast<uint32_t>(__popc(pend));
             }
             listed += static_cast<uint32_t>(__popcll(found));
+            wave_sync();
         }
         // rounds of triangle tests: whenever the ring holds enough for one, or what there is once
         // too few lanes can still walk
@@ -1161,6 +1170,7 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
                 }
             }
             if (part) ringM[at] = static_cast<uint8_t>(m);
+            wave_sync();
             const uint32_t done = static_cast<uint32_t>(__popcll(__ballot(lane < listed && m == 0)));
             first = (first + done) & (kTri8Ring - 1u);
             listed -= done;
@@ -1182,6 +1192,7 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
                     h = rt::w8_confirm<true>(sc.nodes, sc.parent, sc.treeNested != 0, sc.treeTight != 0, va, vb, vc, ro, rd);
             }
             if (mine) atomicAdd(&tal[o], h ? 257u : 256u);
+            wave_sync();
             const uint32_t r = atomicExch(&tal[lane], 0u);  // after this wave's adds (LDS keeps a wave's order)
             waiting -= r >> 8;
             if (r & 0xffu) {
