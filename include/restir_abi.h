@@ -315,9 +315,10 @@ int restir_build_alias_table(const restir_point_light *points, uint32_t n_point,
 
 /* createAliasTable (misc.cpp:418-497) on the device, for lights whose power changes: the columns
  * restir_build_alias_table makes, bit for bit, from device light records (point lights if
- * n_point > 0, else triangle lights; plain arrays, no SSBO header) into device columns[n]. One
- * workgroup, one launch, no host round trip (it may be captured into a graph); the work is
- * ordered on `stream`. Context scratch: 20 bytes per light. */
+ * n_point > 0, else triangle lights; plain arrays, no SSBO header) into device columns[n]. No host
+ * round trip (it may be captured into a graph once a build of that size has sized the scratch; with
+ * 20 bytes per light of it, in one workgroup); the work is ordered on `stream`. Context scratch: 20
+ * bytes per light up to 4,096 lights, above that about 29. */
 int restir_build_alias_table_device(restir_ctx *ctx, const restir_point_light *points,
                                     uint32_t n_point, const restir_tri_light *tris, uint32_t n_tri,
                                     restir_alias_table_column *columns, void *stream);
