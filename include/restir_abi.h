@@ -399,7 +399,9 @@ int restir_mlp_init(restir_ctx *ctx, restir_mlp *mlp, uint64_t seed, const float
 /* Binds the cluster tables of restir_build_light_clusters (device copies) for the proposal.
  * Validates them (copying them to the host, synchronously) and builds from them a context-owned
  * device table of 32 bytes per light (each cluster slot's light, p_within and p_src, for its
- * column and its alias); the caller's buffers must stay alive while the context uses them.
+ * column and its alias); the caller's buffers must stay alive while the context uses them. For
+ * k > 256 (a multiple of 128) the context also allocates the proposal's working memory, at most
+ * 544 * k bytes per compute unit (570 MB at k = 4,096), less where that cannot be had.
  * Call it after restir_set_lights: the slot table snapshots the bound alias table, and binding
  * new lights unbinds the clusters. */
 int restir_set_light_clusters(restir_ctx *ctx, uint32_t k, const int32_t *light_cluster,

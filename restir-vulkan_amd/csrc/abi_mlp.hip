@@ -59,6 +59,36 @@ int restir_mlp_init(restir_ctx *ctx, restir_mlp *m, uint64_t seed, const float *
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "mlp_init launch");
 }
 
+// Slots of the wide proposal for networks of k clusters, where that kernel takes them: as many as
+// the device holds workgroups, half as many as often as they do not fit, down to kMinSlots.
+static int ensure_slots(restir_ctx *ctx, uint32_t k) {
+    constexpr uint32_t kMinSlots = 16;
+    if (k <= 256 || k % rm::kSuper != 0 || k > static_cast<uint32_t>(rm::kMaxClusters) || k <= ctx->slotClusters)
+        return RESTIR_OK;
+    if (ctx->slotsInGraph) {  // a graph may replay launches over the old ones: kept to the end
+        ctx->retired.push_back(ctx->slots);
+    } else if (ctx->slots) {
+        (void)hipFree(ctx->slots);
+    }
+    ctx->slots = nullptr;
+    ctx->slotCount = ctx->slotClusters = 0;
+    ctx->slotsInGraph = false;
+    const size_t each = rk::wide_slot_bytes(k);
+    for (uint32_t n = rk::wide_slots(ctx->cus);; n /= 2) {
+        hipError_t e = hipMalloc(&ctx->slots, n * (each + sizeof(uint32_t)));
+        if (e == hipSuccess) {
+            e = hipMemset(static_cast<uint8_t *>(ctx->slots) + n * each, 0, n * sizeof(uint32_t));
+            if (e != hipSuccess) return hip_fail(ctx, e, "set_light_clusters: slots");
+            ctx->slotCount = n;
+            ctx->slotClusters = k;
+            return RESTIR_OK;
+        }
+        ctx->slots = nullptr;
+        if (n / 2 < kMinSlots) return hip_fail(ctx, e, "set_light_clusters: slots");
+        (void)hipGetLastError();
+    }
+}
+
 int restir_set_light_clusters(restir_ctx *ctx, uint32_t k, const int32_t *lightCluster,
                               const float *lightPWithin, const int32_t *clusterBegin,
                               const int32_t *clusterCount, const int32_t *clusterLights,
@@ -134,6 +164,7 @@ int restir_set_light_clusters(restir_ctx *ctx, uint32_t k, const int32_t *lightC
     if (int r = ensure(ctx, &ctx->clusterFused, &ctx->clusterFusedBytes, sizeof(float4) * fused.size())) return r;
     const hipError_t e = hipMemcpy(ctx->clusterFused, fused.data(), sizeof(float4) * fused.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(ctx, e, "set_light_clusters: fused slot records");
+    if (int r = ensure_slots(ctx, k)) return r;
     ctx->clustersSet = true;
     return RESTIR_OK;
 }
@@ -160,11 +191,19 @@ int restir_learned_candidates(restir_ctx *ctx, const restir_uniforms *u, const r
     if (int r = use_device(ctx)) return r;
     const rt::f3 cam{u->cameraPos[0], u->cameraPos[1], u->cameraPos[2]};
     const uint32_t seed = u->frame * 0x9e3779b1u + 0x7f4a7c15u;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) (void)hipGetLastError();
+    if (st != hipStreamCaptureStatusNone) ctx->slotsInGraph = ctx->slots != nullptr;
+    uint8_t *slots = static_cast<uint8_t *>(ctx->slots);
+    const rk::WideSlots wide{slots,
+                             slots ? reinterpret_cast<uint32_t *>(slots + ctx->slotCount * rk::wide_slot_bytes(ctx->slotClusters))
+                                   : nullptr,
+                             ctx->slotCount};
     const hipError_t e = rk::mlp_propose(*m, view_of(g), cam, lo, hi, ctx->scene, ctx->lightCluster,
                                          ctx->lightPWithin, ctx->clusterBegin, ctx->clusterCount,
                                          ctx->clusterLights, ctx->clusterAlias,
-                                         static_cast<const float4 *>(ctx->clusterFused), M, mix, seed, candLight,
-                                         candQ, static_cast<hipStream_t>(stream));
+                                         static_cast<const float4 *>(ctx->clusterFused), M, mix, seed, wide,
+                                         candLight, candQ, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "learned_candidates launch");
 }
 

@@ -38,7 +38,7 @@ struct restir_ctx {
     void *scratch = nullptr;       // ray queues of the queued Pass C schedule
     size_t scratchBytes = 0;
     bool scratchInGraph = false;   // a stream capture recorded multi-view launches that use it
-    std::vector<void *> retired;   // earlier scratches that captured graphs still use
+    std::vector<void *> retired;   // earlier scratches and slots that captured graphs still use
     uint32_t queuedNpx = 0;        // shape of the last queued Pass C (its rays stay in scratch)
     const restir_reservoir *queuedOut = nullptr;  // its output (the light end of its neighbour rays)
     int queuedK = 0;
@@ -77,6 +77,11 @@ struct restir_ctx {
     // alias, p_within of the column}, {p_within of the alias, p_src of both lights, 0}
     void *clusterFused = nullptr;
     size_t clusterFusedBytes = 0;
+    // the wide proposal's workgroup slots (then a word per slot: held or not), for up to
+    // slotClusters clusters
+    void *slots = nullptr;
+    uint32_t slotCount = 0, slotClusters = 0;
+    bool slotsInGraph = false;     // a stream capture recorded launches that use them
     ~restir_ctx() {
         if (counters) (void)hipFree(counters);
         if (scratch) (void)hipFree(scratch);
@@ -89,6 +94,7 @@ struct restir_ctx {
         if (aliasScratch) (void)hipFree(aliasScratch);
         if (wide) (void)hipFree(wide);
         if (clusterFused) (void)hipFree(clusterFused);
+        if (slots) (void)hipFree(slots);
     }
 };
 

@@ -189,12 +189,22 @@ hipError_t mlp_train(restir_mlp &m, const GView &g, rt::f3 cam, const float lo[3
                      uint32_t seed, float *lossOut, void *scratch, hipStream_t s);
 hipError_t mlp_adam(restir_mlp &m, const float *gw, const float *gb, const uint32_t *nValid, float lr,
                     hipStream_t s);
+// k_propose_wide's memory for workgroups in flight: n slots of wide_slot_bytes each, and a word per
+// slot that is 1 while a workgroup holds it (all 0 between launches)
+struct WideSlots {
+    void *base;
+    uint32_t *busy;
+    uint32_t n;
+};
+size_t wide_slot_bytes(uint32_t K);
+uint32_t wide_slots(uint32_t cus);  // workgroups that the device holds at a time
 hipError_t mlp_propose(const restir_mlp &m, const GView &g, rt::f3 cam, const float lo[3],
                        const float hi[3], const SceneView &sc, const int32_t *lightCluster,
                        const float *lightPWithin, const int32_t *clusterBegin,
                        const int32_t *clusterCount, const int32_t *clusterLights,
                        const restir_alias_table_column *clusterAlias, const float4 *clusterFused, uint32_t M,
-                       float mix, uint32_t seed, int32_t *candLight, float *candQ, hipStream_t s);
+                       float mix, uint32_t seed, const WideSlots &slots, int32_t *candLight, float *candQ,
+                       hipStream_t s);
 
 // ---- FP64 ground truth (truth.hip)
 constexpr uint32_t kTruthChunk = 128;  // lights per workgroup row

@@ -21,7 +21,7 @@ constexpr int kIn = 128;      // feature width (114 used, zero padded)
 constexpr int kHidden = 128;  // hidden width
 constexpr int kFeatures = 114;
 // cluster counts: 64, 128 or 256 (k_propose holds a quad's numerators in LDS), or a multiple of
-// kSuper up to kMaxClusters (k_propose_wide streams them in column blocks of kSuper), with at most
+// kSuper up to kMaxClusters (k_propose_wide keeps a running sum after each kSuper), with at most
 // kWideCand candidates per pixel
 constexpr int kSuper = 128;
 constexpr int kMaxClusters = 4096;

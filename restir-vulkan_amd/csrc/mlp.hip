@@ -10,7 +10,7 @@
 // Kernels:
 //   k_propose      fused inference per 2x2 pixel quad: features -> 4 MFMA layers -> softmax ->
 //                  M candidates (l, q) for each of its pixels (K <= 256)
-//   k_propose_wide the same for K up to 4096: the output layer streamed in 128-cluster blocks
+//   k_propose_wide the same for K up to 4096: the output layer streamed in 64-cluster blocks
 //   k_features     features of listed pixels (bf16), for training and tests
 //   k_gemm         strided C = A*B with bias / ReLU / ReLU-gate epilogues (training fwd/bwd),
 //                  or split-K fp32 partials for the weight gradients
@@ -419,11 +419,11 @@ struct ProposeArgs {
     const float4 *clusterFused;  // per slot: {prob, light, alias light, p_within}, {alias p_within, p_src, alias p_src, 0}
     int32_t *candLight;
     float *candQ;
+    uint8_t *slots;      // k_propose_wide: nSlots workgroups' numerators and running sums,
+    uint32_t *slotBusy;  // and which of them a workgroup holds
+    uint32_t nSlots;
 };
 
-// pixel quads per workgroup of k_propose_wide: 128 quads, 256 lanes and 69.6 KB of LDS, so that
-// two workgroups share a CU and one's barriers and weight loads overlap the other's work
-constexpr int kTilePx = 128;
 constexpr int kRow = kIn + 8;                // padded LDS row (bf16) against bank conflicts
 
 __device__ __forceinline__ void stage_weights(uint16_t *wbuf, const uint16_t *src, int rows) {
@@ -740,256 +740,432 @@ __global__ __launch_bounds__(2 * kProposeTile) void k_propose(const ProposeArgs 
 
 // ----------------------------------------------------------- fused inference, many clusters --
 // k_propose keeps all K softmax numerators of a quad in LDS, which has room for K <= 256. For
-// larger K (a multiple of 128, at most 4096) the output layer streams through LDS in column
-// blocks of kSuper = 128 clusters, three times over the same H3 rows:
-//   1. the row maxima of the logits;
-//   2. the numerators e = fp16(exp(z - max)) and their row sum se, accumulated as in k_propose:
-//      blocks of 32 numerators summed in order, block sums added to se in cluster order;
-//   3. the same numerators again: each of the lane's pending draws t = u * se selects the first
-//      block whose running sum exceeds t (the last block if rounding leaves none) and the first
-//      cluster in it whose running sum from the block's start exceeds t (the block's last if
-//      none), exactly k_propose's pick_cluster over all K / 32 blocks; every candidate picks
-//      up the numerator of its cluster, whether drawn from the MLP or the cluster of a light
-//      drawn from the source table.
-// Then each pixel's random stream is replayed to draw the lights and write (l, q) as k_propose
-// does, with the same draws in the same order. At most kWideCand candidates per pixel.
-constexpr int kERow = kSuper + 4;  // fp16 numerators per LDS row
+// larger K (a multiple of 128, at most 4096) the output layer streams through LDS in blocks of
+// 64 clusters, twice over the same hidden activations:
+//   1. the maximum of a quad's logits;
+//   2. the numerators e = fp16(exp(z - max)), written to global memory with the running sum after
+//      each 32 of them, accumulated as in k_propose: blocks of 32 numerators summed in order,
+//      block sums added in cluster order.
+// Then each pixel's draws t = u * se select the first block whose running sum exceeds t (the last
+// block if rounding leaves none) and the first cluster in it whose running sum from the block's
+// start exceeds t (the block's last if none), exactly k_propose's pick_cluster over all K / 32
+// blocks; every candidate picks up the numerator of its cluster, whether drawn from the MLP or the
+// cluster of a light drawn from the source table. At most kWideCand candidates per pixel.
+//
+// What bounds it: the matrix cores in the first pass, the exponentials and the 16-bit stores of the
+// second. Each wave holds 32 quads in the columns of its products (A = the weights' rows, B = the
+// activations): a lane then has 16 logits of one quad, its partner (lane ^ 32) the other 16, the
+// maximum stays in the lane, two blocks of 32 are exchanged between the partners' halves and
+// summed in order in registers, and a layer's output turns into the next layer's operand by the
+// same exchange. LDS holds nothing but two blocks of weights (the next one on its way in registers
+// while one is multiplied). Before, activations, logits and draws went through 69.6 KB of LDS, the
+// output layer ran a third time to meet the draws, and a lane's draws were searched block by block
+// while the other lanes waited. At 1280x720, M = 8: K = 4,096 3.16 -> 1.13 ms, of which the maximum's
+// pass takes 0.33 ms, the stores 0.25 and the draws 0.2. Two workgroups on a CU (245 registers, none
+// spilled): three are 11% slower, four spill and are slower yet.
+//
+// The numerators and sums (272 * K bytes a workgroup) live in one of `nSlots` slots. There are at
+// most as many workgroups as slots, each taking every gridDim-th tile of quads. A workgroup takes a
+// free slot when it starts and gives it back when it ends, so launches on any number of streams
+// share them; where they run short, the later workgroups wait for running ones to end.
+constexpr int kWideQuads = 128;                 // pixel quads per workgroup: 32 per wave
+constexpr int kWideRows = 64;                   // clusters per staged weight block
+constexpr int kWideTile = kWideRows * kRow;     // bf16 elements of a staged block
+constexpr int kWideResident = 2;                // workgroups on a CU: a wave of each per SIMD
+// bytes of a slot: K fp16 numerators and K / 32 running sums for each quad
+__host__ __device__ constexpr size_t wide_slot_bytes(int K) {
+    return static_cast<size_t>(kWideQuads) * (2 * static_cast<size_t>(K) + static_cast<size_t>(K) / 32 * 4);
+}
+static_assert(wide_slot_bytes(kMaxClusters) == 272u * kMaxClusters, "the slot size named above");
+static_assert(kMaxClusters / kSuper * kWideQuads * 4 <= 2 * kWideTile * 2, "a sum per 128 clusters fits the weight buffers");
 
-__device__ __forceinline__ void super_block_sums(const uint2 *row, float (&bs)[kSuper / 32]) {
-#pragma unroll
-    for (int b = 0; b < kSuper / 32; ++b) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const float4 f = unpack_h4(row[8 * b + q]);
-            sum += f.x;
-            sum += f.y;
-            sum += f.z;
-            sum += f.w;
-        }
-        bs[b] = sum;
-    }
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// lanes 32..63 of x change places with lanes 0..31 of y
+__device__ __forceinline__ void swap_halves(uint32_t &x, uint32_t &y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = r[0];
+    y = r[1];
+}
+__device__ __forceinline__ void swap_halves(float &x, float &y) {
+    uint32_t a = __float_as_uint(x), b = __float_as_uint(y);
+    swap_halves(a, b);
+    x = __uint_as_float(a);
+    y = __uint_as_float(b);
 }
 
-__global__ __launch_bounds__(2 * kTilePx) void k_propose_wide(const ProposeArgs a) {
-    __shared__ __align__(16) uint16_t lds[2 * kTilePx * kRow];
-    static_assert(kTilePx * kERow <= kTilePx * kRow, "a column block's numerators fit the weight buffer");
-    static_assert(kTilePx % 32 == 0, "32 quads per wave in the MFMA layers, two lanes per quad");
-    uint16_t *act = lds;
-    uint16_t *wbuf = lds + kTilePx * kRow;
-    __half *etile = reinterpret_cast<__half *>(wbuf);
+// a barrier for LDS alone: __syncthreads would also wait for the global stores under way
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// 64 outputs of a layer for the wave's 32 quads: rows of staged weights times the activations, on
+// top of the bias. The first half's weights are all read before its products and the second's while
+// they run: a read takes as long as four products, and left to itself the compiler puts each read
+// right before its product.
+__device__ __forceinline__ void wide_blocks(const uint16_t *w, const float *bias, const bf16x8 (&h)[kIn / 16], int lane,
+                                            f32x16 &z0, f32x16 &z1) {
+    constexpr int kSteps = kIn / 16;
+    auto start = [&](f32x16 &z, const float *b) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const float4 v = *reinterpret_cast<const float4 *>(b + 8 * g + 4 * (lane >> 5));
+            z[4 * g] = v.x;
+            z[4 * g + 1] = v.y;
+            z[4 * g + 2] = v.z;
+            z[4 * g + 3] = v.w;
+        }
+    };
+    const uint16_t *at = w + (lane & 31) * kRow + 8 * (lane >> 5);
+    bf16x8 f0[kSteps], f1[kSteps];
+    start(z0, bias);
+    start(z1, bias + 32);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) f0[s] = *reinterpret_cast<const bf16x8 *>(at + 16 * s);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+        z0 = mfma32(f0[s], h[s], z0);
+        f1[s] = *reinterpret_cast<const bf16x8 *>(at + 32 * kRow + 16 * s);
+    }
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) z1 = mfma32(f1[s], h[s], z1);
+    __builtin_amdgcn_sched_group_barrier(0x100, 8 + kSteps, 0);  // LDS reads: both biases, the first half
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    // a product
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
+    }
+    __builtin_amdgcn_sched_group_barrier(0x8, kSteps, 0);
+}
+
+__global__ __launch_bounds__(2 * kWideQuads, kWideResident) void k_propose_wide(const ProposeArgs a) {
+    __shared__ __align__(16) uint16_t lds[2 * kWideTile];
+    __shared__ __align__(16) float bias[2 * kWideRows];
+    __shared__ uint32_t slotShared;
+    static_assert(kWideQuads * kRow <= 2 * kWideTile && kHidden == 2 * kWideRows, "features and hidden layers fit the weight buffers");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t W = a.f.g.W, H = a.f.g.H, QW = (W + 1) / 2, QH = (H + 1) / 2;
-    const uint32_t q0 = blockIdx.x * kTilePx;
-    const int nSuper = a.K / kSuper;
     const uint16_t *w4 = a.wbf + w_off(3);
     const float *b4 = a.bias + b_off(3);
-    propose_hidden<kTilePx>(a, act, wbuf, q0, QW, QH, kSuper);
 
-    // 1. row maxima: each lane covers 16 rows x 4 columns of every block, then the 32 lanes
-    // sharing a row reduce
-    float rmax[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) rmax[i] = -INFINITY;
-    for (int sb = 0; sb < nSuper; ++sb) {
-        if (sb > 0) {
-            stage_weights(wbuf, w4 + static_cast<size_t>(sb) * kSuper * kIn, kSuper);
-            __syncthreads();
+    if (wave == 0) {  // a slot; an acquire: nothing that an earlier workgroup left of it is read
+        const uint32_t chunks = (a.nSlots + 63) / 64;
+        uint32_t c = blockIdx.x / 64 % chunks, slot = 0;
+        for (bool taken = false; !taken; c = c + 1 < chunks ? c + 1 : 0) {
+            const uint32_t i = 64 * c + lane;
+            uint32_t busy = 1;
+            if (i < a.nSlots) busy = __hip_atomic_load(a.slotBusy + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint64_t open = __ballot(busy == 0);
+            while (open && !taken) {
+                // workgroups start their search at different slots
+                const uint64_t later = open >> (blockIdx.x & 63) << (blockIdx.x & 63);
+                const int pick = __ffsll(static_cast<unsigned long long>(later ? later : open)) - 1;
+                uint32_t was = 1;
+                if (lane == pick) was = atomicExch(a.slotBusy + i, 1u);
+                taken = __shfl(was, pick) == 0;
+                slot = 64 * c + pick;
+                open &= ~(1ull << pick);
+            }
         }
-        f32x16 acc[4];
-        layer_mfma<4>(act, wbuf, b4 + sb * kSuper, wave, lane, acc);
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) rmax[i] = fmaxf(rmax[i], acc[nb][i]);
+        if (lane == 0) slotShared = slot;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
+    __syncthreads();
+    const uint32_t slot = slotShared;
+    const uint32_t tiles = (QW * QH + kWideQuads - 1) / kWideQuads;
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint32_t q0 = tile * kWideQuads;
+    // the quads' features, a lane each, by way of LDS into the B operand of the first layer
+    if (tid < kWideQuads) {
+        const uint32_t qd = q0 + tid;
+        uint16_t *row = lds + tid * kRow;
+        if (qd < QW * QH) pixel_features(a.f, quad_pixel(a.f.g, qd % QW, qd / QW), row);
+        else for (int k = 0; k < kIn; ++k) row[k] = 0;
+    }
+    __syncthreads();
+    bf16x8 h[kIn / 16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-#pragma unroll
-        for (int off = 16; off > 0; off >>= 1) rmax[i] = fmaxf(rmax[i], __shfl_xor(rmax[i], off));
+    for (int s = 0; s < kIn / 16; ++s)
+        h[s] = *reinterpret_cast<const bf16x8 *>(&lds[(32 * wave + (lane & 31)) * kRow + 16 * s + 8 * (lane >> 5)]);
 
-    // one column block's numerators into the LDS tile (which overlays the staged weights)
-    auto numerators = [&](int sb) {
-        stage_weights(wbuf, w4 + static_cast<size_t>(sb) * kSuper * kIn, kSuper);
+    // the hidden layers
+    for (int L = 0; L < 3; ++L) {
         __syncthreads();
-        f32x16 acc[4];
-        layer_mfma<4>(act, wbuf, b4 + sb * kSuper, wave, lane, acc);
+        stage_weights(lds, a.wbf + w_off(L), kHidden);
+        if (tid < kHidden) bias[tid] = a.bias[b_off(L) + tid];
         __syncthreads();
+        bf16x8 out[kIn / 16];
+        f32x16 z[2];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int row = 32 * wave + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+        for (int nb = 0; nb < kHidden / 32; ++nb) {
+            if (nb % 2 == 0) wide_blocks(lds + 32 * nb * kRow, bias + 32 * nb, h, lane, z[0], z[1]);
+            const f32x16 &acc = z[nb % 2];
+            uint32_t d[8];
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-                etile[row * kERow + 32 * nb + (lane & 31)] = __float2half(__expf(acc[nb][i] - rmax[i]));
+            for (int i = 0; i < 8; ++i) {
+                const float lo = acc[2 * i], hi = acc[2 * i + 1];
+                d[i] = f2bf2(lo > 0.0f ? lo : 0.0f, hi > 0.0f ? hi : 0.0f);
+            }
+            // outputs 8g + 4 * (lane / 32) + 0..3 lie in d[2g], d[2g + 1]; the operand wants
+            // 8 * (lane / 32) + 0..7 of each 16
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                swap_halves(d[4 * s], d[4 * s + 2]);
+                swap_halves(d[4 * s + 1], d[4 * s + 3]);
+                out[2 * nb + s] = __builtin_bit_cast(bf16x8, make_uint4(d[4 * s], d[4 * s + 1], d[4 * s + 2], d[4 * s + 3]));
+            }
         }
+#pragma unroll
+        for (int s = 0; s < kIn / 16; ++s) h[s] = out[s];
+    }
+    __syncthreads();
+
+    // the output layer, 64 clusters at a time: body(step, logits of the first 32, of the second)
+    auto sweep = [&](auto &&body) {
+        constexpr int kPer = kWideRows * kIn / 8 / (2 * kWideQuads);  // 16-byte pieces per lane
+        u32x4 next[kPer];
+        float nextBias = 0.0f;
+        auto fetch = [&](int step) {
+            const u32x4 *src = reinterpret_cast<const u32x4 *>(w4 + static_cast<size_t>(step) * kWideRows * kIn);
+#pragma unroll
+            for (int e = 0; e < kPer; ++e) next[e] = src[e * 2 * kWideQuads + tid];
+            if (tid < kWideRows) nextBias = b4[step * kWideRows + tid];
+        };
+        auto put = [&](int buf) {
+#pragma unroll
+            for (int e = 0; e < kPer; ++e) {
+                const int at = e * 2 * kWideQuads + tid;
+                *reinterpret_cast<u32x4 *>(&lds[buf * kWideTile + at / (kIn / 8) * kRow + at % (kIn / 8) * 8]) = next[e];
+            }
+            if (tid < kWideRows) bias[buf * kWideRows + tid] = nextBias;
+        };
+        const int steps = a.K / kWideRows;
+        fetch(0);
+        put(0);
         __syncthreads();
+        for (int step = 0; step < steps; ++step) {
+            const int buf = step & 1;
+            if (step + 1 < steps) fetch(step + 1);
+            const uint16_t *w = lds + buf * kWideTile;
+            f32x16 z0, z1;
+            wide_blocks(w, bias + buf * kWideRows, h, lane, z0, z1);
+            body(step, z0, z1);
+            if (step + 1 < steps) put(buf ^ 1);  // read last before the barrier of the step before
+            lds_barrier();
+        }
     };
 
-    // lane pair per quad from here on, each lane drawing for one row of its 2x2 pixels
-    const uint32_t qd = q0 + (tid >> 1);
-    const bool quadOk = qd < QW * QH;
-    const uint32_t qx = quadOk ? qd % QW : 0, qy = quadOk ? qd / QW : 0;
-    const uint32_t py = 2 * qy + static_cast<uint32_t>(tid & 1);
-    const uint2 *erow = reinterpret_cast<const uint2 *>(etile + (tid >> 1) * kERow);
-    const __half *erowh = etile + (tid >> 1) * kERow;
+    // 1. the maximum
+    float zmax = -INFINITY;
+    sweep([&](int, const f32x16 &z0, const f32x16 &z1) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) zmax = fmaxf(zmax, fmaxf(z0[i], z1[i]));
+    });
+    zmax = fmaxf(zmax, __shfl_xor(zmax, 32));
 
-    // 2. the row sum
+    // 2. numerators and running sums. The wave's part of the slot: 16 bytes for each 8
+    // clusters of a quad, so placed that the 64 lanes store 1 KB without gaps (a draw then reads its
+    // block's 64 bytes in four places, but draws are few: 1.27 -> 1.24 ms, and 1.18 ms with stores
+    // that don't stay in the L2; with a block's 64 bytes together those took 2.70 ms); then four
+    // running sums per quad and 128 clusters.
+    const int quad = lane & 31;
+    uint8_t *part = a.slots + slot * wide_slot_bytes(a.K) + wave * (wide_slot_bytes(a.K) / 4);
+    u32x4 *num = reinterpret_cast<u32x4 *>(part);
+    float4 *sums = reinterpret_cast<float4 *>(part + static_cast<size_t>(64) * a.K);
+    auto piece = [&](int b, int g) { return static_cast<size_t>(b >> 1) * 256 + 64 * g + 32 * (b & 1) + quad; };
     float se = 0.0f;
-    for (int sb = 0; sb < nSuper; ++sb) {
-        numerators(sb);
-        float bs[kSuper / 32];
-        super_block_sums(erow, bs);
+    float4 four = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    sweep([&](int step, const f32x16 &z0, const f32x16 &z1) {
+        uint32_t p0[8], p1[8];
 #pragma unroll
-        for (int b = 0; b < kSuper / 32; ++b) se += bs[b];
-        __syncthreads();  // the next block's weights overwrite the tile
-    }
+        for (int i = 0; i < 8; ++i) {
+            const f32x2 e0 = {__expf(z0[2 * i] - zmax), __expf(z0[2 * i + 1] - zmax)};
+            const f32x2 e1 = {__expf(z1[2 * i] - zmax), __expf(z1[2 * i + 1] - zmax)};
+            p0[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e0, f16x2));
+            p1[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e1, f16x2));
+        }
+        // lanes 0..31 get all of the first block of their quad, lanes 32..63 all of the second
+        float s0 = 0.0f;
+        u32x4 *to = num + piece(2 * step, 0) + (lane & 32);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            swap_halves(p0[2 * g], p1[2 * g]);
+            swap_halves(p0[2 * g + 1], p1[2 * g + 1]);
+            const u32x4 v = {p0[2 * g], p0[2 * g + 1], p1[2 * g], p1[2 * g + 1]};
+            __builtin_nontemporal_store(v, to + 64 * g);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const f16x2 e = __builtin_bit_cast(f16x2, static_cast<uint32_t>(v[k]));
+                s0 += static_cast<float>(e[0]);
+                s0 += static_cast<float>(e[1]);
+            }
+        }
+        float s1 = s0;
+        swap_halves(s0, s1);
+        if ((step & 1) == 0) {
+            four.x = se + s0;
+            four.y = four.x + s1;
+            se = four.y;
+        } else {
+            four.z = se + s0;
+            four.w = four.z + s1;
+            se = four.w;
+            if (lane < 32) sums[(step >> 1) * 32 + quad] = four;
+        }
+    });
     const float rse = 1.0f / se;
+    // the wave's lanes read what its other lanes wrote; the sweep's last barrier freed the weights
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    const int nSuper = a.K / kSuper;
+    float *superSum = reinterpret_cast<float *>(lds) + 32 * wave + quad;
+    for (int sb = lane >> 5; sb < nSuper; sb += 2) superSum[sb * kWideQuads] = sums[sb * 32 + quad].w;
+    __syncthreads();
 
-    // the lane's candidates: slot k = s * kWideCand + j for pixel s of its row, candidate j.
-    // MLP draws carry their target t; source draws the cluster of the drawn light.
+    // 3. the draws: lane l for row l / 32 of its quad's pixels
+    const __half *numh = reinterpret_cast<const __half *>(part);
+    auto numerator_at = [&](int c) { return numh[piece(c >> 5, (c >> 3) & 3) * 8 + (c & 7)]; };
+    const uint32_t qd = q0 + 32 * wave + quad;
     const int M = static_cast<int>(a.M);
-    const FeatArgs &f = a.f;
-    uint32_t pix[2];
-    bool pixOk[2];
+    if (qd < QW * QH) {
+        const uint32_t qx = qd % QW, py = 2 * (qd / QW) + static_cast<uint32_t>(lane >> 5);
+        for (uint32_t px = 2 * qx; px < 2 * qx + 2; ++px) {
+            if (px >= W || py >= H) continue;
+            const uint32_t p = py * W + px;
+            const f3 n = rk::load_normal(a.f.g, p);
+            if (rt::dot(n, n) == 0.0f) continue;  // background: Pass A draws no candidates there
+            rt::Pcg rng = rt::pcg_seed(a.seed, p);
+            // Each step does all candidates at once, without branches where a load must not wait for
+            // another candidate's: one that needs no cluster (a source candidate, one beyond M)
+            // searches for t = 0.
+            float t[kWideCand], r1[kWideCand], r2[kWideCand];
+            int32_t ck[kWideCand], l[kWideCand];  // the cluster; a source candidate's light, else -1
+            float pw[kWideCand], ps[kWideCand], ek[kWideCand];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const uint32_t px = 2 * qx + s;
-        pix[s] = py * W + px;
-        pixOk[s] = false;
-        if (quadOk && px < W && py < H) {
-            const uint32_t p = pix[s];
-            const f3 n = rk::load_normal(f.g, p);
-            pixOk[s] = rt::dot(n, n) != 0.0f;  // background: Pass A draws no candidates there
-        }
-    }
-    float tk[2 * kWideCand], ek[2 * kWideCand];
-    int32_t ck[2 * kWideCand];
-    uint32_t pend = 0u;  // MLP draws whose cluster is not found yet
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        rt::Pcg rng = rt::pcg_seed(a.seed, pix[s]);
-#pragma unroll
-        for (int j = 0; j < kWideCand; ++j) {
-            const int k = s * kWideCand + j;
-            tk[k] = 0.0f;
-            ek[k] = 0.0f;
-            ck[k] = -1;
-            if (!pixOk[s] || j >= M) continue;
-            const bool src = rt::pcg_float(rng) < a.mix;
-            if (!src) {
-                tk[k] = rt::pcg_float(rng) * se;
-                ck[k] = a.K - 1;
-                pend |= 1u << k;
-            }
-            const float r1 = rt::pcg_float(rng), r2 = rt::pcg_float(rng);
-            if (src) {
-                int32_t c = static_cast<int32_t>(static_cast<float>(a.nAlias) * r1);
-                c = c < a.nAlias - 1 ? c : a.nAlias - 1;
-                const float4 t4 = a.alias[c];
-                const int32_t l = t4.x > r2 ? c : __float_as_int(t4.y);
-                ck[k] = a.lightCluster[l];
-            }
-        }
-    }
-
-    // 3. find the drawn clusters and pick up every candidate's numerator
-    float cum = 0.0f;
-    for (int sb = 0; sb < nSuper; ++sb) {
-        numerators(sb);
-        float bs[kSuper / 32];
-        super_block_sums(erow, bs);
-        float nx[kSuper / 32];
-        float c2 = cum;
-#pragma unroll
-        for (int b = 0; b < kSuper / 32; ++b) {
-            c2 += bs[b];
-            nx[b] = c2;
-        }
-        const bool last = sb == nSuper - 1;
-        const int c0 = sb * kSuper;
-#pragma unroll
-        for (int k = 0; k < 2 * kWideCand; ++k) {
-            if (pend & (1u << k)) {
-                if (tk[k] < nx[kSuper / 32 - 1] || last) {
-                    int blk = kSuper / 32 - 1;
-                    float base = nx[kSuper / 32 - 2];
-                    bool found = false;
-#pragma unroll
-                    for (int b = 0; b < kSuper / 32; ++b) {
-                        if (!found && (tk[k] < nx[b] || b == kSuper / 32 - 1)) {
-                            blk = b;
-                            base = b == 0 ? cum : nx[b - 1];
-                            found = true;
-                        }
-                    }
-                    int c = 32 * blk + 31;
-                    float run = base;
-                    bool hit = false;
-                    for (int q = 0; q < 8 && !hit; ++q) {
-                        const float4 e4 = unpack_h4(erow[8 * blk + q]);
-                        const float ev[4] = {e4.x, e4.y, e4.z, e4.w};
-#pragma unroll
-                        for (int kk = 0; kk < 4; ++kk) {
-                            run += ev[kk];
-                            if (!hit && tk[k] < run) {
-                                c = 32 * blk + 4 * q + kk;
-                                hit = true;
-                            }
-                        }
-                    }
-                    ck[k] = c0 + c;
-                    ek[k] = __half2float(erowh[c]);
-                    pend &= ~(1u << k);
-                }
-            } else if (ck[k] >= c0 && ck[k] < c0 + kSuper) {
-                ek[k] = __half2float(erowh[ck[k] - c0]);
-            }
-        }
-        cum = nx[kSuper / 32 - 1];
-        __syncthreads();
-    }
-
-    // replay each pixel's stream: the lights and their q, as k_propose draws them
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        if (!pixOk[s]) continue;
-        const uint32_t p = pix[s];
-        rt::Pcg rng = rt::pcg_seed(a.seed, p);
-#pragma unroll
-        for (int j = 0; j < kWideCand; ++j) {
-            if (j >= M) continue;
-            const int k = s * kWideCand + j;
-            const bool src = rt::pcg_float(rng) < a.mix;
-            if (!src) (void)rt::pcg_float(rng);
-            const float r1 = rt::pcg_float(rng), r2 = rt::pcg_float(rng);
-            int32_t l = -1;
-            float pw = 0.0f, ps = 0.0f;
-            if (src) {
-                int32_t c = static_cast<int32_t>(static_cast<float>(a.nAlias) * r1);
-                c = c < a.nAlias - 1 ? c : a.nAlias - 1;
-                const float4 t4 = a.alias[c];
-                const bool keep = t4.x > r2;
-                l = keep ? c : __float_as_int(t4.y);
-                ps = keep ? t4.z : t4.w;
-                pw = a.lightPWithin[l];
-            } else {
-                const int32_t cnt = a.clusterCount[ck[k]], beg = a.clusterBegin[ck[k]];
-                if (cnt > 0) {
-                    int32_t c = static_cast<int32_t>(static_cast<float>(cnt) * r1);
-                    c = c < cnt - 1 ? c : cnt - 1;
-                    const float4 t4 = a.clusterAlias[beg + c];
-                    const bool keep = t4.x > r2;
-                    l = a.clusterLights[beg + (keep ? c : __float_as_int(t4.y))];
-                    pw = keep ? t4.z : t4.w;
-                    ps = a.alias[l].z;
+            for (int j = 0; j < kWideCand; ++j) {
+                t[j] = r1[j] = r2[j] = pw[j] = ps[j] = 0.0f;
+                l[j] = -1;
+                if (j >= M) continue;
+                const bool src = rt::pcg_float(rng) < a.mix;
+                if (!src) t[j] = rt::pcg_float(rng) * se;
+                r1[j] = rt::pcg_float(rng);
+                r2[j] = rt::pcg_float(rng);
+                if (src) {
+                    const int32_t c = static_cast<int32_t>(static_cast<float>(a.nAlias) * r1[j]);
+                    l[j] = c < a.nAlias - 1 ? c : a.nAlias - 1;
                 }
             }
-            const float q = l >= 0 ? (1.0f - a.mix) * (ek[k] * rse) * pw + a.mix * ps : 0.0f;
-            a.candLight[static_cast<size_t>(j) * a.npx + p] = l;
-            a.candQ[static_cast<size_t>(j) * a.npx + p] = q;
+            float4 four[kWideCand];
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j)
+                if (l[j] >= 0) four[j] = a.alias[l[j]];
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                if (l[j] < 0) continue;
+                const bool keep = four[j].x > r2[j];
+                l[j] = keep ? l[j] : __float_as_int(four[j].y);
+                ps[j] = keep ? four[j].z : four[j].w;
+            }
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                ck[j] = -1;
+                if (l[j] < 0) continue;
+                ck[j] = a.lightCluster[l[j]];
+                pw[j] = a.lightPWithin[l[j]];
+            }
+            // the number of running sums, but the last, that t does not lie below: they never fall,
+            // so bisection finds it
+            int at[kWideCand];
+            float base[kWideCand];
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                int sb = 0;
+#pragma unroll
+                for (int w = kMaxClusters / kSuper / 2; w > 0; w >>= 1) {
+                    const int next = sb + w < nSuper ? sb + w : nSuper;  // nSuper: past the last but one
+                    const float sum = superSum[(next - 1) * kWideQuads];
+                    if (next < nSuper && !(t[j] < sum)) sb = next;
+                }
+                at[j] = sb;
+                base[j] = sb > 0 ? superSum[(sb > 0 ? sb - 1 : 0) * kWideQuads] : 0.0f;
+                four[j] = sums[sb * 32 + quad];
+            }
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                const bool past0 = !(t[j] < four[j].x), past1 = past0 && !(t[j] < four[j].y), past2 = past1 && !(t[j] < four[j].z);
+                base[j] = past2 ? four[j].z : past1 ? four[j].y : past0 ? four[j].x : base[j];
+                at[j] = at[j] * (kSuper / 32) + (past0 ? 1 : 0) + (past1 ? 1 : 0) + (past2 ? 1 : 0);
+            }
+#pragma unroll
+            for (int j0 = 0; j0 < kWideCand; j0 += 4) {
+                u32x4 raw[4][4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) raw[j][g] = num[piece(at[j0 + j], g)];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float run = base[j0 + j];
+                    int below = 0;
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const f16x2 e = __builtin_bit_cast(f16x2, static_cast<uint32_t>(raw[j][g][k]));
+                            run += static_cast<float>(e[0]);
+                            below += !(t[j0 + j] < run);
+                            run += static_cast<float>(e[1]);
+                            below += !(t[j0 + j] < run);
+                        }
+                    if (ck[j0 + j] < 0) ck[j0 + j] = 32 * at[j0 + j] + (below < 31 ? below : 31);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) ek[j] = __half2float(numerator_at(ck[j]));
+            // the light of a cluster's own alias table
+            int32_t cnt[kWideCand], beg[kWideCand];
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                cnt[j] = 0;
+                if (j >= M || l[j] >= 0) continue;
+                cnt[j] = a.clusterCount[ck[j]];
+                beg[j] = a.clusterBegin[ck[j]];
+            }
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                if (cnt[j] <= 0) continue;
+                const int32_t c = static_cast<int32_t>(static_cast<float>(cnt[j]) * r1[j]);
+                at[j] = c < cnt[j] - 1 ? c : cnt[j] - 1;
+                four[j] = a.clusterAlias[beg[j] + at[j]];
+            }
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                if (cnt[j] <= 0) continue;
+                const bool keep = four[j].x > r2[j];
+                l[j] = a.clusterLights[beg[j] + (keep ? at[j] : __float_as_int(four[j].y))];
+                pw[j] = keep ? four[j].z : four[j].w;
+            }
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j)
+                if (cnt[j] > 0) ps[j] = a.alias[l[j]].z;
+#pragma unroll
+            for (int j = 0; j < kWideCand; ++j) {
+                if (j >= M) continue;
+                const float q = l[j] >= 0 ? (1.0f - a.mix) * (ek[j] * rse) * pw[j] + a.mix * ps[j] : 0.0f;
+                a.candLight[static_cast<size_t>(j) * a.npx + p] = l[j];
+                a.candQ[static_cast<size_t>(j) * a.npx + p] = q;
+            }
         }
     }
+    __syncthreads();  // the next tile's features overwrite the sums
+    }  // tiles
+    __syncthreads();
+    // a release: all writes to the slot are in memory before another workgroup may take it
+    if (tid == 0) __hip_atomic_store(a.slotBusy + slot, 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace rm
@@ -1268,11 +1444,15 @@ hipError_t mlp_adam(restir_mlp &m, const float *gw, const float *gb, const uint3
     return hipGetLastError();
 }
 
+size_t wide_slot_bytes(uint32_t K) { return rm::wide_slot_bytes(static_cast<int>(K)); }
+uint32_t wide_slots(uint32_t cus) { return rm::kWideResident * cus; }
+
 hipError_t mlp_propose(const restir_mlp &m, const GView &g, f3 cam, const float lo[3], const float hi[3],
                        const SceneView &sc, const int32_t *lightCluster, const float *lightPWithin,
                        const int32_t *clusterBegin, const int32_t *clusterCount, const int32_t *clusterLights,
                        const restir_alias_table_column *clusterAlias, const float4 *clusterFused, uint32_t M,
-                       float mix, uint32_t seed, int32_t *candLight, float *candQ, hipStream_t s) {
+                       float mix, uint32_t seed, const WideSlots &slots, int32_t *candLight, float *candQ,
+                       hipStream_t s) {
     rm::ProposeArgs a{};
     a.f = rm::FeatArgs{g, cam, {lo[0], lo[1], lo[2]}, {hi[0], hi[1], hi[2]}};
     a.wbf = m.weights_bf16;
@@ -1295,7 +1475,11 @@ hipError_t mlp_propose(const restir_mlp &m, const GView &g, f3 cam, const float 
     a.candQ = candQ;
     const uint32_t quads = ((g.W + 1) / 2) * ((g.H + 1) / 2);
     const dim3 grid((quads + rm::kProposeTile - 1) / rm::kProposeTile), block(2 * rm::kProposeTile);
-    const dim3 gridW((quads + rm::kTilePx - 1) / rm::kTilePx), blockW(2 * rm::kTilePx);
+    const uint32_t tilesW = (quads + rm::kWideQuads - 1) / rm::kWideQuads;
+    const dim3 gridW(tilesW < slots.n ? tilesW : slots.n), blockW(2 * rm::kWideQuads);
+    a.slots = static_cast<uint8_t *>(slots.base);
+    a.slotBusy = slots.busy;
+    a.nSlots = slots.n;
     switch (a.K) {
         case 64: RK_LAUNCH("k_propose", (rm::k_propose<64>), grid, block, 0, s, a); break;
         case 128: RK_LAUNCH("k_propose", (rm::k_propose<128>), grid, block, 0, s, a); break;
