@@ -156,6 +156,30 @@ int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, vo
     return RESTIR_OK;
 }
 
+// The memory for Pass A's light records over sc's tables, or null where they would not pay or
+// cannot be had (the device is out of memory; a captured stream, when they would have to grow).
+void *light_records(restir_ctx *ctx, const rk::SceneView &sc, const restir_uniforms &u, hipStream_t s) {
+    if (!rk::light_records_pay(sc, u.screenSize[0] * u.screenSize[1], u.initialLightSampleCount)) return nullptr;
+    const size_t bytes = rk::light_record_bytes(sc);
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        if (bytes > ctx->recordBytes) return nullptr;
+        ctx->recordsInGraph = true;
+        return ctx->records;
+    }
+    if (bytes > ctx->recordBytes && ctx->recordsInGraph) {  // a graph may replay launches over the old ones
+        ctx->retired.push_back(ctx->records);
+        ctx->records = nullptr;
+        ctx->recordBytes = 0;
+        ctx->recordsInGraph = false;
+    }
+    if (ensure(ctx, &ctx->records, &ctx->recordBytes, bytes) == RESTIR_OK) return ctx->records;
+    (void)hipGetLastError();
+    ctx->error.clear();
+    return nullptr;
+}
+
 int pick_tile(restir_ctx *ctx, const restir_launch *l, int *tile) {
     if (!l || (l->tile_x == 0 && l->tile_y == 0)) {
         *tile = 0;
@@ -354,9 +378,10 @@ int restir_initial_temporal(restir_ctx *ctx, const restir_uniforms *u, const res
     if (int r = pick_tile(ctx, launch, &tile)) return r;
     void *queues = nullptr;
     if (int r = pass_a_queues(ctx, launch, W * H, &queues)) return r;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    void *records = queues ? light_records(ctx, ctx->scene, *u, s) : nullptr;
     const hipError_t e = rk::launch_pass_a(tile, ctx->stack, *u, ctx->scene, view_of(cur), view_of(prev),
-                                           prevRes, out, nullptr, nullptr, queues, ctx->persistentBlocks,
-                                           static_cast<hipStream_t>(stream));
+                                           prevRes, out, nullptr, nullptr, queues, ctx->persistentBlocks, s, records);
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "initial_temporal launch");
 }
 

@@ -130,7 +130,8 @@ int restir_initial_temporal_views(restir_ctx *ctx, const restir_view *views, uin
             const int st = views[v].scene->stack;
             const hipError_t e = rk::launch_pass_a(tile, st, w.u, own_counters(ctx, w.sc), w.cur, w.prev, w.prevRes,
                                                    w.out, nullptr, nullptr, ctx->scratch,
-                                                   persistent_blocks(ctx->cus, st), s);
+                                                   persistent_blocks(ctx->cus, st), s,
+                                                   light_records(ctx, w.sc, w.u, s));
             if (e != hipSuccess) return hip_fail(ctx, e, "initial_temporal_views launch");
         }
         return RESTIR_OK;

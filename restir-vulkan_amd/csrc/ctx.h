@@ -38,7 +38,7 @@ struct restir_ctx {
     void *scratch = nullptr;       // ray queues of the queued Pass C schedule
     size_t scratchBytes = 0;
     bool scratchInGraph = false;   // a stream capture recorded multi-view launches that use it
-    std::vector<void *> retired;   // earlier scratches and slots that captured graphs still use
+    std::vector<void *> retired;   // earlier scratches, slots and records that captured graphs still use
     uint32_t queuedNpx = 0;        // shape of the last queued Pass C (its rays stay in scratch)
     const restir_reservoir *queuedOut = nullptr;  // its output (the light end of its neighbour rays)
     int queuedK = 0;
@@ -66,6 +66,9 @@ struct restir_ctx {
     size_t aliasScratchBytes = 0;
     void *wide = nullptr;          // the bound tree's 4-entry nodes (+ the nesting flag)
     size_t wideBytes = 0;
+    void *records = nullptr;       // Pass A's light records (k_light_records)
+    size_t recordBytes = 0;
+    bool recordsInGraph = false;   // a stream capture recorded launches that use them
     // light clusters of the learned proposal (device pointers, caller-owned)
     bool clustersSet = false;
     int32_t nClusters = 0;
@@ -95,6 +98,7 @@ struct restir_ctx {
         if (wide) (void)hipFree(wide);
         if (clusterFused) (void)hipFree(clusterFused);
         if (slots) (void)hipFree(slots);
+        if (records) (void)hipFree(records);
     }
 };
 
@@ -112,6 +116,7 @@ int pick_tile(restir_ctx *ctx, const restir_launch *l, int *tile);
 int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, void **queues);
 int ensure(restir_ctx *ctx, void **buf, size_t *have, size_t bytes);
 int ensure_scratch(restir_ctx *ctx, size_t bytes);
+void *light_records(restir_ctx *ctx, const rk::SceneView &sc, const restir_uniforms &u, hipStream_t s);
 uint32_t resident_blocks(uint32_t cus, uint32_t ldsBytes);
 uint32_t persistent_blocks(uint32_t cus, int stack);
 int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *tris, uint32_t depth, hipStream_t s);

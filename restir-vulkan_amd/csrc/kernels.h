@@ -95,10 +95,15 @@ constexpr uint32_t kTraceListEntries = 64 + 4 * 64;
 constexpr uint32_t kTraceExtraLds = 4u * kTraceListEntries * 5u + 256u * 4u;
 constexpr uint32_t kTrace8Lds = rt::kW8Stack * 1024u + 4u * 128u * 5u + 2u * 256u * 4u;  // the 8-entry tracer's workgroup
 constexpr uint32_t kTrace8PerCu = 5;  // its 92 VGPRs allow 5 waves per SIMD (its LDS 6 workgroups)
+// Columns of 64 bytes for k_light_records, and whether a queued Pass A over npx pixels with M
+// candidates each is worth building them
+size_t light_record_bytes(const SceneView &sc);
+bool light_records_pay(const SceneView &sc, uint32_t npx, uint32_t M);
 hipError_t launch_pass_a(int tile, int stack, const restir_uniforms &u, const SceneView &sc,
                          const GView &cur, const GView &prev, const restir_reservoir *prevRes,
                          restir_reservoir *out, const int32_t *candLight, const float *candQ,
-                         void *queueScratch, uint32_t gridCap, hipStream_t s);
+                         void *queueScratch, uint32_t gridCap, hipStream_t s,
+                         void *records = nullptr);
 size_t pass_a_queue_bytes(uint32_t npx);
 hipError_t launch_pass_b(int tile, const restir_uniforms &u, int iter, float cosThr,
                          const GView &g, const restir_reservoir *in, restir_reservoir *out,

@@ -119,6 +119,7 @@ struct PassAArgs {
     // reference's alias-table candidates
     const int32_t *candLight;
     const float *candQ;
+    const float4 *records;  // k_light_records of the alias table, or null
 };
 
 // Pass A in pieces (restirOmni.glsl:86-212), shared by the inline kernel and the queued schedule.
@@ -194,7 +195,28 @@ __device__ __forceinline__ int32_t alias_column(const SceneView &sc, float r1) {
     return col < sc.nAlias - 1 ? col : sc.nAlias - 1;
 }
 
+// A column of the alias table; with RECORDS its light's and its alias's point-light data too, which
+// k_light_records put next to it: `records` holds 64 bytes per column.
+template <bool RECORDS>
+struct AliasColumn {
+    float4 c, own, other;
+};
+template <bool RECORDS>
+__device__ __forceinline__ AliasColumn<RECORDS> load_column(const SceneView &sc, const float4 *records, int32_t col) {
+    AliasColumn<RECORDS> k;
+    if constexpr (RECORDS) {
+        const float4 *r = records + 4 * static_cast<size_t>(col);
+        k.c = r[0];
+        k.own = r[1];
+        k.other = r[2];
+    } else {
+        k.c = sc.alias[col];
+    }
+    return k;
+}
+
 // Initial RIS over M candidates (alias table or the learned proposal's list).
+template <bool RECORDS>
 __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurface &ps, Res &res, Pcg &rng) {
     const uint32_t W = a.u.screenSize[0], H = a.u.screenSize[1];
     const size_t idx = ps.idx;
@@ -205,7 +227,7 @@ __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurfac
     const SceneView &sc = a.sc;
     const bool standard = (a.u.flags & RESTIR_STANDARD_WEIGHTS_FLAG) != 0;
     const uint32_t M = a.u.initialLightSampleCount;
-    if (dot(n, n) != 0.0f && a.candLight) {
+    if (!RECORDS && dot(n, n) != 0.0f && a.candLight) {
         // RIS over the learned proposal's candidates: weight p_hat / q with the proposal's own
         // density q; a candidate from an empty cluster (l < 0) has weight 0 but still counts in M.
         // Candidates index the lights the alias table indexes (the union: point lights first).
@@ -247,37 +269,40 @@ __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurfac
             bool tri;
             float4 point;  // a point light's record
         };
-        const auto resolve = [&](int32_t col, float4 cv, float r2) {
+        const auto resolve = [&](int32_t col, const AliasColumn<RECORDS> &cv, float r2) {
             Cand k;
             int32_t li;
-            if (cv.x > r2) {
+            if (cv.c.x > r2) {
                 li = col;
-                k.prob = cv.z;
+                k.prob = cv.c.z;
             } else {
-                li = __float_as_int(cv.y);
-                k.prob = cv.w;
+                li = __float_as_int(cv.c.y);
+                k.prob = cv.c.w;
             }
             k.tri = sc.mixed ? li >= sc.nPoints : sc.nPoints == 0;
             k.li = sc.mixed && k.tri ? li - sc.nPoints : li;
-            k.point = k.tri ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : point_light(sc, k.li);
+            if constexpr (RECORDS)
+                k.point = cv.c.x > r2 ? cv.own : cv.other;  // zeros for a triangle light
+            else
+                k.point = k.tri ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : point_light(sc, k.li);
             return k;
         };
         uint64_t st = rng.state;  // candidate i's first state
         int32_t col = alias_column(sc, pcg_float_at(st));
-        Cand cur = resolve(col, sc.alias[col], pcg_float_at(st * kPcgMul + inc));
+        Cand cur = resolve(col, load_column<RECORDS>(sc, a.records, col), pcg_float_at(st * kPcgMul + inc));
         uint64_t stN = after(st, cur.tri);  // candidate i + 1's first state
         int32_t colN = alias_column(sc, pcg_float_at(stN));
-        float4 cN = sc.alias[colN];  // candidate i + 1's column
+        AliasColumn<RECORDS> cN = load_column<RECORDS>(sc, a.records, colN);  // candidate i + 1's column
         for (uint32_t i = 0; i < M; ++i) {
             Cand nxt = cur;
             uint64_t stNN = stN;
             int32_t colNN = colN;
-            float4 cNN = cN;
+            AliasColumn<RECORDS> cNN = cN;
             if (i + 1 < M) {
                 nxt = resolve(colN, cN, pcg_float_at(stN * kPcgMul + inc));
                 stNN = after(stN, nxt.tri);
                 colNN = alias_column(sc, pcg_float_at(stNN));
-                cNN = sc.alias[colNN];
+                cNN = load_column<RECORDS>(sc, a.records, colNN);
             }
             const uint64_t s2 = st * pcg_mul_pow(2) + inc * pcg_mul_sum(2), s3 = s2 * kPcgMul + inc;
             float ra = 0.0f, rb = 0.0f, u;
@@ -353,7 +378,7 @@ __device__ __forceinline__ void pass_a_px(const PassAArgs &a, uint32_t x, uint32
     const SceneView &sc = a.sc;
     Res res;
     Pcg rng = pass_a_rng(a, x, y);
-    pass_a_ris(a, ps, res, rng);
+    pass_a_ris<false>(a, ps, res, rng);
     // Visibility reuse, restirOmni.glsl:148-160. A reservoir with sumWeights == 0 already has
     // w == 0 and is unchanged by a shadow hit, so its ray is skipped.
     if ((a.u.flags & RESTIR_VISIBILITY_REUSE_FLAG) && res.sumW != 0.0f) {
@@ -1236,7 +1261,25 @@ struct AQueues {
     uint32_t *occ;      // per pixel: kBitCentreShadowed once its ray hit
 };
 
-template <int TX, int TY>
+// The alias table's columns with the point lights that each can draw: a candidate then reads one
+// 64-byte record instead of a column and a light somewhere else. Those dependent
+// reads, which miss the L1 and then the L2, bound the pass as soon as the tables outgrow them:
+// 1920x1080, M = 32, 12,000 lights 0.63 -> 0.54 ms, 3840x2160, 1M lights 8.70 -> 4.19 ms. An alias
+// that names no point light gets zeros, as a triangle light does: a column that never draws it may
+// hold anything there.
+__global__ __launch_bounds__(256) void k_light_records(const SceneView sc, float4 *records) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= static_cast<uint32_t>(sc.nAlias)) return;
+    const float4 c = sc.alias[i];
+    const int32_t other = __float_as_int(c.y);
+    float4 *r = records + 4 * static_cast<size_t>(i);
+    r[0] = c;
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    r[1] = static_cast<int32_t>(i) < sc.nPoints ? point_light(sc, static_cast<int32_t>(i)) : zero;
+    r[2] = other >= 0 && other < sc.nPoints ? point_light(sc, other) : zero;
+}
+
+template <int TX, int TY, bool RECORDS>
 __global__ __launch_bounds__(TX *TY) void k_pass_a_ris(const PassAArgs a, const AQueues q) {
     uint32_t x, y;
     tile_pixel<TX, TY>(a.tilesX, a.nTiles, x, y);
@@ -1250,7 +1293,7 @@ __global__ __launch_bounds__(TX *TY) void k_pass_a_ris(const PassAArgs a, const 
         pos = ps.pos;
         Res res;
         Pcg rng = pass_a_rng(a, x, y);
-        pass_a_ris(a, ps, res, rng);
+        pass_a_ris<RECORDS>(a, ps, res, rng);
         store_res(a.out, idx, res);
         q.rng[idx] = rng.state;
         q.occ[idx] = 0u;
@@ -1724,7 +1767,13 @@ static hipError_t run_a_queued(PassAArgs args, const AQueues &q, uint32_t gridCa
     grid_for<TX, TY>(args.u.screenSize[0], args.u.screenSize[1], args.tilesX, args.nTiles);
     const dim3 tiles(args.nTiles), block(TX * TY);
     RK_LAUNCH("k_zero_counters", k_zero_counters, dim3(1), dim3(64), 0, s, q.counter, 2u, args.sc.traceHeads);
-    RK_LAUNCH("k_pass_a_ris", (k_pass_a_ris<TX, TY>), tiles, block, 0, s, args, q);
+    if (args.records) {
+        RK_LAUNCH("k_light_records", k_light_records, dim3((args.sc.nAlias + 255) / 256), dim3(256), 0, s, args.sc,
+                  const_cast<float4 *>(args.records));
+        RK_LAUNCH("k_pass_a_ris", (k_pass_a_ris<TX, TY, true>), tiles, block, 0, s, args, q);
+    } else {
+        RK_LAUNCH("k_pass_a_ris", (k_pass_a_ris<TX, TY, false>), tiles, block, 0, s, args, q);
+    }
     if (args.u.flags & RESTIR_VISIBILITY_REUSE_FLAG) {
         CQueues cq{};
         cq.bits = q.occ;  // a shadowed ray sets kBitCentreShadowed in occ[pixel]
@@ -1746,11 +1795,26 @@ static hipError_t dispatch_a_queued(int tile, const PassAArgs &args, const AQueu
     }
 }
 
+size_t light_record_bytes(const SceneView &sc) { return 64 * static_cast<size_t>(sc.nAlias); }
+// Where the records pay. k_pass_a_ris without and with them, M = 32 at 1920x1080 unless said:
+//   lights              1,500: 383 -> 383 us (+ 4 for the records)   2,000: 440 -> 387
+//                       10,000: 595 -> 390   100,000: 804 -> 715   1,000,000: 2,163 -> 1,098 (+ 55)
+//   most are triangles  500 + 5,000 triangle lights: 763 -> 869      10,000 + 2,000: 633 -> 544
+//   few candidates      256x256, M = 32: 36 -> 36   640x360, M = 32, 3,000 lights: 73 -> 61
+// So: tables (48 bytes a light) well beyond a CU's 32 KB L1, three quarters of them point lights, and
+// enough candidates to win back the records' launch (4 us) and, beyond it, 55 us per million lights.
+bool light_records_pay(const SceneView &sc, uint32_t npx, uint32_t M) {
+    const uint64_t n = static_cast<uint64_t>(sc.nAlias);
+    return n >= 2048 && 4 * static_cast<uint64_t>(sc.nPoints) >= 3 * n &&
+           static_cast<uint64_t>(npx) * M >= (4u << 20) + 3 * n;
+}
+
 hipError_t launch_pass_a(int tile, int stack, const restir_uniforms &u, const SceneView &sc,
                          const GView &cur, const GView &prev, const restir_reservoir *prevRes,
                          restir_reservoir *out, const int32_t *candLight, const float *candQ,
-                         void *queueScratch, uint32_t gridCap, hipStream_t s) {
-    PassAArgs args{u, sc, cur, prev, prevRes, out, 0, 0, candLight, candQ};
+                         void *queueScratch, uint32_t gridCap, hipStream_t s, void *records) {
+    PassAArgs args{u, sc, cur, prev, prevRes, out, 0, 0, candLight, candQ,
+                   queueScratch && !candLight ? static_cast<const float4 *>(records) : nullptr};
     if (queueScratch) {
         const AQueues q = carve_a_queues(queueScratch, u.screenSize[0] * u.screenSize[1]);
         return by_stack(stack, [&](auto S) {
