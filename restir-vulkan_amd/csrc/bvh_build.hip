@@ -3,16 +3,24 @@
 // launches.
 //
 // The reference pops index ranges of one primitive-order array from a FIFO, so node ids are
-// breadth-first and each tree level is a list of disjoint ranges in position order. One round
-// handles a whole level:
-//   classify + scan    ranges of >= 2 primitives take the next node ids (breadth-first order),
-//                      ranges of >= 3 are split; 1- and 2-primitive ranges become leaves
-//   bounds             centroid and box bounds of each split range
+// breadth-first and each tree level is a list of disjoint ranges in position order. Ranges of more
+// than kSub primitives are split level by level, one round of launches for all of a level:
+//   level              ranks the ranges to split; smaller ones go to the subtree list
+//   bounds             centroid and box bounds of each range (and of its halves)
 //   bin                bucket of each primitive on the range's longest centroid axis; box and
 //                      count per bucket
-//   choose             the reference's SAH sweep over the 12 buckets, one lane per range
+//   choose             the reference's SAH sweep over the 12 buckets, 16 lanes per range
 //   partition          the reference's swap partition, reproduced exactly (below)
-// and the host reads back only the level's node and split counts.
+// and the host reads back only the number of ranges to split. Each smaller range then becomes a
+// whole subtree in one workgroup's LDS (k_bvh_subtrees). A split at position mid makes node mid - 1
+// of a temporary array: every inner position is split at once, and position order is the order of a
+// level's nodes, so the breadth-first ids are a stable sort of that array by level.
+//
+// Where the time goes: a level costs its launches (about 5 us each) and its readback, whatever its
+// size, and the lower half of a tree's levels holds ranges of a few primitives. 136,000 triangles
+// (23 levels): 3.2 ms with every level split that way, in 20 launches each; 1.15 ms with the last 12
+// to 13 levels in k_bvh_subtrees (0.22 ms) and 8 launches for each of the others. 1,200 triangles
+// 1.52 -> 0.47 ms, 2.3 million 18.6 -> 6.6 ms (all with the traversal's nodes, bind_tree).
 //
 // Exact min/max. nv_min(a, b) = a < b ? a : b (nvmath.inl:2414-2420) folded in primitive order
 // returns, among equal values, the LAST one; equal floats differ in bits only as +0/-0. Each fold
@@ -45,28 +53,41 @@ using namespace rki;
 namespace {
 
 constexpr int kBuckets = 12;
-constexpr int kBoundWords = 12;                 // centroid lo/hi, box lo/hi keys
+constexpr int kBoundWords = 24;                 // centroid lo/hi, box lo/hi keys; the halves' box lo/hi
 constexpr int kBinWords = 7;                    // box lo/hi keys + count
 constexpr int kAcc = kBoundWords + kBuckets * kBinWords;  // 64-bit words per split range
 constexpr int kSlots = 4;  // split ranges a 256-lane group pre-reduces in LDS
+// Primitives of a range that one workgroup finishes. 136,000 triangles (2.3 million): with 256 1.21
+// (6.94) ms, with 512 1.25 (6.61), with 1024 1.25 (7.12): longer subtrees against more levels.
+constexpr uint32_t kSub = 512;
+constexpr uint32_t kSubWide = 32;  // and those from which on its 16 lanes fold parts of them, not components
+constexpr uint32_t kScanGroup = rscan::kItems;  // positions per block of the partition's prefix sums
 
 struct Seg {  // a range of the level; link = parent node * 2 + side, -1 for the root
     uint32_t first, last;
     int32_t link, pad;
 };
-struct Split {  // a range of >= 3 primitives being split at this level
-    uint32_t id, first, last, mid;
+struct Split {  // a range being split at this level
+    uint32_t first, last, mid;
     uint32_t bucket;      // last bucket of the left side
     uint32_t degenerate;  // the sweep put everything on one side: halved instead
+    int32_t link;
     uint32_t pad[2];
+};
+struct Sub {  // a range of 2..kSub primitives, its level and link
+    uint32_t first, last;
+    int32_t link;
+    uint32_t level;
 };
 struct Params {
     int32_t axis;
     float lo, width, parentArea;
 };
 struct Info {
-    unsigned long long totals;  // node count (low 32 bits) and split count (high 32 bits)
-    uint32_t bad;               // a vertex coordinate is not finite
+    uint32_t splits;  // ranges to split at this level
+    uint32_t subs;    // ranges in the subtree list
+    uint32_t bad;     // a vertex coordinate is not finite
+    uint32_t depth;   // deepest level of a node
 };
 
 using u64 = unsigned long long;
@@ -85,7 +106,8 @@ __device__ inline u64 key_min(float v, uint32_t p) { return (static_cast<u64>(co
 __device__ inline u64 key_max(float v, uint32_t p) { return (static_cast<u64>(code(v)) << 32) | p; }
 
 // word layout of a split range's accumulator: [0,3) centroid lo, [3,6) centroid hi, [6,9) box
-// lo, [9,12) box hi; then per bucket b at 12 + 7b: [0,3) box lo, [3,6) box hi, [6] count
+// lo, [9,12) box hi, [12,18) box lo, hi of the positions before (first + last) / 2, [18,24) of the
+// others; then per bucket b at 24 + 7b: [0,3) box lo, [3,6) box hi, [6] count
 __host__ __device__ inline bool is_min_word(int w) { return w < kBoundWords ? ((w / 3) & 1) == 0 : ((w - kBoundWords) % kBinWords) < 3; }
 __host__ __device__ inline bool is_count_word(int w) { return w >= kBoundWords && (w - kBoundWords) % kBinWords == 6; }
 __device__ inline u64 word_init(int w) { return (!is_count_word(w) && is_min_word(w)) ? ~0ull : 0ull; }
@@ -115,26 +137,97 @@ __device__ inline float half_area(const float lo[3], const float hi[3]) {  // su
     return sx * sy + sx * sz + sy * sz;
 }
 
+// Bucket axis and placement of a range (aabbTreeBuilder.cpp:95-121) from its bounds.
+__device__ inline Params make_params(const float cLo[3], const float cHi[3], const float bLo[3], const float bHi[3]) {
+    Params q;
+    q.parentArea = half_area(bLo, bHi);
+    float extent[3];
+    for (int k = 0; k < 3; ++k) extent[k] = cHi[k] - cLo[k];
+    int axis = extent[0] > extent[1] ? 0 : 1;
+    if ((axis == 0 ? extent[0] : extent[1]) < extent[2]) axis = 2;
+    q.axis = axis;
+    q.lo = axis == 0 ? cLo[0] : axis == 1 ? cLo[1] : cLo[2];
+    q.width = (axis == 0 ? extent[0] : axis == 1 ? extent[1] : extent[2]) / static_cast<float>(kBuckets);
+    return q;
+}
+__device__ inline uint32_t bucket_of(const Params &q, float c) {
+    float f = (c - q.lo) / q.width;
+    f = f < 0.5f ? 0.5f : f;  // nv_clamp(f, 0.5, numBuckets - 0.5)
+    f = f > static_cast<float>(kBuckets) - 0.5f ? static_cast<float>(kBuckets) - 0.5f : f;
+    // coincident centroids give 0/0 (undefined in the reference): bucket 0
+    return f == f ? static_cast<uint32_t>(f) : 0u;
+}
+
+// Lane i of a row of 16 gets v of lane i - D (shr) or i + D (shl), `none` where the row ends.
+template <int D>
+__device__ inline float row_shr(float none, float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(none), __float_as_int(v), 0x110 + D, 0xf, 0xf, false));
+}
+template <int D>
+__device__ inline float row_shl(float none, float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(none), __float_as_int(v), 0x100 + D, 0xf, 0xf, false));
+}
 struct Bin {  // Bucket (aabbTreeBuilder.cpp:33-50)
     float lo[3], hi[3];
-    u64 count;
+    uint32_t count;
 };
-__device__ inline void bin_empty(Bin &b) {
-    for (int k = 0; k < 3; ++k) {
-        b.lo[k] = FLT_MAX;
-        b.hi[k] = -FLT_MAX;
-    }
-    b.count = 0;
-}
-__device__ inline Bin bin_merged(Bin a, const Bin &b) {
-    a.count += b.count;
-    for (int k = 0; k < 3; ++k) {
-        a.lo[k] = nv_min(a.lo[k], b.lo[k]);
-        a.hi[k] = nv_max(a.hi[k], b.hi[k]);
-    }
-    return a;
+__device__ inline Bin bin_empty() {
+    return Bin{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}, 0u};
 }
 __device__ inline float bin_cost(const Bin &b) { return static_cast<float>(b.count) * half_area(b.lo, b.hi); }
+// One step of a row's ordered prefix (suffix) fold. The folds keep the last of equal values, so
+// folding blocks of buckets in their order gives what folding the buckets one by one gives.
+template <int D>
+__device__ inline void fold_left(Bin &b) {
+    for (int k = 0; k < 3; ++k) {
+        b.lo[k] = nv_min(row_shr<D>(FLT_MAX, b.lo[k]), b.lo[k]);
+        b.hi[k] = nv_max(row_shr<D>(-FLT_MAX, b.hi[k]), b.hi[k]);
+    }
+    b.count += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b.count), 0x110 + D, 0xf, 0xf, false));
+}
+template <int D>
+__device__ inline void fold_right(Bin &b) {
+    for (int k = 0; k < 3; ++k) {
+        b.lo[k] = nv_min(row_shl<D>(FLT_MAX, b.lo[k]), b.lo[k]);
+        b.hi[k] = nv_max(row_shl<D>(-FLT_MAX, b.hi[k]), b.hi[k]);
+    }
+    b.count += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b.count), 0x100 + D, 0xf, 0xf, false));
+}
+// The SAH sweep (aabbTreeBuilder.cpp:131-175) by a row of 16 lanes, lane b holding bucket b (empty
+// beyond the last): left and right end as the two sides of a split after bucket b, and the result is
+// the first cheapest split, or -1 where no cost is a number below FLT_MAX.
+__device__ inline int sah_sweep(Bin &left, Bin &right, float parentArea) {
+    const int b = threadIdx.x & 15;
+    fold_left<1>(left);
+    fold_left<2>(left);
+    fold_left<4>(left);
+    fold_left<8>(left);
+    fold_right<1>(right);
+    fold_right<2>(right);
+    fold_right<4>(right);
+    fold_right<8>(right);
+    for (int k = 0; k < 3; ++k) {
+        right.lo[k] = row_shl<1>(FLT_MAX, right.lo[k]);
+        right.hi[k] = row_shl<1>(-FLT_MAX, right.hi[k]);
+    }
+    right.count = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(right.count), 0x101, 0xf, 0xf, false));
+    float cost = 0.125f + (bin_cost(left) + bin_cost(right)) / parentArea;
+    int split = b;
+    if (!(b < kBuckets - 1 && cost < FLT_MAX)) {
+        cost = INFINITY;
+        split = 16;
+    }
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) {
+        const float c = __shfl_xor(cost, d);
+        const int o = __shfl_xor(split, d);
+        if (c < cost || (c == cost && o < split)) {
+            cost = c;
+            split = o;
+        }
+    }
+    return split < 16 ? split : -1;
+}
 
 __device__ inline void write_box(float *dst, const float *v) {  // vec4(vec3) sets w = 1
     dst[0] = v[0];
@@ -145,10 +238,14 @@ __device__ inline void write_box(float *dst, const float *v) {  // vec4(vec3) se
 
 // ---- kernels ----
 
-// triangles out (w = 1), primitive boxes (aabbForTriangle), the identity order, one root range
+// triangles out (w = 1), primitive boxes (aabbForTriangle), the identity order, one root range, its
+// accumulator
 __global__ __launch_bounds__(256) void k_bvh_prep(uint32_t n, const float *xyz, restir_triangle *tris,
-                                                  float4 *box, uint32_t *idx, int32_t *segOf, Info *info) {
+                                                  float4 *box, uint32_t *idx, int32_t *segOf, u64 *acc, Seg *root,
+                                                  Info *info) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < kAcc) acc[i] = word_init(static_cast<int>(i));
+    if (i == 0) *root = Seg{0u, n, -1, 0};
     if (i >= n) return;
     float v[9];
     bool finite = true;
@@ -180,65 +277,49 @@ __global__ __launch_bounds__(256) void k_bvh_prep(uint32_t n, const float *xyz, 
     segOf[i] = 0;
 }
 
-__global__ __launch_bounds__(256) void k_bvh_classify(uint32_t S, const Seg *segs, u64 *flags) {
-    const uint32_t s = blockIdx.x * 256u + threadIdx.x;
-    if (s >= S) return;
-    const uint32_t len = segs[s].last - segs[s].first;
-    flags[s] = static_cast<u64>(len >= 2) | (static_cast<u64>(len >= 3) << 32);
+__device__ inline void set_child(restir_aabb_tree_node *tmp, int32_t link, int32_t value) {
+    if (link < 0) return;
+    restir_aabb_tree_node &parent = tmp[link >> 1];
+    if (link & 1) parent.rightChild = value;
+    else parent.leftChild = value;
 }
 
-// node ids, links from the parents, leaf pairs, the split list
-__global__ __launch_bounds__(256) void k_bvh_setup(uint32_t S, const Seg *segs, const u64 *scan, uint32_t nodeBase,
-                                                   const uint32_t *idx, const float4 *box, restir_aabb_tree_node *nodes,
-                                                   Split *splits) {
-    const uint32_t s = blockIdx.x * 256u + threadIdx.x;
-    if (s >= S) return;
-    const Seg g = segs[s];
-    const uint32_t len = g.last - g.first;
-    const uint32_t id = nodeBase + static_cast<uint32_t>(scan[s]);
-    const int32_t value = len == 1 ? ~static_cast<int32_t>(idx[g.first]) : static_cast<int32_t>(id);
-    if (g.link >= 0) {
-        restir_aabb_tree_node &parent = nodes[g.link >> 1];
-        if (g.link & 1) parent.rightChild = value;
-        else parent.leftChild = value;
+// One workgroup: the level's ranges in order. Those to split get consecutive ranks, ranges of one
+// primitive become leaves, the others go to the subtree list.
+__global__ __launch_bounds__(256) void k_bvh_level(uint32_t S, uint32_t level, const Seg *segs, const uint32_t *idx,
+                                                   restir_aabb_tree_node *tmp, int32_t *segRank, Split *splits, Sub *subs,
+                                                   Info *info) {
+    __shared__ uint32_t waveCount[4];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t base = 0;
+    for (uint32_t s0 = 0; s0 < S; s0 += 256u) {
+        const uint32_t s = s0 + threadIdx.x;
+        Seg g{};
+        if (s < S) g = segs[s];
+        const uint32_t len = g.last - g.first;
+        const bool big = len > kSub;
+        const uint64_t m = __ballot(big);
+        if (lane == 0) waveCount[wave] = static_cast<uint32_t>(__popcll(m));
+        __syncthreads();
+        uint32_t r = base + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
+        for (uint32_t w = 0; w < 4; ++w) {
+            if (w < wave) r += waveCount[w];
+            base += waveCount[w];
+        }
+        __syncthreads();
+        if (s >= S) continue;
+        segRank[s] = big ? static_cast<int32_t>(r) : -1;
+        if (big) splits[r] = Split{g.first, g.last, 0u, 0u, 0u, g.link, {0u, 0u}};
+        else if (len == 1) set_child(tmp, g.link, ~static_cast<int32_t>(idx[g.first]));
+        else subs[atomicAdd(&info->subs, 1u)] = Sub{g.first, g.last, g.link, level};
     }
-    if (len == 2) {
-        const uint32_t a = idx[g.first], b = idx[g.first + 1];
-        restir_aabb_tree_node node;
-        const float4 alo = box[2 * a], ahi = box[2 * a + 1], blo = box[2 * b], bhi = box[2 * b + 1];
-        const float la[3] = {alo.x, alo.y, alo.z}, ha[3] = {ahi.x, ahi.y, ahi.z};
-        const float lb[3] = {blo.x, blo.y, blo.z}, hb[3] = {bhi.x, bhi.y, bhi.z};
-        write_box(node.leftAabbMin, la);
-        write_box(node.leftAabbMax, ha);
-        write_box(node.rightAabbMin, lb);
-        write_box(node.rightAabbMax, hb);
-        node.leftChild = ~static_cast<int32_t>(a);
-        node.rightChild = ~static_cast<int32_t>(b);
-        node._pad[0] = node._pad[1] = 0;
-        nodes[id] = node;
-    } else if (len >= 3) {
-        Split sp{};
-        sp.id = id;
-        sp.first = g.first;
-        sp.last = g.last;
-        splits[scan[s] >> 32] = sp;
-    }
+    if (threadIdx.x == 0) info->splits = base;
 }
 
-__global__ __launch_bounds__(256) void k_bvh_init_acc(uint32_t words, u64 *acc) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i < words) acc[i] = word_init(static_cast<int>(i % kAcc));
-}
-
-// rank of the split range holding each position (-1: a finished or 1-2 primitive range)
-__global__ __launch_bounds__(256) void k_bvh_rank(uint32_t n, const int32_t *segOf, const Seg *segs, const u64 *scan,
-                                                  int32_t *rank) {
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-    if (p >= n) return;
-    const int32_t s = segOf[p];
-    int32_t r = -1;
-    if (s >= 0 && segs[s].last - segs[s].first >= 3) r = static_cast<int32_t>(scan[s] >> 32);
-    rank[p] = r;
+// rank of the split range holding position p (-1: a range that is not split any more)
+__device__ inline int rank_of(uint32_t p, uint32_t n, const int32_t *segOf, const int32_t *segRank) {
+    const int32_t s = p < n ? segOf[p] : -1;
+    return s >= 0 ? segRank[s] : -1;
 }
 
 // Adds `nw` keys (words w0.. of range r's accumulator) through LDS when r is one of the first
@@ -289,31 +370,74 @@ __device__ inline void group_flush(const u64 *sh, int r0, int base, u64 *acc) {
     }
 }
 
-__global__ __launch_bounds__(256) void k_bvh_bounds(uint32_t n, const uint32_t *idx, const int32_t *rank, const float4 *box,
-                                                    u64 *acc) {
+// The extreme of v over a wave's lanes (the same on every lane), and from it the key of the last
+// lane that holds it: lanes hold consecutive positions, p0 is lane 0's.
+template <bool MIN>
+__device__ inline u64 wave_key(float v, bool active, uint32_t p0) {
+    const float none = MIN ? INFINITY : -INFINITY;
+    const float mine = active ? v : none;
+    float x = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const float o = __shfl_xor(x, d);
+        x = MIN ? (o < x ? o : x) : (o > x ? o : x);
+    }
+    const uint64_t at = __ballot(active && mine == x);
+    const uint32_t p = p0 + 63u - static_cast<uint32_t>(__clzll(static_cast<long long>(at)));
+    return MIN ? key_min(x, p) : key_max(x, p);
+}
+
+__global__ __launch_bounds__(256) void k_bvh_bounds(uint32_t n, const uint32_t *idx, const int32_t *segOf,
+                                                    const int32_t *segRank, const Split *splits, const float4 *box, u64 *acc) {
     __shared__ u64 sh[kSlots * kBoundWords];
     __shared__ int shR;
     const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-    const int r = p < n ? rank[p] : -1;
+    const int r = rank_of(p, n, segOf, segRank);
     if (threadIdx.x < kSlots * kBoundWords) sh[threadIdx.x] = word_init(threadIdx.x % kBoundWords);
     const int r0 = group_min_rank(r, &shR);
+    float v[kBoundWords / 2] = {};
+    bool lower = false;
     if (r >= 0) {
         const uint32_t t = idx[p];
         const float4 lo = box[2 * t], hi = box[2 * t + 1];
-        const float cx = 0.5f * (lo.x + hi.x), cy = 0.5f * (lo.y + hi.y), cz = 0.5f * (lo.z + hi.z);
-        const u64 keys[kBoundWords] = {key_min(cx, p),   key_min(cy, p),   key_min(cz, p),   key_max(cx, p),
-                                       key_max(cy, p),   key_max(cz, p),   key_min(lo.x, p), key_min(lo.y, p),
-                                       key_min(lo.z, p), key_max(hi.x, p), key_max(hi.y, p), key_max(hi.z, p)};
+        v[0] = v[3] = 0.5f * (lo.x + hi.x);
+        v[1] = v[4] = 0.5f * (lo.y + hi.y);
+        v[2] = v[5] = 0.5f * (lo.z + hi.z);
+        v[6] = lo.x, v[7] = lo.y, v[8] = lo.z;
+        v[9] = hi.x, v[10] = hi.y, v[11] = hi.z;
+        lower = p < static_cast<uint32_t>((static_cast<uint64_t>(splits[r].first) + splits[r].last) / 2);
+    }
+    // A wave inside one range and one half of it reduces its keys in registers; LDS atomics of all
+    // lanes on the same words would be served one lane at a time.
+    const uint64_t in = __ballot(r >= 0);
+    if (in) {
+        const int lead = __ffsll(static_cast<unsigned long long>(in)) - 1;
+        const int rr = __shfl(r, lead), side = __shfl(lower ? 0 : 1, lead);
+        const bool same = __ballot(r >= 0 && (r != rr || (lower ? 0 : 1) != side)) == 0;
         GroupAcc<kBoundWords> g{sh, r0, 0};
-        g.add(acc, r, 0, keys, kBoundWords);
+        if (same) {
+            const uint32_t lane = threadIdx.x & 63u;
+            u64 mine = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < 12; ++w) {
+                const u64 k = ((w / 3) & 1) == 0 ? wave_key<true>(v[w], r >= 0, p - lane) : wave_key<false>(v[w], r >= 0, p - lane);
+                // words 6..11 are also the half's
+                if (lane == w || (w >= 6 && lane == w + 6)) mine = k;
+            }
+            if (lane < 18) g.add(acc, rr, static_cast<int>(lane) + (lane >= 12 ? 6 * side : 0), &mine, 1);
+        } else if (r >= 0) {
+            u64 keys[12];
+#pragma unroll
+            for (int w = 0; w < 12; ++w) keys[w] = ((w / 3) & 1) == 0 ? key_min(v[w], p) : key_max(v[w], p);
+            g.add(acc, r, 0, keys, 12);
+            g.add(acc, r, lower ? 12 : 18, keys + 6, 6);
+        }
     }
     group_flush<kBoundWords>(sh, r0, 0, acc);
 }
 
-__global__ __launch_bounds__(256) void k_bvh_params(uint32_t nSplits, const uint32_t *idx, const float4 *box,
-                                                    const u64 *acc, Params *par) {
-    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
-    if (r >= nSplits) return;
+// the bounds of range r as k_bvh_bounds left them
+__device__ inline Params params_of(int r, const uint32_t *idx, const float4 *box, const u64 *acc) {
     const u64 *a = acc + static_cast<size_t>(r) * kAcc;
     float cLo[3], cHi[3], bLo[3], bHi[3];
     for (int k = 0; k < 3; ++k) {
@@ -322,37 +446,24 @@ __global__ __launch_bounds__(256) void k_bvh_params(uint32_t nSplits, const uint
         bLo[k] = decode(a[6 + k], true, idx, box, 1, k);
         bHi[k] = decode(a[9 + k], false, idx, box, 2, k);
     }
-    Params q;
-    q.parentArea = half_area(bLo, bHi);
-    float extent[3];
-    for (int k = 0; k < 3; ++k) extent[k] = cHi[k] - cLo[k];
-    int axis = extent[0] > extent[1] ? 0 : 1;
-    if (extent[2] > extent[axis]) axis = 2;
-    q.axis = axis;
-    q.lo = cLo[axis];
-    q.width = extent[axis] / static_cast<float>(kBuckets);
-    par[r] = q;
+    return make_params(cLo, cHi, bLo, bHi);
 }
 
-__global__ __launch_bounds__(256) void k_bvh_bin(uint32_t n, const uint32_t *idx, const int32_t *rank, const float4 *box,
-                                                 const Params *par, uint8_t *bucket, u64 *acc) {
+__global__ __launch_bounds__(256) void k_bvh_bin(uint32_t n, const uint32_t *idx, const int32_t *segOf,
+                                                 const int32_t *segRank, const float4 *box, uint8_t *bucket, u64 *acc) {
     constexpr int NW = kBuckets * kBinWords;
     __shared__ u64 sh[kSlots * NW];
     __shared__ int shR;
     const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-    const int r = p < n ? rank[p] : -1;
+    const int r = rank_of(p, n, segOf, segRank);
     for (int i = threadIdx.x; i < kSlots * NW; i += 256) sh[i] = word_init(kBoundWords + i % NW);
     const int r0 = group_min_rank(r, &shR);
     if (r >= 0) {
-        const Params q = par[r];
+        const Params q = params_of(r, idx, box, acc);
         const uint32_t t = idx[p];
         const float4 lo = box[2 * t], hi = box[2 * t + 1];
         const float c = q.axis == 0 ? 0.5f * (lo.x + hi.x) : (q.axis == 1 ? 0.5f * (lo.y + hi.y) : 0.5f * (lo.z + hi.z));
-        float f = (c - q.lo) / q.width;
-        f = f < 0.5f ? 0.5f : f;  // nv_clamp(f, 0.5, numBuckets - 0.5)
-        f = f > static_cast<float>(kBuckets) - 0.5f ? static_cast<float>(kBuckets) - 0.5f : f;
-        // coincident centroids give 0/0 (undefined in the reference): bucket 0
-        const uint32_t b = f == f ? static_cast<uint32_t>(f) : 0u;
+        const uint32_t b = bucket_of(q, c);
         bucket[p] = static_cast<uint8_t>(b);
         const u64 keys[kBinWords] = {key_min(lo.x, p), key_min(lo.y, p), key_min(lo.z, p), key_max(hi.x, p),
                                      key_max(hi.y, p), key_max(hi.z, p), 1ull};
@@ -362,144 +473,107 @@ __global__ __launch_bounds__(256) void k_bvh_bin(uint32_t n, const uint32_t *idx
     group_flush<NW>(sh, r0, kBoundWords, acc);
 }
 
-// the SAH sweep of one range (aabbTreeBuilder.cpp:131-175), the split point, the next level's
-// two ranges
-__global__ __launch_bounds__(256) void k_bvh_choose(uint32_t nSplits, const uint32_t *idx, const float4 *box,
-                                                    const Params *par, u64 *acc, Split *splits,
-                                                    restir_aabb_tree_node *nodes, Seg *next) {
-    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
+// the sweep of one range per 16 lanes, the split point, its node, the next level's two ranges
+__global__ __launch_bounds__(256) void k_bvh_choose(uint32_t nSplits, uint32_t level, const uint32_t *idx, const float4 *box,
+                                                    const u64 *acc, Split *splits, restir_aabb_tree_node *tmp, uint8_t *levels,
+                                                    Seg *next) {
+    const uint32_t r = blockIdx.x * 16u + (threadIdx.x >> 4);
     if (r >= nSplits) return;
-    u64 *a = acc + static_cast<size_t>(r) * kAcc;
-    Bin bins[kBuckets];
-#pragma unroll
-    for (int b = 0; b < kBuckets; ++b) {
-        const u64 *w = a + kBoundWords + b * kBinWords;
-        bin_empty(bins[b]);
-        bins[b].count = w[6];
-        if (w[6] == 0) continue;
-        for (int k = 0; k < 3; ++k) {  // the bucket's fold starts from the empty box
-            bins[b].lo[k] = nv_min(FLT_MAX, decode(w[k], true, idx, box, 1, k));
-            bins[b].hi[k] = nv_max(-FLT_MAX, decode(w[3 + k], false, idx, box, 2, k));
-        }
-    }
-    Bin right[kBuckets - 1];
-    {
-        Bin cur = bins[kBuckets - 1];
-#pragma unroll
-        for (int s = kBuckets - 1; s > 0;) {
-            right[--s] = cur;
-            cur = bin_merged(cur, bins[s]);
-        }
-    }
-    const float parentArea = par[r].parentArea;
-    uint32_t split = 0;
-    float lLo[3] = {0, 0, 0}, lHi[3] = {0, 0, 0}, rLo[3] = {0, 0, 0}, rHi[3] = {0, 0, 0};
-    {
-        float best = FLT_MAX;
-        Bin left;
-        bin_empty(left);
-#pragma unroll
-        for (int s = 0; s < kBuckets - 1; ++s) {
-            left = bin_merged(left, bins[s]);
-            const float cost = 0.125f + (bin_cost(left) + bin_cost(right[s])) / parentArea;
-            if (cost < best) {
-                best = cost;
-                split = static_cast<uint32_t>(s);
-                for (int k = 0; k < 3; ++k) {
-                    lLo[k] = left.lo[k];
-                    lHi[k] = left.hi[k];
-                    rLo[k] = right[s].lo[k];
-                    rHi[k] = right[s].hi[k];
-                }
-            }
-        }
-    }
-    Split sp = splits[r];
-    u64 nLeft = 0;
-    for (int b = 0; b < kBuckets; ++b)
-        if (static_cast<uint32_t>(b) <= split) nLeft += bins[b].count;
-    uint32_t mid = sp.first + static_cast<uint32_t>(nLeft);
-    const bool degenerate = mid == sp.first || mid == sp.last;
-    if (degenerate) {
-        mid = static_cast<uint32_t>((static_cast<uint64_t>(sp.first) + sp.last) / 2);
-        for (int w = 0; w < kBoundWords; ++w) a[w] = word_init(w);  // reused for the two halves' boxes
-    }
-    restir_aabb_tree_node &node = nodes[sp.id];
-    if (!degenerate) {
-        write_box(node.leftAabbMin, lLo);
-        write_box(node.leftAabbMax, lHi);
-        write_box(node.rightAabbMin, rLo);
-        write_box(node.rightAabbMax, rHi);
-    }
-    node._pad[0] = node._pad[1] = 0;
-    sp.mid = mid;
-    sp.bucket = split;
-    sp.degenerate = degenerate ? 1u : 0u;
-    splits[r] = sp;
-    next[2 * r] = Seg{sp.first, mid, static_cast<int32_t>(2 * sp.id), 0};
-    next[2 * r + 1] = Seg{mid, sp.last, static_cast<int32_t>(2 * sp.id + 1), 0};
-}
-
-// boxes of the two halves of a range the sweep could not split (aabbTreeBuilder.cpp:186-203)
-__global__ __launch_bounds__(256) void k_bvh_halves(uint32_t n, const uint32_t *idx, const int32_t *rank, const float4 *box,
-                                                    const Split *splits, u64 *acc) {
-    __shared__ u64 sh[kSlots * kBoundWords];
-    __shared__ int shR;
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-    int r = p < n ? rank[p] : -1;
-    if (r >= 0 && !splits[r].degenerate) r = -1;
-    if (threadIdx.x < kSlots * kBoundWords) sh[threadIdx.x] = word_init(threadIdx.x % kBoundWords);
-    const int r0 = group_min_rank(r, &shR);
-    if (r >= 0) {
-        const uint32_t t = idx[p];
-        const float4 lo = box[2 * t], hi = box[2 * t + 1];
-        const u64 keys[6] = {key_min(lo.x, p), key_min(lo.y, p), key_min(lo.z, p),
-                             key_max(hi.x, p), key_max(hi.y, p), key_max(hi.z, p)};
-        GroupAcc<kBoundWords> g{sh, r0, 0};
-        g.add(acc, r, p < splits[r].mid ? 0 : 6, keys, 6);
-    }
-    group_flush<kBoundWords>(sh, r0, 0, acc);
-}
-
-__global__ __launch_bounds__(256) void k_bvh_halves_write(uint32_t nSplits, const uint32_t *idx, const float4 *box,
-                                                          const Split *splits, const u64 *acc,
-                                                          restir_aabb_tree_node *nodes) {
-    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
-    if (r >= nSplits || !splits[r].degenerate) return;
+    const int b = threadIdx.x & 15, row = static_cast<int>(threadIdx.x & 48u);
     const u64 *a = acc + static_cast<size_t>(r) * kAcc;
-    float v[4][3];
-    for (int h = 0; h < 4; ++h)  // left lo, left hi, right lo, right hi
-        for (int k = 0; k < 3; ++k) v[h][k] = decode(a[3 * h + k], (h & 1) == 0, idx, box, (h & 1) ? 2 : 1, k);
-    restir_aabb_tree_node &node = nodes[splits[r].id];
-    write_box(node.leftAabbMin, v[0]);
-    write_box(node.leftAabbMax, v[1]);
-    write_box(node.rightAabbMin, v[2]);
-    write_box(node.rightAabbMax, v[3]);
+    Bin left = bin_empty();
+    if (b < kBuckets) {
+        const u64 *w = a + kBoundWords + b * kBinWords;
+        left.count = static_cast<uint32_t>(w[6]);
+        if (left.count != 0)
+            for (int k = 0; k < 3; ++k) {  // the bucket's fold starts from the empty box
+                left.lo[k] = nv_min(FLT_MAX, decode(w[k], true, idx, box, 1, k));
+                left.hi[k] = nv_max(-FLT_MAX, decode(w[3 + k], false, idx, box, 2, k));
+            }
+    }
+    Bin right = left;
+    const Params q = params_of(static_cast<int>(r), idx, box, acc);
+    const int best = sah_sweep(left, right, q.parentArea);
+    const int split = best < 0 ? 0 : best;
+    Split sp = splits[r];
+    uint32_t mid = sp.first + static_cast<uint32_t>(__shfl(static_cast<int>(left.count), row + split));
+    const bool degenerate = mid == sp.first || mid == sp.last;
+    if (degenerate) mid = static_cast<uint32_t>((static_cast<uint64_t>(sp.first) + sp.last) / 2);
+    const uint32_t t = mid - 1;
+    restir_aabb_tree_node &node = tmp[t];
+    if (b == split) {
+        if (degenerate) {
+            float v[4][3];
+            for (int h = 0; h < 4; ++h)  // left lo, left hi, right lo, right hi
+                for (int k = 0; k < 3; ++k) v[h][k] = decode(a[12 + 3 * h + k], (h & 1) == 0, idx, box, (h & 1) ? 2 : 1, k);
+            write_box(node.leftAabbMin, v[0]);
+            write_box(node.leftAabbMax, v[1]);
+            write_box(node.rightAabbMin, v[2]);
+            write_box(node.rightAabbMax, v[3]);
+        } else {
+            const float zero[3] = {0.0f, 0.0f, 0.0f};
+            write_box(node.leftAabbMin, best < 0 ? zero : left.lo);
+            write_box(node.leftAabbMax, best < 0 ? zero : left.hi);
+            write_box(node.rightAabbMin, best < 0 ? zero : right.lo);
+            write_box(node.rightAabbMax, best < 0 ? zero : right.hi);
+        }
+        node._pad[0] = node._pad[1] = 0;
+        levels[t] = static_cast<uint8_t>(level);
+        set_child(tmp, sp.link, static_cast<int32_t>(t));
+        sp.mid = mid;
+        sp.bucket = static_cast<uint32_t>(split);
+        sp.degenerate = degenerate ? 1u : 0u;
+        splits[r] = sp;
+        next[2 * r] = Seg{sp.first, mid, static_cast<int32_t>(2 * t), 0};
+        next[2 * r + 1] = Seg{mid, sp.last, static_cast<int32_t>(2 * t + 1), 0};
+    }
 }
 
 __device__ inline bool goes_left(const Split &sp, const uint8_t *bucket, uint32_t p) {
     return !sp.degenerate && bucket[p] <= sp.bucket;
 }
 
-__global__ __launch_bounds__(256) void k_bvh_left_flags(uint32_t n, const int32_t *rank, const Split *splits,
-                                                        const uint8_t *bucket, uint32_t *flag) {
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-    if (p >= n) return;
-    const int r = rank[p];
-    flag[p] = (r >= 0 && goes_left(splits[r], bucket, p)) ? 1u : 0u;
+// left primitives before each position in its block of kScanGroup positions, and the blocks' totals
+__global__ __launch_bounds__(256) void k_bvh_left_count(uint32_t n, const int32_t *segOf, const int32_t *segRank,
+                                                        const Split *splits, const uint8_t *bucket, uint32_t *before,
+                                                        uint32_t *sums) {
+    __shared__ uint32_t waveTotal[4];
+    const uint32_t base = blockIdx.x * kScanGroup + threadIdx.x * 4u;
+    uint32_t v[4], run = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const int r = rank_of(base + i, n, segOf, segRank);
+        v[i] = run;
+        if (r >= 0 && goes_left(splits[r], bucket, base + i)) ++run;
+    }
+    const uint32_t incl = rscan::wave_inclusive(run);
+    const uint32_t w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63u) == 63u) waveTotal[w] = incl;
+    __syncthreads();
+    uint32_t off = incl - run;
+    for (uint32_t k = 0; k < w; ++k) off += waveTotal[k];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i)
+        if (base + i < n) before[base + i] = off + v[i];
+    if (threadIdx.x == 255) sums[blockIdx.x] = off + run;
+}
+// the same over all positions, once `sums` holds the totals' exclusive prefix sums
+__device__ inline uint32_t left_before(const uint32_t *before, const uint32_t *sums, uint32_t p) {
+    return before[p] + sums[p / kScanGroup];
 }
 
 // ptr[p]: the position whose placement position p copies (itself when final)
-__global__ __launch_bounds__(256) void k_bvh_chain(uint32_t n, const int32_t *rank, const Split *splits,
-                                                   const uint8_t *bucket, const uint32_t *leftBefore, uint32_t *ptr) {
+__global__ __launch_bounds__(256) void k_bvh_chain(uint32_t n, const int32_t *segOf, const int32_t *segRank,
+                                                   const Split *splits, const uint8_t *bucket, const uint32_t *before,
+                                                   const uint32_t *sums, uint32_t *ptr) {
     const uint32_t p = blockIdx.x * 256u + threadIdx.x;
     if (p >= n) return;
-    const int r = rank[p];
+    const int r = rank_of(p, n, segOf, segRank);
     uint32_t q = p;
     if (r >= 0) {
         const Split sp = splits[r];
         if (goes_left(sp, bucket, p)) {
-            const uint32_t g = sp.first + (leftBefore[p] - leftBefore[sp.first]);
+            const uint32_t g = sp.first + (left_before(before, sums, p) - left_before(before, sums, sp.first));
             q = g < p ? g : p;
         }
     }
@@ -510,28 +584,18 @@ __global__ __launch_bounds__(256) void k_bvh_chain(uint32_t n, const int32_t *ra
 // ptr[p] always names a position further down p's chain, whatever the order in which the lanes' reads
 // and writes land, and the chain ends at a position that names itself. While a lane jumps, the lanes
 // whose positions it meets shorten the rest of its chain, so long chains take about log2 of their
-// length. (One launch per round, ceil(log2(longest range)) a level, took 214 launches and 0.54 ms
-// of a 136,000-triangle build; the whole build went from 3.25 to 2.76 ms.)
-__global__ __launch_bounds__(256) void k_bvh_jump(uint32_t n, volatile uint32_t *ptr) {
+// length. Each lane then places what its position holds in the level's new order, notes the
+// position's range at the next level, and clears the accumulators of that level's ranges.
+__global__ __launch_bounds__(256) void k_bvh_scatter(uint32_t n, uint32_t nSplits, const int32_t *segOf, const int32_t *segRank,
+                                                     const Split *splits, const uint8_t *bucket, const uint32_t *before,
+                                                     const uint32_t *sums, volatile uint32_t *ptr, const uint32_t *idx,
+                                                     uint32_t *idxOut, int32_t *segOut, u64 *acc) {
     const uint32_t p = blockIdx.x * 256u + threadIdx.x;
     if (p >= n) return;
-    uint32_t q = ptr[p];
-    for (;;) {
-        const uint32_t r = ptr[q];
-        if (r == q) break;
-        ptr[p] = r;
-        q = r;
-    }
-}
-
-// the level's new primitive order and each position's range at the next level
-__global__ __launch_bounds__(256) void k_bvh_scatter(uint32_t n, const int32_t *rank, const Split *splits,
-                                                     const uint8_t *bucket, const uint32_t *leftBefore,
-                                                     const uint32_t *src, const uint32_t *idx, uint32_t *idxOut,
-                                                     int32_t *segOut) {
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-    if (p >= n) return;
-    const int r = rank[p];
+    // fewer words than positions: a split range has more than kSub of them
+    static_assert(2 * kAcc < kSub, "a lane clears one word at most");
+    if (p < 2 * nSplits * kAcc) acc[p] = word_init(static_cast<int>(p % kAcc));
+    const int r = rank_of(p, n, segOf, segRank);
     if (r < 0) {
         idxOut[p] = idx[p];
         segOut[p] = -1;
@@ -544,14 +608,322 @@ __global__ __launch_bounds__(256) void k_bvh_scatter(uint32_t n, const int32_t *
         return;
     }
     if (goes_left(sp, bucket, p)) {
-        const uint32_t q = sp.first + (leftBefore[p] - leftBefore[sp.first]);
+        const uint32_t q = sp.first + (left_before(before, sums, p) - left_before(before, sums, sp.first));
         idxOut[q] = idx[p];
         segOut[q] = 2 * r;
     }
+    uint32_t q = ptr[p];
+    for (;;) {
+        const uint32_t f = ptr[q];
+        if (f == q) break;
+        ptr[p] = f;
+        q = f;
+    }
     if (p >= sp.mid) {
-        idxOut[p] = idx[src[p]];
+        idxOut[p] = idx[q];
         segOut[p] = 2 * r + 1;
     }
+}
+
+// A subtree of at most kSub primitives, level by level, in one workgroup: 16 lanes take a range at a
+// time. Bounds: a lane per component folds the primitives in order; bins: a lane per bucket; then the
+// sweep of k_bvh_choose and the partition, 16 positions at a time: the chains of a position lead to
+// earlier ones, which are resolved already. Everything is read and written in LDS but the nodes.
+// Only order within a fold matters, and each fold is one lane's. Bound by the chain of levels: a
+// 512-primitive range takes 512 steps of its first fold, its children half of that, and so on.
+struct SubQueue {
+    uint16_t first, last;
+    int32_t link;
+};
+// a node's four boxes as 16 words
+__device__ inline float *box_words(restir_aabb_tree_node &node) { return reinterpret_cast<float *>(&node); }
+// LDS accesses of a wave's lanes happen in program order; this keeps the compiler to it
+__device__ inline void row_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__global__ __launch_bounds__(256) void k_bvh_subtrees(const Sub *subs, const uint32_t *idx, const float4 *box,
+                                                      restir_aabb_tree_node *tmp, uint8_t *levels, Info *info) {
+    __shared__ float bx[kSub * 6];
+    __shared__ uint32_t prim[kSub];
+    __shared__ uint16_t order[2][kSub], ptr[kSub];
+    __shared__ uint8_t bucket[kSub];
+    __shared__ u64 bins[16][kBuckets * kBinWords];
+    __shared__ SubQueue queue[2][kSub / 2];
+    __shared__ uint32_t queued[2];
+    const Sub sub = subs[blockIdx.x];
+    const uint32_t n = sub.last - sub.first;
+    for (uint32_t i = threadIdx.x; i < n; i += 256u) {
+        const uint32_t t = idx[sub.first + i];
+        const float4 lo = box[2 * t], hi = box[2 * t + 1];
+        prim[i] = t;
+        order[0][i] = static_cast<uint16_t>(i);
+        bx[6 * i] = lo.x, bx[6 * i + 1] = lo.y, bx[6 * i + 2] = lo.z;
+        bx[6 * i + 3] = hi.x, bx[6 * i + 4] = hi.y, bx[6 * i + 5] = hi.z;
+    }
+    if (threadIdx.x == 0) {
+        queue[0][0] = SubQueue{0, static_cast<uint16_t>(n), sub.link};
+        queued[0] = 1;
+        queued[1] = 0;
+    }
+    __syncthreads();
+    const uint32_t L = threadIdx.x & 15u;
+    const int row = static_cast<int>(threadIdx.x & 48u);
+    uint32_t level = sub.level;
+    for (uint32_t cur = 0;; cur ^= 1u, ++level) {
+        const uint32_t count = queued[cur];
+        const uint16_t *ord = order[cur];
+        uint16_t *out = order[cur ^ 1u];
+        for (uint32_t i = threadIdx.x >> 4; i < count; i += 16u) {
+            const uint32_t f = queue[cur][i].first, l = queue[cur][i].last;
+            const int32_t link = queue[cur][i].link;
+            if (l - f == 2) {  // a pair of leaves
+                const uint32_t a = ord[f], b = ord[f + 1], t = sub.first + f;
+                restir_aabb_tree_node &node = tmp[t];
+                const uint32_t o = L < 8 ? a : b;
+                box_words(node)[L] = (L & 3u) == 3u ? 1.0f : bx[6 * o + ((L >> 2) & 1u) * 3 + (L & 3u)];
+                if (L == 0) {
+                    node.leftChild = ~static_cast<int32_t>(prim[a]);
+                    node.rightChild = ~static_cast<int32_t>(prim[b]);
+                    node._pad[0] = node._pad[1] = 0;
+                    levels[t] = static_cast<uint8_t>(level);
+                    set_child(tmp, link, static_cast<int32_t>(t));
+                }
+                continue;
+            }
+            float cLo[3], cHi[3], bLo[3], bHi[3];
+            const bool wide = l - f > kSubWide;
+            if (wide) {  // a lane per sixteenth of the primitives, then the lanes' folds in order
+                float v[12];
+#pragma unroll
+                for (int w = 0; w < 12; ++w) v[w] = ((w / 3) & 1) ? -INFINITY : INFINITY;
+                const uint32_t each = (l - f + 15u) / 16u, from = f + L * each, to = from + each < l ? from + each : l;
+#pragma unroll 4
+                for (uint32_t p = from; p < to; ++p) {
+                    const float *e = bx + 6u * ord[p];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const float lo = e[c], hi = e[c + 3], mid = 0.5f * (lo + hi);
+                        v[c] = nv_min(v[c], mid);
+                        v[3 + c] = nv_max(v[3 + c], mid);
+                        v[6 + c] = nv_min(v[6 + c], lo);
+                        v[9 + c] = nv_max(v[9 + c], hi);
+                    }
+                }
+#pragma unroll
+                for (int w = 0; w < 12; ++w) {
+                    if ((w / 3) & 1) {
+                        v[w] = nv_max(v[w], row_shl<1>(-INFINITY, v[w]));
+                        v[w] = nv_max(v[w], row_shl<2>(-INFINITY, v[w]));
+                        v[w] = nv_max(v[w], row_shl<4>(-INFINITY, v[w]));
+                        v[w] = nv_max(v[w], row_shl<8>(-INFINITY, v[w]));
+                    } else {
+                        v[w] = nv_min(v[w], row_shl<1>(INFINITY, v[w]));
+                        v[w] = nv_min(v[w], row_shl<2>(INFINITY, v[w]));
+                        v[w] = nv_min(v[w], row_shl<4>(INFINITY, v[w]));
+                        v[w] = nv_min(v[w], row_shl<8>(INFINITY, v[w]));
+                    }
+                    v[w] = __shfl(v[w], row);
+                }
+#pragma unroll
+                for (int c = 0; c < 3; ++c) cLo[c] = v[c], cHi[c] = v[3 + c], bLo[c] = v[6 + c], bHi[c] = v[9 + c];
+            } else {
+                // lanes 0..2 centroid lo, 3..5 centroid hi, 6..8 box lo, 9..11 box hi
+                const uint32_t k = L % 3u, kind = L / 3u;
+                float v = (kind & 1u) ? -INFINITY : INFINITY;
+                for (uint32_t p = f; p < l; p += 8u) {  // beyond the end: the last one again, which changes nothing
+                    float x[8];
+#pragma unroll
+                    for (uint32_t e = 0; e < 8; ++e) {
+                        const uint32_t o = 6u * ord[p + e < l ? p + e : l - 1] + k;
+                        const float lo = bx[o], hi = bx[o + 3];
+                        x[e] = kind < 2u ? 0.5f * (lo + hi) : kind == 2u ? lo : hi;
+                    }
+#pragma unroll
+                    for (uint32_t e = 0; e < 8; ++e) v = (kind & 1u) ? nv_max(v, x[e]) : nv_min(v, x[e]);
+                }
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    cLo[c] = __shfl(v, row + c);
+                    cHi[c] = __shfl(v, row + 3 + c);
+                    bLo[c] = __shfl(v, row + 6 + c);
+                    bHi[c] = __shfl(v, row + 9 + c);
+                }
+            }
+            const Params q = make_params(cLo, cHi, bLo, bHi);
+            Bin left = bin_empty();
+            if (wide) {  // keys as in k_bvh_bin
+                u64 *a = bins[threadIdx.x >> 4];
+                for (uint32_t w = L; w < kBuckets * kBinWords; w += 16u) a[w] = word_init(kBoundWords + static_cast<int>(w));
+                row_sync();
+                for (uint32_t p = f + L; p < l; p += 16u) {
+                    const float *e = bx + 6u * ord[p];
+                    const uint32_t b = bucket_of(q, 0.5f * (e[q.axis] + e[q.axis + 3]));
+                    bucket[p] = static_cast<uint8_t>(b);
+                    u64 *w = a + b * kBinWords;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        atomicMin(&w[c], key_min(e[c], p));
+                        atomicMax(&w[3 + c], key_max(e[3 + c], p));
+                    }
+                    atomicAdd(&w[6], 1ull);
+                }
+                row_sync();
+                if (L < kBuckets) left.count = static_cast<uint32_t>(a[L * kBinWords + 6]);
+                if (left.count != 0)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const u64 lo = a[L * kBinWords + c], hi = a[L * kBinWords + 3 + c];
+                        const float vl = uncode(static_cast<uint32_t>(lo >> 32)), vh = uncode(static_cast<uint32_t>(hi >> 32));
+                        left.lo[c] = nv_min(FLT_MAX, vl != 0.0f ? vl : bx[6u * ord[~static_cast<uint32_t>(lo)] + c]);
+                        left.hi[c] = nv_max(-FLT_MAX, vh != 0.0f ? vh : bx[6u * ord[static_cast<uint32_t>(hi)] + 3 + c]);
+                    }
+            } else {
+                for (uint32_t p = f + L; p < l; p += 16u) {
+                    const uint32_t o = 6u * ord[p] + static_cast<uint32_t>(q.axis);
+                    bucket[p] = static_cast<uint8_t>(bucket_of(q, 0.5f * (bx[o] + bx[o + 3])));
+                }
+                row_sync();
+                // a lane per bucket
+                for (uint32_t p = f; p < l; p += 4u) {
+                    float x[4][6];
+                    bool mine[4];
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) {
+                        const uint32_t at = p + e < l ? p + e : l - 1, o = 6u * ord[at];
+                        mine[e] = p + e < l && bucket[at] == L;
+#pragma unroll
+                        for (int c = 0; c < 6; ++c) x[e][c] = bx[o + c];
+                    }
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) {
+                        // read in any case, so that the loads of all four are under way together: left
+                        // alone the compiler puts each behind a branch on its bucket
+#pragma unroll
+                        for (int c = 0; c < 6; ++c) asm volatile("" : "+v"(x[e][c]));
+                        left.count += mine[e] ? 1u : 0u;
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) {
+                            left.lo[c] = mine[e] ? nv_min(left.lo[c], x[e][c]) : left.lo[c];
+                            left.hi[c] = mine[e] ? nv_max(left.hi[c], x[e][3 + c]) : left.hi[c];
+                        }
+                    }
+                }
+            }
+            Bin right = left;
+            const int best = sah_sweep(left, right, q.parentArea);
+            const uint32_t split = best < 0 ? 0u : static_cast<uint32_t>(best);
+            uint32_t mid = f + static_cast<uint32_t>(__shfl(static_cast<int>(left.count), row + static_cast<int>(split)));
+            const bool degenerate = mid == f || mid == l;
+            if (degenerate) mid = (f + l) / 2;
+            const uint32_t t = sub.first + mid - 1;
+            restir_aabb_tree_node &node = tmp[t];
+            if (degenerate) {
+                // a lane per component of the halves' boxes, in the node's order; w = 1
+                const uint32_t c = L & 3u, from = L < 8u ? f : mid, to = L < 8u ? mid : l;
+                float x = 1.0f;
+                if (c < 3u)
+                    for (uint32_t p = from; p < to; ++p) {
+                        const float e = bx[6u * ord[p] + ((L >> 2) & 1u) * 3 + c];
+                        x = p == from ? e : ((L >> 2) & 1u) ? nv_max(x, e) : nv_min(x, e);
+                    }
+                box_words(node)[L] = x;
+                for (uint32_t p = f + L; p < l; p += 16u) out[p] = ord[p];
+            } else {
+                if (L == split) {
+                    const float zero[3] = {0.0f, 0.0f, 0.0f};
+                    write_box(node.leftAabbMin, best < 0 ? zero : left.lo);
+                    write_box(node.leftAabbMax, best < 0 ? zero : left.hi);
+                    write_box(node.rightAabbMin, best < 0 ? zero : right.lo);
+                    write_box(node.rightAabbMax, best < 0 ? zero : right.hi);
+                }
+                uint32_t run = f;  // the next left primitive's place
+                for (uint32_t p0 = f; p0 < l; p0 += 16u) {
+                    const uint32_t p = p0 + L;
+                    const bool in = p < l, goes = in && bucket[p] <= split;
+                    const uint32_t m = static_cast<uint32_t>(__ballot(goes) >> row) & 0xffffu;
+                    const uint32_t g = run + static_cast<uint32_t>(__popc(m & ((1u << L) - 1u)));
+                    uint32_t at = p;
+                    if (goes) {
+                        out[g] = ord[p];
+                        at = g < p ? g : p;
+                    }
+                    if (in) ptr[p] = static_cast<uint16_t>(at);
+                    row_sync();
+                    if (in)
+                        for (uint32_t to = ptr[at]; to != at; to = ptr[at]) at = to;
+                    row_sync();
+                    if (in) {
+                        ptr[p] = static_cast<uint16_t>(at);
+                        if (p >= mid) out[p] = ord[at];
+                    }
+                    run += static_cast<uint32_t>(__popc(m));
+                }
+            }
+            row_sync();
+            if (L == 0) {
+                node._pad[0] = node._pad[1] = 0;
+                levels[t] = static_cast<uint8_t>(level);
+                set_child(tmp, link, static_cast<int32_t>(t));
+            }
+            if (L < 2) {
+                const uint32_t a = L == 0 ? f : mid, b = L == 0 ? mid : l;
+                const int32_t to = static_cast<int32_t>(2 * t + L);
+                if (b - a == 1) set_child(tmp, to, ~static_cast<int32_t>(prim[out[a]]));
+                else queue[cur ^ 1u][atomicAdd(&queued[cur ^ 1u], 1u)] = SubQueue{static_cast<uint16_t>(a), static_cast<uint16_t>(b), to};
+            }
+        }
+        __syncthreads();
+        if (queued[cur ^ 1u] == 0) break;
+        __syncthreads();
+        if (threadIdx.x == 0) queued[cur] = 0;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) atomicMax(&info->depth, level);
+}
+
+// Breadth-first ids: the temporary nodes, sorted by level, in their order within one. Nodes of each
+// level in each block of 256 ...
+__global__ __launch_bounds__(256) void k_bvh_level_counts(uint32_t nNodes, uint32_t depth, const uint8_t *levels,
+                                                          uint32_t *counts) {
+    __shared__ uint32_t sh[64];
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (threadIdx.x < 64) sh[threadIdx.x] = 0;
+    __syncthreads();
+    if (t < nNodes) atomicAdd(&sh[levels[t] - 1u], 1u);
+    __syncthreads();
+    if (threadIdx.x < depth) counts[threadIdx.x * gridDim.x + blockIdx.x] = sh[threadIdx.x];
+}
+// ... then, from their exclusive prefix sums (level after level), each node's id.
+__global__ __launch_bounds__(256) void k_bvh_ids(uint32_t nNodes, const uint8_t *levels, const uint32_t *counts, uint32_t *ids) {
+    __shared__ uint32_t sh[4][64];
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    sh[wave][lane] = 0;
+    __syncthreads();
+    const uint32_t l = t < nNodes ? levels[t] - 1u : 0u;
+    uint64_t same = __ballot(t < nNodes);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+        const uint64_t m = __ballot((l >> b) & 1u);
+        same &= ((l >> b) & 1u) ? m : ~m;
+    }
+    const uint32_t before = static_cast<uint32_t>(__popcll(same & ((1ull << lane) - 1ull)));
+    if (t < nNodes && before == 0) sh[wave][l] = static_cast<uint32_t>(__popcll(same));
+    __syncthreads();
+    if (t >= nNodes) return;
+    uint32_t id = counts[l * gridDim.x + blockIdx.x] + before;
+    for (uint32_t w = 0; w < wave; ++w) id += sh[w][l];
+    ids[t] = id;
+}
+__global__ __launch_bounds__(256) void k_bvh_write(uint32_t nNodes, const restir_aabb_tree_node *tmp, const uint32_t *ids,
+                                                   restir_aabb_tree_node *nodes) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t >= nNodes) return;
+    restir_aabb_tree_node node = tmp[t];
+    if (node.leftChild >= 0) node.leftChild = static_cast<int32_t>(ids[node.leftChild]);
+    if (node.rightChild >= 0) node.rightChild = static_cast<int32_t>(ids[node.rightChild]);
+    nodes[ids[t]] = node;
 }
 
 inline uint32_t groups(uint64_t n) { return static_cast<uint32_t>((n + 255) / 256); }
@@ -559,12 +931,13 @@ inline uint32_t groups(uint64_t n) { return static_cast<uint32_t>((n + 255) / 25
 inline size_t align_up(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 struct Layout {
-    size_t box, idx0, idx1, seg0, seg1, rank, bucket, flag, ptr, temp32, segs0, segs1, flags64, temp64, splits,
-        params, acc, info, total;
+    size_t box, idx0, idx1, seg0, seg1, bucket, before, ptr, temp32, segs0, segs1, segRank, splits, subs, acc, tmp, levels,
+        counts, info, total;
 };
 
 Layout layout(uint32_t n) {
-    const size_t maxSplits = n / 3 + 1, maxSegs = 2 * maxSplits + 1;
+    const size_t maxSplits = n / (kSub + 1) + 1, maxSegs = 2 * maxSplits + 1;
+    const size_t sums = (static_cast<size_t>(n) + kScanGroup - 1) / kScanGroup, counts = 64ull * groups(n);
     Layout L{};
     size_t o = 0;
     auto take = [&o](size_t bytes) {
@@ -577,18 +950,19 @@ Layout layout(uint32_t n) {
     L.idx1 = take(4ull * n);
     L.seg0 = take(4ull * n);
     L.seg1 = take(4ull * n);
-    L.rank = take(4ull * n);
     L.bucket = take(n);
-    L.flag = take(4ull * n);
-    L.ptr = take(4ull * n);
-    L.temp32 = take(4 * rscan::temp_items(n));
+    L.before = take(4ull * n);
+    L.ptr = take(4ull * n);  // then the nodes' ids
+    L.temp32 = take(4 * (sums + rscan::temp_items(static_cast<uint32_t>(sums)) + rscan::temp_items(static_cast<uint32_t>(counts))));
     L.segs0 = take(sizeof(Seg) * maxSegs);
     L.segs1 = take(sizeof(Seg) * maxSegs);
-    L.flags64 = take(8 * maxSegs);
-    L.temp64 = take(8 * rscan::temp_items(static_cast<uint32_t>(maxSegs)));
+    L.segRank = take(4 * maxSegs);
     L.splits = take(sizeof(Split) * maxSplits);
-    L.params = take(sizeof(Params) * maxSplits);
-    L.acc = take(8ull * kAcc * maxSplits);
+    L.subs = take(sizeof(Sub) * (n / 2 + 1));
+    L.acc = take(8ull * kAcc * (2 * maxSplits));
+    L.tmp = take(sizeof(restir_aabb_tree_node) * n);
+    L.levels = take(n);
+    L.counts = take(4 * counts);
     L.info = take(sizeof(Info));
     L.total = o;
     return L;
@@ -898,17 +1272,23 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     const bool w8Fits = maxW8 <= (1u << 23) && nTris <= (1u << 26);
     // a level of 8-entry nodes covers at least one level of the tree
     const uint32_t levels = depth < static_cast<uint32_t>(kW8Levels) ? depth : static_cast<uint32_t>(kW8Levels);
-    if (w8Fits)
-        for (uint32_t l = 0; l < levels; ++l)
-            RK_LAUNCH("k_w8_collapse", k_w8_collapse, dim3(1024), dim3(64), 0, s, bn, bt, l, maxW8, nTris, p.flags,
-                      p.w8, p.tris, p.work, p.info);
     struct {
         uint32_t flags[4];
         W8Info w8;
     } host{{1u, 0x7fc00000u, 1u, 1u}, {}};
     static_assert(sizeof host == 16 + sizeof(W8Info), "flags and counters are copied together");
-    if (int r = hip(hipMemcpyAsync(&host, p.flags, sizeof host, hipMemcpyDeviceToHost, s), "bind tree: read")) return r;
-    if (int r = hip(hipStreamSynchronize(s), "bind tree: finish")) return r;
+    // Usually 8-entry levels are about a third as many: after the first launches the counters say
+    // whether there are more (an empty launch takes 4 us, 13 of them in a tree of 23 levels).
+    uint32_t done = 0;
+    for (uint32_t batch = 4 + (32u - static_cast<uint32_t>(__builtin_clz(nTris))) / 3;; batch = 4) {
+        const uint32_t end = !w8Fits ? 0u : (done + batch < levels ? done + batch : levels);
+        for (; done < end; ++done)
+            RK_LAUNCH("k_w8_collapse", k_w8_collapse, dim3(1024), dim3(64), 0, s, bn, bt, done, maxW8, nTris, p.flags,
+                      p.w8, p.tris, p.work, p.info);
+        if (int r = hip(hipMemcpyAsync(&host, p.flags, sizeof host, hipMemcpyDeviceToHost, s), "bind tree: read")) return r;
+        if (int r = hip(hipStreamSynchronize(s), "bind tree: finish")) return r;
+        if (!w8Fits || done == levels || host.w8.nodes[done] == 0) break;
+    }
     float maxCoord;
     std::memcpy(&maxCoord, &host.flags[1], sizeof maxCoord);
     ctx->scene.nodes = bn;
@@ -921,7 +1301,7 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     ctx->scene.w8Tris = p.tris;
     ctx->scene.treeTight = host.flags[3] == 0 ? 1 : 0;
     // the bounds on the coordinates keep every product of the walk finite and its slack normal
-    ctx->scene.w8Ok = w8Fits && host.flags[2] == 0 && host.w8.overflow == 0 && host.w8.nodes[levels] == 0 &&
+    ctx->scene.w8Ok = w8Fits && host.flags[2] == 0 && host.w8.overflow == 0 && host.w8.nodes[done] == 0 &&
                               host.w8.tris == nTris && maxCoord > 1e-18f && maxCoord < 1e18f
                           ? 1
                           : 0;
@@ -962,70 +1342,70 @@ extern "C" int restir_build_bvh(restir_ctx *ctx, const float *triXyz, uint32_t n
     float4 *box = reinterpret_cast<float4 *>(base + L.box);
     uint32_t *idx[2] = {reinterpret_cast<uint32_t *>(base + L.idx0), reinterpret_cast<uint32_t *>(base + L.idx1)};
     int32_t *segOf[2] = {reinterpret_cast<int32_t *>(base + L.seg0), reinterpret_cast<int32_t *>(base + L.seg1)};
-    int32_t *rank = reinterpret_cast<int32_t *>(base + L.rank);
     uint8_t *bucket = reinterpret_cast<uint8_t *>(base + L.bucket);
-    uint32_t *flag = reinterpret_cast<uint32_t *>(base + L.flag);
-    uint32_t *ptr = reinterpret_cast<uint32_t *>(base + L.ptr);
-    uint32_t *temp32 = reinterpret_cast<uint32_t *>(base + L.temp32);
+    uint32_t *before = reinterpret_cast<uint32_t *>(base + L.before);
+    uint32_t *ptr = reinterpret_cast<uint32_t *>(base + L.ptr), *ids = ptr;
     Seg *segs[2] = {reinterpret_cast<Seg *>(base + L.segs0), reinterpret_cast<Seg *>(base + L.segs1)};
-    u64 *flags64 = reinterpret_cast<u64 *>(base + L.flags64);
-    u64 *temp64 = reinterpret_cast<u64 *>(base + L.temp64);
+    int32_t *segRank = reinterpret_cast<int32_t *>(base + L.segRank);
     Split *splits = reinterpret_cast<Split *>(base + L.splits);
-    Params *params = reinterpret_cast<Params *>(base + L.params);
+    Sub *subs = reinterpret_cast<Sub *>(base + L.subs);
     u64 *acc = reinterpret_cast<u64 *>(base + L.acc);
+    restir_aabb_tree_node *tmp = reinterpret_cast<restir_aabb_tree_node *>(base + L.tmp);
+    uint8_t *levels = reinterpret_cast<uint8_t *>(base + L.levels);
+    uint32_t *counts = reinterpret_cast<uint32_t *>(base + L.counts);
     Info *info = reinterpret_cast<Info *>(base + L.info);
     Info *host = static_cast<Info *>(ctx->bvhInfoHost);
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint32_t n = nTris;
+    const uint32_t n = nTris, nSums = (n + kScanGroup - 1) / kScanGroup;
+    uint32_t *sums = reinterpret_cast<uint32_t *>(base + L.temp32), *temp32 = sums + nSums;
 
     auto hip = [&](hipError_t e, const char *what) { return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, what); };
+    auto read_info = [&](const char *what) {
+        if (int r = hip(hipMemcpyAsync(host, info, sizeof(Info), hipMemcpyDeviceToHost, s), what)) return r;
+        return hip(hipStreamSynchronize(s), what);
+    };
     if (int r = hip(hipMemsetAsync(info, 0, sizeof(Info), s), "build_bvh: clear")) return r;
-    RK_LAUNCH("k_bvh_prep", k_bvh_prep, dim3(groups(n)), dim3(256), 0, s, n, triXyz, tris, box, idx[0], segOf[0], info);
-    const Seg root{0u, n, -1, 0};
-    if (int r = hip(hipMemcpyAsync(segs[0], &root, sizeof(Seg), hipMemcpyHostToDevice, s), "build_bvh: root")) return r;
+    RK_LAUNCH("k_bvh_prep", k_bvh_prep, dim3(groups(n)), dim3(256), 0, s, n, triXyz, tris, box, idx[0], segOf[0], acc,
+              segs[0], info);
 
-    uint32_t S = 1, nodeBase = 0, depth = 0, cur = 0;
-    for (uint32_t level = 1; S > 0; ++level) {
-        RK_LAUNCH("k_bvh_classify", k_bvh_classify, dim3(groups(S)), dim3(256), 0, s, S, segs[cur], flags64);
-        if (int r = hip(rscan::exclusive_scan<u64>(flags64, flags64, S, temp64, &info->totals, s), "build_bvh: scan"))
-            return r;
-        if (int r = hip(hipMemcpyAsync(host, info, sizeof(Info), hipMemcpyDeviceToHost, s), "build_bvh: read counts"))
-            return r;
-        if (int r = hip(hipStreamSynchronize(s), "build_bvh: level")) return r;
+    uint32_t S = 1, cur = 0;
+    for (uint32_t level = 1;; ++level) {
+        RK_LAUNCH("k_bvh_level", k_bvh_level, dim3(1), dim3(256), 0, s, S, level, segs[cur], idx[cur], tmp, segRank, splits,
+                  subs, info);
+        if (int r = read_info("build_bvh: level")) return r;
         if (host->bad) return fail(ctx, RESTIR_E_INVALID_ARGUMENT, "build_bvh: a vertex coordinate is not finite");
-        const uint32_t nodesHere = static_cast<uint32_t>(host->totals & 0xffffffffu);
-        const uint32_t nSplits = static_cast<uint32_t>(host->totals >> 32);
-        if (nodesHere > 0) depth = level;
-        RK_LAUNCH("k_bvh_setup", k_bvh_setup, dim3(groups(S)), dim3(256), 0, s, S, segs[cur], flags64, nodeBase,
-                  idx[cur], box, nodes, splits);
-        nodeBase += nodesHere;
+        const uint32_t nSplits = host->splits;
         if (nSplits == 0) break;
-        const uint32_t words = nSplits * static_cast<uint32_t>(kAcc);
-        RK_LAUNCH("k_bvh_init_acc", k_bvh_init_acc, dim3(groups(words)), dim3(256), 0, s, words, acc);
-        RK_LAUNCH("k_bvh_rank", k_bvh_rank, dim3(groups(n)), dim3(256), 0, s, n, segOf[cur], segs[cur], flags64, rank);
-        RK_LAUNCH("k_bvh_bounds", k_bvh_bounds, dim3(groups(n)), dim3(256), 0, s, n, idx[cur], rank, box, acc);
-        RK_LAUNCH("k_bvh_params", k_bvh_params, dim3(groups(nSplits)), dim3(256), 0, s, nSplits, idx[cur], box, acc,
-                  params);
-        RK_LAUNCH("k_bvh_bin", k_bvh_bin, dim3(groups(n)), dim3(256), 0, s, n, idx[cur], rank, box, params, bucket, acc);
-        RK_LAUNCH("k_bvh_choose", k_bvh_choose, dim3(groups(nSplits)), dim3(256), 0, s, nSplits, idx[cur], box, params,
-                  acc, splits, nodes, segs[cur ^ 1]);
-        RK_LAUNCH("k_bvh_halves", k_bvh_halves, dim3(groups(n)), dim3(256), 0, s, n, idx[cur], rank, box, splits, acc);
-        RK_LAUNCH("k_bvh_halves_write", k_bvh_halves_write, dim3(groups(nSplits)), dim3(256), 0, s, nSplits, idx[cur],
-                  box, splits, acc, nodes);
-        RK_LAUNCH("k_bvh_left_flags", k_bvh_left_flags, dim3(groups(n)), dim3(256), 0, s, n, rank, splits, bucket, flag);
-        if (int r = hip(rscan::exclusive_scan<uint32_t>(flag, flag, n, temp32, nullptr, s), "build_bvh: scan")) return r;
-        RK_LAUNCH("k_bvh_chain", k_bvh_chain, dim3(groups(n)), dim3(256), 0, s, n, rank, splits, bucket, flag, ptr);
-        RK_LAUNCH("k_bvh_jump", k_bvh_jump, dim3(groups(n)), dim3(256), 0, s, n, ptr);
-        RK_LAUNCH("k_bvh_scatter", k_bvh_scatter, dim3(groups(n)), dim3(256), 0, s, n, rank, splits, bucket, flag,
-                  ptr, idx[cur], idx[cur ^ 1], segOf[cur ^ 1]);
+        RK_LAUNCH("k_bvh_bounds", k_bvh_bounds, dim3(groups(n)), dim3(256), 0, s, n, idx[cur], segOf[cur], segRank, splits,
+                  box, acc);
+        RK_LAUNCH("k_bvh_bin", k_bvh_bin, dim3(groups(n)), dim3(256), 0, s, n, idx[cur], segOf[cur], segRank, box, bucket,
+                  acc);
+        RK_LAUNCH("k_bvh_choose", k_bvh_choose, dim3((nSplits + 15) / 16), dim3(256), 0, s, nSplits, level, idx[cur], box,
+                  acc, splits, tmp, levels, segs[cur ^ 1]);
+        RK_LAUNCH("k_bvh_left_count", k_bvh_left_count, dim3(nSums), dim3(256), 0, s, n, segOf[cur], segRank, splits, bucket,
+                  before, sums);
+        if (int r = hip(rscan::exclusive_scan<uint32_t>(sums, sums, nSums, temp32, nullptr, s), "build_bvh: scan")) return r;
+        RK_LAUNCH("k_bvh_chain", k_bvh_chain, dim3(groups(n)), dim3(256), 0, s, n, segOf[cur], segRank, splits, bucket,
+                  before, sums, ptr);
+        RK_LAUNCH("k_bvh_scatter", k_bvh_scatter, dim3(groups(n)), dim3(256), 0, s, n, nSplits, segOf[cur], segRank, splits,
+                  bucket, before, sums, ptr, idx[cur], idx[cur ^ 1], segOf[cur ^ 1], acc);
         if (int r = hip(hipGetLastError(), "build_bvh: launch")) return r;
         S = 2 * nSplits;
         cur ^= 1;
     }
-    if (int r = hip(hipStreamSynchronize(s), "build_bvh: finish")) return r;
-    if (nodeBase != n - 1) return fail(ctx, RESTIR_E_BAD_TREE, "build_bvh: %u nodes for %u triangles", nodeBase, n);
+    // every level ends in smaller ranges: the deepest nodes are theirs
+    RK_LAUNCH("k_bvh_subtrees", k_bvh_subtrees, dim3(host->subs), dim3(256), 0, s, subs, idx[cur], box, tmp, levels, info);
+    if (int r = read_info("build_bvh: subtrees")) return r;
+    const uint32_t depth = host->depth;
     if (depth > 64)
         return fail(ctx, RESTIR_E_BAD_TREE, "build_bvh: tree depth %u exceeds the 64-entry traversal stack", depth);
+    const uint32_t nBlocks = groups(n - 1);
+    RK_LAUNCH("k_bvh_level_counts", k_bvh_level_counts, dim3(nBlocks), dim3(256), 0, s, n - 1, depth, levels, counts);
+    if (int r = hip(rscan::exclusive_scan<uint32_t>(counts, counts, depth * nBlocks, temp32, nullptr, s), "build_bvh: scan"))
+        return r;
+    RK_LAUNCH("k_bvh_ids", k_bvh_ids, dim3(nBlocks), dim3(256), 0, s, n - 1, levels, counts, ids);
+    RK_LAUNCH("k_bvh_write", k_bvh_write, dim3(nBlocks), dim3(256), 0, s, n - 1, tmp, ids, nodes);
+    if (int r = hip(hipGetLastError(), "build_bvh: launch")) return r;
     if (depthOut) *depthOut = depth;
     return bind_tree(ctx, nodes, n - 1, tris, depth, s);
 }

@@ -61,7 +61,7 @@ struct restir_ctx {
     size_t viewTableBytes = 0;
     void *bvhScratch = nullptr;    // primitive order, keys and ranges of the GPU tree build
     size_t bvhScratchBytes = 0;
-    void *bvhInfoHost = nullptr;   // pinned: each tree level's node and split counts
+    void *bvhInfoHost = nullptr;   // pinned: the counters of the tree build
     void *aliasScratch = nullptr;  // powers, weights and queues of the device alias-table build
     size_t aliasScratchBytes = 0;
     void *wide = nullptr;          // the bound tree's 4-entry nodes (+ the nesting flag)
