@@ -12,10 +12,10 @@
 //                  M candidates (l, q) for each of its pixels (K <= 256)
 //   k_propose_wide the same for K up to 4096: the output layer streamed in 64-cluster blocks
 //   k_features     features of listed pixels (bf16), for training and tests
-//   k_gemm         strided C = A*B with bias / ReLU / ReLU-gate epilogues (training fwd/bwd),
-//                  or split-K fp32 partials for the weight gradients
+//   k_mlp_forward, k_mlp_backward, k_mlp_grads   training: a tile of samples through all layers and
+//                  back, and the weight and bias gradients as partial sums over ranges of samples
 //   k_softmax_ce   mean cross-entropy of the logits against target clusters, and dlogits
-//   k_colsum_partial, k_sum_partials   bias gradients and the split-K reduction, in fixed order
+//   k_sum_partials the partial sums of the gradients and the loss, in fixed order
 //   k_adam         Adam step on fp32 master weights, refreshes the bf16 copy
 //   k_mlp_init     seeded He-uniform initialisation
 #include "../../include/restir_abi.h"
@@ -90,116 +90,230 @@ __global__ __launch_bounds__(256) void k_features(const FeatArgs f, const uint32
     }
 }
 
-// -------------------------------------------------------------------------------- GEMM ------
-struct GemmArgs {
-    const uint16_t *A;
-    int64_t sam, sak;
-    const uint16_t *B;
-    int64_t sbk, sbn;
-    int M, N, K;
-    const float *bias;     // per output column, or null
-    int relu;              // clamp at 0
-    const uint16_t *gate;  // out *= (gate(m, n) > 0), or null
-    int64_t sgm, sgn;
-    float *Cf;             // fp32 output, or null
-    uint16_t *Cb;          // bf16 output, or null
-    int64_t scm, scn;
-    int kChunk;            // split-K: workgroup z covers K range [z*kChunk, (z+1)*kChunk) and
-    int64_t scz;           // writes its fp32 partial at Cf + z*scz (no bias/relu/gate); 0 = off
-};
+// ----------------------------------------------------------------- forward and backward ------
+// Training works on a few thousand samples: what bounds it is the chain of launches and, inside
+// one, of memory round trips, not the products (0.9 GFLOP at 4,096 samples and 256 clusters). So a
+// workgroup takes 32 samples through all layers, its activations in LDS, each wave with all of a
+// layer's weights for its 32 columns under way at once; and the weight gradients of all layers are
+// one launch. As 11 launches of a 64x64-tile product (8.6 us each) and 8 others a step of 4,096
+// samples took 144 us, now 56: forward 12, backward 14, gradients 13, their sums 8. 4,096 clusters
+// 375 -> 277 us, 16,384 samples 320 -> 125, 64 samples 97 -> 40.
+constexpr int kMlpRows = 32;     // samples per workgroup
+constexpr int kRow = kIn + 8;    // padded LDS row (bf16) against bank conflicts
 
-// 64x64 output tile per 256-lane workgroup; each wave owns a 32x32 quarter. K advances in steps
-// of 32 through LDS tiles As[64][32] and Bt[64][32] (B staged transposed so every fragment is
-// eight consecutive bf16). Requires M, N multiples of 64, K a multiple of 32 and 16-byte aligned
-// operands whose strides are multiples of 8 elements.
-__global__ __launch_bounds__(256) void k_gemm(const GemmArgs g) {
-    __shared__ __align__(16) uint16_t As[64][40];
-    __shared__ __align__(16) uint16_t Bt[64][40];
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    const int kBeg = g.kChunk ? static_cast<int>(blockIdx.z) * g.kChunk : 0;
-    const int kEnd = g.kChunk ? kBeg + g.kChunk : g.K;
-    // staging order: consecutive lanes read consecutive addresses of whichever operand index is
-    // contiguous in memory
-    const bool aRowFast = g.sak != 1, bRowFast = g.sbn == 1;
+// the product's operands and result are laid out as mlp.h says; row of a lane's result element i
+__device__ __forceinline__ int acc_row(int lane, int i) { return 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3); }
+__device__ __forceinline__ f32x16 acc_zero() {
     f32x16 acc;
+#pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-    // 16-byte loads where one operand index is contiguous (every launch here): a lane loads 8
-    // consecutive k of one row, or 8 consecutive rows of one k and scatters them to LDS
-    const bool vecA = g.sak == 1 || g.sam == 1, vecB = g.sbk == 1 || g.sbn == 1;
-    for (int k0 = kBeg; k0 < kEnd; k0 += 32) {
-        if (vecA) {
-            if (g.sak == 1) {
-                const int r = tid >> 2, c = (tid & 3) * 8;
-                *reinterpret_cast<uint4 *>(&As[r][c]) = *reinterpret_cast<const uint4 *>(&g.A[(m0 + r) * g.sam + k0 + c]);
-            } else {
-                const int kk = tid >> 3, r = (tid & 7) * 8;
-                const uint4 v = *reinterpret_cast<const uint4 *>(&g.A[(k0 + kk) * g.sak + m0 + r]);
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    return acc;
+}
+// a 32-sample LDS tile to rows of kHidden
+__device__ __forceinline__ void store_tile(const uint16_t (*tile)[kRow], uint16_t *dst) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    As[r + 2 * i][kk] = static_cast<uint16_t>(w[i] & 0xffffu);
-                    As[r + 2 * i + 1][kk] = static_cast<uint16_t>(w[i] >> 16);
-                }
-            }
-        }
-        if (vecB) {
-            if (g.sbk == 1) {
-                const int r = tid >> 2, c = (tid & 3) * 8;
-                *reinterpret_cast<uint4 *>(&Bt[r][c]) = *reinterpret_cast<const uint4 *>(&g.B[k0 + c + (n0 + r) * g.sbn]);
-            } else {
-                const int kk = tid >> 3, r = (tid & 7) * 8;
-                const uint4 v = *reinterpret_cast<const uint4 *>(&g.B[(k0 + kk) * g.sbk + n0 + r]);
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    Bt[r + 2 * i][kk] = static_cast<uint16_t>(w[i] & 0xffffu);
-                    Bt[r + 2 * i + 1][kk] = static_cast<uint16_t>(w[i] >> 16);
-                }
-            }
-        }
-        if (!vecA || !vecB) {
-            for (int e = tid; e < 64 * 32; e += 256) {
-                if (!vecA) {
-                    const int ra = aRowFast ? (e & 63) : (e >> 5), ca = aRowFast ? (e >> 6) : (e & 31);
-                    As[ra][ca] = g.A[(m0 + ra) * g.sam + (k0 + ca) * g.sak];
-                }
-                if (!vecB) {
-                    const int rb = bRowFast ? (e & 63) : (e >> 5), cb = bRowFast ? (e >> 6) : (e & 31);
-                    Bt[rb][cb] = g.B[(k0 + cb) * g.sbk + (n0 + rb) * g.sbn];
-                }
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < 32; ks += 16) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&As[wm + (lane & 31)][ks + 8 * (lane >> 5)]);
-            const bf16x8 b = *reinterpret_cast<const bf16x8 *>(&Bt[wn + (lane & 31)][ks + 8 * (lane >> 5)]);
-            acc = mfma32(a, b, acc);
-        }
-        __syncthreads();
+    for (int e = threadIdx.x; e < kMlpRows * (kHidden / 8); e += 256) {
+        const int r = e / (kHidden / 8), c = (e % (kHidden / 8)) * 8;
+        *reinterpret_cast<uint4 *>(dst + static_cast<size_t>(r) * kHidden + c) = *reinterpret_cast<const uint4 *>(&tile[r][c]);
     }
-    const int col = n0 + wn + (lane & 31);
-    if (g.kChunk) {
-        float *P = g.Cf + blockIdx.z * g.scz;
+}
+
+struct ForwardArgs {
+    const uint16_t *X, *wbf;
+    const float *bias;
+    uint16_t *H[3];  // hidden activations
+    float *Z;        // logits
+    int K, cols;     // clusters; those that a workgroup computes (blockIdx.y-th group)
+};
+// Workgroup (x, y): the hidden layers of samples 32x .. 32x + 31 (kept by y = 0), then their logits
+// of clusters cols * y .. : with thousands of clusters the output layer needs more workgroups than
+// there are tiles of samples, and the hidden layers are cheap to repeat.
+__global__ __launch_bounds__(256) void k_mlp_forward(const ForwardArgs a) {
+    __shared__ __align__(16) uint16_t act[2][kMlpRows][kRow];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r0 = blockIdx.x * kMlpRows;
+    const int row = lane & 31, k8 = 8 * (lane >> 5);
+    bf16x8 x[kIn / 16], w[kIn / 16];
+    auto load_w = [&](const uint16_t *W, int col) {
+#pragma unroll
+        for (int s = 0; s < kIn / 16; ++s) w[s] = *reinterpret_cast<const bf16x8 *>(W + static_cast<size_t>(col) * kIn + 16 * s + k8);
+    };
+#pragma unroll
+    for (int s = 0; s < kIn / 16; ++s)
+        x[s] = *reinterpret_cast<const bf16x8 *>(a.X + static_cast<size_t>(r0 + row) * kIn + 16 * s + k8);
+    load_w(a.wbf + w_off(0), 32 * wave + row);
+    for (int l = 0; l < 3; ++l) {
+        f32x16 acc = acc_zero();
+#pragma unroll
+        for (int s = 0; s < kIn / 16; ++s) acc = mfma32(x[s], w[s], acc);
+        // the next layer's weights while this one's results go through LDS
+        if (l < 2) load_w(a.wbf + w_off(l + 1), 32 * wave + row);
+        const int col = 32 * wave + row;
+        const float bias = a.bias[b_off(l) + col];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const int row = m0 + wm + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-            P[row * g.scm + col * g.scn] = acc[i];
+            const float v = acc[i] + bias;
+            act[l & 1][acc_row(lane, i)][col] = f2bf(v > 0.0f ? v : 0.0f);
         }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < kIn / 16; ++s) x[s] = *reinterpret_cast<const bf16x8 *>(&act[l & 1][row][16 * s + k8]);
+        if (blockIdx.y == 0) store_tile(act[l & 1], a.H[l] + static_cast<size_t>(r0) * kHidden);
+    }
+    for (int c = 32 * wave; c < a.cols; c += 128) {
+        const int col = blockIdx.y * a.cols + c + row;
+        load_w(a.wbf + w_off(3), col);
+        f32x16 acc = acc_zero();
+#pragma unroll
+        for (int s = 0; s < kIn / 16; ++s) acc = mfma32(x[s], w[s], acc);
+        const float bias = a.bias[b_off(3) + col];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) a.Z[static_cast<size_t>(r0 + acc_row(lane, i)) * a.K + col] = acc[i] + bias;
+    }
+}
+
+struct BackwardArgs {
+    const uint16_t *dZ, *wbf;
+    const uint16_t *H[3];
+    uint16_t *dH[3];  // gradients at the hidden layers' outputs before their ReLU
+    int K;
+};
+// dIn[b][k] = sum over o of dY[b][o] W[o][k], where the layer below was positive: the output layer's
+// weights come through LDS 128 clusters at a time, then the hidden layers' (a wave reads a column of
+// them there, eight consecutive o as eight 16-bit reads), the next ones on their way in registers.
+__global__ __launch_bounds__(256) void k_mlp_backward(const BackwardArgs a) {
+    __shared__ __align__(16) uint16_t wt[kHidden][kRow];
+    __shared__ __align__(16) uint16_t dy[kMlpRows][kRow];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r0 = blockIdx.x * kMlpRows;
+    const int row = lane & 31, k8 = 8 * (lane >> 5), col = 32 * wave + row;
+    const int chunks = (a.K + kHidden - 1) / kHidden;  // of 128 clusters; one of 64 if K = 64
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 next[8];
+    auto rows_of = [&](int c) { return c < chunks && a.K < kHidden ? a.K : kHidden; };
+    auto fetch = [&](int c) {  // chunk c of the output layer, then layers 2 and 1
+        const uint16_t *src = c < chunks ? a.wbf + w_off(3) + static_cast<size_t>(c) * kHidden * kIn : a.wbf + w_off(2 - (c - chunks));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int at = e * 256 + threadIdx.x;
+            if (at / (kIn / 8) < rows_of(c)) next[e] = *reinterpret_cast<const u32x4 *>(src + at * 8);
+        }
+    };
+    fetch(0);
+    f32x16 acc = acc_zero();
+    for (int c = 0; c < chunks + 2; ++c) {
+        const int rows = rows_of(c);
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int at = e * 256 + threadIdx.x, r = at / (kIn / 8);
+            if (r < rows) *reinterpret_cast<u32x4 *>(&wt[r][(at % (kIn / 8)) * 8]) = next[e];
+        }
+        __syncthreads();
+        if (c + 1 < chunks + 2) fetch(c + 1);
+        const int below = c < chunks ? 2 : 1 - (c - chunks);  // the hidden layer that receives the gradient
+        const bool ends = c >= chunks - 1;
+        uint16_t gate[16];
+        if (ends)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) gate[i] = a.H[below][static_cast<size_t>(r0 + acc_row(lane, i)) * kHidden + col];
+        bf16x8 x[kHidden / 16];
+#pragma unroll
+        for (int s = 0; s < kHidden / 16; ++s)
+            if (16 * s < rows)
+                x[s] = c < chunks ? *reinterpret_cast<const bf16x8 *>(a.dZ + static_cast<size_t>(r0 + row) * a.K + c * kHidden + 16 * s + k8)
+                                  : *reinterpret_cast<const bf16x8 *>(&dy[row][16 * s + k8]);
+#pragma unroll
+        for (int s = 0; s < kHidden / 16; ++s) {
+            if (16 * s >= rows) continue;
+            uint32_t d[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                d[j] = static_cast<uint32_t>(wt[16 * s + k8 + 2 * j][col]) | (static_cast<uint32_t>(wt[16 * s + k8 + 2 * j + 1][col]) << 16);
+            acc = mfma32(x[s], __builtin_bit_cast(bf16x8, make_uint4(d[0], d[1], d[2], d[3])), acc);
+        }
+        if (!ends) continue;
+        __syncthreads();  // the other waves' reads of dy
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dy[acc_row(lane, i)][col] = bf2f(gate[i]) > 0.0f ? f2bf(acc[i] + 0.0f) : 0;
+        acc = acc_zero();
+        __syncthreads();
+        store_tile(dy, a.dH[below] + static_cast<size_t>(r0) * kHidden);
+    }
+}
+
+// The gradients of all layers' weights and biases over the samples, as partial sums that
+// k_sum_partials adds in a fixed order: gW[o][k] = sum over b of dY[b][o] in[b][k] in `split` ranges
+// of b, 64x64 per workgroup, and gb[o] = sum over b of dY[b][o] in ranges of 64.
+struct GradLayer {
+    const uint16_t *dY, *in;  // [n][N], [n][kIn]
+    float *pw, *pb;
+    int N, split;
+    uint32_t firstW, firstB;  // workgroups before this layer's
+};
+struct GradArgs {
+    GradLayer layer[4];
+    int n;
+    uint32_t weightGroups;  // workgroups of the weights, then those of the biases
+};
+// 64x64 outputs per 256-lane workgroup; each wave owns a 32x32 quarter. The samples advance in steps
+// of 32 through LDS, both operands transposed on the way in so that every fragment is eight
+// consecutive bf16; the next step's are on their way in registers.
+__global__ __launch_bounds__(256) void k_mlp_grads(const GradArgs a) {
+    __shared__ __align__(16) uint16_t As[64][40];
+    __shared__ __align__(16) uint16_t Bt[64][40];
+    __shared__ float red[4][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (blockIdx.x >= a.weightGroups) {
+        const uint32_t job = blockIdx.x - a.weightGroups;
+        int l = 3;
+        while (l > 0 && job >= a.layer[l - 1].firstB) --l;
+        const GradLayer &g = a.layer[l];
+        const uint32_t local = job - g.firstB, tiles = static_cast<uint32_t>(g.N) / 64u;
+        const int c = static_cast<int>(local % tiles) * 64 + lane, chunk = static_cast<int>(local / tiles);
+        float sum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum += bf2f(g.dY[static_cast<size_t>(chunk * 64 + wave + 4 * r) * g.N + c]);
+        red[wave][lane] = sum;
+        __syncthreads();
+        if (wave == 0) g.pb[static_cast<size_t>(chunk) * g.N + c] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
         return;
     }
-    const float bias = g.bias ? g.bias[col] : 0.0f;
+    int l = 3;
+    while (l > 0 && blockIdx.x >= a.layer[l - 1].firstW) --l;
+    const GradLayer &g = a.layer[l];
+    const uint32_t local = blockIdx.x - g.firstW, tiles = 2u * static_cast<uint32_t>(g.N) / 64u;
+    const int m0 = static_cast<int>(local % tiles) / 2 * 64, n0 = static_cast<int>(local % 2u) * 64;
+    const int part = static_cast<int>(local / tiles), each = a.n / g.split, kBeg = part * each, kEnd = kBeg + each;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int kk = tid >> 3, r = (tid & 7) * 8;
+    uint4 va, vb;
+    auto fetch = [&](int k0) {
+        va = *reinterpret_cast<const uint4 *>(&g.dY[static_cast<size_t>(k0 + kk) * g.N + m0 + r]);
+        vb = *reinterpret_cast<const uint4 *>(&g.in[static_cast<size_t>(k0 + kk) * kIn + n0 + r]);
+    };
+    fetch(kBeg);
+    f32x16 acc = acc_zero();
+    for (int k0 = kBeg; k0 < kEnd; k0 += 32) {
+        const uint32_t wa[4] = {va.x, va.y, va.z, va.w}, wb[4] = {vb.x, vb.y, vb.z, vb.w};
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int row = m0 + wm + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-        float v = acc[i] + bias;
-        if (g.relu) v = v > 0.0f ? v : 0.0f;
-        if (g.gate && !(bf2f(g.gate[row * g.sgm + col * g.sgn]) > 0.0f)) v = 0.0f;
-        if (g.Cf) g.Cf[row * g.scm + col * g.scn] = v;
-        if (g.Cb) g.Cb[row * g.scm + col * g.scn] = f2bf(v);
+        for (int i = 0; i < 4; ++i) {
+            As[r + 2 * i][kk] = static_cast<uint16_t>(wa[i] & 0xffffu);
+            As[r + 2 * i + 1][kk] = static_cast<uint16_t>(wa[i] >> 16);
+            Bt[r + 2 * i][kk] = static_cast<uint16_t>(wb[i] & 0xffffu);
+            Bt[r + 2 * i + 1][kk] = static_cast<uint16_t>(wb[i] >> 16);
+        }
+        __syncthreads();
+        if (k0 + 32 < kEnd) fetch(k0 + 32);
+#pragma unroll
+        for (int ks = 0; ks < 32; ks += 16) {
+            const bf16x8 fa = *reinterpret_cast<const bf16x8 *>(&As[wm + (lane & 31)][ks + 8 * (lane >> 5)]);
+            const bf16x8 fb = *reinterpret_cast<const bf16x8 *>(&Bt[wn + (lane & 31)][ks + 8 * (lane >> 5)]);
+            acc = mfma32(fa, fb, acc);
+        }
+        __syncthreads();
     }
+    float *P = g.pw + static_cast<size_t>(part) * g.N * kIn;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) P[static_cast<size_t>(m0 + wm + acc_row(lane, i)) * kIn + n0 + wn + (lane & 31)] = acc[i];
 }
 
 // ----------------------------------------------------------------------------- loss/grad ----
@@ -244,50 +358,63 @@ __global__ __launch_bounds__(256) void k_softmax_ce(const float *Z, int K, const
     if (threadIdx.x == 0) lossPart[blockIdx.x] = ((wl[0] + wl[1]) + wl[2]) + wl[3];
 }
 
-__global__ __launch_bounds__(256) void k_count_mask(const uint32_t *mask, uint32_t n, uint32_t *count) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    const bool on = i < n && mask[i] != 0u;
-    const uint64_t b = __ballot(on);
-    if ((threadIdx.x & 63u) == 0u && b) atomicAdd(count, static_cast<uint32_t>(__popcll(b)));
+// samples that train, by one workgroup
+__global__ __launch_bounds__(1024) void k_count_mask(const uint32_t *mask, uint32_t n, uint32_t *count) {
+    __shared__ uint32_t waves[16];
+    uint32_t c = 0;
+    for (uint32_t i = threadIdx.x; i < n; i += 1024u) c += mask[i] != 0u ? 1u : 0u;
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
+    if ((threadIdx.x & 63u) == 0u) waves[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    uint32_t sum = 0;
+    for (int w = 0; w < 16; ++w) sum += waves[w];
+    *count = sum;
 }
 
 __global__ void k_copy_f32(const float *src, float *dst) { *dst = *src; }
 
-// Column sums of a bf16 [rows][cols] matrix in two deterministic steps: workgroup (x, y) sums
-// rows [y*chunk, (y+1)*chunk) of columns [64x, 64x+64) into part[y][col]; k_sum_partials adds
-// the partials of each column in order.
-__global__ __launch_bounds__(256) void k_colsum_partial(const uint16_t *G, int cols, int chunk,
-                                                        float *part) {
-    __shared__ float red[4][64];
-    const int c = blockIdx.x * 64 + static_cast<int>(threadIdx.x & 63);
-    const int r0 = blockIdx.y * chunk, q = static_cast<int>(threadIdx.x >> 6);
-    float sum = 0.0f;
-    for (int r = r0 + q; r < r0 + chunk; r += 4) sum += bf2f(G[static_cast<size_t>(r) * cols + c]);
-    red[q][threadIdx.x & 63] = sum;
-    __syncthreads();
-    if (q == 0) part[static_cast<size_t>(blockIdx.y) * cols + c] = ((red[0][c & 63] + red[1][c & 63]) + red[2][c & 63]) + red[3][c & 63];
-}
-
-// Up to 9 reductions in one launch: for segment j, out_j[i] = sum over s < nParts_j of
+// 8 reductions in one launch: for segment j, out_j[i] = sum over s < nParts_j of
 // part_j[s * count_j + i], in order of s. Lane t of the grid takes element t of the segments laid
-// end to end.
+// end to end; a last workgroup adds the loss, one number of nLoss parts, through LDS (as one lane's
+// loads from memory these took 22 us of 4,096 samples' 1,024).
 struct SumSegments {
-    const float *part[9];
-    float *out[9];
-    int nParts[9];
-    int64_t count[9];
-    int n;
+    const float *part[8];
+    float *out[8];
+    int nParts[8];
+    int64_t count[8];
+    const float *lossPart;
+    float *loss;
+    int nLoss;
 };
 __global__ __launch_bounds__(256) void k_sum_partials(const SumSegments a) {
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ float v[1024];
+        float sum = 0.0f;
+        for (int s0 = 0; s0 < a.nLoss; s0 += 1024) {
+#pragma unroll
+            for (int e = threadIdx.x; e < 1024; e += 256)
+                if (s0 + e < a.nLoss) v[e] = a.lossPart[s0 + e];
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                const int end = a.nLoss - s0 < 1024 ? a.nLoss - s0 : 1024;
+#pragma unroll 16
+                for (int e = 0; e < end; ++e) sum += v[e];
+            }
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) *a.loss = sum;
+        return;
+    }
     int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     int j = 0;
-    while (j < a.n && i >= a.count[j]) i -= a.count[j++];
-    if (j >= a.n) return;
+    while (j < 8 && i >= a.count[j]) i -= a.count[j++];
+    if (j >= 8) return;
     const float *part = a.part[j];
     const int64_t count = a.count[j];
     float sum = 0.0f;
-    // unrolled so that the loads of 8 parts are in flight together; the additions stay in order
-#pragma unroll 8
+    // unrolled so that the loads of 16 parts are in flight together; the additions stay in order
+#pragma unroll 16
     for (int s = 0; s < a.nParts[j]; ++s) sum += part[s * count + i];
     a.out[j][i] = sum;
 }
@@ -424,7 +551,6 @@ struct ProposeArgs {
     uint32_t nSlots;
 };
 
-constexpr int kRow = kIn + 8;                // padded LDS row (bf16) against bank conflicts
 
 __device__ __forceinline__ void stage_weights(uint16_t *wbuf, const uint16_t *src, int rows) {
     // rows x 128 bf16 from global into LDS rows of kRow, 16 bytes per lane per step
@@ -1173,25 +1299,13 @@ __global__ __launch_bounds__(2 * kWideQuads, kWideResident) void k_propose_wide(
 // ----------------------------------------------------------------------------- launchers ----
 namespace rk {
 
-using rm::GemmArgs;
 using rm::kHidden;
 using rm::kIn;
 using rt::f3;
 
-static void gemm(const GemmArgs &g, hipStream_t s) {
-    RK_LAUNCH("k_gemm", rm::k_gemm, dim3(g.N / 64, g.M / 64), dim3(256), 0, s, g);
-}
-static GemmArgs gemm_args(int M, int N, int K) {
-    GemmArgs g{};
-    g.M = M;
-    g.N = N;
-    g.K = K;
-    return g;
-}
-
 // Training tensors carved from one scratch allocation.
 struct MlpScratch {
-    uint16_t *X, *H[3], *dA, *dB, *dZ;
+    uint16_t *X, *H[3], *dH[3], *dZ;
     float *Z, *gw, *gb, *loss;
     float *part;      // split-K and column-sum partials
     float *lossPart;  // per-workgroup loss sums of k_softmax_ce
@@ -1221,8 +1335,7 @@ static MlpScratch carve_mlp(void *base, uint32_t n, int K, size_t *bytes = nullp
     MlpScratch m;
     m.X = c.take<uint16_t>(2 * nn * kIn);
     for (int l = 0; l < 3; ++l) m.H[l] = c.take<uint16_t>(2 * nn * kHidden);
-    m.dA = c.take<uint16_t>(2 * nn * kHidden);
-    m.dB = c.take<uint16_t>(2 * nn * kHidden);
+    for (int l = 0; l < 3; ++l) m.dH[l] = c.take<uint16_t>(2 * nn * kHidden);
     m.dZ = c.take<uint16_t>(2 * nn * kk);
     m.Z = c.take<float>(4 * nn * kk);
     m.target = c.take<int32_t>(4 * nn);
@@ -1243,32 +1356,12 @@ size_t mlp_scratch_bytes(uint32_t n, int K) {
     return bytes;
 }
 
-// forward through the GEMM path, keeping the hidden activations for the backward pass
+// forward, keeping the hidden activations for the backward pass
 static void mlp_fwd(const restir_mlp &m, const uint16_t *X, uint32_t n, const MlpScratch &t, float *logits,
                     hipStream_t s) {
     const int K = static_cast<int>(m.n_clusters);
-    const uint16_t *in = X;
-    for (int l = 0; l < 4; ++l) {
-        const int N = l < 3 ? kHidden : K;
-        GemmArgs g = gemm_args(static_cast<int>(n), N, kIn);
-        g.A = in;
-        g.sam = kIn;
-        g.sak = 1;
-        g.B = m.weights_bf16 + rm::w_off(l);  // B(k, o) = W[o][k]
-        g.sbk = 1;
-        g.sbn = kIn;
-        g.bias = m.bias + rm::b_off(l);
-        g.scm = N;
-        g.scn = 1;
-        if (l < 3) {
-            g.relu = 1;
-            g.Cb = t.H[l];
-            in = t.H[l];
-        } else {
-            g.Cf = logits;
-        }
-        gemm(g, s);
-    }
+    rm::ForwardArgs a{X, m.weights_bf16, m.bias, {t.H[0], t.H[1], t.H[2]}, logits, K, K <= 256 ? K : (K % 256 == 0 ? 256 : 128)};
+    RK_LAUNCH("k_mlp_forward", rm::k_mlp_forward, dim3(n / rm::kMlpRows, K / a.cols), dim3(256), 0, s, a);
 }
 
 hipError_t mlp_forward(const restir_mlp &m, const uint16_t *X, uint32_t n, float *logits, void *scratch,
@@ -1284,80 +1377,44 @@ static void mlp_loss_grad_impl(const restir_mlp &m, const uint16_t *X, const int
                                float *loss, bool countMask, hipStream_t s) {
     const int K = static_cast<int>(m.n_clusters);
     const int nn = static_cast<int>(n);
-    if (countMask) {
-        RK_LAUNCH("k_zero_u32", k_zero_u32, dim3(1), dim3(64), 0, s, t.nValid, 1u);
-        RK_LAUNCH("k_count_mask", rm::k_count_mask, dim3((n + 255) / 256), dim3(256), 0, s, mask, n, t.nValid);
-    }
+    if (countMask)
+        RK_LAUNCH("k_count_mask", rm::k_count_mask, dim3(1), dim3(1024), 0, s, mask, n, t.nValid);
     mlp_fwd(m, X, n, t, t.Z, s);
     RK_LAUNCH("k_softmax_ce", rm::k_softmax_ce, dim3((n + 3) / 4), dim3(256), 0, s, t.Z, K, target, mask, nn,
                        t.nValid, t.dZ, t.lossPart);
-    // layer 4: gW4[o][k] = sum_b dZ[b][o] H3[b][k]
-    const uint16_t *dY = t.dZ;
-    int N = K;
-    rm::SumSegments sums{};
-    // the loss: the workgroups' sums of k_softmax_ce, in order
-    sums.part[0] = t.lossPart;
-    sums.nParts[0] = (nn + 3) / 4;
-    sums.count[0] = 1;
-    sums.out[0] = loss;
-    sums.n = 1;
-    int64_t sumCount = 1;
+    const rm::BackwardArgs back{t.dZ, m.weights_bf16, {t.H[0], t.H[1], t.H[2]}, {t.dH[0], t.dH[1], t.dH[2]}, K};
+    RK_LAUNCH("k_mlp_backward", rm::k_mlp_backward, dim3(n / rm::kMlpRows), dim3(256), 0, s, back);
+    // the gradients' partial sums of all four layers, then each summed in a fixed order, with the
+    // loss: the workgroups' sums of k_softmax_ce, in order
     const int chunks = nn / 64;
     float *partB = t.part + static_cast<size_t>(kMaxSplit) * (3 * static_cast<size_t>(kHidden) + K) * kIn;
-    for (int l = 3; l >= 0; --l) {
+    rm::GradArgs ga{};
+    rm::SumSegments sums{};
+    ga.n = nn;
+    uint32_t biasGroups = 0;
+    int64_t sumCount = 0;
+    for (int l = 3; l >= 0; --l) {  // the largest first
+        const int j = 3 - l, N = l == 3 ? K : kHidden, sp = split_for(N, kIn, nn);
         float *pw = t.part + static_cast<size_t>(kMaxSplit) * rows_before(l) * kIn;
         float *pb = partB + static_cast<size_t>(chunks) * rows_before(l);
-        const uint16_t *in = l > 0 ? t.H[l - 1] : X;
-        // split-K partials over the samples, then an in-order reduction (deterministic)
-        const int sp = split_for(N, kIn, nn);
-        GemmArgs gwA = gemm_args(N, kIn, nn);
-        gwA.A = dY;      // A(o, b) = dY[b][o]
-        gwA.sam = 1;
-        gwA.sak = N;
-        gwA.B = in;      // B(b, k) = in[b][k]
-        gwA.sbk = kIn;
-        gwA.sbn = 1;
-        gwA.Cf = pw;
-        gwA.scm = kIn;
-        gwA.scn = 1;
-        gwA.kChunk = nn / sp;
-        gwA.scz = static_cast<int64_t>(N) * kIn;
-        RK_LAUNCH("k_gemm_splitk", rm::k_gemm, dim3(kIn / 64, N / 64, sp), dim3(256), 0, s, gwA);
-        // bias gradients: column sums of dY over 64-row chunks (added in order below)
-        RK_LAUNCH("k_colsum_partial", rm::k_colsum_partial, dim3(N / 64, chunks), dim3(256), 0, s, dY, N, 64, pb);
-        const int seg = sums.n;
-        sums.part[seg] = pw;
-        sums.nParts[seg] = sp;
-        sums.count[seg] = static_cast<int64_t>(N) * kIn;
-        sums.out[seg] = gw + rm::w_off(l);
-        sums.part[seg + 1] = pb;
-        sums.nParts[seg + 1] = chunks;
-        sums.count[seg + 1] = N;
-        sums.out[seg + 1] = gb + rm::b_off(l);
-        sums.n = seg + 2;
-        sumCount += sums.count[seg] + sums.count[seg + 1];
-        if (l == 0) break;
-        // dIn[b][k] = sum_o dY[b][o] W[o][k], gated by the ReLU of the layer below
-        uint16_t *dIn = (dY == t.dA) ? t.dB : t.dA;
-        GemmArgs gd = gemm_args(nn, kIn, N);
-        gd.A = dY;
-        gd.sam = N;
-        gd.sak = 1;
-        gd.B = m.weights_bf16 + rm::w_off(l);  // B(o, k) = W[o][k]
-        gd.sbk = kIn;
-        gd.sbn = 1;
-        gd.gate = t.H[l - 1];
-        gd.sgm = kIn;
-        gd.sgn = 1;
-        gd.Cb = dIn;
-        gd.scm = kIn;
-        gd.scn = 1;
-        gemm(gd, s);
-        dY = dIn;
-        N = kHidden;
+        ga.layer[l] = rm::GradLayer{l == 3 ? t.dZ : t.dH[l], l > 0 ? t.H[l - 1] : X, pw, pb, N, sp, ga.weightGroups, biasGroups};
+        ga.weightGroups += static_cast<uint32_t>(kIn / 64 * (N / 64) * sp);
+        biasGroups += static_cast<uint32_t>(N / 64 * chunks);
+        sums.part[2 * j] = pw;
+        sums.nParts[2 * j] = sp;
+        sums.count[2 * j] = static_cast<int64_t>(N) * kIn;
+        sums.out[2 * j] = gw + rm::w_off(l);
+        sums.part[2 * j + 1] = pb;
+        sums.nParts[2 * j + 1] = chunks;
+        sums.count[2 * j + 1] = N;
+        sums.out[2 * j + 1] = gb + rm::b_off(l);
+        sumCount += sums.count[2 * j] + N;
     }
-    // the split-K and bias partials of all four layers, each summed in a fixed order
-    RK_LAUNCH("k_sum_partials", rm::k_sum_partials, dim3(static_cast<uint32_t>((sumCount + 255) / 256)), dim3(256), 0,
+    RK_LAUNCH("k_mlp_grads", rm::k_mlp_grads, dim3(ga.weightGroups + biasGroups), dim3(256), 0, s, ga);
+    sums.lossPart = t.lossPart;
+    sums.loss = loss;
+    sums.nLoss = (nn + 3) / 4;
+    RK_LAUNCH("k_sum_partials", rm::k_sum_partials, dim3(static_cast<uint32_t>((sumCount + 255) / 256) + 1), dim3(256), 0,
               s, sums);
 }
 
