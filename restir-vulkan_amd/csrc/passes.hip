@@ -215,6 +215,14 @@ __device__ __forceinline__ AliasColumn<RECORDS> load_column(const SceneView &sc,
     return k;
 }
 
+// The reservoir's W once RIS has seen all candidates.
+__device__ __forceinline__ void finish_ris(const PassAArgs &a, const RisTaken &taken, Res &res) {
+    res.w = ris_w(taken, res.pHat);
+    // the standard RIS contribution weight instead of the selection-time one
+    if ((a.u.flags & RESTIR_STANDARD_WEIGHTS_FLAG) && res.w > 0.0f)
+        res.w = res.sumW / (static_cast<float>(res.M) * res.pHat);
+}
+
 // Initial RIS over M candidates (alias table or the learned proposal's list).
 template <bool RECORDS>
 __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurface &ps, Res &res, Pcg &rng) {
@@ -322,9 +330,7 @@ __device__ __forceinline__ void pass_a_ris(const PassAArgs &a, const PassASurfac
         }
         rng.state = st;
     }
-    res.w = ris_w(taken, res.pHat);
-    // the standard RIS contribution weight instead of the selection-time one
-    if (standard && res.w > 0.0f) res.w = res.sumW / (static_cast<float>(res.M) * res.pHat);
+    finish_ris(a, taken, res);
 }
 
 // Temporal reuse of the previous frame's reservoir at the reprojected pixel.
@@ -1310,6 +1316,104 @@ __global__ __launch_bounds__(TX *TY) void k_pass_a_ris(const PassAArgs a, const 
     }
 }
 
+// Lane j of each four lanes' value.
+template <int J>
+__device__ __forceinline__ float quad_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x55 * J, 0xf, 0xf, false));
+}
+
+// k_pass_a_ris for small images and tables of point lights alone: four lanes per pixel, each drawing
+// and evaluating every fourth candidate (3 draws each, so candidate i's first state is a jump of 3 i);
+// the reservoir's updates follow in order on all four, from each other's weights. With a lane per
+// pixel, a small image's few waves wait for 32 candidates one after another: 256x256, M = 32, 64
+// lights 36 -> 25 us (split_pays has the limits).
+constexpr int kSplitX = 8, kSplitY = 8;
+__global__ __launch_bounds__(256) void k_pass_a_ris_split(const PassAArgs a, const AQueues q) {
+    const uint32_t pixel = threadIdx.x >> 2, sub = threadIdx.x & 3u;
+    const uint32_t t = xcd_tile(blockIdx.x, a.nTiles);
+    const uint32_t x = t % a.tilesX * kSplitX + pixel % kSplitX, y = t / a.tilesX * kSplitY + pixel / kSplitX;
+    const bool inside = x < a.u.screenSize[0] && y < a.u.screenSize[1];
+    bool emit = false;
+    size_t idx = 0;
+    f3 pos{0.0f, 0.0f, 0.0f}, lp{0.0f, 0.0f, 0.0f};
+    if (inside) {  // the same for a pixel's four lanes
+        const PassASurface ps = pass_a_surface(a, x, y);
+        idx = ps.idx;
+        pos = ps.pos;
+        Res res = res_zero();
+        RisTaken taken;
+        Pcg rng = pass_a_rng(a, x, y);
+        const uint32_t M = a.u.initialLightSampleCount;
+        if (dot(ps.n, ps.n) != 0.0f && M > 0) {
+            const SceneView &sc = a.sc;
+            const uint64_t inc = rng.inc;
+            const uint64_t mul = sub == 0 ? 1ull : sub == 1 ? pcg_mul_pow(3) : sub == 2 ? pcg_mul_pow(6) : pcg_mul_pow(9);
+            const uint64_t add = sub == 0 ? 0ull : sub == 1 ? pcg_mul_sum(3) : sub == 2 ? pcg_mul_sum(6) : pcg_mul_sum(9);
+            uint64_t st = rng.state * mul + inc * add, before = st;  // the lane's candidate's first state
+            f3 L{0.0f, 0.0f, 0.0f};                                  // of the lane's candidate taken last
+            float lum = 0.0f, pHat = 0.0f;
+            int32_t light = 0;
+            for (uint32_t i = 0; i < M; i += 4) {
+                const uint64_t s1 = st * kPcgMul + inc;
+                const int32_t col = alias_column(sc, pcg_float_at(st));
+                const float4 c = sc.alias[col];
+                const bool keep = c.x > pcg_float_at(s1);
+                const int32_t li = keep ? col : __float_as_int(c.y);
+                const float4 point = point_light(sc, li);
+                const float ph = eval_phat(ps.s, xyz(point), f3{0.0f, 0.0f, 0.0f}, false, point.w);
+                const float weight = ris_weight(ph, keep ? c.z : c.w), u = pcg_float_at(s1 * kPcgMul + inc);
+                const auto update = [&](uint32_t j, float wj, float uj) {
+                    if (i + j >= M) return;
+                    res.M += 1u;
+                    if (!res_takes(res, wj, uj)) return;
+                    taken.sumW = res.sumW;
+                    taken.M = res.M;
+                    if (j != sub) return;
+                    L = xyz(point);
+                    lum = point.w;
+                    pHat = ph;
+                    light = li;
+                };
+                update(0, quad_lane<0>(weight), quad_lane<0>(u));
+                update(1, quad_lane<1>(weight), quad_lane<1>(u));
+                update(2, quad_lane<2>(weight), quad_lane<2>(u));
+                update(3, quad_lane<3>(weight), quad_lane<3>(u));
+                before = st;
+                st = st * pcg_mul_pow(12) + inc * pcg_mul_sum(12);
+            }
+            // candidate M's first state, and the candidate taken last, from the lanes that have them
+            const int quad = static_cast<int>(threadIdx.x & 60u), at = quad + static_cast<int>(M & 3u);
+            const uint64_t mine = (M & 3u) ? before : st;
+            rng.state = static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(mine), at))) |
+                        static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(mine >> 32), at))) << 32;
+            if (taken.M) {
+                const int w = quad + static_cast<int>((taken.M - 1u) & 3u);
+                res.pos = f3{__shfl(L.x, w), __shfl(L.y, w), __shfl(L.z, w)};
+                res.emLum = __shfl(lum, w);
+                res.pHat = __shfl(pHat, w);
+                res.lightIndex = __shfl(light, w);
+                res.normal = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                res.w = 0.0f;
+            }
+        }
+        finish_ris(a, taken, res);
+        if (sub == 0) {
+            store_res(a.out, idx, res);
+            q.rng[idx] = rng.state;
+            q.occ[idx] = 0u;
+            emit = (a.u.flags & RESTIR_VISIBILITY_REUSE_FLAG) && res.sumW != 0.0f;
+            lp = res.pos;
+        }
+    }
+    __shared__ uint2 reserve[5];
+    const uint2 rank = wave_rank(emit);
+    const uint32_t slot = group_reserve<4>(reinterpret_cast<unsigned long long *>(q.counter), rank.y, 0u, reserve).x + rank.x;
+    if (emit) {
+        q.p1[slot] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(static_cast<uint32_t>(idx)));
+        q.p2[slot] = make_float4(lp.x, lp.y, lp.z, 0.0f);
+    }
+}
+
 template <int TX, int TY>
 __global__ __launch_bounds__(TX *TY) void k_pass_a_finish(const PassAArgs a, const AQueues q) {
     uint32_t x, y;
@@ -1762,6 +1866,16 @@ size_t pass_a_queue_bytes(uint32_t npx) {
     return bytes;
 }
 
+// Where four lanes per pixel pay (k_pass_a_ris_split): while the image leaves most of the chip idle,
+// and with enough candidates to make up for the surface that all four lanes set up. A lane per pixel
+// against four, M = 32, 64 lights: 64x64 33 against 14 us, 256x256 36 against 25, 400x300 41 against
+// 38, 512x512 63 against 67, 1920x1080 351 against 397; 256x256, M = 8: 14 against 16, M = 16:
+// 21 against 18; 416x312, M = 16: 27 against 29.
+static bool split_pays(const PassAArgs &a) {
+    return !a.candLight && a.sc.nPoints > 0 && !a.sc.mixed && a.u.initialLightSampleCount >= 16 &&
+           static_cast<uint64_t>(a.u.screenSize[0]) * a.u.screenSize[1] <= 98304u;
+}
+
 template <int TX, int TY, int STACK>
 static hipError_t run_a_queued(PassAArgs args, const AQueues &q, uint32_t gridCap, hipStream_t s) {
     grid_for<TX, TY>(args.u.screenSize[0], args.u.screenSize[1], args.tilesX, args.nTiles);
@@ -1771,6 +1885,10 @@ static hipError_t run_a_queued(PassAArgs args, const AQueues &q, uint32_t gridCa
         RK_LAUNCH("k_light_records", k_light_records, dim3((args.sc.nAlias + 255) / 256), dim3(256), 0, s, args.sc,
                   const_cast<float4 *>(args.records));
         RK_LAUNCH("k_pass_a_ris", (k_pass_a_ris<TX, TY, true>), tiles, block, 0, s, args, q);
+    } else if (split_pays(args)) {
+        PassAArgs split = args;
+        grid_for<kSplitX, kSplitY>(args.u.screenSize[0], args.u.screenSize[1], split.tilesX, split.nTiles);
+        RK_LAUNCH("k_pass_a_ris_split", k_pass_a_ris_split, dim3(split.nTiles), dim3(256), 0, s, split, q);
     } else {
         RK_LAUNCH("k_pass_a_ris", (k_pass_a_ris<TX, TY, false>), tiles, block, 0, s, args, q);
     }

@@ -380,15 +380,18 @@ RT_HD Res res_zero() {
     r.M = 0u;
     return r;
 }
-// updateReservoirAt, reservoir.glsl:6-26
-// u: the update's uniform draw; returns true when the sample is taken
-__device__ __forceinline__ bool res_update_u(Res &r, float weight, f3 pos, float4 n, float emLum, int32_t li, float pHat,
-                                             float w, float u) {
+// updateReservoirAt, reservoir.glsl:6-26, in two parts: whether the sample is taken (u: the update's
+// uniform draw), and the update, which returns that
+__device__ __forceinline__ bool res_takes(Res &r, float weight, float u) {
     r.sumW += weight;
     if (weight == 0.0f) return false;  // u < 0 / sumW never holds
     const float rp = mid_range(weight) && mid_range(r.sumW) ? div_near(weight, r.sumW, rcp_near(r.sumW))
                                                             : weight / r.sumW;
-    if (u < rp) {
+    return u < rp;
+}
+__device__ __forceinline__ bool res_update_u(Res &r, float weight, f3 pos, float4 n, float emLum, int32_t li, float pHat,
+                                             float w, float u) {
+    if (res_takes(r, weight, u)) {
         r.pos = pos;
         r.emLum = emLum;
         r.normal = n;
@@ -409,13 +412,15 @@ struct RisTaken {
     float sumW = 0.0f;
     uint32_t M = 0u;  // 0: none was taken
 };
+__device__ __forceinline__ float ris_weight(float pHat, float sampleP) {
+    return (mid_range(pHat) || __float_as_uint(pHat) == 0u) && mid_range(sampleP)
+               ? div_near(pHat, sampleP, rcp_near(sampleP))
+               : pHat / sampleP;
+}
 __device__ __forceinline__ void res_add_sample_u(Res &r, RisTaken &taken, f3 pos, float4 n, float emLum, int32_t li,
                                                  float pHat, float sampleP, float u) {
-    const float weight = (mid_range(pHat) || __float_as_uint(pHat) == 0u) && mid_range(sampleP)
-                             ? div_near(pHat, sampleP, rcp_near(sampleP))
-                             : pHat / sampleP;
     r.M += 1u;
-    if (res_update_u(r, weight, pos, n, emLum, li, pHat, 0.0f, u)) {
+    if (res_update_u(r, ris_weight(pHat, sampleP), pos, n, emLum, li, pHat, 0.0f, u)) {
         taken.sumW = r.sumW;
         taken.M = r.M;
     }
