@@ -560,25 +560,6 @@ __device__ __forceinline__ void stage_weights(uint16_t *wbuf, const uint16_t *sr
     }
 }
 
-template <int NB>
-__device__ __forceinline__ void layer_mfma(const uint16_t *act, const uint16_t *wbuf, const float *bias,
-                                           int wave, int lane, f32x16 (&acc)[NB]) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        const float bv = bias[32 * nb + (lane & 31)];
-        for (int i = 0; i < 16; ++i) acc[nb][i] = bv;
-    }
-#pragma unroll
-    for (int s = 0; s < kIn / 16; ++s) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&act[(32 * wave + (lane & 31)) * kRow + 16 * s + 8 * (lane >> 5)]);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const bf16x8 b = *reinterpret_cast<const bf16x8 *>(&wbuf[(32 * nb + (lane & 31)) * kRow + 16 * s + 8 * (lane >> 5)]);
-            acc[nb] = mfma32(a, b, acc[nb]);
-        }
-    }
-}
-
 __device__ __forceinline__ float4 unpack_h4(uint2 v) {  // four fp16 -> float
     const float2 lo = __half22float2(__builtin_bit_cast(__half2, v.x));
     const float2 hi = __half22float2(__builtin_bit_cast(__half2, v.y));
@@ -599,100 +580,188 @@ __device__ __forceinline__ uint32_t quad_pixel(const rk::GView &g, uint32_t qx, 
     return y0 * g.W + x0;
 }
 
-// Features of the workgroup's TILE quads (2 * TILE lanes, a wave per 32 quads) and the three
-// hidden layers: leaves H3 in `act` (bf16 rows of kRow) and the first `outRows` rows of W4 staged
-// in `wbuf`. Ends with a barrier.
-template <int TILE>
-__device__ __forceinline__ void propose_hidden(const ProposeArgs &a, uint16_t *act, uint16_t *wbuf, uint32_t q0,
-                                               uint32_t QW, uint32_t QH, int outRows) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // features (lanes 0..TILE-1) while the other TILE lanes stage W1
-    if (tid < TILE) {
-        const uint32_t qd = q0 + tid;
-        uint16_t *row = act + tid * kRow;
-        if (qd < QW * QH) pixel_features(a.f, quad_pixel(a.f.g, qd % QW, qd / QW), row);
-        else for (int k = 0; k < kIn; ++k) row[k] = 0;
-    } else {
-        for (int e = tid - TILE; e < kHidden * (kIn / 8); e += TILE) {
-            const int r = e / (kIn / 8), c = (e % (kIn / 8)) * 8;
-            *reinterpret_cast<uint4 *>(&wbuf[r * kRow + c]) = *reinterpret_cast<const uint4 *>(&a.wbf[r * kIn + c]);
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// lanes 32..63 of x change places with lanes 0..31 of y
+__device__ __forceinline__ void swap_halves(uint32_t &x, uint32_t &y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = r[0];
+    y = r[1];
+}
+__device__ __forceinline__ void swap_halves(float &x, float &y) {
+    uint32_t a = __float_as_uint(x), b = __float_as_uint(y);
+    swap_halves(a, b);
+    x = __uint_as_float(a);
+    y = __uint_as_float(b);
+}
+
+// a barrier for LDS alone: __syncthreads would also wait for the global stores under way
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// 64 outputs of a layer for the wave's 32 quads: rows of staged weights times the activations, on
+// top of the bias. The first half's weights are all read before its products and the second's while
+// they run: a read takes as long as four products, and left to itself the compiler puts each read
+// right before its product.
+__device__ __forceinline__ void wide_blocks(const uint16_t *w, const float *bias, const bf16x8 (&h)[kIn / 16], int lane,
+                                            f32x16 &z0, f32x16 &z1) {
+    constexpr int kSteps = kIn / 16;
+    auto start = [&](f32x16 &z, const float *b) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const float4 v = *reinterpret_cast<const float4 *>(b + 8 * g + 4 * (lane >> 5));
+            z[4 * g] = v.x;
+            z[4 * g + 1] = v.y;
+            z[4 * g + 2] = v.z;
+            z[4 * g + 3] = v.w;
+        }
+    };
+    const uint16_t *at = w + (lane & 31) * kRow + 8 * (lane >> 5);
+    bf16x8 f0[kSteps], f1[kSteps];
+    start(z0, bias);
+    start(z1, bias + 32);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) f0[s] = *reinterpret_cast<const bf16x8 *>(at + 16 * s);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+        z0 = mfma32(f0[s], h[s], z0);
+        f1[s] = *reinterpret_cast<const bf16x8 *>(at + 32 * kRow + 16 * s);
+    }
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) z1 = mfma32(f1[s], h[s], z1);
+    __builtin_amdgcn_sched_group_barrier(0x100, 8 + kSteps, 0);  // LDS reads: both biases, the first half
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    // a product
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
+    }
+    __builtin_amdgcn_sched_group_barrier(0x8, kSteps, 0);
+}
+
+// A hidden layer for the wave's 32 quads: its 128 outputs, clamped, as the next layer's operand.
+__device__ __forceinline__ void wide_hidden(const uint16_t *w, const float *bias, bf16x8 (&h)[kIn / 16], int lane) {
+    bf16x8 out[kIn / 16];
+    f32x16 z[2];
+#pragma unroll
+    for (int nb = 0; nb < kHidden / 32; ++nb) {
+        if (nb % 2 == 0) wide_blocks(w + 32 * nb * kRow, bias + 32 * nb, h, lane, z[0], z[1]);
+        const f32x16 &acc = z[nb % 2];
+        uint32_t d[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float lo = acc[2 * i], hi = acc[2 * i + 1];
+            d[i] = f2bf2(lo > 0.0f ? lo : 0.0f, hi > 0.0f ? hi : 0.0f);
+        }
+        // outputs 8g + 4 * (lane / 32) + 0..3 lie in d[2g], d[2g + 1]; the operand wants
+        // 8 * (lane / 32) + 0..7 of each 16
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            swap_halves(d[4 * s], d[4 * s + 2]);
+            swap_halves(d[4 * s + 1], d[4 * s + 3]);
+            out[2 * nb + s] = __builtin_bit_cast(bf16x8, make_uint4(d[4 * s], d[4 * s + 1], d[4 * s + 2], d[4 * s + 3]));
         }
     }
-    __syncthreads();
-    for (int L = 0; L < 3; ++L) {
-        f32x16 acc[4];
-        layer_mfma<4>(act, wbuf, a.bias + b_off(L), wave, lane, acc);
-        __syncthreads();
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int row = 32 * wave + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-                const float v = acc[nb][i];
-                act[row * kRow + 32 * nb + (lane & 31)] = f2bf(v > 0.0f ? v : 0.0f);
-            }
-        stage_weights(wbuf, a.wbf + w_off(L + 1), L + 1 < 3 ? kHidden : outRows);
-        __syncthreads();
-    }
+    for (int s = 0; s < kIn / 16; ++s) h[s] = out[s];
 }
 
 // One workgroup of 256 lanes (4 waves) proposes for kProposeTile = 128 pixel quads (2x2 pixels
 // each): one MLP evaluation per quad, each pixel drawing its own candidates from the quad's
-// distribution with its own random stream (q is that distribution, so RIS stays unbiased). LDS
-// holds the activations [128][136] bf16 and 128 rows of one layer's weights (W4 of K = 256 in two
-// halves); after the last layer the same LDS holds the fp16 softmax numerators [128][K + 4].
-// 69.6 KB of LDS lets two workgroups share a CU, so one's barriers and loads overlap the other's
-// work.
+// distribution with its own random stream (q is that distribution, so RIS stays unbiased). A wave
+// holds 32 quads in the columns of its products (wide_blocks), so activations and logits stay in
+// registers; LDS holds the features and the first layer's weights, then one layer's weights (128
+// rows) while the next one's arrive, and last the fp16 softmax numerators [128][K + 4]. 72 KB of LDS
+// let two workgroups share a CU, so one's barriers and loads overlap the other's work. 1920x1080,
+// K = 256, M = 8: 403 -> 344 us against activations kept in LDS, 208 of them for the draws, which
+// wait for the tables.
 constexpr int kProposeTile = 128;
 template <int KC>
-__global__ __launch_bounds__(2 * kProposeTile) void k_propose(const ProposeArgs a) {
-    constexpr int T = kProposeTile;
+__global__ __launch_bounds__(2 * kProposeTile, 2) void k_propose(const ProposeArgs a) {
+    constexpr int T = kProposeTile, kOut = KC < 128 ? KC : 128;  // rows of W4 staged at a time
     __shared__ __align__(16) uint16_t lds[2 * T * kRow];
+    __shared__ __align__(16) float bias[3 * kHidden + KC];
     static_assert(T * (KC + 4) <= 2 * T * kRow, "softmax numerators fit the LDS tile");
-    uint16_t *act = lds;
-    uint16_t *wbuf = lds + T * kRow;
+    static_assert(KC == 64 || KC % 128 == 0, "W4 in whole blocks");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // one MLP row per 2x2 pixel quad: the quad's first surface pixel in the order (0,0), (1,0),
     // (0,1), (1,1) stands for it (quad_pixel)
     const uint32_t W = a.f.g.W, H = a.f.g.H, QW = (W + 1) / 2, QH = (H + 1) / 2;
     const uint32_t q0 = blockIdx.x * T;
-    propose_hidden<T>(a, act, wbuf, q0, QW, QH, KC < 128 ? KC : 128);
-    {
-        f32x16 acc[KC / 32];
-        if constexpr (KC <= 128) {
-            layer_mfma<KC / 32>(act, wbuf, a.bias + b_off(3), wave, lane, acc);
+    // features by the first T lanes while the others stage W1
+    for (int e = tid; e < 3 * kHidden + KC; e += 2 * T) bias[e] = a.bias[e];
+    if (tid < T) {
+        const uint32_t qd = q0 + tid;
+        uint16_t *row = lds + tid * kRow;
+        if (qd < QW * QH) pixel_features(a.f, quad_pixel(a.f.g, qd % QW, qd / QW), row);
+        else for (int k = 0; k < kIn; ++k) row[k] = 0;
+    } else {
+        for (int e = tid - T; e < kHidden * (kIn / 8); e += T)
+            *reinterpret_cast<u32x4 *>(&lds[(T + e / (kIn / 8)) * kRow + e % (kIn / 8) * 8]) =
+                *reinterpret_cast<const u32x4 *>(a.wbf + e * 8);
+    }
+    __syncthreads();
+    bf16x8 h[kIn / 16];
+#pragma unroll
+    for (int s = 0; s < kIn / 16; ++s)
+        h[s] = *reinterpret_cast<const bf16x8 *>(&lds[(32 * wave + (lane & 31)) * kRow + 16 * s + 8 * (lane >> 5)]);
+    __syncthreads();
+    // step L multiplies the weights in buffer (L + 1) & 1 and brings the next ones to the other: the
+    // hidden layers, then the output layer 128 clusters at a time
+    constexpr int kSteps = 3 + KC / kOut;
+    f32x16 acc[KC / 32];
+#pragma unroll
+    for (int L = 0; L < kSteps; ++L) {
+        constexpr int kPer = kHidden * kIn / 8 / (2 * T);  // 16-byte pieces per lane
+        u32x4 next[kPer];
+        const int rows = L + 1 < 3 ? kHidden : kOut;
+        const uint16_t *src = a.wbf + (L + 1 < 3 ? w_off(L + 1) : w_off(3) + static_cast<size_t>(L + 1 - 3) * kOut * kIn);
+        if (L + 1 < kSteps)
+#pragma unroll
+            for (int e = 0; e < kPer; ++e)
+                if ((e * 2 * T) / (kIn / 8) < rows) next[e] = *reinterpret_cast<const u32x4 *>(src + (e * 2 * T + tid) * 8);
+        const uint16_t *w = lds + ((L + 1) & 1) * T * kRow;
+        if (L < 3) {
+            wide_hidden(w, bias + b_off(L), h, lane);
         } else {
-            static_assert(KC == 256, "W4 in two halves of 128 rows");
-            f32x16 lo[4], hi[4];
-            layer_mfma<4>(act, wbuf, a.bias + b_off(3), wave, lane, lo);
-            __syncthreads();
-            stage_weights(wbuf, a.wbf + w_off(3) + 128 * kIn, 128);
-            __syncthreads();
-            layer_mfma<4>(act, wbuf, a.bias + b_off(3) + 128, wave, lane, hi);
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                acc[nb] = lo[nb];
-                acc[nb + 4] = hi[nb];
+            for (int nb = 0; nb < kOut / 32; nb += 2)
+                wide_blocks(w + 32 * nb * kRow, bias + b_off(3) + (L - 3) * kOut + 32 * nb, h, lane,
+                            acc[(L - 3) * (kOut / 32) + nb], acc[(L - 3) * (kOut / 32) + nb + 1]);
+        }
+        if (L + 1 < kSteps)
+#pragma unroll
+            for (int e = 0; e < kPer; ++e) {
+                const int at = e * 2 * T + tid;
+                if ((e * 2 * T) / (kIn / 8) < rows)
+                    *reinterpret_cast<u32x4 *>(&lds[((L & 1) * T + at / (kIn / 8)) * kRow + at % (kIn / 8) * 8]) = next[e];
             }
-        }
         __syncthreads();
-        // softmax numerators e = exp(z - rowmax) as fp16 rows of KC + 4 halves: the row maximum
-        // is reduced across the 32 lanes holding a row's columns; the padding keeps rows 8-byte
-        // aligned and spreads the per-pixel scans below over the banks (lane t reads dwords
-        // 130 t + c/2, c/2 + 1)
-        __half *e = reinterpret_cast<__half *>(lds);
+    }
+    {
+        // softmax numerators e = exp(z - rowmax) as fp16 rows of KC + 4 halves; the padding keeps
+        // rows 8-byte aligned and spreads these stores and the per-pixel scans below over the banks
+        float m = acc[0][0];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float m = acc[0][i];
+        for (int nb = 0; nb < KC / 32; ++nb)
 #pragma unroll
-            for (int nb = 1; nb < KC / 32; ++nb) m = fmaxf(m, acc[nb][i]);
+            for (int i = 0; i < 16; ++i) m = fmaxf(m, acc[nb][i]);
+        m = fmaxf(m, __shfl_xor(m, 32));
+        __half *row = reinterpret_cast<__half *>(lds) + (32 * wave + (lane & 31)) * (KC + 4) + 4 * (lane >> 5);
 #pragma unroll
-            for (int off = 16; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-            const int row = 32 * wave + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+        for (int nb = 0; nb < KC / 32; ++nb)
 #pragma unroll
-            for (int nb = 0; nb < KC / 32; ++nb)
-                e[row * (KC + 4) + 32 * nb + (lane & 31)] = __float2half(__expf(acc[nb][i] - m));
-        }
+            for (int g = 0; g < 4; ++g) {
+                const f32x2 e0 = {__expf(acc[nb][4 * g] - m), __expf(acc[nb][4 * g + 1] - m)};
+                const f32x2 e1 = {__expf(acc[nb][4 * g + 2] - m), __expf(acc[nb][4 * g + 3] - m)};
+                *reinterpret_cast<uint2 *>(row + 32 * nb + 8 * g) =
+                    make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(e0, f16x2)),
+                               __builtin_bit_cast(uint32_t, __builtin_convertvector(e1, f16x2)));
+            }
         __syncthreads();
     }
     // two lanes per quad, each drawing for one row of its 2x2 pixels
@@ -905,69 +974,6 @@ __host__ __device__ constexpr size_t wide_slot_bytes(int K) {
 static_assert(wide_slot_bytes(kMaxClusters) == 272u * kMaxClusters, "the slot size named above");
 static_assert(kMaxClusters / kSuper * kWideQuads * 4 <= 2 * kWideTile * 2, "a sum per 128 clusters fits the weight buffers");
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-// lanes 32..63 of x change places with lanes 0..31 of y
-__device__ __forceinline__ void swap_halves(uint32_t &x, uint32_t &y) {
-    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-    x = r[0];
-    y = r[1];
-}
-__device__ __forceinline__ void swap_halves(float &x, float &y) {
-    uint32_t a = __float_as_uint(x), b = __float_as_uint(y);
-    swap_halves(a, b);
-    x = __uint_as_float(a);
-    y = __uint_as_float(b);
-}
-
-// a barrier for LDS alone: __syncthreads would also wait for the global stores under way
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// 64 outputs of a layer for the wave's 32 quads: rows of staged weights times the activations, on
-// top of the bias. The first half's weights are all read before its products and the second's while
-// they run: a read takes as long as four products, and left to itself the compiler puts each read
-// right before its product.
-__device__ __forceinline__ void wide_blocks(const uint16_t *w, const float *bias, const bf16x8 (&h)[kIn / 16], int lane,
-                                            f32x16 &z0, f32x16 &z1) {
-    constexpr int kSteps = kIn / 16;
-    auto start = [&](f32x16 &z, const float *b) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const float4 v = *reinterpret_cast<const float4 *>(b + 8 * g + 4 * (lane >> 5));
-            z[4 * g] = v.x;
-            z[4 * g + 1] = v.y;
-            z[4 * g + 2] = v.z;
-            z[4 * g + 3] = v.w;
-        }
-    };
-    const uint16_t *at = w + (lane & 31) * kRow + 8 * (lane >> 5);
-    bf16x8 f0[kSteps], f1[kSteps];
-    start(z0, bias);
-    start(z1, bias + 32);
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) f0[s] = *reinterpret_cast<const bf16x8 *>(at + 16 * s);
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-        z0 = mfma32(f0[s], h[s], z0);
-        f1[s] = *reinterpret_cast<const bf16x8 *>(at + 32 * kRow + 16 * s);
-    }
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) z1 = mfma32(f1[s], h[s], z1);
-    __builtin_amdgcn_sched_group_barrier(0x100, 8 + kSteps, 0);  // LDS reads: both biases, the first half
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    // a product
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
-    }
-    __builtin_amdgcn_sched_group_barrier(0x8, kSteps, 0);
-}
-
 __global__ __launch_bounds__(2 * kWideQuads, kWideResident) void k_propose_wide(const ProposeArgs a) {
     __shared__ __align__(16) uint16_t lds[2 * kWideTile];
     __shared__ __align__(16) float bias[2 * kWideRows];
@@ -1024,29 +1030,7 @@ __global__ __launch_bounds__(2 * kWideQuads, kWideResident) void k_propose_wide(
         stage_weights(lds, a.wbf + w_off(L), kHidden);
         if (tid < kHidden) bias[tid] = a.bias[b_off(L) + tid];
         __syncthreads();
-        bf16x8 out[kIn / 16];
-        f32x16 z[2];
-#pragma unroll
-        for (int nb = 0; nb < kHidden / 32; ++nb) {
-            if (nb % 2 == 0) wide_blocks(lds + 32 * nb * kRow, bias + 32 * nb, h, lane, z[0], z[1]);
-            const f32x16 &acc = z[nb % 2];
-            uint32_t d[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float lo = acc[2 * i], hi = acc[2 * i + 1];
-                d[i] = f2bf2(lo > 0.0f ? lo : 0.0f, hi > 0.0f ? hi : 0.0f);
-            }
-            // outputs 8g + 4 * (lane / 32) + 0..3 lie in d[2g], d[2g + 1]; the operand wants
-            // 8 * (lane / 32) + 0..7 of each 16
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                swap_halves(d[4 * s], d[4 * s + 2]);
-                swap_halves(d[4 * s + 1], d[4 * s + 3]);
-                out[2 * nb + s] = __builtin_bit_cast(bf16x8, make_uint4(d[4 * s], d[4 * s + 1], d[4 * s + 2], d[4 * s + 3]));
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < kIn / 16; ++s) h[s] = out[s];
+        wide_hidden(lds, bias, h, lane);
     }
     __syncthreads();
 
