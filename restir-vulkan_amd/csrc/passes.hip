@@ -667,7 +667,15 @@ __device__ __forceinline__ uint2 wave_rank(bool emit) {
 // Position and normal of every pixel in one 32-byte record: the merge's horizon test and the
 // neighbour-ray emission gather them for random neighbours, one sector per neighbour instead of
 // one line per plane.
-__global__ __launch_bounds__(256) void k_pack_surface(const GView g, uint32_t npx, float4 *surf) {
+// A queued pass's work counters, cleared by the first workgroup of a kernel ahead of their first use
+__device__ __forceinline__ void clear_counters(uint32_t *counter, uint32_t *heads) {
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x < 2) counter[threadIdx.x] = 0u;
+    if (threadIdx.x < kTraceShards) heads[threadIdx.x * kTraceShardStride] = 0u;
+}
+__global__ __launch_bounds__(256) void k_pack_surface(const GView g, uint32_t npx, float4 *surf, uint32_t *counter,
+                                                      uint32_t *heads) {
+    clear_counters(counter, heads);
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= npx) return;
     const f3 p = plane3(g.pos, i, g.P), n = load_normal(g, i);
@@ -1047,7 +1055,8 @@ constexpr uint32_t kTri8Ring = 128, kTri8Round = 48;  // a round starts at kTri8
 template <int MODE>
 __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4 *__restrict__ p1,
                                                 const float4 *__restrict__ p2, const uint32_t *__restrict__ count,
-                                                uint32_t nBatch, CQueues q, uint32_t *__restrict__ out) {
+                                                uint32_t nBatch, uint32_t perWave, CQueues q,
+                                                uint32_t *__restrict__ out) {
     constexpr bool PER_PIXEL = MODE == kTracePassA, BATCH = MODE == kTraceBatch;
     __shared__ uint32_t stack[rt::kW8Stack * 256];
     __shared__ uint32_t ringTri[4 * kTri8Ring];
@@ -1078,9 +1087,16 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
     const uint32_t nChunks = (n + kTraceChunk - 1) / kTraceChunk;
     // wave-uniform; no more waves than chunks are needed (each takes at least one)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
-    if (wave >= nChunks) return;
     uint32_t shard = wave % kTraceShards;
     bool drained = false;            // wave-uniform: every shard is exhausted
+    if (BATCH && perWave) {          // a small batch: the wave's own rays and no others
+        next = wave * perWave;
+        end = n - next < perWave ? n : next + perWave;
+        drained = true;
+        if (next >= n) return;
+    } else if (wave >= nChunks) {
+        return;
+    }
     for (;;) {
         const uint64_t idle = __ballot(ray < 0);
         const uint32_t nIdle = static_cast<uint32_t>(__popcll(idle));
@@ -1243,16 +1259,29 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
     }
 }
 
+// Rays that each wave of k_trace8 takes of a batch that fits the grid (no counters to clear and to
+// ask), 0 for a larger one, whose chunks are handed out. A small batch takes as long as its slowest
+// wave, and a wave's time grows with its rays: a wave per ray up to the grid's workgroups in number,
+// then as many rays per wave as that leaves, up to 32; from there on full waves. Against chunks of
+// 64 with counters: 64 rays 41 -> 31 us, 1,021 rays 49 -> 34, 20,000 rays 81 -> 76 (60,000 rays in
+// waves of 47 take 91 us, in full ones 83).
+static uint32_t rays_per_wave(const SceneView &sc, uint32_t n) {
+    if (!sc.w8Ok || n > 256u * sc.w8Grid) return 0u;
+    const uint32_t per = (n + sc.w8Grid - 1u) / sc.w8Grid;
+    return per > 32u ? 64u : per;
+}
+
 // Launches the queue tracer over the nodes that cover the scene's tree.
 template <int STACK, int MODE>
 static void launch_tracer(const char *name, uint32_t gridCap, const SceneView &sc, const float4 *p1, const float4 *p2,
                           const uint32_t *count, uint32_t nBatch, const CQueues &q, uint32_t *out, hipStream_t s) {
-    // nBatch rays need no more workgroups than one lane each
-    const uint32_t grid = MODE == kTraceBatch && (nBatch + 255) / 256 < sc.w8Grid ? (nBatch + 255) / 256 : sc.w8Grid;
-    if (sc.w8Ok)
-        RK_LAUNCH(name, k_trace8<MODE>, dim3(grid), dim3(256), 0, s, sc, p1, p2, count, nBatch, q, out);
-    else
+    if (sc.w8Ok) {
+        const uint32_t per = MODE == kTraceBatch ? rays_per_wave(sc, nBatch) : 0u;
+        const uint32_t grid = per ? ((nBatch + per - 1) / per + 3) / 4 : sc.w8Grid;
+        RK_LAUNCH(name, k_trace8<MODE>, dim3(grid), dim3(256), 0, s, sc, p1, p2, count, nBatch, per, q, out);
+    } else {
         RK_LAUNCH(name, (k_trace_queue<STACK, MODE>), dim3(gridCap), dim3(256), 0, s, sc, p1, p2, count, nBatch, q, out);
+    }
 }
 
 // ---------------------------------------------------------------- Pass A, ray queue ---
@@ -1273,7 +1302,8 @@ struct AQueues {
 // 1920x1080, M = 32, 12,000 lights 0.63 -> 0.54 ms, 3840x2160, 1M lights 8.70 -> 4.19 ms. An alias
 // that names no point light gets zeros, as a triangle light does: a column that never draws it may
 // hold anything there.
-__global__ __launch_bounds__(256) void k_light_records(const SceneView sc, float4 *records) {
+__global__ __launch_bounds__(256) void k_light_records(const SceneView sc, float4 *records, uint32_t *counter) {
+    clear_counters(counter, sc.traceHeads);
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= static_cast<uint32_t>(sc.nAlias)) return;
     const float4 c = sc.alias[i];
@@ -1880,10 +1910,11 @@ template <int TX, int TY, int STACK>
 static hipError_t run_a_queued(PassAArgs args, const AQueues &q, uint32_t gridCap, hipStream_t s) {
     grid_for<TX, TY>(args.u.screenSize[0], args.u.screenSize[1], args.tilesX, args.nTiles);
     const dim3 tiles(args.nTiles), block(TX * TY);
-    RK_LAUNCH("k_zero_counters", k_zero_counters, dim3(1), dim3(64), 0, s, q.counter, 2u, args.sc.traceHeads);
+    if (!args.records)
+        RK_LAUNCH("k_zero_counters", k_zero_counters, dim3(1), dim3(64), 0, s, q.counter, 2u, args.sc.traceHeads);
     if (args.records) {
         RK_LAUNCH("k_light_records", k_light_records, dim3((args.sc.nAlias + 255) / 256), dim3(256), 0, s, args.sc,
-                  const_cast<float4 *>(args.records));
+                  const_cast<float4 *>(args.records), q.counter);
         RK_LAUNCH("k_pass_a_ris", (k_pass_a_ris<TX, TY, true>), tiles, block, 0, s, args, q);
     } else if (split_pays(args)) {
         PassAArgs split = args;
@@ -1983,11 +2014,13 @@ static hipError_t run_c_queued(PassCArgs args, const CQueues &q, uint32_t gridCa
     static_assert((kCentreTag & 0x07ffffffu) == 0 && (kCentreTag >> 27) > 15u, "the centre tag is no pixel or slot");
     grid_for<TX, TY>(args.u.screenSize[0], args.u.screenSize[1], args.tilesX, args.nTiles);
     const dim3 tiles(args.nTiles), block(TX * TY);
-    RK_LAUNCH("k_zero_counters", k_zero_counters, dim3(1), dim3(64), 0, s, q.counter, 2u, args.sc.traceHeads);
     const uint32_t npx = args.u.screenSize[0] * args.u.screenSize[1];
     // packSurface false: q.surf already holds this G-buffer's records (the previous Pass C's)
     if (packSurface)
-        RK_LAUNCH("k_pack_surface", k_pack_surface, dim3((npx + 255) / 256), dim3(256), 0, s, args.g, npx, q.surf);
+        RK_LAUNCH("k_pack_surface", k_pack_surface, dim3((npx + 255) / 256), dim3(256), 0, s, args.g, npx, q.surf, q.counter,
+                  args.sc.traceHeads);
+    else
+        RK_LAUNCH("k_zero_counters", k_zero_counters, dim3(1), dim3(64), 0, s, q.counter, 2u, args.sc.traceHeads);
     RK_LAUNCH("k_pass_c_merge", (k_pass_c_merge<TX, TY>), tiles, block, 0, s, args, q);
     if (args.u.flags & RESTIR_VISIBILITY_REUSE_FLAG) {
         launch_tracer<STACK, kTracePassC>("k_trace_queue(pass_c)", gridCap, args.sc, nullptr, nullptr, q.counter + 0, 0u,
@@ -2309,9 +2342,11 @@ static void run_trace(bool persistent, uint32_t gridCap, uint32_t *counter, cons
         RK_LAUNCH("k_trace", (k_trace<STACK, REF>), dim3(blocks), dim3(256), 0, s, args);
         return;
     }
-    RK_LAUNCH("k_zero_counters", k_zero_counters, dim3(1), dim3(64), 0, s, counter, 1u, args.sc.traceHeads);
+    const bool queue = !REF && !args.visits && !args.tests;
+    if (!queue || rays_per_wave(args.sc, args.n) == 0)
+        RK_LAUNCH("k_zero_counters", k_zero_counters, dim3(1), dim3(64), 0, s, counter, 1u, args.sc.traceHeads);
     const uint32_t grid = blocks < gridCap ? blocks : gridCap;
-    if (!REF && !args.visits && !args.tests) {
+    if (queue) {
         // no counts asked for: the passes' queue tracer (gathered triangle tests)
         launch_tracer<STACK, kTraceBatch>("k_trace_queue(batch)", grid, args.sc, args.p1, args.p2, nullptr, args.n,
                                           CQueues{}, args.shadowed, s);
