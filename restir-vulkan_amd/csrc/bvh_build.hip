@@ -19,8 +19,9 @@
 // Where the time goes: a level costs its launches (about 5 us each) and its readback, whatever its
 // size, and the lower half of a tree's levels holds ranges of a few primitives. 136,000 triangles
 // (23 levels): 3.2 ms with every level split that way, in 20 launches each; 1.15 ms with the last 12
-// to 13 levels in k_bvh_subtrees (0.22 ms) and 8 launches for each of the others. 1,200 triangles
-// 1.52 -> 0.47 ms, 2.3 million 18.6 -> 6.6 ms (all with the traversal's nodes, bind_tree).
+// to 13 levels in k_bvh_subtrees (0.22 ms) and 8 launches for each of the others, 1.05 with the 8-entry
+// nodes' collapse on 8 lanes a node. 1,200 triangles
+// 1.52 -> 0.39 ms, 2.3 million 18.6 -> 6.4 ms (all with the traversal's nodes, bind_tree).
 //
 // Exact min/max. nv_min(a, b) = a < b ? a : b (nvmath.inl:2414-2420) folded in primitive order
 // returns, among equal values, the LAST one; equal floats differ in bits only as +0/-0. Each fold
@@ -1057,170 +1058,203 @@ __global__ __launch_bounds__(256) void k_wide_build(const rt::Node *__restrict__
 }
 
 // ---- 8-entry nodes (rt_wide8.h), collapsed top-down from the binary tree, one level of 8-entry
-// nodes per launch: each lane makes one node. Its entries start as the two sides of its binary
-// node; while fewer than 8, the largest internal entry (by box area) is replaced by its own two
+// nodes per launch: 8 lanes make one node, an entry each. The entries start as the two sides of the
+// binary node; while fewer than 8, the largest internal entry (by box area) is replaced by its own two
 // sides. Children of one node are consecutive; the order of the nodes of a level is the order of
 // the atomics and changes no answer. One triangle per leaf entry: groups of up to 2, 3 and 4 made
-// the tracer 0-1%, 5% and 12% slower (more triangle tests than boxes saved). Latency bound (each
-// lane's expansions wait for one node after another): 0.17 ms for 136,000 triangles.
+// the tracer 0-1%, 5% and 12% slower (more triangle tests than boxes saved). Latency bound (a node's
+// expansions wait for one node after another): a lane per node, which
+// chose, ordered and rounded its entries one after another, took the builds of 1,200, 136,000 and 2.3
+// million triangles 0.49, 1.25 and 6.62 ms, this 0.39, 1.08 and 6.40.
 constexpr int kW8Levels = rt::kW8Stack + 1;
 struct W8Info {
     uint32_t nodes[kW8Levels + 1];  // nodes per level; [0] = 1
     uint32_t tris, overflow;
 };
 
-__global__ __launch_bounds__(64) void k_w8_collapse(const rt::Node *__restrict__ nodes,
-                                                    const float4 *__restrict__ tris, uint32_t level,
-                                                    uint32_t maxNodes, uint32_t maxTris,
-                                                    const uint32_t *__restrict__ bounds, rt::W8Node *__restrict__ out,
-                                                    float4 *__restrict__ outTris, uint32_t *__restrict__ work,
-                                                    W8Info *__restrict__ info) {
-    __shared__ float box[6][8][64];
-    __shared__ int32_t ref[8][64];    // >= 0 internal node, < 0 ~triangle
-    __shared__ uint32_t slot[8][64];  // where it is stored: 2 node + side
-    __shared__ float area[8][64];     // of an internal entry's box
-    const uint32_t lane = threadIdx.x;
+__global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict__ nodes,
+                                                     const float4 *__restrict__ tris, uint32_t level,
+                                                     uint32_t maxNodes, uint32_t maxTris,
+                                                     const uint32_t *__restrict__ bounds, rt::W8Node *__restrict__ out,
+                                                     float4 *__restrict__ outTris, uint32_t *__restrict__ work,
+                                                     W8Info *__restrict__ info) {
+    __shared__ __align__(16) rt::W8Node made[64];
+    __shared__ uint2 reserve[9];
+    const uint32_t lane = threadIdx.x & 63u, k = lane & 7u;
+    const int row = static_cast<int>(lane & 56u);
     uint32_t begin = 0;
     for (uint32_t l = 0; l < level; ++l) begin += info->nodes[l];
     const uint32_t n = info->nodes[level], next = begin + n;
     const double grow = static_cast<double>(rt::kW8Grow) * static_cast<double>(__uint_as_float(bounds[1]));
     if (bounds[2] != 0) return;  // a box is not finite: no 8-entry nodes
     for (uint32_t i0 = blockIdx.x * 64u; i0 < n; i0 += gridDim.x * 64u) {
-        const bool on = i0 + lane < n;
-        const uint32_t me = begin + i0 + lane;
-        int cnt = 0;
-        const auto put = [&](int at, float4 mn, float4 mx, int32_t c, uint32_t from) {
-            box[0][at][lane] = mn.x;
-            box[1][at][lane] = mn.y;
-            box[2][at][lane] = mn.z;
-            box[3][at][lane] = mx.x;
-            box[4][at][lane] = mx.y;
-            box[5][at][lane] = mx.z;
-            const float sx = mx.x - mn.x, sy = mx.y - mn.y, sz = mx.z - mn.z;
-            area[at][lane] = c >= 0 ? sx * sy + sx * sz + sy * sz : -1.0f;
-            ref[at][lane] = c;
-            slot[at][lane] = from;
+        const uint32_t i = i0 + (threadIdx.x >> 3), me = begin + i;
+        const bool on = i < n;  // the same for a node's 8 lanes
+        uint32_t cnt = 0;
+        float mn[3] = {}, mx[3] = {};  // this lane's entry: its box,
+        int32_t ref = 0;               // >= 0 internal node, < 0 ~triangle,
+        uint32_t slot = 0;             // where it is stored: 2 node + side,
+        float area = -2.0f;            // and its box's area, -2 unless it is internal
+        const auto put = [&](float4 lo, float4 hi, int32_t c, uint32_t from) {
+            mn[0] = lo.x, mn[1] = lo.y, mn[2] = lo.z;
+            mx[0] = hi.x, mx[1] = hi.y, mx[2] = hi.z;
+            const float sx = hi.x - lo.x, sy = hi.y - lo.y, sz = hi.z - lo.z;
+            area = c >= 0 ? sx * sy + sx * sz + sy * sz : -2.0f;
+            ref = c;
+            slot = from;
         };
         if (on) {
             int32_t x = level == 0 ? 0 : static_cast<int32_t>(work[me]);
-            int at = 0;
+            uint32_t at = 0;
             for (;;) {  // entry `at` becomes the left side of node x, a new entry its right side
                 const rt::Node nd = rt::load_node(nodes, x);
-                put(at, nd.lmin, nd.lmax, nd.left, 2u * static_cast<uint32_t>(x));
-                if (cnt == 0) cnt = 1;
-                put(cnt++, nd.rmin, nd.rmax, nd.right, 2u * static_cast<uint32_t>(x) + 1u);
+                const uint32_t add = cnt == 0 ? 1u : cnt;
+                if (k == at) put(nd.lmin, nd.lmax, nd.left, 2u * static_cast<uint32_t>(x));
+                if (k == add) put(nd.rmin, nd.rmax, nd.right, 2u * static_cast<uint32_t>(x) + 1u);
+                cnt = add + 1u;
                 if (cnt == 8) break;
-                at = -1;
-                float best = -1.0f;
-                for (int k = 0; k < cnt; ++k) {
-                    const float v = area[k][lane];
-                    if (ref[k][lane] >= 0 && (at < 0 || v > best)) {
-                        at = k;
+                float best = area;  // the first of the largest
+                at = k;
+#pragma unroll
+                for (int d = 1; d < 8; d <<= 1) {
+                    const float v = __shfl_xor(best, d);
+                    const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(at), d));
+                    if (v > best || (v == best && o < at)) {
                         best = v;
+                        at = o;
                     }
                 }
-                if (at < 0) break;
-                x = ref[at][lane];
+                if (best == -2.0f) break;
+                x = __shfl(ref, row + static_cast<int>(at));
             }
         }
-        // slots: internal entries first, then the triangles
-        int order[8], nInt = 0;
-        for (int k = 0; k < cnt; ++k)
-            if (ref[k][lane] >= 0) order[nInt++] = k;
-        const int nTri = cnt - nInt;
-        int at = nInt;
-        for (int k = 0; k < cnt; ++k)
-            if (ref[k][lane] < 0) order[at++] = k;
-        // the internal entries along the axis on which their centres spread most, the largest
+        const bool internal = k < cnt && ref >= 0, leaf = k < cnt && ref < 0;
+        const uint32_t intMask = static_cast<uint32_t>(__ballot(internal) >> row) & 0xffu;
+        const uint32_t triMask = static_cast<uint32_t>(__ballot(leaf) >> row) & 0xffu;
+        const uint32_t nInt = static_cast<uint32_t>(__popc(intMask)), nTri = static_cast<uint32_t>(__popc(triMask));
+        // slots: internal entries first, then the triangles.
+        // The internal entries along the axis on which their centres spread most, the largest
         // centre first: the primary rays take them from the side they come from. The shadow rays
         // take them in this order (1-11% faster on the terrains than the other way round)
         uint32_t axis = 0;
         float spread = -1.0f;
+#pragma unroll
         for (uint32_t a = 0; a < 3; ++a) {
-            float lo = __builtin_huge_valf(), hi = -__builtin_huge_valf();
-            for (int k = 0; k < nInt; ++k) {
-                const float c = box[a][order[k]][lane] + box[3 + a][order[k]][lane];
-                lo = fminf(lo, c);
-                hi = fmaxf(hi, c);
+            const float c = mn[a] + mx[a];
+            float lo = internal ? c : __builtin_huge_valf(), hi = internal ? c : -__builtin_huge_valf();
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) {
+                lo = fminf(lo, __shfl_xor(lo, d));
+                hi = fmaxf(hi, __shfl_xor(hi, d));
             }
             if (hi - lo > spread) {
                 spread = hi - lo;
                 axis = a;
             }
         }
-        for (int k = 1; k < nInt; ++k)
-            for (int j = k; j > 0; --j) {
-                const int u = order[j - 1], v = order[j];
-                if (!(box[axis][u][lane] + box[3 + axis][u][lane] < box[axis][v][lane] + box[3 + axis][v][lane])) break;
-                order[j - 1] = v;
-                order[j] = u;
-            }
-        // room in the next level and among the triangles, one atomic pair per wave
-        const uint32_t inclInt = rscan::wave_inclusive(static_cast<uint32_t>(nInt));
-        const uint32_t inclTri = rscan::wave_inclusive(static_cast<uint32_t>(nTri));
-        const uint32_t totInt = __shfl(inclInt, 63), totTri = __shfl(inclTri, 63);
-        uint32_t baseInt = 0, baseTri = 0;
-        if (lane == 0) {
-            if (totInt) baseInt = atomicAdd(&info->nodes[level + 1], totInt);
-            if (totTri) baseTri = atomicAdd(&info->tris, totTri);
+        const float centre = axis == 0 ? mn[0] + mx[0] : axis == 1 ? mn[1] + mx[1] : mn[2] + mx[2];
+        uint32_t rank = k;  // an empty entry keeps its place at the end
+        if (leaf) rank = nInt + static_cast<uint32_t>(__popc(triMask & ((1u << k) - 1u)));
+        uint32_t before = 0;
+#pragma unroll
+        for (uint32_t o = 0; o < 8; ++o) {
+            const float c = __shfl(centre, row + static_cast<int>(o));
+            if (((intMask >> o) & 1u) && (c > centre || (c == centre && o < k))) ++before;
         }
-        baseInt = next + __shfl(baseInt, 0) + inclInt - static_cast<uint32_t>(nInt);
-        baseTri = __shfl(baseTri, 0) + inclTri - static_cast<uint32_t>(nTri);
+        if (internal) rank = before;
+        // room in the next level and among the triangles, one atomic pair per workgroup (an atomic is
+        // served in 11 ns: one per wave, of 8 nodes, made 2.3 million triangles 0.7 ms slower)
+        const uint32_t inclInt = rscan::wave_inclusive(k == 0 ? nInt : 0u);
+        const uint32_t inclTri = rscan::wave_inclusive(k == 0 ? nTri : 0u);
+        const uint32_t wave = threadIdx.x >> 6;
+        if (lane == 63) reserve[wave] = make_uint2(inclInt, inclTri);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint2 sum = make_uint2(0u, 0u);
+            for (uint32_t v = 0; v < 8; ++v) {
+                const uint2 t = reserve[v];
+                reserve[v] = sum;
+                sum.x += t.x;
+                sum.y += t.y;
+            }
+            if (sum.x) sum.x = atomicAdd(&info->nodes[level + 1], sum.x);
+            if (sum.y) sum.y = atomicAdd(&info->tris, sum.y);
+            reserve[8] = sum;
+        }
+        __syncthreads();
+        const uint32_t baseInt = next + reserve[8].x + reserve[wave].x + inclInt - nInt;
+        const uint32_t baseTri = reserve[8].y + reserve[wave].y + inclTri - nTri;
         if (!on) continue;
-        if (baseInt + static_cast<uint32_t>(nInt) > maxNodes || baseTri + static_cast<uint32_t>(nTri) > maxTris ||
-            me >= maxNodes) {
-            atomicOr(&info->overflow, 1u);
+        if (baseInt + nInt > maxNodes || baseTri + nTri > maxTris || me >= maxNodes) {
+            if (k == 0) atomicOr(&info->overflow, 1u);
             continue;
         }
-        rt::W8Node w;
-        w.child = (baseInt << 8) | ((1u << nInt) - 1u);
-        w.triBase = baseTri - static_cast<uint32_t>(nInt);
-        w.exps = (((1u << cnt) - 1u) & ~((1u << nInt) - 1u)) << 24;
-        w.axis = axis;
-        w.pad = 0;
-        for (int k = 0; k < nInt; ++k) work[baseInt + static_cast<uint32_t>(k)] = static_cast<uint32_t>(ref[order[k]][lane]);
+        if (internal) work[baseInt + rank] = static_cast<uint32_t>(ref);
+        // per axis, by a lane each: the origin p below the node's planes, and e, the smallest step 2^e
+        // (down to 2^-100) whose 2047 multiples span the node
+        float least[3], most[3];
+#pragma unroll
         for (int a = 0; a < 3; ++a) {
-            double lo = 1e300, hi = -1e300;
-            for (int k = 0; k < cnt; ++k) {
-                lo = fmin(lo, static_cast<double>(box[a][k][lane]) - grow);
-                hi = fmax(hi, static_cast<double>(box[3 + a][k][lane]) + grow);
-            }
-            float p = static_cast<float>(lo);
-            if (static_cast<double>(p) > lo) p = nextafterf(p, -__builtin_huge_valf());
-            const double ext = hi - static_cast<double>(p);
-            int e = -100;  // the smallest step 2^e (down to 2^-100) whose 2047 multiples span the node
-            if (ext > 0.0) {
-                const int f = ilogb(ext) - 11;
-                if (f > e) e = f;
-            }
-            while (ext > 2047.0 * ldexp(1.0, e)) ++e;
-            w.p[a] = p;
-            w.exps |= (static_cast<uint32_t>(e) & 0xffu) << (8 * a);
-            const double inv = ldexp(1.0, -e);
-            for (int k = 0; k < 8; ++k) {
-                double ql = 0.0, qh = 0.0;
-                if (k < cnt) {
-                    ql = floor((static_cast<double>(box[a][order[k]][lane]) - grow - static_cast<double>(p)) * inv);
-                    qh = ceil((static_cast<double>(box[3 + a][order[k]][lane]) + grow - static_cast<double>(p)) * inv);
-                    ql = fmin(fmax(ql, 0.0), 2047.0);
-                    qh = fmin(fmax(qh, 0.0), 2047.0);
-                }
-                w.plane[a][0][k] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(ql)));
-                w.plane[a][1][k] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(qh)));
+            least[a] = k < cnt ? mn[a] : __builtin_huge_valf();
+            most[a] = k < cnt ? mx[a] : -__builtin_huge_valf();
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) {
+                least[a] = fminf(least[a], __shfl_xor(least[a], d));
+                most[a] = fmaxf(most[a], __shfl_xor(most[a], d));
             }
         }
-        out[me] = w;
-        for (int k = nInt; k < cnt; ++k) {
-            const size_t t = static_cast<size_t>(~ref[order[k]][lane]), to = baseTri + static_cast<uint32_t>(k - nInt);
+        const double lo = static_cast<double>(k == 0 ? least[0] : k == 1 ? least[1] : least[2]) - grow;
+        const double hi = static_cast<double>(k == 0 ? most[0] : k == 1 ? most[1] : most[2]) + grow;
+        float p = static_cast<float>(lo);
+        if (static_cast<double>(p) > lo) p = nextafterf(p, -__builtin_huge_valf());
+        const double ext = hi - static_cast<double>(p);
+        int e = -100;
+        if (ext > 0.0) {
+            const int f = ilogb(ext) - 11;
+            if (f > e) e = f;
+        }
+        while (ext > 2047.0 * ldexp(1.0, e)) ++e;
+        rt::W8Node &w = made[threadIdx.x >> 3];
+        uint32_t exps = (((1u << cnt) - 1u) & ~((1u << nInt) - 1u)) << 24;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float pa = __shfl(p, row + a);
+            const int ea = __shfl(e, row + a);
+            exps |= (static_cast<uint32_t>(ea) & 0xffu) << (8 * a);
+            const double inv = ldexp(1.0, -ea);
+            double ql = 0.0, qh = 0.0;
+            if (k < cnt) {
+                ql = floor((static_cast<double>(mn[a]) - grow - static_cast<double>(pa)) * inv);
+                qh = ceil((static_cast<double>(mx[a]) + grow - static_cast<double>(pa)) * inv);
+                ql = fmin(fmax(ql, 0.0), 2047.0);
+                qh = fmin(fmax(qh, 0.0), 2047.0);
+            }
+            w.plane[a][0][rank] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(ql)));
+            w.plane[a][1][rank] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(qh)));
+            if (k == 0) w.p[a] = pa;
+        }
+        if (k == 0) {
+            w.child = (baseInt << 8) | ((1u << nInt) - 1u);
+            w.triBase = baseTri - nInt;
+            w.exps = exps;
+            w.axis = axis;
+            w.pad = 0;
+        }
+        row_sync();
+        // the node by way of LDS: 16 bytes a lane
+        static_assert(sizeof(rt::W8Node) == 128, "8 lanes store a node");
+        reinterpret_cast<float4 *>(out + me)[k] = reinterpret_cast<const float4 *>(&w)[k];
+        row_sync();
+        if (leaf) {
+            const size_t t = static_cast<size_t>(~ref), to = baseTri + rank - nInt;
             const float4 v0 = tris[3 * t], v1 = tris[3 * t + 1], v2 = tris[3 * t + 2];
-            outTris[3 * to] = make_float4(v0.x, v0.y, v0.z, __uint_as_float(slot[order[k]][lane]));
+            outTris[3 * to] = make_float4(v0.x, v0.y, v0.z, __uint_as_float(slot));
             outTris[3 * to + 1] = make_float4(v1.x, v1.y, v1.z, __int_as_float(static_cast<int32_t>(t)));
             outTris[3 * to + 2] = make_float4(v2.x, v2.y, v2.z, 0.0f);
         }
     }
 }
 
-// clears the flags of k_wide_build and the counters of the collapse
 __global__ void k_w8_clear(uint32_t *flags, W8Info *info) {
     uint32_t *w = reinterpret_cast<uint32_t *>(info);
     const uint32_t t = threadIdx.x;
@@ -1283,7 +1317,7 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     for (uint32_t batch = 4 + (32u - static_cast<uint32_t>(__builtin_clz(nTris))) / 3;; batch = 4) {
         const uint32_t end = !w8Fits ? 0u : (done + batch < levels ? done + batch : levels);
         for (; done < end; ++done)
-            RK_LAUNCH("k_w8_collapse", k_w8_collapse, dim3(1024), dim3(64), 0, s, bn, bt, done, maxW8, nTris, p.flags,
+            RK_LAUNCH("k_w8_collapse", k_w8_collapse, dim3(1024), dim3(512), 0, s, bn, bt, done, maxW8, nTris, p.flags,
                       p.w8, p.tris, p.work, p.info);
         if (int r = hip(hipMemcpyAsync(&host, p.flags, sizeof host, hipMemcpyDeviceToHost, s), "bind tree: read")) return r;
         if (int r = hip(hipStreamSynchronize(s), "bind tree: finish")) return r;
