@@ -20,8 +20,8 @@
 // size, and the lower half of a tree's levels holds ranges of a few primitives. 136,000 triangles
 // (23 levels): 3.2 ms with every level split that way, in 20 launches each; 1.15 ms with the last 12
 // to 13 levels in k_bvh_subtrees (0.22 ms) and 8 launches for each of the others, 1.05 with the 8-entry
-// nodes' collapse on 8 lanes a node. 1,200 triangles
-// 1.52 -> 0.39 ms, 2.3 million 18.6 -> 6.4 ms (all with the traversal's nodes, bind_tree).
+// nodes' collapse on 8 lanes a node. 1,200 triangles 1.52 -> 0.39 ms, 2.3 million 18.6 -> 6.4 ms (all
+// with the traversal's nodes, bind_tree).
 //
 // Exact min/max. nv_min(a, b) = a < b ? a : b (nvmath.inl:2414-2420) folded in primitive order
 // returns, among equal values, the LAST one; equal floats differ in bits only as +0/-0. Each fold
@@ -35,7 +35,7 @@
 // arrives. After the pass, a position p >= mid holds what was placed there at step p: the
 // primitive itself if it is a right one, else the front of the block at that step, which sat at
 // first + (left primitives before p) and is resolved the same way. That chain only moves to
-// smaller positions; it is followed by pointer jumping in place (k_bvh_jump).
+// smaller positions; it is followed by pointer jumping in place (k_bvh_scatter).
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
