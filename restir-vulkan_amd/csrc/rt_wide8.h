@@ -18,8 +18,13 @@
 // every node on the path of a triangle whose path passes. 1/d is clamped to +-K (SceneView::invMax,
 // s K >= 4): for |d| < 1/K a segment that starts inside the grown slab keeps near < 0 and far > 1,
 // and one that starts outside cannot reach the box itself (its distance exceeds s K), so zero,
-// denormal (the hardware's reciprocal is then infinite) and tiny components are covered too. Segments with a non-finite component or |o| > 16 C walk the
-// binary tree (occluded_slow). The same holds for unbounded rays (the primary rays) of unit
+// denormal (the hardware's reciprocal is then infinite) and tiny components are covered too. Long
+// segments are another matter: the hardware flushes the reciprocal of a component above 2^126 to
+// zero, which puts all its distances at 0, and shorter ones leave S and the slack without bits in a
+// small scene. With |d| <= min(2^99, 2^96 C) the reciprocal is normal, S is at least 2^-123 (a
+// node's step 2^e is at least 2^-27 C) and the slack s / |d| at least 2^-113, far above what N's product
+// loses below the normal range. Segments beyond that, with a non-finite component or with |o| > 16 C
+// walk the binary tree (occluded_slow). The same holds for unbounded rays (the primary rays) of unit
 // direction, whose boxes all lie within 31 C of the origin: s K >= 31 C.
 #pragma once
 
@@ -30,6 +35,7 @@ namespace rt {
 constexpr int kW8Stack = 16;  // entries of a lane's stack: trees of at most 17 levels of 8-entry nodes
 constexpr float kW8Grow = 192.0f * 5.9604645e-8f;  // s / C
 constexpr float kW8Reach = 16.0f;                  // |o| / C at most
+constexpr float kW8Long = 0x1p96f, kW8Longest = 0x1p99f;  // |d| / C and |d| at most
 
 struct alignas(128) W8Node {
     float p[3];         // the node's corner: plane q of axis a lies at p[a] + q 2^e[a]
@@ -52,7 +58,6 @@ struct W8Seg {
 };
 // False for a segment the walk does not cover.
 __device__ __forceinline__ bool make_w8seg(W8Seg &w, f3 o, f3 d, float maxCoord, float invMax) {
-    constexpr float kInf = __builtin_huge_valf();
     w.o = o;
     w.d = d;
     const f3 inv{__builtin_amdgcn_rcpf(d.x), __builtin_amdgcn_rcpf(d.y), __builtin_amdgcn_rcpf(d.z)};
@@ -61,9 +66,9 @@ __device__ __forceinline__ bool make_w8seg(W8Seg &w, f3 o, f3 d, float maxCoord,
     w.ox = w.inv.x > 0.0f ? 0u : 16u;
     w.oy = w.inv.y > 0.0f ? 0u : 16u;
     w.oz = w.inv.z > 0.0f ? 0u : 16u;
-    const float reach = kW8Reach * maxCoord;
+    const float reach = kW8Reach * maxCoord, longest = fminf(kW8Long * maxCoord, kW8Longest);
     // comparisons are false for NaN
-    return fabsf(d.x) < kInf && fabsf(d.y) < kInf && fabsf(d.z) < kInf && fabsf(o.x) <= reach &&
+    return fabsf(d.x) <= longest && fabsf(d.y) <= longest && fabsf(d.z) <= longest && fabsf(o.x) <= reach &&
            fabsf(o.y) <= reach && fabsf(o.z) <= reach;
 }
 

@@ -192,3 +192,39 @@ def test_wide8_spine_tree(torch, levels):
     ref = _check(torch, ctx, osc, p1, p2, f"spine of {levels}")
     assert 0.02 < ref.mean() < 0.999
     del keep
+
+
+def _long_segments(rng, lo, hi, n, reach):
+    """Segments from the scene to `reach` times its size and beyond, up to the largest float, along one
+    axis, two or all three (whose other components keep the scene's size), through its middle."""
+    size = float((hi - lo).max())
+    p1, p2 = random_segments(rng, lo, hi, n)
+    axes = rng.integers(1, 8, size=n)
+    length = np.exp(rng.uniform(np.log(size * reach), np.log(3.3e38), size=n))
+    for a in range(3):
+        far = (axes >> a) & 1 != 0
+        sign = rng.choice((-1.0, 1.0), size=n)
+        p2[far, a] = (sign * length * rng.uniform(0.2, 1.0, size=n))[far].astype(np.float32)
+    return p1, p2
+
+
+@pytest.mark.parametrize("size", [1.0, 1e-8, 1e-12])
+def test_wide8_long_segments(torch, size):
+    """A segment's component above 2^126 has a reciprocal that the hardware flushes to zero, and far
+    shorter ones leave a tiny scene's slab distances without bits: the binary walk takes those."""
+    sc = scenes.terrain(5, grid=64, n_boxes=100, n_point_lights=10)
+    lo, hi = sc.aabb()
+    scale = size / float((hi - lo).max())
+    xyz = (sc.tri_xyz.reshape(-1, 9).astype(np.float64) * scale).astype(np.float32)
+    lo, hi = lo.astype(np.float64) * scale, hi.astype(np.float64) * scale
+    nodes, tris, _ = abi.build_aabb_tree(xyz)
+    osc = oracle.Scene(nodes, tris, None, None, None)
+    ctx = abi.Context(0)
+    keep = _bind(torch, ctx, nodes, tris)
+    rng = np.random.default_rng(23)
+    p1, p2 = _long_segments(rng, lo, hi, 60000, 1e2)
+    ref = _check(torch, ctx, osc, p1, p2, f"long, size {size}")
+    # what the walk over rounded slab distances gets wrong is occluded segments
+    top = np.abs(p2[:, :3] - p1[:, :3]).max(axis=1) > 2.0 ** 126
+    assert ref.sum() > 200 and (size != 1.0 or ref[top].sum() > 20), (ref.sum(), ref[top].sum())
+    del keep
