@@ -845,13 +845,13 @@ __global__ __launch_bounds__(TX *TY) void k_pass_c_finish(const PassCArgs a, con
 // walk. A lane's ray ends when no test of its is waiting and a test hit or its walk is over; the
 // lane takes no new ray before, and the tests of a ray already known to hit are skipped.
 //
-// MODE kTracePassA: the rays are Pass A's visibility rays (p1, p2: end points; *count of them),
-// and one that is shadowed sets kBitCentreShadowed in bits[pixel]. kTracePassC: the rays are a
-// Pass C's: its count[0] centre rays (q.c1), then its count[1] neighbour rays (q.n1), both
-// ending at the light sample of merged[pixel]. A shadowed centre ray sets kBitCentreShadowed in
-// bits[pixel]; a shadowed neighbour ray sets bit `slot` of occ[pixel], and is not traced when its
-// pixel's centre ray is already known to be shadowed (the centre rays come first in the index
-// space, so that holds for nearly all of them; tracing the others too changes nothing).
+// MODE kTracePassA: the rays are Pass A's visibility rays (p1, p2: end points; *count of them; the
+// tag is the pixel, of up to 2^31), and one that is shadowed sets kBitCentreShadowed in bits[pixel].
+// kTracePassC: the rays are a Pass C's: its count[0] centre rays (q.c1), then its count[1] neighbour
+// rays (q.n1), both ending at the light sample of merged[pixel]. A shadowed centre ray sets
+// kBitCentreShadowed in bits[pixel]; a shadowed neighbour ray sets bit `slot` of occ[pixel], and is
+// not traced when its pixel's centre ray is already known to be shadowed (the centre rays come first
+// in the index space, so that holds for nearly all of them; tracing the others too changes nothing).
 // kTraceBatch: nBatch rays p1[i] -> p2[i] (restir_trace_shadow); out[i] gets 1 if shadowed, else 0.
 constexpr uint32_t kTraceRefill = 32;
 constexpr uint32_t kTriList = kTraceListEntries, kTriRoundWalkers = 32;
@@ -1002,7 +1002,8 @@ __global__ __launch_bounds__(256) void k_trace_queue(const SceneView sc, const f
             if (BATCH) {
                 out[tag] = w.hit ? 1u : 0u;
             } else if (w.hit) {
-                if (PER_PIXEL || (tag & kCentreTag)) q.bits[tag & 0x07ffffffu] |= kBitCentreShadowed;
+                if (PER_PIXEL) q.bits[tag] |= kBitCentreShadowed;
+                else if (tag & kCentreTag) q.bits[tag & 0x07ffffffu] |= kBitCentreShadowed;
                 else atomicOr(&q.occ[tag & 0x07ffffffu], 1u << (tag >> 27));
             }
             ray = -1;
@@ -1251,7 +1252,8 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
             if (BATCH) {
                 out[tag] = hit ? 1u : 0u;
             } else if (hit) {
-                if (PER_PIXEL || (tag & kCentreTag)) q.bits[tag & 0x07ffffffu] |= kBitCentreShadowed;
+                if (PER_PIXEL) q.bits[tag] |= kBitCentreShadowed;
+                else if (tag & kCentreTag) q.bits[tag & 0x07ffffffu] |= kBitCentreShadowed;
                 else atomicOr(&q.occ[tag & 0x07ffffffu], 1u << (tag >> 27));
             }
             ray = -1;
