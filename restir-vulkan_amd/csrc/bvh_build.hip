@@ -1085,11 +1085,15 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
     uint32_t begin = 0;
     for (uint32_t l = 0; l < level; ++l) begin += info->nodes[l];
     const uint32_t n = info->nodes[level], next = begin + n;
-    const double grow = static_cast<double>(rt::kW8Grow) * static_cast<double>(__uint_as_float(bounds[1]));
-    if (bounds[2] != 0) return;  // a box is not finite: no 8-entry nodes
+    const float maxCoord = __uint_as_float(bounds[1]);
+    const double grow = static_cast<double>(rt::kW8Grow) * static_cast<double>(maxCoord);
+    // a box is not finite, or too large or small: no 8-entry nodes. Areas are then finite: from about
+    // 1.7e38 on a flat box's would be inf * 0, and no lane's NaN agrees with another's choice
+    if (bounds[2] != 0 || !rt::w8_covers(maxCoord)) return;
     for (uint32_t i0 = blockIdx.x * 64u; i0 < n; i0 += gridDim.x * 64u) {
         const uint32_t i = i0 + (threadIdx.x >> 3), me = begin + i;
-        const bool on = i < n;  // the same for a node's 8 lanes
+        // the same for a node's 8 lanes; nodes beyond maxNodes are counted but have no work entry
+        const bool on = i < n && me < maxNodes;
         uint32_t cnt = 0;
         float mn[3] = {}, mx[3] = {};  // this lane's entry: its box,
         int32_t ref = 0;               // >= 0 internal node, < 0 ~triangle,
@@ -1185,7 +1189,7 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
         const uint32_t baseInt = next + reserve[8].x + reserve[wave].x + inclInt - nInt;
         const uint32_t baseTri = reserve[8].y + reserve[wave].y + inclTri - nTri;
         if (!on) continue;
-        if (baseInt + nInt > maxNodes || baseTri + nTri > maxTris || me >= maxNodes) {
+        if (baseInt + nInt > maxNodes || baseTri + nTri > maxTris) {
             if (k == 0) atomicOr(&info->overflow, 1u);
             continue;
         }
@@ -1334,9 +1338,8 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     ctx->scene.w8 = p.w8;
     ctx->scene.w8Tris = p.tris;
     ctx->scene.treeTight = host.flags[3] == 0 ? 1 : 0;
-    // the bounds on the coordinates keep every product of the walk finite and its slack normal
     ctx->scene.w8Ok = w8Fits && host.flags[2] == 0 && host.w8.overflow == 0 && host.w8.nodes[done] == 0 &&
-                              host.w8.tris == nTris && maxCoord > 1e-18f && maxCoord < 1e18f
+                              host.w8.tris == nTris && rt::w8_covers(maxCoord)
                           ? 1
                           : 0;
     ctx->scene.w8Grid = ctx->cus * rk::kTrace8PerCu;

@@ -35,6 +35,8 @@ namespace rt {
 constexpr int kW8Stack = 16;  // entries of a lane's stack: trees of at most 17 levels of 8-entry nodes
 constexpr float kW8Grow = 192.0f * 5.9604645e-8f;  // s / C
 constexpr float kW8Reach = 16.0f;                  // |o| / C at most
+// Trees whose largest |box coordinate| C keeps every product of the walk finite and its slack normal
+__host__ __device__ inline bool w8_covers(float c) { return c > 1e-18f && c < 1e18f; }
 constexpr float kW8Long = 0x1p96f, kW8Longest = 0x1p99f;  // |d| / C and |d| at most
 
 struct alignas(128) W8Node {

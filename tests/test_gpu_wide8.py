@@ -228,3 +228,30 @@ def test_wide8_long_segments(torch, size):
     top = np.abs(p2[:, :3] - p1[:, :3]).max(axis=1) > 2.0 ** 126
     assert ref.sum() > 200 and (size != 1.0 or ref[top].sum() > 20), (ref.sum(), ref[top].sum())
     del keep
+
+
+@pytest.mark.parametrize("how", ["host", "device"])
+@pytest.mark.parametrize("size", [1e17, 1e19, 3.3e38])
+def test_wide8_enormous_boxes(torch, size, how):
+    """Boxes up to the largest float, flat ones among them (whose area would be inf * 0): beyond the
+    coordinates that the 8-entry nodes cover, the tree keeps its 4-entry nodes."""
+    rng = np.random.default_rng(31)
+    n = 300
+    xyz = np.zeros((n, 3, 3))
+    xyz[:, :, 0] = rng.uniform(-1, 1, size=(n, 1)) + rng.uniform(-0.2, 0.2, size=(n, 3))
+    xyz[:, :, 2] = rng.uniform(-1, 1, size=(n, 1)) + rng.uniform(-0.2, 0.2, size=(n, 3))
+    xyz[n // 2:, :, 1] = rng.uniform(-1e-3, 1e-3, size=(n - n // 2, 3))  # the first half is flat
+    xyz = (np.clip(xyz, -1, 1) * size).astype(np.float32)
+    nodes, tris, _ = abi.build_aabb_tree(xyz.reshape(-1, 9))
+    osc = oracle.Scene(nodes, tris, None, None, None)
+    ctx = abi.Context(0)
+    if how == "host":
+        keep = _bind(torch, ctx, nodes, tris)
+    else:
+        keep = (torch.from_numpy(xyz).cuda(), torch.zeros(nodes.nbytes, dtype=torch.uint8, device="cuda"),
+                torch.zeros(tris.nbytes, dtype=torch.uint8, device="cuda"))
+        ctx.build_bvh(keep[0], n, keep[1], keep[2])
+        assert keep[1].cpu().numpy().tobytes() == nodes.tobytes()
+    lo, hi = np.array([-1, -1e-3, -1]) * size * 0.5, np.array([1, 1e-3, 1]) * size * 0.5
+    _check(torch, ctx, osc, *random_segments(rng, lo, hi, 20000), f"size {size}")
+    del keep
