@@ -125,30 +125,45 @@ uint32_t persistent_blocks(uint32_t cus, int stack) {
     return resident_blocks(cus, static_cast<uint32_t>(stack) * 256u * 4u + rk::kTraceExtraLds);
 }
 
-int ensure_scratch(restir_ctx *ctx, size_t bytes) {
-    if (bytes > ctx->scratchBytes) {
-        ctx->surfValid = false;  // a new allocation holds no records
-        if (ctx->scratchInGraph) {  // a graph may replay launches over the old one: kept to the end
-            ctx->retired.push_back(ctx->scratch);
-            ctx->scratch = nullptr;
-            ctx->scratchBytes = 0;
-            ctx->scratchInGraph = false;
-        }
+// Whether s is being captured into a graph (so too a stream that cannot be asked).
+bool in_capture(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
+// ensure for memory that launches on s will use: what a capture recorded launches over (*inGraph) is
+// kept to the context's end when it has to grow, since a graph may replay them.
+int ensure_kept(restir_ctx *ctx, void **buf, size_t *have, bool *inGraph, size_t bytes, hipStream_t s) {
+    const bool capture = in_capture(s);
+    if (bytes > *have && *inGraph) {
+        ctx->retired.push_back(*buf);
+        *buf = nullptr;
+        *have = 0;
+        *inGraph = false;
     }
-    return ensure(ctx, &ctx->scratch, &ctx->scratchBytes, bytes);
+    if (int r = ensure(ctx, buf, have, bytes)) return r;
+    *inGraph = *inGraph || capture;
+    return RESTIR_OK;
+}
+
+int ensure_scratch(restir_ctx *ctx, size_t bytes, hipStream_t s) {
+    if (bytes > ctx->scratchBytes) ctx->surfValid = false;  // a new allocation holds no records
+    return ensure_kept(ctx, &ctx->scratch, &ctx->scratchBytes, &ctx->scratchInGraph, bytes, s);
 }
 
 // Binds the device and, for the queued schedule (the default), sizes the context scratch for
 // Pass A's ray queue; *queues stays null for the inline schedule. The Pass C ray export is
 // invalidated: the queues share the scratch.
-int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, void **queues) {
+int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, void **queues, hipStream_t s) {
     const uint32_t schedule = launch ? launch->schedule : RESTIR_SCHEDULE_QUEUED;
     if (schedule != RESTIR_SCHEDULE_QUEUED && schedule != RESTIR_SCHEDULE_INLINE)
         return fail(ctx, RESTIR_E_INVALID_ARGUMENT, "unknown schedule %u", schedule);
     if (int r = use_device(ctx)) return r;
     *queues = nullptr;
     if (schedule == RESTIR_SCHEDULE_QUEUED) {
-        if (int r = ensure_scratch(ctx, rk::pass_a_queue_bytes(npx))) return r;
+        if (int r = ensure_scratch(ctx, rk::pass_a_queue_bytes(npx), s)) return r;
         *queues = ctx->scratch;
         ctx->queuedNpx = 0;
         ctx->surfValid = false;
@@ -161,20 +176,8 @@ int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, vo
 void *light_records(restir_ctx *ctx, const rk::SceneView &sc, const restir_uniforms &u, hipStream_t s) {
     if (!rk::light_records_pay(sc, u.screenSize[0] * u.screenSize[1], u.initialLightSampleCount)) return nullptr;
     const size_t bytes = rk::light_record_bytes(sc);
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        if (bytes > ctx->recordBytes) return nullptr;
-        ctx->recordsInGraph = true;
-        return ctx->records;
-    }
-    if (bytes > ctx->recordBytes && ctx->recordsInGraph) {  // a graph may replay launches over the old ones
-        ctx->retired.push_back(ctx->records);
-        ctx->records = nullptr;
-        ctx->recordBytes = 0;
-        ctx->recordsInGraph = false;
-    }
-    if (ensure(ctx, &ctx->records, &ctx->recordBytes, bytes) == RESTIR_OK) return ctx->records;
+    if (bytes > ctx->recordBytes && in_capture(s)) return nullptr;
+    if (ensure_kept(ctx, &ctx->records, &ctx->recordBytes, &ctx->recordsInGraph, bytes, s) == RESTIR_OK) return ctx->records;
     (void)hipGetLastError();
     ctx->error.clear();
     return nullptr;
@@ -377,8 +380,8 @@ int restir_initial_temporal(restir_ctx *ctx, const restir_uniforms *u, const res
     int tile;
     if (int r = pick_tile(ctx, launch, &tile)) return r;
     void *queues = nullptr;
-    if (int r = pass_a_queues(ctx, launch, W * H, &queues)) return r;
     const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (int r = pass_a_queues(ctx, launch, W * H, &queues, s)) return r;
     void *records = queues ? light_records(ctx, ctx->scene, *u, s) : nullptr;
     const hipError_t e = rk::launch_pass_a(tile, ctx->stack, *u, ctx->scene, view_of(cur), view_of(prev),
                                            prevRes, out, nullptr, nullptr, queues, ctx->persistentBlocks, s, records);
@@ -455,7 +458,7 @@ int restir_unbiased(restir_ctx *ctx, const restir_uniforms *u, int k, int iter,
     bool pack = true;
     const rk::GView gv = view_of(g);
     if (schedule == RESTIR_SCHEDULE_QUEUED) {
-        if (int r = ensure_scratch(ctx, rk::pass_c_queue_bytes(W * H, k))) return r;
+        if (int r = ensure_scratch(ctx, rk::pass_c_queue_bytes(W * H, k), static_cast<hipStream_t>(stream))) return r;
         queues = ctx->scratch;
         // RESTIR_INPUT_VISIBLE_FLAG promises the previous Pass C's output over the same G-buffer:
         // when that Pass C ran here on these planes, size and k, its surface records are reused

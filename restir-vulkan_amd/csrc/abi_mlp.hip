@@ -191,9 +191,7 @@ int restir_learned_candidates(restir_ctx *ctx, const restir_uniforms *u, const r
     if (int r = use_device(ctx)) return r;
     const rt::f3 cam{u->cameraPos[0], u->cameraPos[1], u->cameraPos[2]};
     const uint32_t seed = u->frame * 0x9e3779b1u + 0x7f4a7c15u;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) (void)hipGetLastError();
-    if (st != hipStreamCaptureStatusNone) ctx->slotsInGraph = ctx->slots != nullptr;
+    if (ctx->slots && in_capture(static_cast<hipStream_t>(stream))) ctx->slotsInGraph = true;
     uint8_t *slots = static_cast<uint8_t *>(ctx->slots);
     const rk::WideSlots wide{slots,
                              slots ? reinterpret_cast<uint32_t *>(slots + ctx->slotCount * rk::wide_slot_bytes(ctx->slotClusters))
@@ -232,7 +230,7 @@ int restir_initial_temporal_candidates(restir_ctx *ctx, const restir_uniforms *u
     int tile;
     if (int r = pick_tile(ctx, launch, &tile)) return r;
     void *queues = nullptr;
-    if (int r = pass_a_queues(ctx, launch, W * H, &queues)) return r;
+    if (int r = pass_a_queues(ctx, launch, W * H, &queues, static_cast<hipStream_t>(stream))) return r;
     const hipError_t e = rk::launch_pass_a(tile, ctx->stack, *u, ctx->scene, view_of(cur), view_of(prev), prevRes,
                                            out, candLight, candQ, queues, ctx->persistentBlocks,
                                            static_cast<hipStream_t>(stream));

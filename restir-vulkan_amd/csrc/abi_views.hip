@@ -66,14 +66,8 @@ bool queued_views(restir_ctx *ctx, const restir_launch *launch, size_t bytes, hi
     // what the scratch held of a single-view Pass C will be overwritten
     ctx->queuedNpx = 0;
     ctx->surfValid = false;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        if (bytes > ctx->scratchBytes) return false;
-        ctx->scratchInGraph = true;
-        return true;
-    }
-    if (ensure_scratch(ctx, bytes) == RESTIR_OK) return true;
+    if (bytes > ctx->scratchBytes && in_capture(s)) return false;
+    if (ensure_scratch(ctx, bytes, s) == RESTIR_OK) return true;
     (void)hipGetLastError();
     ctx->error.clear();
     return false;

@@ -37,7 +37,7 @@ struct restir_ctx {
     void *noallocScratch = nullptr;  // this device's copy of abi.hip's static `scratch` array
     void *scratch = nullptr;       // ray queues of the queued Pass C schedule
     size_t scratchBytes = 0;
-    bool scratchInGraph = false;   // a stream capture recorded multi-view launches that use it
+    bool scratchInGraph = false;   // a stream capture recorded launches that use it
     std::vector<void *> retired;   // earlier scratches, slots and records that captured graphs still use
     uint32_t queuedNpx = 0;        // shape of the last queued Pass C (its rays stay in scratch)
     const restir_reservoir *queuedOut = nullptr;  // its output (the light end of its neighbour rays)
@@ -113,9 +113,11 @@ int check_gbuffer(restir_ctx *ctx, const restir_gbuffer *g, uint32_t W, uint32_t
 rk::GView view_of(const restir_gbuffer *g);
 int check_frame(restir_ctx *ctx, const restir_uniforms *u, const char *name);
 int pick_tile(restir_ctx *ctx, const restir_launch *l, int *tile);
-int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, void **queues);
+int pass_a_queues(restir_ctx *ctx, const restir_launch *launch, uint32_t npx, void **queues, hipStream_t s);
 int ensure(restir_ctx *ctx, void **buf, size_t *have, size_t bytes);
-int ensure_scratch(restir_ctx *ctx, size_t bytes);
+bool in_capture(hipStream_t s);
+int ensure_kept(restir_ctx *ctx, void **buf, size_t *have, bool *inGraph, size_t bytes, hipStream_t s);
+int ensure_scratch(restir_ctx *ctx, size_t bytes, hipStream_t s);
 void *light_records(restir_ctx *ctx, const rk::SceneView &sc, const restir_uniforms &u, hipStream_t s);
 uint32_t resident_blocks(uint32_t cus, uint32_t ldsBytes);
 uint32_t persistent_blocks(uint32_t cus, int stack);

@@ -85,3 +85,34 @@ def test_routes_agree_and_graphs_survive_growth(sizes):
                 t.zero_()
         g.replay()
         assert all(torch.equal(a, b) for a, b in zip(p.out(torch), ref))
+
+
+def test_single_view_graph_survives_growth():
+    """A graph of single-view passes A and C keeps its ray queues when later eager calls on the same
+    context need larger ones: a multi-view call with a larger view, then a larger single view."""
+    import torch
+
+    def single(ctx, p, stream=None):
+        (u,), (g,), (bufs,) = p.us, p.gs, p.bufs
+        ctx.initial_temporal(u, g, g, None, bufs[0], None, stream)
+        for j in range(PASSES):
+            ctx.unbiased(u, K, j, g, bufs[j % 2], bufs[1 - j % 2], None, stream)
+
+    p, large, larger = (_Passes(torch, [size]) for size in ((200, 120), (520, 400), (900, 700)))
+    ctx = p.b.views[0]["ctx"]  # holds the room, the scene of all three
+    single(ctx, p)  # eager: sizes the queues
+    ref = p.out(torch)[0]
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        single(ctx, p, s)
+    large.b.ctx = ctx
+    for step in (large.run, lambda: single(ctx, larger)):
+        step()
+        for _ in range(3):
+            for t in p.bufs[0]:
+                t.zero_()
+            graph.replay()
+            assert torch.equal(p.out(torch)[0], ref)
+            step()
