@@ -386,15 +386,11 @@ extern "C" int restir_build_alias_table_device(restir_ctx *ctx, const restir_poi
     // the device-wide steps, unless the larger scratch cannot be had under capture
     bool many = n > kMany;
     size_t bytes = carve(nullptr, many);
-    if (many && bytes > ctx->aliasScratchBytes) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            many = false;
-            bytes = carve(nullptr, many);
-        }
+    if (many && bytes > ctx->aliasScratchBytes && in_capture(s)) {
+        many = false;
+        bytes = carve(nullptr, many);
     }
-    if (int r = ensure(ctx, &ctx->aliasScratch, &ctx->aliasScratchBytes, bytes)) return r;
+    if (int r = ensure_kept(ctx, &ctx->aliasScratch, &ctx->aliasScratchBytes, &ctx->aliasInGraph, bytes, s)) return r;
     carve(ctx->aliasScratch, many);
     if (!many) {
         RK_LAUNCH("k_alias_build", k_alias_build, dim3(1), dim3(kLanes), 0, s, pts, tls, n, columns, p.power, p.scaled,

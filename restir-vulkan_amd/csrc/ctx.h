@@ -38,7 +38,7 @@ struct restir_ctx {
     void *scratch = nullptr;       // ray queues of the queued Pass C schedule
     size_t scratchBytes = 0;
     bool scratchInGraph = false;   // a stream capture recorded launches that use it
-    std::vector<void *> retired;   // earlier scratches, slots and records that captured graphs still use
+    std::vector<void *> retired;   // what had to grow while captured graphs still use it (ensure_kept)
     uint32_t queuedNpx = 0;        // shape of the last queued Pass C (its rays stay in scratch)
     const restir_reservoir *queuedOut = nullptr;  // its output (the light end of its neighbour rays)
     int queuedK = 0;
@@ -64,6 +64,7 @@ struct restir_ctx {
     void *bvhInfoHost = nullptr;   // pinned: the counters of the tree build
     void *aliasScratch = nullptr;  // powers, weights and queues of the device alias-table build
     size_t aliasScratchBytes = 0;
+    bool aliasInGraph = false;     // a stream capture recorded a build that uses it
     void *wide = nullptr;          // the bound tree's 4-entry nodes (+ the nesting flag)
     size_t wideBytes = 0;
     void *records = nullptr;       // Pass A's light records (k_light_records)

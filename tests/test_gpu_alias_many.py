@@ -81,3 +81,37 @@ def test_captured_with_and_without_the_large_scratch():
             g.replay()
             torch.cuda.synchronize()
             assert np.array_equal(cols.cpu().numpy(), want)
+
+
+def test_graph_of_the_small_scratch_survives_its_growth():
+    """Above 4,096 lights with scratch for one workgroup only, a capture records that route; an eager
+    build of the same size then needs the larger scratch, and the graph keeps the one it has."""
+    import torch
+    n = 6000
+    ctx = abi.Context(0)
+    want = {}
+    for m in (5000, n, 20000):
+        pts = np.zeros(m, dtype=abi.POINT_LIGHT_DTYPE)
+        pts["color_lum"][:, 3] = _powers("log_uniform", m, np.random.default_rng(m))
+        want[m] = (abi.build_alias_table(pts, None).view(np.uint8),
+                   torch.from_numpy(pts.view(np.uint8).reshape(-1).copy()).cuda(),
+                   torch.zeros(16 * m, dtype=torch.uint8, device="cuda"))
+
+    def check(m):
+        torch.cuda.synchronize()
+        assert np.array_equal(want[m][2].cpu().numpy(), want[m][0]), m
+        want[m][2].zero_()
+
+    _build(torch, ctx, *want[5000][1:])  # device-wide: more than 6,000 lights take in one workgroup
+    check(5000)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        ctx.build_alias_table(want[n][1], n, None, 0, want[n][2], stream=s)
+    for m in (n, 20000):
+        for _ in range(3):
+            _build(torch, ctx, *want[m][1:])
+            check(m)
+            g.replay()
+            check(n)
