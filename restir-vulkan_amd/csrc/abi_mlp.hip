@@ -78,6 +78,9 @@ static int ensure_slots(restir_ctx *ctx, uint32_t k) {
         hipError_t e = hipMalloc(&ctx->slots, n * (each + sizeof(uint32_t)));
         if (e == hipSuccess) {
             e = hipMemset(static_cast<uint8_t *>(ctx->slots) + n * each, 0, n * sizeof(uint32_t));
+            // a memset may return before it has run: launches on a stream that does not wait for the null
+            // stream would find words that are not 0, or lose theirs to it
+            if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
             if (e != hipSuccess) return hip_fail(ctx, e, "set_light_clusters: slots");
             ctx->slotCount = n;
             ctx->slotClusters = k;

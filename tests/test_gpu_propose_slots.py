@@ -106,3 +106,19 @@ def test_graph_outlives_its_slots(torch):
         eager = f.outputs()
         f.propose(wide.mlp, eager)
         f.check(eager, want)
+
+
+def test_slots_are_ready_on_return(torch):
+    """set_light_clusters leaves nothing of the slots' set-up under way: a launch on a stream that does
+    not wait for the default one may follow at once."""
+    f = Frame(torch, 257, 129, 8)
+    want = f.narrow()
+    for k in (512, 1024, 2048, 4096):  # larger slots each time
+        e = Embedded(torch, f.lp, k, k // 2)
+        out, s = f.outputs(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        f.r.ctx.set_light_clusters(k, *e.tables)
+        assert torch.cuda.default_stream().query()
+        f.propose(e.mlp, out, s)
+        torch.cuda.synchronize()
+        f.check(out, want)
