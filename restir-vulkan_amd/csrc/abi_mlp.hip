@@ -196,10 +196,9 @@ int restir_learned_candidates(restir_ctx *ctx, const restir_uniforms *u, const r
     const uint32_t seed = u->frame * 0x9e3779b1u + 0x7f4a7c15u;
     if (ctx->slots && in_capture(static_cast<hipStream_t>(stream))) ctx->slotsInGraph = true;
     uint8_t *slots = static_cast<uint8_t *>(ctx->slots);
-    const rk::WideSlots wide{slots,
-                             slots ? reinterpret_cast<uint32_t *>(slots + ctx->slotCount * rk::wide_slot_bytes(ctx->slotClusters))
-                                   : nullptr,
-                             ctx->slotCount};
+    const size_t each = rk::wide_slot_bytes(ctx->slotClusters);
+    const rk::WideSlots wide{slots, slots ? reinterpret_cast<uint32_t *>(slots + ctx->slotCount * each) : nullptr,
+                             ctx->slotCount, each};
     const hipError_t e = rk::mlp_propose(*m, view_of(g), cam, lo, hi, ctx->scene, ctx->lightCluster,
                                          ctx->lightPWithin, ctx->clusterBegin, ctx->clusterCount,
                                          ctx->clusterLights, ctx->clusterAlias,

@@ -194,12 +194,14 @@ hipError_t mlp_train(restir_mlp &m, const GView &g, rt::f3 cam, const float lo[3
                      uint32_t seed, float *lossOut, void *scratch, hipStream_t s);
 hipError_t mlp_adam(restir_mlp &m, const float *gw, const float *gb, const uint32_t *nValid, float lr,
                     hipStream_t s);
-// k_propose_wide's memory for workgroups in flight: n slots of wide_slot_bytes each, and a word per
-// slot that is 1 while a workgroup holds it (all 0 between launches)
+// k_propose_wide's memory for workgroups in flight: n slots of `each` bytes (wide_slot_bytes of the most
+// clusters they were made for, whatever the network's: launches of several sizes may share them), and a
+// word per slot that is 1 while a workgroup holds it (all 0 between launches)
 struct WideSlots {
     void *base;
     uint32_t *busy;
     uint32_t n;
+    size_t each;
 };
 size_t wide_slot_bytes(uint32_t K);
 uint32_t wide_slots(uint32_t cus);  // workgroups that the device holds at a time

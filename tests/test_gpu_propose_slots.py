@@ -122,3 +122,28 @@ def test_slots_are_ready_on_return(torch):
         f.propose(e.mlp, out, s)
         torch.cuda.synchronize()
         f.check(out, want)
+
+
+def test_two_networks_share_the_slots(torch):
+    """Launches of 4,096 and 512 clusters in flight at a time, over the slots made for 4,096."""
+    f = Frame(torch, 1031, 517, 3)
+    want = f.narrow()
+    big, small = Embedded(torch, f.lp, 4096, 1024), Embedded(torch, f.lp, 512, 256)
+    f.r.ctx.set_light_clusters(4096, *big.tables)
+    out, got = f.outputs(), [f.outputs() for _ in range(6)]
+    f.propose(big.mlp, out)
+    torch.cuda.synchronize()
+    graph, streams = torch.cuda.CUDAGraph(), [torch.cuda.Stream(), torch.cuda.Stream()]
+    with torch.cuda.graph(graph, stream=streams[0]):
+        f.propose(big.mlp, out, streams[0])
+    f.r.ctx.set_light_clusters(512, *small.tables)
+    for o in out:
+        o.fill_(-7)
+    torch.cuda.synchronize()
+    for o in got:
+        with torch.cuda.stream(streams[0]):
+            graph.replay()
+        f.propose(small.mlp, o, streams[1])
+    torch.cuda.synchronize()
+    for o in [out, *got]:
+        f.check(o, want)
