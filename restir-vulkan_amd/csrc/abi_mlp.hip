@@ -255,7 +255,8 @@ int restir_mlp_train(restir_ctx *ctx, restir_mlp *m, const restir_uniforms *u, c
     const uint32_t W = u->screenSize[0], H = u->screenSize[1];
     if (int r = check_gbuffer(ctx, g, W, H, false, "mlp_train")) return r;
     if (int r = use_device(ctx)) return r;
-    if (int r = ensure(ctx, &ctx->mlpScratch, &ctx->mlpScratchBytes, rk::mlp_scratch_bytes(n, m->n_clusters)))
+    if (int r = ensure_kept(ctx, &ctx->mlpScratch, &ctx->mlpScratchBytes, &ctx->mlpInGraph,
+                            rk::mlp_scratch_bytes(n, m->n_clusters), static_cast<hipStream_t>(stream)))
         return r;
     const rt::f3 cam{u->cameraPos[0], u->cameraPos[1], u->cameraPos[2]};
     const hipError_t e = rk::mlp_train(*m, view_of(g), cam, lo, hi, res, ctx->lightCluster, ctx->scene.nLights,
@@ -288,7 +289,8 @@ int restir_mlp_forward(restir_ctx *ctx, const restir_mlp *m, const uint16_t *X, 
     if (n == 0 || n % 64 != 0 || n > 65536)
         return fail(ctx, RESTIR_E_INVALID_ARGUMENT, "mlp_forward: n=%u (multiple of 64, <= 65536)", n);
     if (int r = use_device(ctx)) return r;
-    if (int r = ensure(ctx, &ctx->mlpScratch, &ctx->mlpScratchBytes, rk::mlp_scratch_bytes(n, m->n_clusters)))
+    if (int r = ensure_kept(ctx, &ctx->mlpScratch, &ctx->mlpScratchBytes, &ctx->mlpInGraph,
+                            rk::mlp_scratch_bytes(n, m->n_clusters), static_cast<hipStream_t>(stream)))
         return r;
     const hipError_t e = rk::mlp_forward(*m, X, n, logits, ctx->mlpScratch, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "mlp_forward launch");
@@ -305,7 +307,8 @@ int restir_mlp_loss_grad(restir_ctx *ctx, const restir_mlp *m, const uint16_t *X
     if (n == 0 || n % 64 != 0 || n > 65536)
         return fail(ctx, RESTIR_E_INVALID_ARGUMENT, "mlp_loss_grad: n=%u (multiple of 64, <= 65536)", n);
     if (int r = use_device(ctx)) return r;
-    if (int r = ensure(ctx, &ctx->mlpScratch, &ctx->mlpScratchBytes, rk::mlp_scratch_bytes(n, m->n_clusters)))
+    if (int r = ensure_kept(ctx, &ctx->mlpScratch, &ctx->mlpScratchBytes, &ctx->mlpInGraph,
+                            rk::mlp_scratch_bytes(n, m->n_clusters), static_cast<hipStream_t>(stream)))
         return r;
     const hipError_t e = rk::mlp_loss_grad(*m, X, target, mask, n, gw, gb, loss, ctx->mlpScratch,
                                            static_cast<hipStream_t>(stream));

@@ -48,9 +48,9 @@ int check_views(restir_ctx *ctx, const restir_view *views, uint32_t n, const cha
     return RESTIR_OK;
 }
 
-int prepare(restir_ctx *ctx, uint32_t n) {
+int prepare(restir_ctx *ctx, uint32_t n, hipStream_t s) {
     if (int r = use_device(ctx)) return r;
-    return ensure(ctx, &ctx->viewTable, &ctx->viewTableBytes, rk::views_table_bytes(n));
+    return ensure_kept(ctx, &ctx->viewTable, &ctx->viewTableBytes, &ctx->viewsInGraph, rk::views_table_bytes(n), s);
 }
 
 uint32_t *view_counter(restir_ctx *ctx) { return ctx->counters + 8; }
@@ -130,7 +130,7 @@ int restir_initial_temporal_views(restir_ctx *ctx, const restir_view *views, uin
         }
         return RESTIR_OK;
     }
-    if (int r = prepare(ctx, n)) return r;
+    if (int r = prepare(ctx, n, s)) return r;
     const hipError_t e = rk::launch_pass_a_views(tile, stack, rec.data(), n, ctx->viewTable, view_counter(ctx),
                                                  resident_blocks(ctx->cus, static_cast<uint32_t>(stack) * 1024u), s);
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "initial_temporal_views launch");
@@ -157,7 +157,7 @@ int restir_spatial_views(restir_ctx *ctx, const restir_view *views, uint32_t n, 
         rec[v] = rk::ViewB{*u, view_of(w.cur), w.in, w.out, rt::cos_degrees(u->spatialNormalThreshold)};
     }
     if (int r = check_disjoint(ctx, outs, ins, "spatial_views")) return r;
-    if (int r = prepare(ctx, n)) return r;
+    if (int r = prepare(ctx, n, static_cast<hipStream_t>(stream))) return r;
     const hipError_t e = rk::launch_pass_b_views(tile, rec.data(), n, iter, ctx->viewTable, view_counter(ctx),
                                                  ctx->persistentBlocks, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "spatial_views launch");
@@ -207,7 +207,7 @@ int restir_unbiased_views(restir_ctx *ctx, const restir_view *views, uint32_t n,
         }
         return RESTIR_OK;
     }
-    if (int r = prepare(ctx, n)) return r;
+    if (int r = prepare(ctx, n, s)) return r;
     const hipError_t e = rk::launch_pass_c_views(tile, stack, rec.data(), n, k, iter, ctx->viewTable,
                                                  view_counter(ctx), resident_blocks(ctx->cus, static_cast<uint32_t>(stack) * 1024u),
                                                  s);
@@ -236,7 +236,7 @@ int restir_shade_views(restir_ctx *ctx, const restir_view *views, uint32_t n, fl
                                view_of(w.cur), w.in, w.rgb, w.rgb_stride};
     }
     if (int r = check_disjoint(ctx, outs, ins, "shade_views")) return r;
-    if (int r = prepare(ctx, n)) return r;
+    if (int r = prepare(ctx, n, static_cast<hipStream_t>(stream))) return r;
     const hipError_t e = rk::launch_shade_views(rec.data(), n, gamma, ctx->viewTable, view_counter(ctx),
                                                 ctx->persistentBlocks, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, "shade_views launch");

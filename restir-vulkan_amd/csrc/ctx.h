@@ -55,10 +55,12 @@ struct restir_ctx {
     rk::Recorder recorder;
     void *mlpScratch = nullptr;    // training tensors of the learned proposal
     size_t mlpScratchBytes = 0;
+    bool mlpInGraph = false;       // a stream capture recorded launches that use it
     void *truthScratch = nullptr;  // per-light-chunk partial sums of the FP64 ground truth
     size_t truthScratchBytes = 0;
     void *viewTable = nullptr;     // per-view records of the batched-view launches
     size_t viewTableBytes = 0;
+    bool viewsInGraph = false;     // a stream capture recorded launches that use it
     void *bvhScratch = nullptr;    // primitive order, keys and ranges of the GPU tree build
     size_t bvhScratchBytes = 0;
     void *bvhInfoHost = nullptr;   // pinned: the counters of the tree build

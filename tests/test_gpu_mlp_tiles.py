@@ -43,3 +43,40 @@ def test_matches_oracle(K, n):
         sl, bl = slice(layer * 128 * 128, (layer * 128 + rows) * 128), slice(layer * 128, layer * 128 + rows)
         assert np.linalg.norm(gW[sl] - rgW[sl]) / np.linalg.norm(rgW[sl]) < 2e-2, layer
         assert np.linalg.norm(gB[bl] - rgB[bl]) / np.linalg.norm(rgB[bl]) < 2e-2, layer
+
+
+def test_graph_keeps_its_scratch():
+    """A captured step's activations and partial sums stay its own when a larger batch needs more."""
+    import torch
+    K, n, larger = 256, 256, 4096
+    ctx = abi.Context(0)
+    nW, nB = mlp_sizes(K)
+    z = lambda m, t=torch.float32: torch.zeros(m, dtype=t, device="cuda")  # noqa: E731
+    w_bf16, w, b, m, v = z(nW, torch.int16), z(nW), z(nB), z(nW + nB), z(nW + nB)
+    mlp = MlpStruct(K, 0, w_bf16.data_ptr(), w.data_ptr(), b.data_ptr(), m.data_ptr(), v.data_ptr())
+    ctx.mlp_init(mlp, 5, z(K))
+    X, tgt, mask = rand_features(torch, larger, 1)[0], z(larger, torch.int32), z(larger, torch.int32) + 1
+    out = z(nW), z(nB), z(1)
+
+    def step(count, stream=None):
+        ctx.mlp_loss_grad(mlp, X, tgt, mask, count, *out, stream=stream)
+
+    def results():
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        for t in out:
+            t.zero_()
+        return got
+
+    step(n)
+    ref = results()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        step(n, s)
+    for _ in range(3):
+        step(larger)
+        assert results()[2].item() > 0
+        graph.replay()
+        assert all(torch.equal(a, c) for a, c in zip(results(), ref))

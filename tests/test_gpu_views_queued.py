@@ -116,3 +116,29 @@ def test_single_view_graph_survives_growth():
             graph.replay()
             assert torch.equal(p.out(torch)[0], ref)
             step()
+
+
+def test_graph_of_views_keeps_its_table():
+    """The per-view records of a captured persistent launch stay its own when a call over more views
+    needs a larger table."""
+    import torch
+    p, more = _Passes(torch, [(64, 48), (33, 21)]), _Passes(torch, [(16 + i, 9) for i in range(12)])
+    inline = abi.Launch(0, 0, abi.SCHEDULE_INLINE)
+    p.run(inline)
+    ref = p.out(torch)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        p.run(inline, s)
+    more.run(inline)
+    want = more.out(torch)
+    more.b.ctx = p.b.ctx
+    for _ in range(3):
+        more.run(inline)
+        assert all(torch.equal(a, b) for a, b in zip(more.out(torch), want))
+        for buf in p.bufs:
+            for t in buf:
+                t.zero_()
+        graph.replay()
+        assert all(torch.equal(a, b) for a, b in zip(p.out(torch), ref))
