@@ -991,8 +991,9 @@ __device__ inline bool inside(float4 mn, float4 mx, float4 outerMn, float4 outer
 // threads together check every box and every parent-child pair; info[1] gets the bits of the
 // largest |coordinate| of any box (non-negative floats order as their bit patterns; a NaN orders
 // above every number).
-// It also writes the parent slot (2 node + side) of each internal child, and sets info[2] when a
-// box is not finite and ordered, info[3] when a leaf's box is not the bounding box of its triangle.
+// It also writes the parent slot (2 node + side) of each internal child (unless parent is null), and
+// sets info[2] when a box is not finite and ordered, info[3] when a leaf's box is not the bounding box
+// of its triangle.
 __global__ __launch_bounds__(256) void k_wide_build(const rt::Node *__restrict__ nodes, uint32_t nNodes,
                                                     const float4 *__restrict__ tris,
                                                     rt::WNode *__restrict__ wide, uint32_t *__restrict__ parent,
@@ -1021,7 +1022,7 @@ __global__ __launch_bounds__(256) void k_wide_build(const rt::Node *__restrict__
                     smn.z == fminf(fminf(v0.z, v1.z), v2.z) && smx.x == fmaxf(fmaxf(v0.x, v1.x), v2.x) &&
                     smx.y == fmaxf(fmaxf(v0.y, v1.y), v2.y) && smx.z == fmaxf(fmaxf(v0.z, v1.z), v2.z);
         } else {
-            parent[c] = 2u * x + static_cast<uint32_t>(side);
+            if (parent) parent[c] = 2u * x + static_cast<uint32_t>(side);
             const rt::Node cn = rt::load_node(nodes, c);
             mn[2 * side] = cn.lmin;
             mx[2 * side] = cn.lmax;
@@ -1090,10 +1091,10 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
     // a box is not finite, or too large or small: no 8-entry nodes. Areas are then finite: from about
     // 1.7e38 on a flat box's would be inf * 0, and no lane's NaN agrees with another's choice
     if (bounds[2] != 0 || !rt::w8_covers(maxCoord)) return;
+    if (info->overflow) return;  // of the levels before: not every node counted has its work entry
     for (uint32_t i0 = blockIdx.x * 64u; i0 < n; i0 += gridDim.x * 64u) {
         const uint32_t i = i0 + (threadIdx.x >> 3), me = begin + i;
-        // the same for a node's 8 lanes; nodes beyond maxNodes are counted but have no work entry
-        const bool on = i < n && me < maxNodes;
+        const bool on = i < n && me < maxNodes;  // the same for a node's 8 lanes
         uint32_t cnt = 0;
         float mn[3] = {}, mx[3] = {};  // this lane's entry: its box,
         int32_t ref = 0;               // >= 0 internal node, < 0 ~triangle,
@@ -1276,8 +1277,13 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     auto hip = [&](hipError_t e, const char *what) { return e == hipSuccess ? RESTIR_OK : hip_fail(ctx, e, what); };
     if (int r = hip(hipDeviceSynchronize(), "bind tree: wait for work in flight")) return r;
     // 8-entry nodes: every node with an internal child has 8 entries, so T triangles need at most
-    // 4 T / 7 + 1 nodes (each of them with two-triangle nodes below)
-    const uint32_t nTris = nNodes + 1, maxW8 = static_cast<uint32_t>(4ull * nTris / 7) + 8;
+    // 4 T / 7 + 1 nodes (each of them with two-triangle nodes below), usually less than half of that.
+    // Node indices take 23 bits of a child word, triangles 26 bits of a tracer's list entry; a tree
+    // that turns out to need more nodes, or for which there is no memory, keeps its 4-entry nodes.
+    const uint32_t nTris = nNodes + 1;
+    const uint64_t most = 4ull * nTris / 7 + 8;
+    const uint32_t maxW8 = static_cast<uint32_t>(most < (1u << 23) ? most : 1u << 23);
+    bool w8Fits = nTris <= (1u << 26);
     const auto carve = [&](void *base, size_t *bytes) {
         struct {
             rt::WNode *wide;
@@ -1285,29 +1291,37 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
             float4 *tris;
             uint32_t *parent, *work, *flags;
             W8Info *info;
-        } p;
+        } p{};
         rk::Carver c(base);
         p.wide = c.take<rt::WNode>(sizeof(rt::WNode) * static_cast<size_t>(nNodes));
-        p.w8 = c.take<rt::W8Node>(sizeof(rt::W8Node) * static_cast<size_t>(maxW8));
-        p.tris = c.take<float4>(48 * static_cast<size_t>(nTris));
-        p.parent = c.take<uint32_t>(4 * static_cast<size_t>(nNodes));
-        p.work = c.take<uint32_t>(4 * static_cast<size_t>(maxW8));
         p.flags = c.take<uint32_t>(16 + sizeof(W8Info));  // 4 flag words, then the counters
+        if (w8Fits) {
+            p.w8 = c.take<rt::W8Node>(sizeof(rt::W8Node) * static_cast<size_t>(maxW8));
+            p.tris = c.take<float4>(48 * static_cast<size_t>(nTris));
+            p.parent = c.take<uint32_t>(4 * static_cast<size_t>(nNodes));
+            p.work = c.take<uint32_t>(4 * static_cast<size_t>(maxW8));
+        }
         p.info = reinterpret_cast<W8Info *>(p.flags + 4);
         if (bytes) *bytes = c.end();
         return p;
     };
     size_t bytes = 0;
     carve(nullptr, &bytes);
-    if (int r = ensure(ctx, &ctx->wide, &ctx->wideBytes, bytes)) return r;
+    int held = ensure(ctx, &ctx->wide, &ctx->wideBytes, bytes);
+    if (held != RESTIR_OK && w8Fits) {  // the 4-entry nodes alone take half
+        (void)hipGetLastError();
+        ctx->error.clear();
+        w8Fits = false;
+        carve(nullptr, &bytes);
+        held = ensure(ctx, &ctx->wide, &ctx->wideBytes, bytes);
+    }
+    if (held != RESTIR_OK) return held;
     const auto p = carve(ctx->wide, nullptr);
     const auto *bn = static_cast<const rt::Node *>(nodes);
     const auto *bt = static_cast<const float4 *>(tris);
     RK_LAUNCH("k_w8_clear", k_w8_clear, dim3(1), dim3(64), 0, s, p.flags, p.info);
     RK_LAUNCH("k_wide_build", k_wide_build, dim3(groups(nNodes)), dim3(256), 0, s, bn, nNodes, bt, p.wide, p.parent,
               p.flags);
-    // node indices take 23 bits of a child word, triangles 26 bits of a tracer's list entry
-    const bool w8Fits = maxW8 <= (1u << 23) && nTris <= (1u << 26);
     // a level of 8-entry nodes covers at least one level of the tree
     const uint32_t levels = depth < static_cast<uint32_t>(kW8Levels) ? depth : static_cast<uint32_t>(kW8Levels);
     struct {
