@@ -1348,6 +1348,7 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     ctx->scene.wide = p.wide;
     ctx->scene.treeNested = host.flags[0] == 0 ? 1 : 0;
     ctx->scene.maxCoord = maxCoord;
+    ctx->scene.quickCoord = nNodes <= (1u << 25) ? maxCoord : __builtin_nanf("");
     ctx->scene.parent = p.parent;
     ctx->scene.w8 = p.w8;
     ctx->scene.w8Tris = p.tris;

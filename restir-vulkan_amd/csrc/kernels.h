@@ -39,6 +39,8 @@ struct SceneView {
     const rt::WNode *wide;  // the 4-entry nodes over `nodes` (same indices), built by the library
     int32_t treeNested;     // 1: every box finite and inside the box stored for its parent
     float maxCoord;         // largest |box coordinate| of the tree
+    float quickCoord;       // the same for the 4-entry walk's quick form, whose byte offsets of nodes take 32
+                            // bits: NaN (no segment is quick) for a tree of more than 2^25 nodes
     // the 8-entry nodes (rt_wide8.h), their triangles (p1.w: the slot that stores the triangle, 2 node
     // + side; p2.w: its index) and the parent slot of each binary node
     const rt::W8Node *w8;

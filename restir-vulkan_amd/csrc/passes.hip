@@ -391,7 +391,7 @@ __device__ __forceinline__ void pass_a_px(const PassAArgs &a, uint32_t x, uint32
         f3 o, d;
         shadow_segment(pos, res.pos, o, d);
         TraceStats st{0, 0};
-        if (occluded_w<STACK>(sc.wide, sc.nodes, sc.tris, sc.treeNested != 0, sc.maxCoord, o, d, stk, kBlock, st)) {
+        if (occluded_w<STACK>(sc.wide, sc.nodes, sc.tris, sc.treeNested != 0, sc.quickCoord, o, d, stk, kBlock, st)) {
             res.w = 0.0f;
             res.sumW = 0.0f;
         }
@@ -566,7 +566,7 @@ __device__ __forceinline__ void pass_c_px(const PassCArgs &a, uint32_t x, uint32
         f3 o, d;
         shadow_segment(pos, lp, o, d);
         TraceStats st{0, 0};
-        centreShadowed = occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.maxCoord, o, d, stk, kBlock, st);
+        centreShadowed = occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.quickCoord, o, d, stk, kBlock, st);
     }
     if (centreShadowed) {
         numSamples = 0;
@@ -580,7 +580,7 @@ __device__ __forceinline__ void pass_c_px(const PassCArgs &a, uint32_t x, uint32
                 f3 o, d;
                 shadow_segment(nwp, lp, o, d);
                 TraceStats st{0, 0};
-                if (occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.maxCoord, o, d, stk, kBlock, st)) continue;
+                if (occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.quickCoord, o, d, stk, kBlock, st)) continue;
             }
             numSamples += nM[j];
         }
@@ -933,7 +933,7 @@ __global__ __launch_bounds__(256) void k_trace_queue(const SceneView sc, const f
                                                   ? p2[i]
                                                   : reinterpret_cast<const float4 *>(q.merged + (tag & 0x07ffffffu))[0];
                             shadow_segment(xyz(a4), xyz(b4), o, d);
-                            wwalk_begin(w, o, d, sc.treeNested != 0, sc.maxCoord);
+                            wwalk_begin(w, o, d, sc.treeNested != 0, sc.quickCoord);
                             ray = static_cast<int32_t>(i);
                         }
                     }
@@ -1525,7 +1525,7 @@ __global__ __launch_bounds__(256) void k_shade(const ShadeArgs a) {
                 f3 o, d;
                 shadow_segment(plane3(a.g.pos, i, a.g.P), r.pos, o, d);
                 TraceStats st{0, 0};
-                occ = occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.maxCoord, o, d,
+                occ = occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.quickCoord, o, d,
                                         stack + threadIdx.x, 256, st);
             }
         }
@@ -1551,7 +1551,7 @@ __global__ __launch_bounds__(256) void k_trace(const TraceArgs a) {
     TraceStats st{0, 0};
     bool occ;
     if constexpr (REF) occ = occluded<STACK, true>(a.sc.nodes, a.sc.tris, o, d, stack + threadIdx.x, 256, st);
-    else occ = occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.maxCoord, o, d, stack + threadIdx.x,
+    else occ = occluded_w<STACK>(a.sc.wide, a.sc.nodes, a.sc.tris, a.sc.treeNested != 0, a.sc.quickCoord, o, d, stack + threadIdx.x,
                                  256, st);
     a.shadowed[i] = occ ? 1u : 0u;
     if (a.visits) a.visits[i] = st.visits;
@@ -1585,7 +1585,7 @@ __global__ __launch_bounds__(256) void k_trace_pool(const TraceArgs a, uint32_t 
                     f3 o, d;
                     shadow_segment(xyz(a.p1[i]), xyz(a.p2[i]), o, d);
                     if constexpr (REF) walk_begin(w, o, d);
-                    else wwalk_begin(w, o, d, a.sc.treeNested != 0, a.sc.maxCoord);
+                    else wwalk_begin(w, o, d, a.sc.treeNested != 0, a.sc.quickCoord);
                     ray = static_cast<int32_t>(i);
                 }
             }

@@ -9,6 +9,7 @@ pytestmark = pytest.mark.gpu
 
 GRID = 2830
 N = 2 * (GRID - 1) ** 2
+HUGE_GRID = 4130  # more than 2^25 triangles
 
 
 @pytest.fixture(scope="module")
@@ -18,20 +19,25 @@ def torch():
     return t
 
 
-@pytest.fixture(scope="module")
-def ground(torch):
+def _field(torch, grid):
     """A height field's triangles, and their tree built by a first context."""
     g = torch.Generator(device="cuda").manual_seed(2)
-    y = torch.rand(GRID, GRID, device="cuda", generator=g) * 2e-3
-    x, z = torch.meshgrid(*[torch.linspace(-1, 1, GRID, device="cuda")] * 2, indexing="ij")
+    y = torch.rand(grid, grid, device="cuda", generator=g) * 2e-3
+    x, z = torch.meshgrid(*[torch.linspace(-1, 1, grid, device="cuda")] * 2, indexing="ij")
     p = torch.stack([x, y, z], dim=2)
     a, b, c, d = p[:-1, :-1], p[1:, :-1], p[:-1, 1:], p[1:, 1:]
     xyz = torch.stack([torch.stack([a, b, c], 2), torch.stack([b, d, c], 2)], 2).reshape(-1, 9).contiguous()
-    nodes = torch.zeros(80 * (N - 1), dtype=torch.uint8, device="cuda")
-    tris = torch.zeros(48 * N, dtype=torch.uint8, device="cuda")
+    n = len(xyz)
+    nodes = torch.zeros(80 * (n - 1), dtype=torch.uint8, device="cuda")
+    tris = torch.zeros(48 * n, dtype=torch.uint8, device="cuda")
     ctx = abi.Context(0)
-    ctx.build_bvh(xyz, N, nodes, tris)
+    ctx.build_bvh(xyz, n, nodes, tris)
     return ctx, nodes, tris
+
+
+@pytest.fixture(scope="module")
+def ground(torch):
+    return _field(torch, GRID)
 
 
 def _segments(torch, n=50000):
@@ -84,3 +90,14 @@ def test_bound_without_room_for_8_entry_nodes(torch, ground):
     ctx.set_bvh(nodes, N - 1, tris, N)  # now there is
     got, covered = _trace(torch, ctx)
     assert torch.equal(got, ref) and covered
+
+
+def test_walks_of_a_tree_beyond_32_bit_offsets(torch):
+    """More than 2^25 nodes of 128 bytes: the 4-entry walk's quick form has 32 bits for their offsets."""
+    assert 2 * (HUGE_GRID - 1) ** 2 - 1 > 1 << 25
+    ctx, nodes, tris = _field(torch, HUGE_GRID)
+    ref, _ = _trace(torch, ctx, reference_loop=True)
+    visits = torch.zeros(len(ref), dtype=torch.int32, device="cuda")
+    for name, kw in (("first hit", {}), ("with counts", {"visits": visits}), ("a ray per lane", {"one_ray_per_lane": True})):
+        got, _ = _trace(torch, ctx, **kw)
+        assert torch.equal(got, ref), name
