@@ -534,9 +534,11 @@ int restir_camera_projection_view(const restir_camera *cam, float aspect, float 
  * (RESTIR_INPUT_VISIBLE_FLAG is ignored here). restir_spatial_views and restir_shade_views are one
  * launch over the tiles of all views, so small and large views share the GPU without a
  * tail per view. The two calls that trace shadow rays run the views one after another on the queued
- * schedule with ctx's scratch and counters; with launch->schedule = RESTIR_SCHEDULE_INLINE, or where
- * the scratch cannot grow (under stream capture, or out of memory), they too are one persistent
- * launch, rays traced per pixel. The per-view records of a persistent launch are written to
+ * schedule with ctx's scratch and counters (growing it to the largest view's, and ending the life of
+ * the rays that a queued restir_unbiased on ctx left there) where that is faster, which their
+ * number, sizes and scenes' triangles decide; with many small views or small trees, with
+ * launch->schedule = RESTIR_SCHEDULE_INLINE, or where the scratch cannot grow (under stream capture,
+ * or out of memory), they too are one persistent launch, rays traced per pixel. The per-view records of a persistent launch are written to
  * context-owned device memory by kernels on `stream` (no host-memory reads at execution), so a
  * sequence of these calls can be captured in a HIP graph; calls on one context must stay on one
  * stream. Outputs may not overlap each other or any view's inputs. */

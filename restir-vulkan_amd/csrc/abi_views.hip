@@ -1,9 +1,10 @@
 // abi_views.hip — batched-view entry points (restir_*_views): per-view validation with the same
-// rules as the single-view entry points, then one persistent launch per pass, or, for the passes that
-// trace shadow rays, the queued schedule view after view.
+// rules as the single-view entry points, then one launch per pass over all views, or, for the passes that
+// trace shadow rays, the queued schedule view after view where that is faster (Route).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "ctx.h"
@@ -55,14 +56,47 @@ int prepare(restir_ctx *ctx, uint32_t n, hipStream_t s) {
 
 uint32_t *view_counter(restir_ctx *ctx) { return ctx->counters + 8; }
 
-// Whether the passes that trace rays run view after view on the queued schedule, with this context's
-// scratch (`bytes`: the largest view's) and work counters: unless the caller asks for the inline
-// schedule, or the scratch is too small and cannot grow (the stream is being captured, or the
-// device is out of memory). Tracing in the pixels' lanes keeps a wave until its longest ray ends
-// and cannot gather triangle tests: 8 views from 640x360 to 1920x1080 over 2 scenes take 21.5 ms of
-// one-launch passes A and C that way, 13.6 ms queued, with a launch sequence per view.
-bool queued_views(restir_ctx *ctx, const restir_launch *launch, size_t bytes, hipStream_t s) {
-    if (launch && launch->schedule == RESTIR_SCHEDULE_INLINE) return false;
+// The two routes of a pass that traces rays: queued, view after view, or inline, one persistent launch
+// over all views with the rays traced in the pixels' lanes. Queued, each view takes a few launches and
+// waits for its longest ray; inline, one launch does, but a wave waits for the longest ray of its pixels and
+// cannot gather triangle tests. All of it grows with the depth of the trees, L = log2(triangles). In us
+//   Pass A:  queued 5.6 L a view more; inline  8.2 L once, 18 (L - 10) - 1.6 (M - 8) a million pixels more
+//   Pass C:  queued 5.6 L a view more; inline  4 (k + 2) L once, 14 (k + 1) (L - 7) a million pixels more
+// (negative over small trees and with many candidates, where inline costs less per pixel too). Fitted to
+// 560 pairs of times for each pass: 1 to 12 views of 64 to 1,080 lines, 34 to 593,000 triangles, M 8 and 32,
+// k 3 and 5. What this picks takes at most 1.3 times what the other route takes (4 pairs above 1.15);
+// always queued takes up to 8.1 times, always inline up to 6.5. Inline against queued, 138,000 triangles:
+//   12 views of      120 lines        240 lines        720 lines       1 view of 120 lines
+//   Pass A, M = 32   0.41, 1.62 ms    0.83, 1.85 ms    5.59, 5.86 ms   0.18, 0.13 ms
+//   Pass C, k = 5    1.19, 1.33       2.62, 2.08       17.3, 6.58      0.56, 0.11
+// Without rays one view takes about as long either way, and more are better inline (12 views of 240 lines:
+// Pass A 0.34, 0.75 ms, Pass C 0.18, 0.26).
+class Route {
+  public:
+    // perMpx: what inline costs more per million pixels of a view, from its L
+    template <class F>
+    void add(const restir_view &w, F perMpx) {
+        const restir_uniforms &u = *w.uniforms;
+        const double L = std::log2(std::max(2u, w.scene->treeTris));
+        ++views_;
+        rays_ = rays_ || (u.flags & RESTIR_VISIBILITY_REUSE_FLAG);
+        deepest_ = std::max(deepest_, L);
+        gain_ += 5.6 * L - 1e-6 * u.screenSize[0] * u.screenSize[1] * perMpx(L);
+    }
+    // once: what the inline launch costs more, per L
+    bool queued(double once) const { return rays_ ? gain_ <= once * deepest_ : views_ == 1; }
+
+  private:
+    double gain_ = 0.0, deepest_ = 0.0;
+    uint32_t views_ = 0;
+    bool rays_ = false;
+};
+
+// Whether the views run queued, with this context's scratch (`bytes`: the largest view's) and work
+// counters: where that is the faster route (`pays`), unless the caller asks for the inline schedule or
+// the scratch is too small and cannot grow (the stream is being captured, or the device is out of memory).
+bool queued_views(restir_ctx *ctx, const restir_launch *launch, bool pays, size_t bytes, hipStream_t s) {
+    if (!pays || (launch && launch->schedule == RESTIR_SCHEDULE_INLINE)) return false;
     // what the scratch held of a single-view Pass C will be overwritten
     ctx->queuedNpx = 0;
     ctx->surfValid = false;
@@ -93,6 +127,7 @@ int restir_initial_temporal_views(restir_ctx *ctx, const restir_view *views, uin
     std::vector<rk::ViewA> rec(n);
     std::vector<Span> outs, ins;
     size_t queueBytes = 0;
+    Route route;
     int stack = 24;  // the smallest compiled stack; raised to the deepest scene's
     for (uint32_t v = 0; v < n; ++v) {
         const restir_view &w = views[v];
@@ -113,12 +148,13 @@ int restir_initial_temporal_views(restir_ctx *ctx, const restir_view *views, uin
         outs.push_back({w.out, bytes});
         if (w.scene->stack > stack) stack = w.scene->stack;
         queueBytes = std::max(queueBytes, rk::pass_a_queue_bytes(W * H));
+        route.add(w, [u](double L) { return 18.0 * (L - 10.0) - 1.6 * (static_cast<double>(u->initialLightSampleCount) - 8.0); });
         rec[v] = rk::ViewA{*u, w.scene->scene, view_of(w.cur), view_of(temporal ? w.prev : nullptr), w.in, w.out};
     }
     if (int r = check_disjoint(ctx, outs, ins, "initial_temporal_views")) return r;
     if (int r = use_device(ctx)) return r;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (queued_views(ctx, launch, queueBytes, s)) {
+    if (queued_views(ctx, launch, route.queued(8.2), queueBytes, s)) {
         for (uint32_t v = 0; v < n; ++v) {
             const rk::ViewA &w = rec[v];
             const int st = views[v].scene->stack;
@@ -173,6 +209,7 @@ int restir_unbiased_views(restir_ctx *ctx, const restir_view *views, uint32_t n,
     std::vector<rk::ViewC> rec(n);
     std::vector<Span> outs, ins;
     size_t queueBytes = 0;
+    Route route;
     bool queueable = true;
     int stack = 24;  // the smallest compiled stack; raised to the deepest scene's
     for (uint32_t v = 0; v < n; ++v) {
@@ -189,6 +226,7 @@ int restir_unbiased_views(restir_ctx *ctx, const restir_view *views, uint32_t n,
         outs.push_back({w.out, bytes});
         if (w.scene->stack > stack) stack = w.scene->stack;
         queueBytes = std::max(queueBytes, rk::pass_c_queue_bytes(W * H, k));
+        route.add(w, [k](double L) { return 14.0 * (k + 1) * (L - 7.0); });
         // a queued neighbour ray carries its pixel in 27 bits of its tag
         queueable = queueable && static_cast<uint64_t>(W) * H < (1ull << 27);
         rec[v] = rk::ViewC{*u, w.scene->scene, view_of(w.cur), w.in, w.out};
@@ -196,7 +234,7 @@ int restir_unbiased_views(restir_ctx *ctx, const restir_view *views, uint32_t n,
     if (int r = check_disjoint(ctx, outs, ins, "unbiased_views")) return r;
     if (int r = use_device(ctx)) return r;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (queueable && queued_views(ctx, launch, queueBytes, s)) {
+    if (queued_views(ctx, launch, queueable && route.queued(4.0 * (k + 2)), queueBytes, s)) {
         for (uint32_t v = 0; v < n; ++v) {
             rk::ViewC &w = rec[v];
             w.u.flags &= ~RESTIR_INPUT_VISIBLE_FLAG;  // these calls make no use of the promise

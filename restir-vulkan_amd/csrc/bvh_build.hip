@@ -1363,6 +1363,7 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     ctx->stack = depth <= 24 ? 24 : (depth <= 32 ? 32 : 64);
     ctx->persistentBlocks = persistent_blocks(ctx->cus, ctx->stack);
     ctx->treeDepth = depth;
+    ctx->treeTris = nTris;
     ctx->bvhSet = true;
     return RESTIR_OK;
 }

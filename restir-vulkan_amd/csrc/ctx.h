@@ -30,7 +30,7 @@ struct restir_ctx {
     bool lightsSet = false;
     bool bvhSet = false;
     int stack = 32;
-    uint32_t treeDepth = 0;
+    uint32_t treeDepth = 0, treeTris = 0;
     uint32_t *counters = nullptr;  // device work counters of the persistent kernels
     uint32_t cus = 256;                // compute units of the device
     uint32_t persistentBlocks = 1280;  // workgroups of the persistent tracers (see persistent_blocks)

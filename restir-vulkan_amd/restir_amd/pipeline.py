@@ -275,10 +275,11 @@ class BatchRenderer:
     the same Scene object share its device tables (one context per distinct scene). Every view
     has its own G-buffers, reservoirs and image; ``rgb`` holds all images back to back and
     ``images[v]`` is view v's [3 * W * H] slice. Pass B and shading of all views run as one
-    persistent launch each (restir_*_views). The passes that trace shadow rays, A and C, run either
+    launch each (restir_*_views). The passes that trace shadow rays, A and C, run either
     through the multi-view entry points too (``rays="persistent"``, the default: queued view after
-    view with this renderer's own scratch, or, with ``launch.schedule`` = SCHEDULE_INLINE, one
-    persistent launch per pass with the rays traced per pixel) or view by view through each scene's
+    view with this renderer's own scratch, or one persistent launch per pass with the rays traced per
+    pixel, whichever is faster for the views; always the latter with ``launch.schedule`` =
+    SCHEDULE_INLINE) or view by view through each scene's
     context (``rays="queued"``). All give each view's output bit-identical to a Renderer of that view
     alone.
 

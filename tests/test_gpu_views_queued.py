@@ -98,7 +98,7 @@ def test_single_view_graph_survives_growth():
         for j in range(PASSES):
             ctx.unbiased(u, K, j, g, bufs[j % 2], bufs[1 - j % 2], None, stream)
 
-    p, large, larger = (_Passes(torch, [size]) for size in ((200, 120), (520, 400), (900, 700)))
+    p, large, larger = (_Passes(torch, [size]) for size in ((200, 120), (320, 200), (900, 700)))
     ctx = p.b.views[0]["ctx"]  # holds the room, the scene of all three
     single(ctx, p)  # eager: sizes the queues
     ref = p.out(torch)[0]
