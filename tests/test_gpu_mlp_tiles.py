@@ -80,3 +80,23 @@ def test_graph_keeps_its_scratch():
         assert results()[2].item() > 0
         graph.replay()
         assert all(torch.equal(a, c) for a, c in zip(results(), ref))
+
+
+@pytest.mark.parametrize("K,n", [(128, 8192), (384, 4096), (384, 8192), (640, 4096), (640, 16384), (1024, 320), (3968, 1088)])
+def test_groups_of_clusters_give_the_same_logits(K, n):
+    """A workgroup's share of the clusters depends on the batch: groups of one to all blocks of 128, the
+    last of them shorter. A sample's logits don't."""
+    import torch
+    ctx = abi.Context(0)
+    nW, nB = mlp_sizes(K)
+    z = lambda m, t=torch.float32: torch.zeros(m, dtype=t, device="cuda")  # noqa: E731
+    w_bf16, w, b, m, v = z(nW, torch.int16), z(nW), z(nB), z(nW + nB), z(nW + nB)
+    mlp = MlpStruct(K, 0, w_bf16.data_ptr(), w.data_ptr(), b.data_ptr(), m.data_ptr(), v.data_ptr())
+    ctx.mlp_init(mlp, 5, z(K) + torch.arange(K, device="cuda") * 0.25)
+    X = rand_features(torch, n, 1)[0]
+    got, piece = z(n * K).view(n, K) - 1, z(64 * K).view(64, K)
+    ctx.mlp_forward(mlp, X, n, got)
+    for i in range(0, n, 64 * (1 + n // 1024)):
+        ctx.mlp_forward(mlp, X[i:i + 64], 64, piece)
+        assert torch.equal(got[i:i + 64], piece), i
+    assert got.std() > 0.1 and not (got == -1).any()
