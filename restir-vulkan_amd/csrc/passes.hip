@@ -1054,10 +1054,10 @@ __device__ __forceinline__ uint32_t wave_sum_inclusive(uint32_t x) {
 // 17% and 5% slower; 6 waves per SIMD (80 VGPRs) spills and is 6% slower.
 constexpr uint32_t kTri8Ring = 128, kTri8Round = 48;  // a round starts at kTri8Round entries
 template <int MODE>
-__global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4 *__restrict__ p1,
-                                                const float4 *__restrict__ p2, const uint32_t *__restrict__ count,
-                                                uint32_t nBatch, uint32_t perWave, CQueues q,
-                                                uint32_t *__restrict__ out) {
+__global__ __launch_bounds__(256, kTrace8PerCu) void k_trace8(const SceneView sc, const float4 *__restrict__ p1,
+                                                              const float4 *__restrict__ p2,
+                                                              const uint32_t *__restrict__ count, uint32_t nBatch,
+                                                              uint32_t perWave, CQueues q, uint32_t *__restrict__ out) {
     constexpr bool PER_PIXEL = MODE == kTracePassA, BATCH = MODE == kTraceBatch;
     __shared__ uint32_t stack[rt::kW8Stack * 256];
     __shared__ uint32_t ringTri[4 * kTri8Ring];
@@ -1077,6 +1077,7 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
     uint32_t *tal = tally + (threadIdx.x & ~63u);
     tally[threadIdx.x] = 0u;  // each wave uses its own 64 words only
     rt::W8Seg w{};
+    constexpr uint32_t kFarRay = 0x80000000u, kOddRay = kFarRay + 0x100u;  // no group: masks of 0
     uint32_t grp = 0;    // the entries to visit: first child << 8 | mask; mask 0: nothing to walk
     int top = 0;         // entries of this lane's stack
     bool hit = false;
@@ -1147,14 +1148,22 @@ __global__ __launch_bounds__(256) void k_trace8(const SceneView sc, const float4
                             hit = false;
                             top = 0;
                             grp = 1u;  // node 0
-                            if (!rt::make_w8seg(w, o, d, sc.maxCoord, sc.invMax)) {
-                                hit = rt::occluded_slow(sc.nodes, sc.tris, sc.parent, o, d);
-                                grp = 0u;
-                            }
+                            const rt::W8Cover cover = rt::make_w8seg(w, o, d, sc.maxCoord, sc.invMax);
+                            if (cover != rt::W8Cover::near) grp = cover == rt::W8Cover::far ? kFarRay : kOddRay;
                         }
                     }
                 }
                 next = end - next < nIdle ? end : next + nIdle;
+                // the rays just taken that the visits below don't cover, out here where few masks are live
+                if (__ballot(grp >= kFarRay) != 0) {
+                    if (grp >= kFarRay) {
+                        hit = BATCH && grp == kFarRay
+                                  ? rt::occluded_far(w, sc.w8, sc.w8Tris, sc.nodes, sc.parent, sc.treeNested != 0,
+                                                     sc.treeTight != 0, stk, 256)
+                                  : rt::occluded_slow(sc.nodes, sc.tris, sc.parent, w.o, w.d);
+                        grp = 0u;
+                    }
+                }
             }
         }
         if (__ballot(ray >= 0) == 0) {

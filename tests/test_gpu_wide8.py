@@ -255,3 +255,32 @@ def test_wide8_enormous_boxes(torch, size, how):
     lo, hi = np.array([-1, -1e-3, -1]) * size * 0.5, np.array([1, 1e-3, 1]) * size * 0.5
     _check(torch, ctx, osc, *random_segments(rng, lo, hi, 20000), f"size {size}")
     del keep
+
+
+@pytest.mark.parametrize("name", ["cornell", "terrain_small"])
+def test_wide8_far_origins(torch, name):
+    """Origins from inside the reach of the grown boxes, over the far ones whose slab distances get a
+    slack per ray, to those that walk the binary tree; each mixed with near ones in its wave."""
+    sc = scenes.cornell_box(1) if name == "cornell" else scenes.terrain(5, grid=64, n_boxes=100, n_point_lights=10)
+    hs = HostScene(sc)
+    ctx = abi.Context(0)
+    keep = _bind(torch, ctx, hs.nodes, hs.tris)
+    lo, hi = sc.aabb()
+    big = max(np.abs(lo).max(), np.abs(hi).max())
+    rng = np.random.default_rng(25)
+    n = 80000
+    p1, p2 = random_segments(rng, lo, hi, n)
+    v = rng.normal(size=(n, 3))
+    v[::5] = np.eye(3)[rng.integers(3, size=len(v[::5]))] * rng.choice([-1, 1], size=(len(v[::5]), 1))  # axis-parallel
+    far = rng.uniform(size=n) < 0.9
+    dist = big * 2.0 ** rng.uniform(2, 27, size=n)
+    ends = p1[:, :3] + v / np.linalg.norm(v, axis=1, keepdims=True) * dist[:, None]
+    p1[far, :3] = ends[far].astype(np.float32)
+    # a segment may also start at the far end's light and lead past the scene
+    past = rng.uniform(size=n) < 0.3
+    p2[past, :3] += (p2[past, :3] - p1[past, :3]) * np.float32(0.5)
+    ref = _check(torch, ctx, hs.oracle, p1, p2, f"{name} far")
+    for k in range(4, 24, 4):
+        some = far & (dist > big * 2.0 ** k) & (dist < big * 2.0 ** (k + 4))
+        assert 0.05 < ref[some].mean() < 0.98, k
+    del keep
