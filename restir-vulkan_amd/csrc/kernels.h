@@ -96,7 +96,7 @@ int tile_index(uint32_t tx, uint32_t ty);  // -1 if not compiled
 constexpr uint32_t kTraceListEntries = 64 + 4 * 64;
 constexpr uint32_t kTraceExtraLds = 4u * kTraceListEntries * 5u + 256u * 4u;
 constexpr uint32_t kTrace8Lds = rt::kW8Stack * 1024u + 4u * 128u * 5u + 2u * 256u * 4u;  // the 8-entry tracer's workgroup
-constexpr uint32_t kTrace8PerCu = 5;  // its 92 VGPRs allow 5 waves per SIMD (its LDS 6 workgroups)
+constexpr uint32_t kTrace8PerCu = 5;  // its 92 to 94 VGPRs allow 5 waves per SIMD (its LDS 7 workgroups)
 // Columns of 64 bytes for k_light_records, and whether a queued Pass A over npx pixels with M
 // candidates each is worth building them
 size_t light_record_bytes(const SceneView &sc);

@@ -43,7 +43,7 @@ RT_HD f3 xyz(float4 v) { return f3{v.x, v.y, v.z}; }
 //   sqrt_near(x)    = RN(sqrt(x)): one residual step on the hardware's reciprocal square root
 //   over_pi(x)      = RN(x / kPi): as div_near, with 1 / kPi rounded at compile time
 // Compared on the MI355X with the IEEE forms for every b in [2^-60, 2^60], every x in [2^-100,
-// 2^100], and every one of the 2^46 pairs of mantissas of a and b: no difference. Scaling by powers of
+// 2^100], and every one of the 2^46 pairs of mantissas of a and b (probe/near_math.hip): no difference. Scaling by powers of
 // two changes no mantissa while nothing under- or overflows, which the bounds below keep away. With
 // them, and W formed once instead of per candidate, k_pass_a_ris (VALU bound: 0.82 of the issue
 // rate) went from 0.75 to 0.635 ms at 1080p, M = 32.
