@@ -45,17 +45,18 @@ for p in (ROOT, ROOT / "restir-vulkan_amd"):
 METRIC = "ms/frame @1080p to equal RMSE vs FP64 ref: learned vs plain RIS; Mrays/s"
 HBM_PEAK_GBS = 8000.0
 VALU_LANE_OPS = 39.3e12  # fp32 lane-ops/s (non-packed), the traversal's ALU ceiling
-# Traversal work per ray: V visits of 128-byte 4-entry nodes and T triangle tests of 48 bytes
-# each (V and T counted by the tracer on the same rays); ALU per visit: 4 box tests of
-# 16 lane-ops (6 FMA + 6 min/max + 4 compares) + 24 of walk control; 45 per triangle test.
-NODE_BYTES, TRI_BYTES = 128, 48
-VISIT_OPS, TEST_OPS = 4 * 16 + 24, 45
+# Traversal work per ray, whatever nodes the tracer walks: that of the reference's loop over the same
+# rays, V visits of its binary nodes (80 bytes) and T triangle tests (48 bytes each), counted by
+# restir_trace_shadow's reference loop; ALU per visit: the boxes of its two sides, 16 lane-ops each (6
+# FMA + 6 min/max + 4 compares); 45 per triangle test.
+NODE_BYTES, TRI_BYTES = 80, 48
+VISIT_OPS, TEST_OPS = 2 * 16, 45
 BYTES_PER_PX_SHADE = 124
 # compulsory bytes per pixel of the resampling passes (each buffer byte read or written once):
 # Pass A = current G 44 + previous G 36 + previous reservoir 64 + output 64; Pass C (without its
 # rays) = G 48 + reservoir in 64 + out 64
 BYTES_PER_PX_PASS_A, BYTES_PER_PX_PASS_C = 208, 176
-PASS_A_KERNELS = ("k_pass_a", "k_pass_a_ris", "k_pass_a_finish")
+PASS_A_KERNELS = ("k_pass_a", "k_light_records", "k_pass_a_ris", "k_pass_a_ris_split", "k_pass_a_finish")
 PASS_C_KERNELS = ("k_pack_surface", "k_pass_c_merge", "k_pass_c_finish", "k_pass_c")
 TRUTH_TRI_SAMPLES = 64  # stratified samples per triangle light in the FP64 ground truth
 # Error study: fixed views of the orbit (0.5 deg/frame), the same whatever --steps and --warmup
@@ -223,8 +224,7 @@ class Frames:
                 self.run(f, M, learned=learned, train=False)
             rows = ctx.profile_read()
             ctx.profile_enable(False)
-            table[name] = sum(rows[k][1] for k in ("k_pass_a", "k_pass_a_ris", "k_trace_queue(pass_a)",
-                                                   "k_pass_a_finish") if k in rows) / reps
+            table[name] = sum(rows[k][1] for k in (*PASS_A_KERNELS, "k_trace_queue(pass_a)") if k in rows) / reps
         best = min(table, key=table.get)
         self.launch_a = abi.Launch(self.launch.tile_x, self.launch.tile_y,
                                    abi.SCHEDULE_QUEUED if best == "queued" else abi.SCHEDULE_INLINE)
@@ -352,7 +352,7 @@ def main():
 
     # ---- the last timed frame again, untimed and bit-identical (same inputs and seeds; a frame
     # does not overwrite the previous frame's reservoirs it reads): export each Pass C's queued
-    # shadow rays and count node visits / triangle tests of exactly those rays
+    # shadow rays and count the reference loop's node visits / triangle tests of exactly those rays
     f_last = nframes - 1
     cap = npx * args.k
     q1 = torch.zeros(cap, 4, dtype=torch.float32, device=dev)
@@ -364,7 +364,7 @@ def main():
     for _j in fr.frame(f_last, args.M):
         for which, key in ((0, "centre"), (1, "neighbour")):
             n = ctx.unbiased_rays(which, q1, q2, cap, stream=stream)
-            ctx.trace_shadow(q1, q2, n, sh, visits, tests, stream=stream)
+            ctx.trace_shadow(q1, q2, n, sh, visits, tests, reference_loop=True, stream=stream)
             torch.cuda.synchronize()
             ray_sets[key].append({"rays": n, "V": float(visits[:n].double().mean()) if n else 0.0,
                                   "T": float(tests[:n].double().mean()) if n else 0.0,
@@ -386,7 +386,7 @@ def main():
     cpu_rays = (q1[:nr].cpu().numpy(), q2[:nr].cpu().numpy()) if not args.no_cpu_baseline else None
     rays_per_s = nr / (trace_ms * 1e-3)
     # Rays/s roofline: the lane-op model is the binding roof. The node and triangle fetches
-    # (128V + 48T bytes per ray) come from L1/L2 and the Infinity Cache: the HBM bytes the counters
+    # come from L1/L2 and the Infinity Cache: the HBM bytes the counters
     # measure per launch are a few percent of them, so the memory roof, priced at the measured
     # bytes per ray when the profile has them, is far above the ALU one.
     valu_rays = VALU_LANE_OPS / (VISIT_OPS * Vn + TEST_OPS * Tn)
@@ -423,8 +423,8 @@ def main():
     dom_ms = kernels[dominant]["avg_ms"]
     dom_traffic = measured_traffic(dominant) if W * H == 1920 * 1080 else None
     if dominant.startswith("k_trace_queue"):
-        # VALU-bound: algorithmic lane-ops per launch (88 per 4-entry visit, 45 per triangle
-        # test, V and T of this kernel's own rays) over the average launch time
+        # VALU-bound: algorithmic lane-ops per launch (32 per binary node and 45 per triangle test
+        # of the reference's loop over this kernel's own rays) over the average launch time
         key = dominant[len("k_trace_queue("):-1]
         ops = float(np.mean([r["rays"] * (VISIT_OPS * r["V"] + TEST_OPS * r["T"]) for r in ray_sets[key]]))
         rays = float(np.mean([r["rays"] for r in ray_sets[key]]))
@@ -440,9 +440,10 @@ def main():
                              "frac": round(dom_traffic / (dom_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                              "bytes": "rocprofv3 FETCH_SIZE + WRITE_SIZE per launch, copy-calibrated"}
                             if dom_traffic else None),
-                    "note": "model: 4 box tests of 16 lane-ops (6 FMA, 6 min/max, 4 compares) + 24 of "
-                            "walk control per 4-entry node visit, 45 per triangle test; node fetches "
-                            "are served by L1/L2, so the HBM roof does not bind"}
+                    "note": "work: that of the reference's loop over the same rays, 2 box tests of 16 "
+                            "lane-ops (6 FMA, 6 min/max, 4 compares) per binary node it visits, 45 per "
+                            "triangle test; the kernel walks 8-entry nodes (about 12 visits of 8 boxes a ray); "
+                            "node fetches are served by L1/L2, so the HBM roof does not bind"}
     else:
         ach = dom_bytes / (dom_ms * 1e-3) / 1e9 if dom_bytes else None
         roofline = {"kernel": dominant, "bound": "hbm", "achieved": round(ach, 1) if ach else None,
@@ -487,7 +488,8 @@ def main():
                   "kernels": rounded(kernels), "resampling_passes": resampling},
         "mrays_per_s": round(rays_per_s / 1e6, 1),
         "traversal": {"rays": nr, "ray_set": "last frame's second Pass C neighbour rays",
-                      "walk": "4-entry nodes (two tree levels per visit), persistent queue tracer, triangle tests gathered per wave",
+                      "walk": "8-entry nodes with 11-bit planes, persistent queue tracer, triangle tests gathered per wave, hits confirmed against the reference's boxes",
+                      "work": "the reference's loop over the same rays: binary node visits and triangle tests",
                       "node_bytes": NODE_BYTES, "ops_per_visit": VISIT_OPS, "ops_per_test": TEST_OPS,
                       "node_visits_per_ray": round(Vn, 2), "tri_tests_per_ray": round(Tn, 2),
                       "ms": round(trace_ms, 4), "roofline_mrays_per_s": round(roof_rays / 1e6, 1),
