@@ -1068,30 +1068,41 @@ __global__ __launch_bounds__(256) void k_wide_build(const rt::Node *__restrict__
 // chose, ordered and rounded its entries one after another, took the builds of 1,200, 136,000 and 2.3
 // million triangles 0.49, 1.25 and 6.62 ms, this 0.39, 1.08 and 6.40.
 constexpr int kW8Levels = rt::kW8Stack + 1;
+// Trees of at most this many nodes (1,120 triangles) take one launch: a launch a level took 300 triangles
+// 101 us to bind, 1,000 103, this 70 and 94; 1,200 triangles 104 and 106, 2,000 116 and 130.
+constexpr uint32_t kW8OneGroup = 640;
 struct W8Info {
     uint32_t nodes[kW8Levels + 1];  // nodes per level; [0] = 1
     uint32_t tris, overflow;
 };
 
+// kAll: all levels, `levels` at most, by one workgroup. Else level `level0` alone.
+template <bool kAll>
 __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict__ nodes,
-                                                     const float4 *__restrict__ tris, uint32_t level,
-                                                     uint32_t maxNodes, uint32_t maxTris,
+                                                     const float4 *__restrict__ tris, uint32_t level0,
+                                                     uint32_t levels, uint32_t maxNodes, uint32_t maxTris,
                                                      const uint32_t *__restrict__ bounds, rt::W8Node *__restrict__ out,
                                                      float4 *__restrict__ outTris, uint32_t *__restrict__ work,
                                                      W8Info *__restrict__ info) {
     __shared__ __align__(16) rt::W8Node made[64];
     __shared__ uint2 reserve[9];
+    __shared__ uint32_t below, spilled;  // kAll: nodes of the next level; whether a node found no room
     const uint32_t lane = threadIdx.x & 63u, k = lane & 7u;
     const int row = static_cast<int>(lane & 56u);
-    uint32_t begin = 0;
-    for (uint32_t l = 0; l < level; ++l) begin += info->nodes[l];
-    const uint32_t n = info->nodes[level], next = begin + n;
     const float maxCoord = __uint_as_float(bounds[1]);
     const double grow = static_cast<double>(rt::kW8Grow) * static_cast<double>(maxCoord);
     // a box is not finite, or too large or small: no 8-entry nodes. Areas are then finite: from about
     // 1.7e38 on a flat box's would be inf * 0, and no lane's NaN agrees with another's choice
     if (bounds[2] != 0 || !rt::w8_covers(maxCoord)) return;
-    if (info->overflow) return;  // of the levels before: not every node counted has its work entry
+    if (!kAll && info->overflow) return;  // of the levels before: not every node counted has its work entry
+    uint32_t begin = 0, n = 1;
+    if (!kAll) {
+        for (uint32_t l = 0; l < level0; ++l) begin += info->nodes[l];
+        n = info->nodes[level0];
+    }
+    for (uint32_t level = level0; n != 0; ++level) {
+    const uint32_t next = begin + n;
+    if (kAll && threadIdx.x == 0) below = spilled = 0;  // read before the last barrier
     for (uint32_t i0 = blockIdx.x * 64u; i0 < n; i0 += gridDim.x * 64u) {
         const uint32_t i = i0 + (threadIdx.x >> 3), me = begin + i;
         const bool on = i < n && me < maxNodes;  // the same for a node's 8 lanes
@@ -1182,6 +1193,7 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
                 sum.x += t.x;
                 sum.y += t.y;
             }
+            if (kAll) below += sum.x;
             if (sum.x) sum.x = atomicAdd(&info->nodes[level + 1], sum.x);
             if (sum.y) sum.y = atomicAdd(&info->tris, sum.y);
             reserve[8] = sum;
@@ -1192,6 +1204,7 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
         if (!on) continue;
         if (baseInt + nInt > maxNodes || baseTri + nTri > maxTris) {
             if (k == 0) atomicOr(&info->overflow, 1u);
+            if (kAll) spilled = 1;
             continue;
         }
         if (internal) work[baseInt + rank] = static_cast<uint32_t>(ref);
@@ -1257,6 +1270,12 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
             outTris[3 * to + 1] = make_float4(v1.x, v1.y, v1.z, __int_as_float(static_cast<int32_t>(t)));
             outTris[3 * to + 2] = make_float4(v2.x, v2.y, v2.z, 0.0f);
         }
+    }
+    if (!kAll) return;
+    __syncthreads();  // the level's work entries and its children's number are whole
+    begin = next;
+    n = level + 1 < levels && !spilled ? below : 0u;
+    __syncthreads();
     }
 }
 
@@ -1331,12 +1350,18 @@ int bind_tree(restir_ctx *ctx, const void *nodes, uint32_t nNodes, const void *t
     static_assert(sizeof host == 16 + sizeof(W8Info), "flags and counters are copied together");
     // Usually 8-entry levels are about a third as many: after the first launches the counters say
     // whether there are more (an empty launch takes 4 us, 13 of them in a tree of 23 levels).
+    // A small tree's are made by one workgroup in one launch.
     uint32_t done = 0;
+    if (w8Fits && maxW8 <= kW8OneGroup) {
+        RK_LAUNCH("k_w8_collapse", k_w8_collapse<true>, dim3(1), dim3(512), 0, s, bn, bt, 0u, levels, maxW8, nTris, p.flags,
+                  p.w8, p.tris, p.work, p.info);
+        done = levels;
+    }
     for (uint32_t batch = 4 + (32u - static_cast<uint32_t>(__builtin_clz(nTris))) / 3;; batch = 4) {
         const uint32_t end = !w8Fits ? 0u : (done + batch < levels ? done + batch : levels);
         for (; done < end; ++done)
-            RK_LAUNCH("k_w8_collapse", k_w8_collapse, dim3(1024), dim3(512), 0, s, bn, bt, done, maxW8, nTris, p.flags,
-                      p.w8, p.tris, p.work, p.info);
+            RK_LAUNCH("k_w8_collapse", k_w8_collapse<false>, dim3(1024), dim3(512), 0, s, bn, bt, done, 1u, maxW8, nTris,
+                      p.flags, p.w8, p.tris, p.work, p.info);
         if (int r = hip(hipMemcpyAsync(&host, p.flags, sizeof host, hipMemcpyDeviceToHost, s), "bind tree: read")) return r;
         if (int r = hip(hipStreamSynchronize(s), "bind tree: finish")) return r;
         if (!w8Fits || done == levels || host.w8.nodes[done] == 0) break;

@@ -26,9 +26,9 @@
 // loses below the normal range.
 //
 // Far origins. With |o| > 16 C the rounding of p - o and b - o outgrows s. Such a walk sets every
-// near distance back and every far one forward by e = 16 u |o| inv per axis (|o|: the largest
-// component): the distances differ by at most u (6 (|q 2^e| + |p - o|) + 2.01 |b - o|) / |d| <=
-// u (32.2 C + 8.01 |o|) / |d|, one rounding more than above included, less than (s + e) / |d|. All
+// near distance back and every far one forward by e = 9 u |o| inv, per axis: the distances differ by
+// at most u (6 (|q 2^e| + |p - o|) + 2.01 |b - o|) / |d| <= u (32.2 C + 8.01 |o|) / |d|, one rounding
+// more than above included, less than (s + e) / |d|. All
 // distances stay finite up to |o| = 2^24 C (2^24 C K < 2^125), where C is an ulp of o. A batch's tracer
 // walks these segments as it takes them (occluded_far): 300,000 from 100 times the scene's size take 0.11
 // ms, through the binary tree 0.40. Its own visits have no slack: 4 million segments took 0.78
@@ -47,7 +47,7 @@ constexpr int kW8Stack = 16;  // entries of a lane's stack: trees of at most 17 
 constexpr float kW8Grow = 192.0f * 5.9604645e-8f;  // s / C
 constexpr float kW8Reach = 16.0f;                  // |o| / C at most, without the slack of far origins
 constexpr float kW8Far = 0x1p24f;                  // and with it
-constexpr float kW8FarSlack = 0x1p-20f;            // 16 u
+constexpr float kW8FarSlack = 9.0f * 5.9604645e-8f;
 // Trees whose largest |box coordinate| C keeps every product of the walk finite and its slack normal
 __host__ __device__ inline bool w8_covers(float c) { return c > 1e-18f && c < 1e18f; }
 constexpr float kW8Long = 0x1p96f, kW8Longest = 0x1p99f;  // |d| / C and |d| at most
@@ -127,8 +127,8 @@ __device__ __forceinline__ W8Visit w8_visit(const W8Seg &w, const W8Node *__rest
     const float bx = (h0.x - w.o.x) * w.inv.x, by = (h0.y - w.o.y) * w.inv.y, bz = (h0.z - w.o.z) * w.inv.z;
     f3 nb{bx, by, bz}, fb = nb;
     if (kFar) {
-        const float e = kW8FarSlack * fmaxf(fmaxf(fabsf(w.o.x), fabsf(w.o.y)), fabsf(w.o.z));
-        const f3 slack{e * fabsf(w.inv.x), e * fabsf(w.inv.y), e * fabsf(w.inv.z)};
+        const f3 slack{kW8FarSlack * fabsf(w.o.x * w.inv.x), kW8FarSlack * fabsf(w.o.y * w.inv.y),
+                       kW8FarSlack * fabsf(w.o.z * w.inv.z)};
         nb = nb - slack;
         fb = fb + slack;
     }

@@ -284,3 +284,27 @@ def test_wide8_far_origins(torch, name):
         some = far & (dist > big * 2.0 ** k) & (dist < big * 2.0 ** (k + 4))
         assert 0.05 < ref[some].mean() < 0.98, k
     del keep
+
+
+@pytest.mark.parametrize("n_tris", [1119, 1120, 1121, 3000])
+def test_wide8_one_workgroup_or_many(torch, n_tris):
+    """Up to 640 possible nodes the collapse is one workgroup's; both sides of that, host and device build."""
+    rng = np.random.default_rng(n_tris)
+    xyz = (rng.uniform(-1, 1, size=(n_tris, 1, 3)) + rng.uniform(-0.1, 0.1, size=(n_tris, 3, 3))).astype(np.float32)
+    nodes, tris, _ = abi.build_aabb_tree(xyz.reshape(-1, 9))
+    osc = oracle.Scene(nodes, tris, None, None, None)
+    lo, hi = np.full(3, -1.1, np.float32), np.full(3, 1.1, np.float32)
+    for how in ("host", "device"):
+        ctx = abi.Context(0)
+        for _ in range(2):  # again over the buffers of the first
+            if how == "host":
+                keep = _bind(torch, ctx, nodes, tris)
+            else:
+                keep = (torch.from_numpy(xyz).cuda(), torch.zeros(nodes.nbytes, dtype=torch.uint8, device="cuda"),
+                        torch.zeros(tris.nbytes, dtype=torch.uint8, device="cuda"))
+                ctx.build_bvh(keep[0], n_tris, keep[1], keep[2])
+        ctx.profile_enable(True)
+        ref = _check(torch, ctx, osc, *random_segments(rng, lo, hi, 20000), f"{n_tris} triangles, {how}")
+        assert "k_zero_counters" not in ctx.profile_read(), "the 8-entry nodes do not cover the tree"
+        assert 0.02 < ref.mean() < 0.98
+        del keep
