@@ -13,13 +13,7 @@
 #include "scan.h"
 
 #define AK_FN __device__ __forceinline__
-// LDS and memory accesses of one wave take effect in order; the barrier keeps the compiler's order
-#define AK_WAVE_SYNC(g)                                        \
-    do {                                                       \
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); \
-        __builtin_amdgcn_wave_barrier();                       \
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); \
-    } while (0)
+#define AK_WAVE_SYNC(g) rk::wave_sync()
 #include "alias_kernel.h"
 
 using namespace rki;

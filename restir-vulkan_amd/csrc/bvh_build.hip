@@ -19,7 +19,7 @@
 // Where the time goes: a level costs its launches (about 5 us each) and its readback, whatever its
 // size, and the lower half of a tree's levels holds ranges of a few primitives. 136,000 triangles
 // (23 levels): 3.2 ms with every level split that way, in 20 launches each; 1.15 ms with the last 12
-// to 13 levels in k_bvh_subtrees (0.22 ms) and 8 launches for each of the others, 1.05 with the 8-entry
+// to 13 levels in k_bvh_subtrees (0.22 ms) and 8 launches for each of the others, 1.06 with the 8-entry
 // nodes' collapse on 8 lanes a node. 1,200 triangles 1.52 -> 0.39 ms, 2.3 million 18.6 -> 6.4 ms (all
 // with the traversal's nodes, bind_tree).
 //
@@ -638,12 +638,6 @@ struct SubQueue {
 };
 // a node's four boxes as 16 words
 __device__ inline float *box_words(restir_aabb_tree_node &node) { return reinterpret_cast<float *>(&node); }
-// LDS accesses of a wave's lanes happen in program order; this keeps the compiler to it
-__device__ inline void row_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 __global__ __launch_bounds__(256) void k_bvh_subtrees(const Sub *subs, const uint32_t *idx, const float4 *box,
                                                       restir_aabb_tree_node *tmp, uint8_t *levels, Info *info) {
     __shared__ float bx[kSub * 6];
@@ -757,7 +751,7 @@ __global__ __launch_bounds__(256) void k_bvh_subtrees(const Sub *subs, const uin
             if (wide) {  // keys as in k_bvh_bin
                 u64 *a = bins[threadIdx.x >> 4];
                 for (uint32_t w = L; w < kBuckets * kBinWords; w += 16u) a[w] = word_init(kBoundWords + static_cast<int>(w));
-                row_sync();
+                rk::wave_sync();
                 for (uint32_t p = f + L; p < l; p += 16u) {
                     const float *e = bx + 6u * ord[p];
                     const uint32_t b = bucket_of(q, 0.5f * (e[q.axis] + e[q.axis + 3]));
@@ -770,7 +764,7 @@ __global__ __launch_bounds__(256) void k_bvh_subtrees(const Sub *subs, const uin
                     }
                     atomicAdd(&w[6], 1ull);
                 }
-                row_sync();
+                rk::wave_sync();
                 if (L < kBuckets) left.count = static_cast<uint32_t>(a[L * kBinWords + 6]);
                 if (left.count != 0)
 #pragma unroll
@@ -785,7 +779,7 @@ __global__ __launch_bounds__(256) void k_bvh_subtrees(const Sub *subs, const uin
                     const uint32_t o = 6u * ord[p] + static_cast<uint32_t>(q.axis);
                     bucket[p] = static_cast<uint8_t>(bucket_of(q, 0.5f * (bx[o] + bx[o + 3])));
                 }
-                row_sync();
+                rk::wave_sync();
                 // a lane per bucket
                 for (uint32_t p = f; p < l; p += 4u) {
                     float x[4][6];
@@ -851,10 +845,10 @@ __global__ __launch_bounds__(256) void k_bvh_subtrees(const Sub *subs, const uin
                         at = g < p ? g : p;
                     }
                     if (in) ptr[p] = static_cast<uint16_t>(at);
-                    row_sync();
+                    rk::wave_sync();
                     if (in)
                         for (uint32_t to = ptr[at]; to != at; to = ptr[at]) at = to;
-                    row_sync();
+                    rk::wave_sync();
                     if (in) {
                         ptr[p] = static_cast<uint16_t>(at);
                         if (p >= mid) out[p] = ord[at];
@@ -862,7 +856,7 @@ __global__ __launch_bounds__(256) void k_bvh_subtrees(const Sub *subs, const uin
                     run += static_cast<uint32_t>(__popc(m));
                 }
             }
-            row_sync();
+            rk::wave_sync();
             if (L == 0) {
                 node._pad[0] = node._pad[1] = 0;
                 levels[t] = static_cast<uint8_t>(level);
@@ -1066,7 +1060,7 @@ __global__ __launch_bounds__(256) void k_wide_build(const rt::Node *__restrict__
 // the tracer 0-1%, 5% and 12% slower (more triangle tests than boxes saved). Latency bound (a node's
 // expansions wait for one node after another): a lane per node, which
 // chose, ordered and rounded its entries one after another, took the builds of 1,200, 136,000 and 2.3
-// million triangles 0.49, 1.25 and 6.62 ms, this 0.39, 1.08 and 6.40.
+// million triangles 0.49, 1.25 and 6.62 ms, this 0.39, 1.06 and 6.40.
 constexpr int kW8Levels = rt::kW8Stack + 1;
 // Trees of at most this many nodes (1,120 triangles) take one launch: a launch a level took 300 triangles
 // 101 us to bind, 1,000 103, this 70 and 94; 1,200 triangles 104 and 106, 2,000 116 and 130.
@@ -1258,11 +1252,11 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
             w.axis = axis;
             w.pad = 0;
         }
-        row_sync();
+        rk::wave_sync();
         // the node by way of LDS: 16 bytes a lane
         static_assert(sizeof(rt::W8Node) == 128, "8 lanes store a node");
         reinterpret_cast<float4 *>(out + me)[k] = reinterpret_cast<const float4 *>(&w)[k];
-        row_sync();
+        rk::wave_sync();
         if (leaf) {
             const size_t t = static_cast<size_t>(~ref), to = baseTri + rank - nInt;
             const float4 v0 = tris[3 * t], v1 = tris[3 * t + 1], v2 = tris[3 * t + 2];

@@ -11,6 +11,15 @@
 
 namespace rk {
 
+// What the wave's lanes stored before it, its other lanes read after it: a wave's accesses of LDS (and
+// of memory, by way of its own L1) take effect in order, and the barrier (no instruction) keeps the compiler
+// from reordering them.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- optional per-kernel timing (restir_profile_enable). Every launch goes through RK_LAUNCH,
 // which hands the kernel a start/stop event pair when the calling thread has a recorder bound;
 // the events bracket exactly that kernel on its stream (hipExtLaunchKernel).

@@ -664,15 +664,15 @@ __device__ __forceinline__ uint2 wave_rank(bool emit) {
     return make_uint2(lanes_below(m), static_cast<uint32_t>(__popcll(m)));
 }
 
-// Position and normal of every pixel in one 32-byte record: the merge's horizon test and the
-// neighbour-ray emission gather them for random neighbours, one sector per neighbour instead of
-// one line per plane.
 // A queued pass's work counters, cleared by the first workgroup of a kernel ahead of their first use
 __device__ __forceinline__ void clear_counters(uint32_t *counter, uint32_t *heads) {
     if (blockIdx.x != 0) return;
     if (threadIdx.x < 2) counter[threadIdx.x] = 0u;
     if (threadIdx.x < kTraceShards) heads[threadIdx.x * kTraceShardStride] = 0u;
 }
+// Position and normal of every pixel in one 32-byte record: the merge's horizon test and the
+// neighbour-ray emission gather them for random neighbours, one sector per neighbour instead of
+// one line per plane.
 __global__ __launch_bounds__(256) void k_pack_surface(const GView g, uint32_t npx, float4 *surf, uint32_t *counter,
                                                       uint32_t *heads) {
     clear_counters(counter, heads);
@@ -1009,14 +1009,6 @@ __global__ __launch_bounds__(256) void k_trace_queue(const SceneView sc, const f
             ray = -1;
         }
     }
-}
-
-// What the wave's lanes stored to LDS before it, its other lanes read after it: a wave's LDS accesses
-// take effect in order, and the barrier (no instruction) keeps the compiler from reordering them.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Inclusive sum over the wave's lanes (all active).
@@ -1805,7 +1797,8 @@ __global__ __launch_bounds__(256) void k_primary(const PrimaryArgs a) {
 // when the walk comes back, in the order of their centres on the node's axis from the side the ray
 // comes from (bit 31 of a stack word: from the last slot down): in storage order the 2.3 M-triangle
 // 4K frame takes 20 ms, by the axis alone 5.0, so 4.4 (the binary walk, whose slabs are IEEE
-// divisions: 7.7); 1080p 0.70 -> 0.35 ms. VALU bound: about 200 instructions a visit.
+// divisions: 7.7); 1080p 0.70 -> 0.35 ms. A lane waits for its one node in flight about as long as it
+// computes (VALU 0.51 to 0.54 busy, about 200 instructions a visit), and a wave for its longest ray.
 __global__ __launch_bounds__(256) void k_primary8(const PrimaryArgs a, uint32_t tilesX, uint32_t nTiles) {
     __shared__ uint32_t stack[rt::kW8Stack * 256];
     uint32_t *stk = stack + threadIdx.x;
