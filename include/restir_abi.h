@@ -198,7 +198,7 @@ void restir_destroy(restir_ctx *ctx);
 const char *restir_last_error(const restir_ctx *ctx);
 /* ABI revision; bumped whenever an entry point's signature or documented behaviour changes. Bindings compare it with the
  * revision they were written against and refuse a mismatched library. */
-#define RESTIR_ABI_VERSION 17
+#define RESTIR_ABI_VERSION 18
 int restir_version(void);
 
 /* Light tables: device pointers to the reference buffer images (header + array). The counts are
@@ -216,7 +216,10 @@ int restir_set_lights(restir_ctx *ctx, const void *point_lights, size_t point_by
                       size_t alias_bytes);
 
 /* BVH: device pointers in the AabbTreeBuffers layout (aabbTreeBuilder.h:25-51). The tree is
- * read back once to validate child indices and to measure its depth. */
+ * read back once to validate child indices and to measure its depth. The context builds the nodes
+ * that its rays walk from the tree: 128 bytes per triangle, and where the device has them another
+ * 127 (for at most 2^23 8-entry nodes and 2^26 triangles); without, rays walk the former alone,
+ * with the same results. Rebind after changing the buffers' contents. */
 int restir_set_bvh(restir_ctx *ctx, const restir_aabb_tree_node *nodes, uint32_t n_nodes,
                    const restir_triangle *tris, uint32_t n_tris);
 
@@ -226,8 +229,8 @@ int restir_set_bvh(restir_ctx *ctx, const restir_aabb_tree_node *nodes, uint32_t
  * device buffers nodes[n_tris - 1] and tris[n_tris] and bound to ctx as restir_set_bvh binds them
  * (the build's own bookkeeping replaces set_bvh's read-back check). depth_out (host, may be NULL)
  * gets the tree depth. The build waits for the stream once per tree level (it reads each level's
- * node count back), so it cannot be captured into a graph. Context scratch: about 380 bytes per
- * triangle. A non-finite coordinate gives RESTIR_E_INVALID_ARGUMENT. */
+ * node count back), so it cannot be captured into a graph. Context scratch: about 230 bytes per
+ * triangle, besides the nodes that restir_set_bvh names. A non-finite coordinate gives RESTIR_E_INVALID_ARGUMENT. */
 int restir_build_bvh(restir_ctx *ctx, const float *tri_xyz, uint32_t n_tris,
                      restir_aabb_tree_node *nodes, restir_triangle *tris, uint32_t *depth_out,
                      void *stream);
@@ -401,7 +404,8 @@ int restir_mlp_init(restir_ctx *ctx, restir_mlp *mlp, uint64_t seed, const float
  * device table of 32 bytes per light (each cluster slot's light, p_within and p_src, for its
  * column and its alias); the caller's buffers must stay alive while the context uses them. For
  * k > 256 (a multiple of 128) the context also allocates the proposal's working memory, at most
- * 544 * k bytes per compute unit (570 MB at k = 4,096), less where that cannot be had.
+ * 544 * k bytes per compute unit (570 MB at k = 4,096), less where that cannot be had (the proposal
+ * is then slower); the call fails with RESTIR_E_HIP where the device cannot give 16 * 272 * k bytes.
  * Call it after restir_set_lights: the slot table snapshots the bound alias table, and binding
  * new lights unbinds the clusters. */
 int restir_set_light_clusters(restir_ctx *ctx, uint32_t k, const int32_t *light_cluster,

@@ -24,7 +24,7 @@ SHADE_VISIBILITY_FLAG = 1  # RESTIR_SHADE_VISIBILITY_FLAG: final shading re-test
 TRACE_FIRST_HIT = 0
 TRACE_REFERENCE_LOOP = 1
 TRACE_ONE_RAY_PER_LANE = 2
-ABI_VERSION = 17  # RESTIR_ABI_VERSION of include/restir_abi.h
+ABI_VERSION = 18  # RESTIR_ABI_VERSION of include/restir_abi.h
 
 ERRORS = {
     -1: "RESTIR_E_INVALID_ARGUMENT",
