@@ -1150,8 +1150,7 @@ __global__ __launch_bounds__(256, kTrace8PerCu) void k_trace8(const SceneView sc
                 if (__ballot(grp >= kFarRay) != 0) {
                     if (grp >= kFarRay) {
                         hit = BATCH && grp == kFarRay
-                                  ? rt::occluded_far(w, sc.w8, sc.w8Tris, sc.nodes, sc.parent, sc.treeNested != 0,
-                                                     sc.treeTight != 0, stk, 256)
+                                  ? rt::occluded_far(w, sc.w8, sc.w8Tris, sc.nodes, sc.parent, sc.treeNested != 0, stk, 256)
                                   : rt::occluded_slow(sc.nodes, sc.tris, sc.parent, w.o, w.d);
                         grp = 0u;
                     }
@@ -1167,7 +1166,7 @@ __global__ __launch_bounds__(256, kTrace8PerCu) void k_trace8(const SceneView sc
         if (grp & 0xffu) {
             const uint32_t node = (grp >> 8) + static_cast<uint32_t>(__builtin_ctz(grp));
             grp &= grp - 1u;
-            const rt::W8Visit v = rt::w8_visit<false>(w, sc.w8, node, 1.0f);
+            const rt::W8Visit v = rt::w8_visit<false, false, BATCH ? 0 : 1>(w, sc.w8, node, 1.0f);
             pend = v.tris;
             triBase = v.triBase;
             const bool more = (grp & 0xffu) != 0;

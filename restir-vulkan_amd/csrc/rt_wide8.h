@@ -98,7 +98,8 @@ struct W8Visit {
 };
 // Visits `node` on [0, tMax]. 12 VALU per box: 6 FMA with half operands, max3, min3, the clamp to
 // the segment, a subtraction whose sign is shifted into the mask. kFar: with the slack of far origins.
-template <bool kOrder, bool kFar = false>
+// kPass: what may be scheduled across the end of the loads (sched_barrier's mask; 0 or 1, as measured).
+template <bool kOrder, bool kFar = false, int kPass = 0>
 __device__ __forceinline__ W8Visit w8_visit(const W8Seg &w, const W8Node *__restrict__ nodes, uint32_t node,
                                             float tMax) {
     const char *base = reinterpret_cast<const char *>(nodes);
@@ -120,7 +121,7 @@ __device__ __forceinline__ W8Visit w8_visit(const W8Seg &w, const W8Node *__rest
     const h8 fz = *reinterpret_cast<const h8 *>(base + (row + (w.oz ^ 16u)) + 96);
     // the eight loads under way together: left to itself the compiler may wait for one after another (4
     // million segments 0.88 ms instead of 0.74, depending on the code around)
-    __builtin_amdgcn_sched_barrier(1);
+    __builtin_amdgcn_sched_barrier(kPass);
     const int32_t e = static_cast<int32_t>(h1.x);
     const float sx = ldexpf(w.inv.x, (e << 24) >> 24), sy = ldexpf(w.inv.y, (e << 16) >> 24),
                 sz = ldexpf(w.inv.z, (e << 8) >> 24);
@@ -238,7 +239,7 @@ __device__ __forceinline__ bool w8_confirm(const Node *__restrict__ nodes, const
 // entries, `stride` apart.
 __device__ __forceinline__ bool occluded_far(const W8Seg &w, const W8Node *__restrict__ w8, const float4 *__restrict__ w8Tris,
                                              const Node *__restrict__ nodes, const uint32_t *__restrict__ parent,
-                                             bool treeNested, bool tight, uint32_t *stk, int stride) {
+                                             bool treeNested, uint32_t *stk, int stride) {
     uint32_t grp = 1u;  // as in the tracer: first child << 8 | mask of the entries to visit
     int top = 0;
     for (;;) {
@@ -253,7 +254,10 @@ __device__ __forceinline__ bool occluded_far(const W8Seg &w, const W8Node *__res
         for (uint32_t m = v.tris; m; m &= m - 1u) {
             const float4 *t = w8Tris + 3 * static_cast<size_t>(v.triBase + static_cast<uint32_t>(__builtin_ctz(m)));
             const float4 a = t[0], b = t[1], c = t[2];
-            if (tri_hit(a, b, c, w.o, w.d) && w8_confirm<true>(nodes, parent, treeNested, tight, a, b, c, w.o, w.d)) return true;
+            // w8_confirm without its quick form, whose registers the tracer would have to find
+            if (tri_hit(a, b, c, w.o, w.d) &&
+                path_passes<true>(nodes, parent, __float_as_uint(a.w), w.o, w.d, treeNested && regular_segment(w.o, w.d)))
+                return true;
         }
         if (v.child & 0xffu) {
             if (grp & 0xffu) {
