@@ -1087,8 +1087,9 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
     const double grow = static_cast<double>(rt::kW8Grow) * static_cast<double>(maxCoord);
     // a box is not finite, or too large or small: no 8-entry nodes. Areas are then finite: from about
     // 1.7e38 on a flat box's would be inf * 0, and no lane's NaN agrees with another's choice
-    if (bounds[2] != 0 || !rt::w8_covers(maxCoord)) return;
-    if (!kAll && info->overflow) return;  // of the levels before: not every node counted has its work entry
+    // (nor below a level that found no room: not every node counted has its work entry). One wait for the three
+    const uint32_t spilledAbove = kAll ? 0u : info->overflow;
+    if ((bounds[2] | spilledAbove) != 0 || !rt::w8_covers(maxCoord)) return;
     uint32_t begin = 0, n = 1;
     if (!kAll) {
         for (uint32_t l = 0; l < level0; ++l) begin += info->nodes[l];
