@@ -1085,9 +1085,10 @@ __global__ __launch_bounds__(512) void k_w8_collapse(const rt::Node *__restrict_
     const int row = static_cast<int>(lane & 56u);
     const float maxCoord = __uint_as_float(bounds[1]);
     const double grow = static_cast<double>(rt::kW8Grow) * static_cast<double>(maxCoord);
-    // a box is not finite, or too large or small: no 8-entry nodes. Areas are then finite: from about
-    // 1.7e38 on a flat box's would be inf * 0, and no lane's NaN agrees with another's choice
-    // (nor below a level that found no room: not every node counted has its work entry). One wait for the three
+    // A box is not finite, or too large or small: no 8-entry nodes. Areas are finite in this range; from about
+    // 1.7e38 on a flat box's would be inf * 0, and no lane's NaN agrees with another's choice. Nor is there
+    // anything to do below a level that found no room: not every node counted there has its work entry. The
+    // three words are read together, one wait for all.
     const uint32_t spilledAbove = kAll ? 0u : info->overflow;
     if ((bounds[2] | spilledAbove) != 0 || !rt::w8_covers(maxCoord)) return;
     uint32_t begin = 0, n = 1;
